@@ -42,15 +42,15 @@ def listed():
     qwen, deginex, roserax = "qwen3_4b", "deginex_4b_moe", "roserax_4b"
     return [
         # one user waits for the next word: every weight is read for one token, launches count
-        _decode("decode, one request", qwen, 1, 2049, 2049, 4),
+        _decode("decode 1", qwen, 1, 2049, 2049, 4),
         # the repository's headline: a batch of eight behind 2,048-token prompts
-        _decode("decode, 8 requests", qwen, 8, 2049, 2049, 8),
+        _decode("decode 8", qwen, 8, 2049, 2049, 8),
         # a busy server: contexts of very unequal lengths
-        _decode("decode, 48 ragged", qwen, 48, 131, 2601, 4),
+        _decode("decode 48 ragged", qwen, 48, 131, 2601, 4),
         # time to the first token of an ordinary prompt
-        _read("read 2,048 tokens", qwen, 1, 2048, 2048, 2048),
+        _read("read 2048", qwen, 1, 2048, 2048, 2048),
         # a long document, read in portions over a growing history; its length divides by nothing
-        _read("read 8,191 in portions", qwen, 1, 8191, 8191, 2048),
+        _read("read 8191 in portions", qwen, 1, 8191, 8191, 2048),
         # continuous batching: portions of prompts beside decoding requests
         {"name": "continuous batching", "kind": "mix", "model": qwen, "dtype": "bfloat16", "requests": 10,
          "shortest": 77, "longest": 1501, "steps": 12, "budget": 512},
@@ -58,14 +58,14 @@ def listed():
         {"name": "score 6 short requests", "kind": "score", "model": qwen, "dtype": "bfloat16", "requests": 6,
          "shortest": 19, "longest": 307, "steps": 16, "budget": 2048},
         # the true 32-bit mode, short prompts and a few tokens: what checks of numerics run
-        {"name": "float32, 2 requests", "kind": "mix", "model": qwen, "dtype": "float32", "requests": 2,
+        {"name": "float32 2 requests", "kind": "mix", "model": qwen, "dtype": "float32", "requests": 2,
          "shortest": 93, "longest": 261, "steps": 6, "budget": 512},
         # routed experts over several residual streams
-        _read("experts: read 3 prompts", deginex, 3, 301, 1151, 2048),
-        _decode("experts: decode, 8 requests", deginex, 8, 1025, 1025, 8),
+        _read("experts read 3 prompts", deginex, 3, 301, 1151, 2048),
+        _decode("experts decode 8", deginex, 8, 1025, 1025, 8),
         # latent attention, retention, windows and experts
-        _read("latent: read 2,047 tokens", roserax, 1, 2047, 2047, 2048),
-        _decode("latent: decode, 8 requests", roserax, 8, 1025, 1025, 8),
+        _read("latent read 2047", roserax, 1, 2047, 2047, 2048),
+        _decode("latent decode 8", roserax, 8, 1025, 1025, 8),
     ]
 
 
