@@ -1,0 +1,63 @@
+"""The float32 kernels at the edges of their tiles: products against float64 within the bound of a
+float32 sum, equal bits however many rows share a launch; attention by tiles against the plain one."""
+
+import math
+
+import pytest
+import torch
+
+from plain import ops_ref as R
+from test_kernels_gpu import DEV, build_attention_case, close, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    return HipOps()
+
+
+# K: less than a chunk of 16, no multiple of 16, the ends of the 4-, 8- and 16-part ranges; N and M: around 16, 64, 128
+@pytest.mark.parametrize("n,k", [(1, 4), (17, 20), (64, 252), (65, 260), (130, 1028), (48, 8188), (33, 8192), (15, 10004)])
+def test_product_against_float64_and_equal_bits_for_any_number_of_rows(ops, n, k):
+    x, w = rnd(200, k, seed=1), rnd(n, k, seed=2, scale=0.05)
+    whole = ops.linear(x, w)
+    want = x.double() @ w.double().T
+    # a sum of k products in any order, each rounded: at most k units of 2^-24 of the sum of magnitudes
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((whole.double() - want).abs() <= bound).all()
+    for m in (1, 16, 17, 32, 33, 64, 65, 129):
+        assert torch.equal(ops.linear(x[70: 70 + m].contiguous(), w), whole[70: 70 + m]), m
+
+
+def test_product_of_many_rows_in_large_tiles(ops):
+    x, w = rnd(4100, 36, seed=3), rnd(4097, 36, seed=4)   # 33 x 33 tiles of 128, the last of one row and one column
+    whole = ops.linear(x, w)
+    bound = 36 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((whole.double() - x.double() @ w.double().T).abs() <= bound).all()
+    assert torch.equal(ops.linear(x[4099:].contiguous(), w), whole[4099:])
+
+
+@pytest.mark.parametrize("seqs,nq,nkv,d,dv,ps,more", [
+    ([(1, 16), (1, 17), (1, 130)], 4, 2, 128, 128, 16, {}),                       # decoding: eight waves share the keys
+    ([(20, 33), (7, 7), (1, 1)], 5, 1, 48, 48, 4, {}),                            # a tile's 16 rows cut a token's heads
+    ([(300, 300), (160, 190)], 8, 8, 32, 16, 24, {}),                             # many tiles: four waves; values of another size
+    ([(40, 90)], 4, 2, 256, 256, 8, {"window": 9, "keep_first": 5, "sink": True}),
+    ([(1, 99), (33, 99)], 6, 2, 64, 80, 16, {"window": 40, "softcap": 5.0}),
+    ([(50, 75)], 4, 4, 16, 32, 12, {"chunk": 24, "gate": True}),
+])
+def test_attention_by_tiles(ops, seqs, nq, nkv, d, dv, ps, more):
+    more = dict(more)
+    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, ps, torch.float32, window=more.get("window"), poison=True)
+    if dv != d:
+        cache.v = rnd(cache.v.shape[0], nkv, dv, ps, seed=7)
+    if more.pop("gate", False):
+        more["gate"] = rnd(ctx.num_tokens, nq * dv, seed=9)
+    window, scale = more.pop("window", None), 1.0 / math.sqrt(d)
+    want = R.paged_attention(q.double(), cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, ps,
+                             nq, nkv, d, scale, window, torch.float64, value_dim=dv, **more)
+    got = ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window, value_dim=dv, **more)
+    # scores of size 3 * sqrt(d) * scale and values of size 3: sums of up to 300 float32 terms
+    close(got, want.float(), 2e-5, 2e-5)
