@@ -1,6 +1,7 @@
-// Paged attention in true 32-bit, any head size: the check path.
+// Paged attention in true 32-bit: a kernel by tiles (below) for the usual sizes in float32, and one for
+// any head size and either type.
 //
-// One wave per (query token, query head). The wave walks the keys its query may
+// The latter: one wave per (query token, query head). The wave walks the keys its query may
 // see in chunks of 64 (one key per lane for the scores), keeps a running
 // maximum and sum (online softmax, float32), and accumulates the context with
 // each lane owning head elements lane, lane + 64, ... Query head h reads key
@@ -34,6 +35,8 @@ struct AttnArgs {
   int keep_first;  // with a window: keys j < keep_first are seen too
   int sink;        // 1: one more term exp(0) in the denominator
   const float* turn;  // [T, Dv] or null: cosines of the token's Dv / 2 angles, then their sines; the output is turned back by them
+  const int* cu_q;    // [S + 1] or null: first token of every sequence (the tile kernel goes by it)
+  int num_seqs, max_q_len;  // sequences, and the most tokens one brings
 };
 
 #define MAX_D 1024
@@ -134,6 +137,170 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
   }
 }
 
+// ---------------------------------------------------------------- float32 by tiles
+// A block takes 16 rows (token * g + head in group) of one sequence and key head, its W waves the
+// sequence's blocks of 16 keys in turn, each with a maximum, a sum and an accumulator of its own, which
+// meet in LDS at the end. Scores are formed transposed, S^T = K Q^T, on the float32 MFMA (whole float32
+// products and sums): a lane then holds four neighbouring keys of its row, exactly the operand that
+// O^T = V^T P^T takes against one 16-byte read of the transposed value page, so nothing crosses lanes but
+// the row's maximum. The kernel before it (a wave per token and head, a key's dot product per lane,
+// uncoalesced) is bound by load latency: 354 tokens of 2 sequences with 32 heads of 128 took 798 us, two
+// decoded tokens behind 267 keys 170 us; this one 43 and 25 us.
+// Head sizes in multiples of 16 up to 256, pages of a multiple of 4 keys; other sizes keep the kernel above.
+template <int ND, int W>
+__global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) {
+  __shared__ __align__(16) f32x4_t hand[W > 1 ? W / 2 : 1][ND * 64];  // accumulators on their way from wave to wave
+  __shared__ float hand_m[W][16], hand_l[W][16];
+  const int lane = threadIdx.x & 63, wave = uniform_wave_number();
+  const int r = lane & 15, q = lane >> 4;
+  const int s = blockIdx.z, kvh = blockIdx.y, g = a.nq / a.nkv;
+  const int t0 = a.cu_q[s], rows = (a.cu_q[s + 1] - t0) * g, row0 = blockIdx.x * 16;
+  if (row0 >= rows) return;  // the whole block alike
+  const int D = a.head_dim, Dv = a.value_dim, ps = a.page_size, nd = D >> 4, nv = Dv >> 4;
+  const int last_row = min(row0 + 15, rows - 1), rr = min(row0 + r, last_row);
+  const int t = t0 + rr / g, h = kvh * g + rr % g;
+  const int pos = a.positions[t], hi = a.positions[t0 + last_row / g], pos0 = a.positions[t0 + row0 / g];
+  const int* table = a.block_table + (size_t)s * a.table_width;
+  const int lo = a.window > 0 ? max(0, pos - a.window + 1) : (a.chunk > 0 ? pos - pos % a.chunk : 0);
+  const int lo0 = a.window > 0 ? max(0, pos0 - a.window + 1) : (a.chunk > 0 ? pos0 - pos0 % a.chunk : 0);
+  const int keep = a.window > 0 ? a.keep_first : 0;
+  // blocks of 16 keys: the kept first ones that lie before the window's, then from the first row's first key on
+  const int main0 = lo0 >> 4, kept = min((keep + 15) >> 4, main0);
+  const int blocks = __builtin_amdgcn_readfirstlane(kept + (hi >> 4) - main0 + 1);
+
+  f32x4_t qv[ND], acc[ND];
+  const float* qr = (const float*)a.q + ((size_t)t * a.nq + h) * D + 4 * q;
+#pragma unroll
+  for (int j = 0; j < ND; ++j) {
+    if (j < nd) qv[j] = *(const f32x4_t*)(qr + 16 * j);
+    acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  float m = -INFINITY, l = 0.f;
+  const float* kc = (const float*)a.k_cache;
+  const float* vc = (const float*)a.v_cache;
+  for (int i = wave; i < blocks; i += W) {
+    const int j0 = 16 * (i < kept ? i : main0 + i - kept);
+    // K: the lane's key j0 + r; V: its keys j0 + 4 q .. + 3 (one page). Places after the last key, and pages
+    // that were given back, are read as the sequence's last key (its page is there) and count for nothing
+    const int kj = min(j0 + r, hi), vj = j0 + 4 * q;
+    int kp = table[kj / ps], vp = table[min(vj, hi) / ps];
+    const int last_page = table[hi / ps];
+    const bool v_there = vj <= hi && vp >= 0;
+    kp = kp < 0 ? last_page : kp;
+    vp = v_there ? vp : last_page;
+    const float* kr = kc + (((size_t)kp * a.nkv + kvh) * ps + kj % ps) * D + 4 * q;
+    const float* vr = vc + ((size_t)vp * a.nkv + kvh) * Dv * ps + (v_there ? vj % ps : 0);
+    f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+      if (j < nd) {
+        const f32x4_t kv = *(const f32x4_t*)(kr + 16 * j);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[c], qv[j][c], sc, 0, 0, 0);
+      }
+    float mx = m;
+    bool seen[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = j0 + 4 * q + e;
+      sc[e] *= a.scale;
+      if (a.softcap > 0.f) sc[e] = a.softcap * tanhf(sc[e] / a.softcap);
+      seen[e] = j <= pos && (j >= lo || j < keep);
+      if (seen[e]) mx = fmaxf(mx, sc[e]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (mx > -INFINITY) {  // false only for rows that have seen no key yet
+      const float corr = expf(m - mx);
+      l *= corr;
+#pragma unroll
+      for (int j = 0; j < ND; ++j) acc[j] *= corr;
+      m = mx;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sc[e] = seen[e] ? expf(sc[e] - m) : 0.f;
+      l += sc[e];
+    }
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+      if (j < nv) {
+        f32x4_t vv = *(const f32x4_t*)(vr + (size_t)(16 * j + r) * ps);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vv[e] = (v_there && vj + e <= hi) ? vv[e] : 0.f;  // never written: not a number, perhaps
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], sc[e], acc[j], 0, 0, 0);
+        }
+      }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (W > 1) {
+    if (q == 0) {
+      hand_m[wave][r] = m;
+      hand_l[wave][r] = l;
+    }
+    __syncthreads();
+    float top = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) top = fmaxf(top, hand_m[w][r]);
+#pragma unroll
+    for (int w = 0; w < W; ++w) sum += hand_m[w][r] > -INFINITY ? hand_l[w][r] * expf(hand_m[w][r] - top) : 0.f;
+    const float corr = m > -INFINITY ? expf(m - top) : 0.f;
+#pragma unroll
+    for (int j = 0; j < ND; ++j) acc[j] *= corr;
+    m = top;
+    l = sum;
+#pragma unroll
+    for (int half = W / 2; half > 0; half >>= 1) {
+      if (wave >= half && wave < 2 * half)
+#pragma unroll
+        for (int j = 0; j < ND; ++j) hand[wave - half][j * 64 + lane] = acc[j];
+      __syncthreads();
+      if (wave < half)
+#pragma unroll
+        for (int j = 0; j < ND; ++j) acc[j] += hand[wave][j * 64 + lane];
+      __syncthreads();
+    }
+  }
+  if (a.sink) {  // a key of score 0 without a value
+    const float top = fmaxf(m, 0.f), corr = m > -INFINITY ? expf(m - top) : 0.f;
+    l = l * corr + expf(-top);
+#pragma unroll
+    for (int j = 0; j < ND; ++j) acc[j] *= corr;
+  }
+  // rows into LDS in order, then out with the block's threads (a turned value's partner lies half a row away)
+  float* out_rows = (float*)hand;
+  if (wave == 0) {
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+      if (j < nv) *(f32x4_t*)(out_rows + r * Dv + 16 * j + 4 * q) = acc[j] * inv;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < (last_row - row0 + 1) * Dv; i += 64 * W) {
+    const int ri = row0 + i / Dv, d = i % Dv, ti = t0 + ri / g, hq = kvh * g + ri % g;
+    float v = out_rows[i];
+    if (a.turn) {
+      const float* angles = a.turn + (size_t)ti * Dv;
+      const int half = Dv >> 1, j = d < half ? d : d - half;
+      const float p = out_rows[d < half ? i + half : i - half], c = angles[j], sn = angles[half + j];
+      v = d < half ? v * c + p * sn : v * c - p * sn;
+    }
+    if (a.gate) v *= 1.0f / (1.0f + expf(-((const float*)a.gate)[(size_t)ti * a.gate_stride + (size_t)hq * Dv + d]));
+    ((float*)a.out)[((size_t)ti * a.nq + hq) * Dv + d] = v;
+  }
+}
+
+// Eight waves a row tile where tiles are few (decoding: the keys are what there is to share), four otherwise.
+template <int ND>
+static void attention_f32_tiles(const AttnArgs& a, hipStream_t stream) {
+  const int tiles = (int)(((long)a.max_q_len * (a.nq / a.nkv) + 15) / 16);
+  dim3 grid(tiles, a.nkv, a.num_seqs);
+  if ((long)tiles * a.nkv * a.num_seqs <= 512) attention_f32_tile_kernel<ND, 8><<<grid, 512, 0, stream>>>(a);
+  else attention_f32_tile_kernel<ND, 4><<<grid, 256, 0, stream>>>(a);
+}
+
 extern "C" int qrt_attention_f32(const AttnArgs* args, int dtype, hipStream_t stream) {
   AttnArgs a = *args;
   QRT_CHECK(a.num_tokens >= 0 && a.nq > 0 && a.nkv > 0 && a.nq % a.nkv == 0,
@@ -148,6 +315,17 @@ extern "C" int qrt_attention_f32(const AttnArgs* args, int dtype, hipStream_t st
   QRT_CHECK(!a.turn || a.value_dim % 2 == 0, "attention: turned values of odd size %d", a.value_dim);
   QRT_CHECK(a.nq <= 65535, "attention: too many heads");
   if (a.num_tokens == 0) return 0;
+  const int widest = a.head_dim > a.value_dim ? a.head_dim : a.value_dim;
+  if (dtype == QRT_F32 && a.cu_q && a.head_dim % 16 == 0 && a.value_dim % 16 == 0 && widest <= 256 && a.page_size % 4 == 0 &&
+      a.num_seqs <= 65535 && a.nkv <= 65535 && a.max_q_len > 0 &&
+      ((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.v_cache) % 16 == 0) {
+    if (widest <= 32) attention_f32_tiles<2>(a, stream);
+    else if (widest <= 64) attention_f32_tiles<4>(a, stream);
+    else if (widest <= 128) attention_f32_tiles<8>(a, stream);
+    else attention_f32_tiles<16>(a, stream);
+    QRT_LAUNCH_CHECK("attention_f32_tiles");
+    return 0;
+  }
   dim3 grid(a.num_tokens, a.nq), block(64);
   if (dtype == QRT_F32) attention_f32_kernel<float><<<grid, block, 0, stream>>>(a);
   else if (dtype == QRT_BF16) attention_f32_kernel<bf16_t><<<grid, block, 0, stream>>>(a);
