@@ -75,8 +75,10 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 
 // ------------------------------------------------------------ the MFMA kernels
 // Parts of K (waves a block of the few-row kernel) and the length of one: more parts for a longer K, so
-// that 160 blocks (the 2,560 rows of a 4B down projection) still keep enough loads in flight.
-static inline int f32_parts(int K) { return K >= 8192 ? 16 : K >= 1024 ? 8 : K >= 256 ? 4 : 1; }
+// that 160 blocks (the 2,560 rows of a 4B down projection) still keep enough loads in flight, and parts
+// for a short one too, since a sum's error grows with the length of its chain: relative to float64 2.0e-7 in one
+// chain and 1.1e-7 in four parts at K 128, 4.1e-7 and 1.6e-7 at 512 (equal up to 32, where there is one part).
+static inline int f32_parts(int K) { return K >= 8192 ? 16 : K >= 256 ? 8 : K > 64 ? 4 : K > 32 ? 2 : 1; }
 static inline int f32_part_len(int K, int parts) { return ((K + parts - 1) / parts + 31) / 32 * 32; }
 
 __device__ __forceinline__ f32x4_t load_f32x4_below(const float* __restrict__ row, int k, int end) {
@@ -254,6 +256,7 @@ static void f32_rows_parts(const float* a, const float* w, float* c, int M, int 
     case 16: return f32_rows<MB, 16>(a, w, c, M, N, K, stream);
     case 8: return f32_rows<MB, 8>(a, w, c, M, N, K, stream);
     case 4: return f32_rows<MB, 4>(a, w, c, M, N, K, stream);
+    case 2: return f32_rows<MB, 2>(a, w, c, M, N, K, stream);
     default: return f32_rows<MB, 1>(a, w, c, M, N, K, stream);
   }
 }
