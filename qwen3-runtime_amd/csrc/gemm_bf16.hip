@@ -9,6 +9,7 @@
 // one vector. A wave owns a (16*MT) x (16*NT) tile; a block is four waves side
 // by side along N. Skinny M (decode) uses MT = 1.
 #include "common.h"
+#include "direct.h"
 #include <type_traits>
 
 template <bool ALIGNED>
@@ -261,14 +262,6 @@ static int skinny(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int 
 // result is plane blockIdx.y of the output (the caller adds the planes: used where the result
 // feeds a residual add); its NW waves take the pairs round-robin and meet in LDS, added in
 // wave order.
-#define QRT_WAIT_LOADS(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
-#define QRT_WAIT_LDS() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
-// A barrier without the fence of __syncthreads(), which would wait for every direct load to LDS
-// in flight: what has to have landed is waited for by hand before it.
-#define QRT_BARRIER() asm volatile("s_barrier" ::: "memory")
-typedef const void __attribute__((address_space(1)))* global_ptr_t;
-typedef void __attribute__((address_space(3)))* lds_ptr_t;
-
 template <int NW, int NT, int U, int GATED, typename TO>
 __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,

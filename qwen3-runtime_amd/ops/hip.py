@@ -945,10 +945,14 @@ class HipOps:
         _need(down, "expert down", x.dtype, (n, h, inter))
         _need(index, "expert index", torch.int32, (t, top))
         _need(weight, "expert weight", torch.float32, (t, top))
+        if out is not None:  # the caller's own float32 rows
+            _need(out, "experts' output", torch.float32, (t, h))
+        if t and self.experts_fit(x, h, inter):
+            planes = self.moe_for_residual(x, gate_up, down, index, weight, activation, limit, weight_on_input)
+            total = planes[0] if top == 1 else self.accumulate(planes[0], planes[1:])
+            return total if out is None else out.copy_(total)
         if out is None:
             out = torch.empty((t, h), dtype=torch.float32, device=x.device)
-        else:  # the caller's own float32 rows (a plane of a sum that the next norm adds up)
-            _need(out, "experts' output", torch.float32, (t, h))
         if t == 0:
             return out
         pairs = t * top
@@ -978,6 +982,50 @@ class HipOps:
                                                      _ptr(act), _ptr(out), _CODE[x.dtype], c_int(t), c_int(h),
                                                      c_int(inter), c_int(n), c_int(top), *kind, c_int(bool(weight_on_input)),
                                                      _stream()))
+        return out
+
+    # Pairs per expert from which the experts' products go by tiles and not as a stream of the weights: 16 experts
+    # of 2,560 x 1,536, 2 a token, both products, us by the stream and by tiles: 77 and 95 at 64 tokens (8 pairs
+    # an expert), 104 and 97 at 96 (12), 263 and 114 at 512
+    experts_tile_pairs_per_expert = 11
+    experts_rows_max_pairs = 8192  # the stream's blocks list their expert's pairs in LDS
+
+    @staticmethod
+    def experts_fit(x, hidden, inter) -> bool:
+        """Whether the experts' MFMA kernels take these operands (rows of whole cache lines)."""
+        return x.dtype == torch.bfloat16 and hidden % 64 == 0 and inter % 64 == 0
+
+    def moe_for_residual(self, x, gate_up, down, index, weight, activation="swiglu", limit=0.0, weight_on_input=False,
+                         out=None):
+        """``moe_swiglu`` for a result that is only ever added to the residual stream: float32 planes
+        [top, T, H], plane ``j`` the output of each token's ``j``-th expert, which the next norm adds up; in ``out``
+        if given. None where the MFMA kernels do not take the operands (``moe_swiglu`` takes all)."""
+        t, h = x.shape
+        n, rows_e, _ = gate_up.shape
+        inter = rows_e if activation == "relu2" else rows_e // 2
+        top = index.shape[1]
+        if not self.experts_fit(x, h, inter):
+            return None
+        if weight_on_input and activation == "relu2":
+            raise OpsError("weights on the experts' input go with gated experts")
+        _need(x, "x")
+        _need(gate_up, "expert gate/up", x.dtype, (n, rows_e, h))
+        _need(down, "expert down", x.dtype, (n, h, inter))
+        _need(index, "expert index", torch.int32, (t, top))
+        _need(weight, "expert weight", torch.float32, (t, top))
+        if out is None:
+            out = torch.empty((top, t, h), dtype=torch.float32, device=x.device)
+        else:
+            _need(out, "experts' planes", torch.float32, (top, t, h))
+        pairs = t * top
+        act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
+        scratch = None
+        if pairs >= self.experts_tile_pairs_per_expert * n or pairs > self.experts_rows_max_pairs:
+            scratch = torch.empty(pairs + n + 2 + 2 * (pairs // 128 + n), dtype=torch.int32, device=x.device)
+        self._check(self.lib, self.lib.qrt_experts(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(index), _ptr(weight), _ptr(act),
+                                                   _ptr(out), _ptr(scratch), c_int(t), c_int(h), c_int(inter), c_int(n),
+                                                   c_int(top), c_int(ACTIVATIONS[activation]), c_float(limit),
+                                                   c_int(bool(weight_on_input)), _stream()))
         return out
 
     # Steps of many tokens run the experts one by one, each on the rows of its own tokens, with
@@ -1163,9 +1211,9 @@ class HipOps:
             c_int(kernel), c_int(parts), _stream()))
         return out
 
-    def linear_planes_with_spare(self, x, w):
-        """``linear_for_residual(x, w)`` as float32 planes ``[P + 1, T, N]`` of which the last is left
-        for the caller to fill with one more addend of the same sum (so that the sum costs no
+    def linear_planes_with_spare(self, x, w, spare=1):
+        """``linear_for_residual(x, w)`` as float32 planes ``[P + spare, T, N]`` of which the last ``spare`` are left
+        for the caller to fill with more addends of the same sum (so that the sum costs no
         kernel of its own); None where the product does not run in the engine's own kernels."""
         m, k = x.shape
         n = w.shape[0]
@@ -1179,7 +1227,7 @@ class HipOps:
             return None
         _need(x, "x", torch.bfloat16)
         _need(w, "weight", torch.bfloat16, (n, k))
-        out = torch.empty((parts + 1, m, n), dtype=torch.float32, device=x.device)
+        out = torch.empty((parts + spare, m, n), dtype=torch.float32, device=x.device)
         self._check(self.lib, self.lib.qrt_gemm_bf16(
             _ptr(x), _ptr(w), _ptr(out), F32, c_int(m), c_int(n), c_int(k), c_int(0),
             c_int(kernel), c_int(parts), _stream()))

@@ -150,7 +150,7 @@ class RoutedSwiGLU(FeedForward):
                  and self.weight_on == "output")
         if plain:
             index, weight = ops.route_top(x, self.router, self.router_bias, self.top)
-            return ops.moe_swiglu(x, self.gate_up, self.down, index, weight)
+            return self._routed(ops, x, index, weight)
         how = {"group_score": self.group_score} if self.group_score != "top2" else {}
         if self.has_correction or self.renormalise or self.weight_scale != 1.0:
             how.update(correction=self.correction, renormalise=self.renormalise, weight_scale=self.weight_scale)
@@ -166,13 +166,26 @@ class RoutedSwiGLU(FeedForward):
         if self.weight_on == "input":
             more["weight_on_input"] = True
         if not self.shared_size:
-            return ops.moe_swiglu(x, self.gate_up, self.down, index, weight, **more)
+            return self._routed(ops, x, index, weight, **more)
         act = ops.gated_linear(x, self.shared_gate_up, activation=self.activation, limit=self.shared_limit, **opened)
-        # few tokens: the shared expert's product leaves float32 planes with one to spare, the routed
-        # experts write theirs into it, and the norm that comes next adds them all up
-        planes = ops.linear_planes_with_spare(act, self.shared_down)
-        if planes is not None:
-            ops.moe_swiglu(x, self.gate_up, self.down, index, weight, out=planes[-1], **more)
-            return planes
+        # few tokens: the shared expert's product leaves float32 planes with some to spare, the routed
+        # experts write theirs into them, and the norm that comes next adds them all up
+        fits = getattr(ops, "experts_fit", None)
+        if fits is not None and fits(x, self.hidden_size, self.intermediate_size):
+            planes = ops.linear_planes_with_spare(act, self.shared_down, self.top)
+            if planes is not None:
+                ops.moe_for_residual(x, self.gate_up, self.down, index, weight, out=planes[-self.top:], **more)
+                return planes
+        else:
+            planes = ops.linear_planes_with_spare(act, self.shared_down)
+            if planes is not None:
+                ops.moe_swiglu(x, self.gate_up, self.down, index, weight, out=planes[-1], **more)
+                return planes
         out = ops.moe_swiglu(x, self.gate_up, self.down, index, weight, **more)
         return ops.accumulate(out, ops.linear_for_residual(act, self.shared_down))
+
+    def _routed(self, ops, x, index, weight, **more):
+        """The routed experts' sum, as the norm that comes next may have it: in planes where the ops make them."""
+        planes = getattr(ops, "moe_for_residual", None) if self.top <= 8 else None
+        out = None if planes is None else planes(x, self.gate_up, self.down, index, weight, **more)
+        return ops.moe_swiglu(x, self.gate_up, self.down, index, weight, **more) if out is None else out

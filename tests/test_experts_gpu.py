@@ -1,0 +1,76 @@
+"""The routed experts' MFMA kernels against the plain experts in float64, in both forms (a stream of the
+weights, tiles), at the edges of their groups of 16 and 128 pairs."""
+
+import pytest
+import torch
+
+from test_kernels_gpu import DEV, close, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def ops():
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    return HipOps()
+
+
+def plain(x, gate_up, down, index, weight, activation, limit, on_input):
+    """float64 [top, T, H]; the activations rounded to bfloat16 between the two products."""
+    t, top = index.shape
+    x, gate_up, down, weight = x.double(), gate_up.double(), down.double(), weight.double()
+    out = torch.zeros(top, t, x.shape[1], dtype=torch.float64, device=x.device)
+    for i in range(t):
+        for j in range(top):
+            e = int(index[i, j])
+            by = weight[i, j] if on_input else 1.0
+            z = gate_up[e] @ x[i] * by
+            if activation == "relu2":
+                a = z.clamp(min=0).square()
+            else:
+                g, u = z.chunk(2)
+                if activation == "clamped":
+                    g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+                    a = g * torch.sigmoid(1.702 * g) * (u + 1)
+                else:
+                    a = g * torch.sigmoid(g) * u
+            out[j, i] = down[e] @ a.bfloat16().double() * (1.0 if on_input else weight[i, j])
+    return out
+
+
+@pytest.mark.parametrize("form", ["stream", "tiles"])
+@pytest.mark.parametrize("t,top,n,h,inter,skew,activation,on_input", [
+    (1, 2, 16, 128, 64, None, "swiglu", False),     # fewer pairs than experts
+    (5, 3, 4, 192, 128, None, "clamped", False),    # K of three pieces of 64, one wave without any
+    (17, 1, 3, 64, 192, 0, "swiglu", True),         # 17 pairs of one expert: two groups of 16; experts without a pair
+    (40, 2, 5, 128, 64, None, "relu2", False),
+    (129, 1, 2, 64, 64, 1, "swiglu", False),        # 129 pairs of one expert: two tiles, the second of one pair
+    (150, 8, 64, 128, 128, None, "swiglu", False),
+])
+def test_experts_against_float64(ops, form, t, top, n, h, inter, skew, activation, on_input):
+    ops.experts_tile_pairs_per_expert = 0 if form == "tiles" else 1 << 20
+    gated = activation != "relu2"
+    x = rnd(t, h, dtype=torch.bfloat16, seed=1)
+    gate_up = rnd(n, (2 if gated else 1) * inter, h, dtype=torch.bfloat16, scale=h ** -0.5, seed=2)
+    down = rnd(n, h, inter, dtype=torch.bfloat16, scale=inter ** -0.5, seed=3)
+    scores = rnd(t, n, seed=4)
+    if skew is not None:
+        scores[:, skew] += 100.0
+    weight, index = scores.topk(top, -1)
+    weight, index = torch.softmax(weight, -1).contiguous(), index.int().contiguous()
+    want = plain(x, gate_up, down, index, weight, activation, 2.0, on_input)
+    got = ops.moe_for_residual(x, gate_up, down, index, weight, activation, 2.0, on_input)
+    # an activation (about one in size) that float32 sums bring to the other side of a bfloat16 boundary is 2^-8 off:
+    # times a weight of size inter^-0.5, and few of an output's terms are
+    close(got, want.float(), 4e-3, 4e-3)
+    close(ops.moe_swiglu(x, gate_up, down, index, weight, activation, 2.0, weight_on_input=on_input), want.sum(0).float(), 8e-3, 8e-3)
+
+
+def test_widths_that_whole_lines_do_not_fit_keep_the_general_form(ops):
+    x, gate_up, down = (rnd(*s, dtype=torch.bfloat16, scale=0.1) for s in ((3, 96), (4, 80, 96), (4, 96, 40)))
+    index = torch.tensor([[0, 3], [1, 0], [2, 1]], dtype=torch.int32, device=DEV)
+    weight = torch.full((3, 2), 0.5, device=DEV)
+    assert ops.moe_for_residual(x, gate_up, down, index, weight) is None
+    want = plain(x, gate_up, down, index, weight, "swiglu", 0.0, False).sum(0)
+    close(ops.moe_swiglu(x, gate_up, down, index, weight), want.float(), 1e-3, 1e-3)
