@@ -28,6 +28,7 @@
 // keep_first keys of the sequence are visible too. With a score cap the scaled scores become
 // cap * tanh(score / cap) before the softmax; with a sink the denominator has one more term, 1.
 #include "common.h"
+#include "direct.h"
 #include <math.h>
 
 #ifndef QRT_HEAD_DIM
@@ -973,6 +974,209 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void attention_bf16_prefil
   }
 }
 
+// Portions with heads wider than 256 (latent rows: one key head for all query heads). A wave's accumulator
+// and queries are 168 registers at 448, so a tile of 16 rows a wave is what fits, and what bounds such a
+// wave reading keys and values for itself (the general kernel) is the loads: 57 KB from the caches for 56
+// MFMAs. Here eight waves, 128 rows, share each block of 32 keys through LDS, two stages filled by direct
+// loads (no registers on the way) during the products of the block before, one barrier a block. The LDS
+// reads, 57 KB a wave and block at 220 B/clk, then take about as long as the products. 2,047 tokens with 32
+// heads of 448: 789 -> 225 us without history, 2,190 -> 438 us with 2,048 tokens of it (0.76 PFLOP/s); LDS and matrix pipes
+// are busy a quarter of the time each: what is left is a wave's own chain, which two waves a SIMD do not hide.
+// A stage holds the keys group by group as they lie in the cache, 8 rows of 2 D bytes, the 16-byte pieces of
+// key k of group p permuted within every 128 bytes (piece c at place c ^ (2 p + k / 2 % 2)), and the values
+// group by group as [DV][8 keys]: neither operand read then meets a bank twice, and a load's source is
+// a scalar base plus a lane's constant. MFMA row 4 q + r of sub-block s is key 8 q + 4 s + r, as above.
+#if QRT_HEAD_DIM % 64 == 0 && QRT_VALUE_DIM % 64 == 0 && (QRT_HEAD_DIM > 256 || QRT_VALUE_DIM > 256)
+#define QRT_WIDE_PREFILL 1
+constexpr int WIDE_STAGE = 64 * D + 64 * DV;  // bytes: 32 keys, 32 values
+template <bool P2>
+__global__ __launch_bounds__(512, 1) void attention_bf16_wide_kernel(AttnTileArgs a) {
+  extern __shared__ __align__(16) unsigned char wide_lds[];  // [2][WIDE_STAGE]
+  const int lane = threadIdx.x & 63, wave = uniform_wave_number();
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int tile = blockIdx.x / a.nkv, kvh = blockIdx.x - tile * a.nkv, split = blockIdx.z;
+  const int seq = a.tile_seq[tile];
+  const int g = a.nq / a.nkv;
+  const int q_begin = a.cu_q[seq];
+  const int q_len = a.cu_q[seq + 1] - q_begin;
+  const int kv_len = a.kv_lens[seq];
+  const int n_rows = q_len * g;
+  const int tile_row0 = a.tile_row0[tile];
+  const int row0 = tile_row0 + 16 * wave;
+  const bool wave_has_rows = row0 < n_rows;
+  const int first_pos = kv_len - q_len;
+  const int ps = a.page_size, psh = __builtin_ctz(ps);
+  const int* table = a.block_table + (size_t)seq * a.table_width;
+
+  const int my_row = row0 + r16;
+  const bool row_valid = my_row < n_rows;
+  const int row_c = min(my_row, n_rows - 1);
+  const int tok = row_c / g, hg = row_c - tok * g;
+  const int qpos = first_pos + tok;
+  const size_t row_index = (size_t)(q_begin + tok) * a.nq + kvh * g + hg;
+  const bf16_t* qp = a.q + row_index * D;
+  bf16x8_t qreg[KFULL];
+#pragma unroll
+  for (int i = 0; i < KFULL; ++i) qreg[i] = *(const bf16x8_t*)(qp + 32 * i + 8 * quad);
+  const int tile_pos_min = __builtin_amdgcn_readfirstlane(first_pos + min(row0, n_rows - 1) / g);
+  const int tile_lo_max = __builtin_amdgcn_readfirstlane(first_seen(first_pos + min(row0 + 15, n_rows - 1) / g, a.window, a.chunk));
+
+  const int blk_last_row = min(tile_row0 + 127, n_rows - 1);
+  const int blk_pos_min = first_pos + tile_row0 / g, blk_pos_max = first_pos + blk_last_row / g;
+  const int lo = max(0, first_seen(blk_pos_min, a.window, a.chunk));
+  const int all_b0 = lo >> 5, all_b1 = (blk_pos_max >> 5) + 1;
+  const int per = (all_b1 - all_b0 + a.num_splits - 1) / a.num_splits;
+  const int b0 = all_b0 + split * per, b1 = min(all_b1, b0 + per);
+  int wb0 = b1, wb1 = b0;  // this wave's blocks: none unless it has rows
+  if (wave_has_rows) {
+    const int row_last = min(row0 + 15, n_rows - 1);
+    wb0 = max(0, first_seen(first_pos + row0 / g, a.window, a.chunk)) >> 5;
+    wb1 = min(((first_pos + row_last / g) >> 5) + 1, b1);
+  }
+  f32x4_t o[DB];
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int i = 0; i < DB; ++i) o[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+  // Wave p of the first four brings the keys of group p of a block, wave 4 + p the values of group p: a group
+  // lies in one page, found with a scalar instruction a round ahead.
+  const size_t k_stride = (size_t)a.nkv * ps * D, v_stride = (size_t)a.nkv * ps * DV;  // elements per page
+  const bf16_t* k_head = a.k_cache + (size_t)kvh * ps * D;
+  const bf16_t* v_head = a.v_cache + (size_t)kvh * DV * ps;
+  const bool brings_keys = wave < 4;
+  const int group = wave & 3;
+  constexpr int PER_KEY = D / 8, K_LOADS = D / 64, V_LOADS = DV / 64;
+  int from[K_LOADS];  // of a load's piece, within the group
+#pragma unroll
+  for (int j = 0; j < K_LOADS; ++j) {
+    const int piece = 64 * j + lane, key = piece / PER_KEY, slot = piece - key * PER_KEY;
+    from[j] = key * D + 8 * ((slot & ~7) | ((slot & 7) ^ (2 * group + ((key >> 1) & 1))));
+  }
+  // A group's first key is clamped into pages the sequence holds; what lies outside is masked with the scores,
+  // and its values are zeroed before they are multiplied.
+  auto group_start = [&](int b) { return min(max((b << 5) + 8 * group, lo & ~7), blk_pos_max & ~7); };
+  auto lookup = [&](int b) { return table[page_div<P2>(group_start(b), ps, psh)]; };
+  auto fetch = [&](int b, int page, int stage) {  // the wave's part of block b into a stage
+    const int off = page_mod<P2>(group_start(b), ps);
+    unsigned char* dst = wide_lds + stage * WIDE_STAGE;
+    if (brings_keys) {
+      const bf16_t* src = k_head + (size_t)page * k_stride + (size_t)off * D;
+#pragma unroll
+      for (int j = 0; j < K_LOADS; ++j)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(src + from[j]), (lds_ptr_t)(dst + 16 * D * group + 1024 * j), 16, 0, 0);
+    } else {
+      const bf16_t* src = v_head + (size_t)page * v_stride + off + (size_t)lane * ps;
+#pragma unroll
+      for (int j = 0; j < V_LOADS; ++j)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(src + (size_t)64 * j * ps), (lds_ptr_t)(dst + 64 * D + 16 * DV * group + 1024 * j), 16, 0, 0);
+    }
+  };
+  const int key_row = 16 * D * (r16 >> 2) + 2 * D * (r16 & 3), key_swap = 2 * (r16 >> 2) + ((r16 >> 1) & 1);
+  const int key_at[2] = {key_row + 16 * (quad ^ key_swap), key_row + 16 * ((4 + quad) ^ key_swap)};
+  const int value_at = 64 * D + 16 * DV * quad + 16 * r16;
+  auto multiply = [&](int b, int stage) {
+    if (b < wb0 || b >= wb1) return;  // uniform over the wave
+    const int base = b << 5;
+    const unsigned char* at = wide_lds + stage * WIDE_STAGE;
+    f32x4_t sc[2];
+    sc[0] = sc[1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    // Operands are read two at a time, AHEAD groups ahead of their products and no further: left alone the
+    // compiler asks for all 28 at once, has no registers for them and spills, and a reload from scratch in
+    // this loop waits for the direct loads in flight.
+    constexpr int AHEAD = DMAX <= 448 ? 3 : 1;
+    bf16x8_t in[AHEAD + 1][2];
+    auto keys = [&](int n) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) in[n % (AHEAD + 1)][e] = *(const bf16x8_t*)(at + key_at[n & 1] + 128 * (n >> 1) + 8 * D * e);
+    };
+    auto values = [&](int n) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) in[n % (AHEAD + 1)][e] = *(const bf16x8_t*)(at + value_at + 256 * (2 * n + e));
+    };
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) keys(n);
+#pragma unroll
+    for (int n = 0; n < KFULL; ++n) {
+      if (n + AHEAD < KFULL) keys(n + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) sc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in[n % (AHEAD + 1)][e], qreg[n], sc[e], 0, 0, 0);
+    }
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) values(n);
+    if (a.cap_in > 0.f) cap_scores(sc, a.cap_in, a.cap_out);  // the same for the whole launch
+    const bool whole = base + 31 <= tile_pos_min && base >= tile_lo_max;
+    float mx = lane_max(sc);
+    if (!whole || __any(mx * a.scale_log2 > m + LAZY)) {
+      if (!whole) {
+        tile_mask(sc, base, quad, row_valid, qpos, a.window, a.chunk, 0, 0);
+        mx = lane_max(sc);
+      }
+      tile_move_reference(mx, a.scale_log2, m, l, o);
+    }
+    bf16x8_t pb;
+    tile_probabilities(sc, a.scale_log2, m, l, pb);
+#pragma unroll
+    for (int n = 0; n < DB / 2; ++n) {
+      if (n + AHEAD < DB / 2) values(n + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        o[2 * n + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in[n % (AHEAD + 1)][e], pb, o[2 * n + e], 0, 0, 0);
+    }
+  };
+  if (b0 < b1) {  // uniform over the block of waves
+    int page = lookup(b0);
+    fetch(b0, page, 0);
+    page = lookup(min(b0 + 1, b1 - 1));
+    for (int b = b0; b < b1; ++b) {
+      const int stage = (b - b0) & 1;
+      QRT_WAIT_LOADS(0);  // this wave's part of block b has landed ...
+      QRT_WAIT_LDS();     // ... and it has read block b - 1,
+      QRT_BARRIER();      // ... as have all others
+      if (b + 1 < b1) {
+        fetch(b + 1, page, stage ^ 1);
+        page = lookup(min(b + 2, b1 - 1));
+      }
+      if ((b << 5) + 31 > blk_pos_max || (b << 5) < lo) {
+        // 0 * NaN is NaN: values of keys no row of the block sees become zeros, in the stage (a test
+        // beside every operand read, or a second copy of the products, cost registers that are not there)
+        for (int i = threadIdx.x; i < 4 * DV; i += 512) {
+          const int g0 = (b << 5) + 8 * (i / DV);
+          bf16x8_t* v = (bf16x8_t*)(wide_lds + stage * WIDE_STAGE + 64 * D + 16 * i);
+          *v = keep_first(*v, g0 + 7 >= lo ? blk_pos_max - g0 + 1 : 0);
+        }
+        QRT_WAIT_LDS();
+        QRT_BARRIER();
+      }
+      multiply(b, stage);
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (!row_valid || !wave_has_rows) return;
+  if (a.sink && a.num_splits == 1) add_sink(m, l, o);
+  if (a.turn && a.num_splits == 1) turn_back(o, a.turn + row_index / a.nq * DV, quad);
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  if (a.num_splits == 1) {
+    bf16_t* op = a.out + row_index * DV;
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      bf16x4_t w;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        w[r] = (bf16_t)(o[i][r] * inv * gate_factor(a.gate, a.gate_stride, a.nq, row_index, 16 * i + 4 * quad + r));
+      *(bf16x4_t*)(op + 16 * i + 4 * quad) = w;
+    }
+  } else {
+    float* op = a.part_o + (row_index * a.num_splits + split) * DV;
+#pragma unroll
+    for (int i = 0; i < DB; ++i) *(f32x4_t*)(op + 16 * i + 4 * quad) = o[i] * inv;
+    if (quad == 0) a.part_lse[row_index * a.num_splits + split] = l > 0.f ? m + log2f(l) : -INFINITY;
+  }
+}
+#endif
+
 // Few splits: every load is asked for before the first is used (clamped indices, so none stands
 // under a branch), one trip to memory instead of two; the sums are those of the kernel's loop.
 // A thread takes elements threadIdx.x and threadIdx.x + blockDim.x of the row; with turned values the two
@@ -1561,6 +1765,10 @@ extern "C" int qrt_attention_bf16(const AttnTileArgs* args, int num_rows_total, 
   QRT_CHECK((a.cap_in > 0.f) == (a.cap_out > 0.f), "attention: a score cap needs both of its factors");
   QRT_CHECK(!a.gate || a.gate_stride >= (long)a.nq * DV, "attention: the gate's rows are %ld elements apart, %d heads of %d need more",
             a.gate_stride, a.nq, DV);
+  QRT_CHECK(a.use_lds >= 0 && a.use_lds <= 3, "attention: unknown way through LDS %d", a.use_lds);
+#ifndef QRT_WIDE_PREFILL
+  QRT_CHECK(a.use_lds != 3, "attention: the kernel for wide heads is not built for heads of %d and values of %d", D, DV);
+#endif
   if (a.num_tiles == 0) return 0;
   const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
   QRT_CHECK((long long)a.num_tiles * a.nkv < (1ll << 31), "attention: %d tiles x %d key heads is too many blocks", a.num_tiles, a.nkv);
@@ -1590,6 +1798,20 @@ extern "C" int qrt_attention_bf16(const AttnTileArgs* args, int num_rows_total, 
     const size_t smem = lds_bytes;
     if (p2) attention_bf16_prefill_kernel<2, true, 1><<<grid, block, smem, stream>>>(a);
     else attention_bf16_prefill_kernel<2, false, 1><<<grid, block, smem, stream>>>(a);
+#ifdef QRT_WIDE_PREFILL
+  } else if (a.use_lds == 3) {  // tiles of 128 rows
+    QRT_CHECK(a.keep_first == 0, "attention: the kernel for wide heads keeps no first keys beside a window");
+    constexpr size_t smem = 2 * (size_t)WIDE_STAGE;
+    static bool allowed = false;
+    if (!allowed) {
+      if (hipFuncSetAttribute((const void*)attention_bf16_wide_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess ||
+          hipFuncSetAttribute((const void*)attention_bf16_wide_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+        return qrt_fail("attention (wide heads): cannot get %zu bytes of LDS", smem);
+      allowed = true;
+    }
+    if (p2) attention_bf16_wide_kernel<true><<<grid, dim3(512), smem, stream>>>(a);
+    else attention_bf16_wide_kernel<false><<<grid, dim3(512), smem, stream>>>(a);
+#endif
   } else if (a.row_tiles == 1 && p2) attention_bf16_kernel<1, true><<<grid, block, 0, stream>>>(a);
   else if (a.row_tiles == 1) attention_bf16_kernel<1, false><<<grid, block, 0, stream>>>(a);
   else if (a.row_tiles == 2 && p2) attention_bf16_kernel<2, true><<<grid, block, 0, stream>>>(a);

@@ -1724,7 +1724,7 @@ class HipOps:
         row_tiles = 1 if max_rows <= 64 or widest > 256 else (self.prefill_row_tiles if widest <= 128 else min(2, self.prefill_row_tiles))
         # the list depends on the rows a tile holds (head geometry and kernel choice): layers of
         # another geometry in the same step get a list of their own
-        key = ("attn_plan", g, nkv, widest, waves, row_tiles, decode, None if subset is None else tuple(subset), reach)
+        key = ("attn_plan", g, nkv, d, dv, waves, row_tiles, decode, None if subset is None else tuple(subset), reach, bool(keep_first))
         plan = ctx.scratch.get(key)
         if plan is None:  # the same for every layer of the step
             dev = out.device
@@ -1735,7 +1735,10 @@ class HipOps:
                 lds = waves == 4 and row_tiles >= 2 and self.prefill_through_lds
                 groups = self.choose_key_groups(q_lens, kv_lens, g, nkv, reach,
                                                 ctx.scratch.get("attn_splits")) if lds else 0
-                host, n_tiles = self.plan_tiles(q_lens, kv_lens, g, 16 * waves * row_tiles, nkv,
+                if (waves == 4 and widest > 256 and d % 64 == 0 and dv % 64 == 0 and not keep_first
+                        and self.prefill_through_lds):
+                    groups = 3  # eight waves of one tile of 16 rows each share keys and values through LDS
+                host, n_tiles = self.plan_tiles(q_lens, kv_lens, g, 128 if groups == 3 else 16 * waves * row_tiles, nkv,
                                                 self.resident_blocks if waves == 4 and row_tiles >= 2 and groups < 2
                                                 else 0, subset)
                 tiles = torch.from_numpy(host).to(dev)
