@@ -1289,6 +1289,9 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_o, const f
 // write-through atomic stores in place of the fence it costs what the second launch
 // costs.)
 constexpr int DW = 4;
+// Floats per row of an accumulator on its way through LDS: rows begin in different banks (at DV itself the 16 rows of
+// every store met in one: the join cost 0.4 to 1 us of a launch, and is stored 16 bytes at a time now).
+constexpr int OROW = DV + 4;
 
 // The 32-key blocks of the cache that a tile of the decode kernel walks: [begin, end). `fused`:
 // the cache holds the keys before the tile's one token (which the kernel adds from registers).
@@ -1426,7 +1429,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   extern __shared__ float lds[];
   float* lds_m = lds;                 // [DW][16]
   float* lds_l = lds + DW * 16;       // [DW][16]
-  float* lds_o = lds + 2 * DW * 16;   // [DW][16][DV]
+  float* lds_o = lds + 2 * DW * 16;   // [DW][16][OROW]
 
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r16 = lane & 15, quad = lane >> 4;
@@ -1595,10 +1598,9 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     lds_m[wave * 16 + r16] = m;
     lds_l[wave * 16 + r16] = l;
   }
+  if (row_valid)
 #pragma unroll
-  for (int i = 0; i < DB; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) lds_o[(wave * 16 + r16) * DV + 16 * i + 4 * quad + r] = o[i][r];
+    for (int i = 0; i < DB; ++i) *(f32x4_t*)(lds_o + (wave * 16 + r16) * OROW + 16 * i + 4 * quad) = o[i];
   __syncthreads();
 
   const size_t tile_row0 = (size_t)q_begin * a.nq;  // rows of this sequence start here, in units of heads
@@ -1615,7 +1617,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
 #pragma unroll
       for (int w = 0; w < DW; ++w) {
         const float f = exp2f(lds_m[w * 16 + row] - mm);
-        num += f * lds_o[(w * 16 + row) * DV + d];
+        num += f * lds_o[(w * 16 + row) * OROW + d];
         den += f * lds_l[w * 16 + row];
       }
     }
@@ -1700,7 +1702,7 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
   const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
   dim3 grid(a.num_tiles, a.nkv, a.num_splits), block(64 * DW);
   if (a.items) grid = dim3(a.nkv, a.max_items, 1);
-  constexpr size_t smem = (size_t)(2 * DW * 16 + DW * 16 * DV) * sizeof(float);
+  constexpr size_t smem = (size_t)(2 * DW * 16 + DW * 16 * OROW) * sizeof(float);
   if (smem > 64 * 1024) {  // head size 256: a little more LDS than a block gets without asking
     static bool allowed = false;  // once: not again inside every stream capture
     if (!allowed) {

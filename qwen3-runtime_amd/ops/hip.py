@@ -1627,13 +1627,17 @@ class HipOps:
         (1 / parts + cost). Counts of blocks that leave some units one block more than others are
         what it avoids: 12 sequences of 2,100 keys on 8 key heads 32 us in 3 parts (288 blocks), 27
         in 2; 24 sequences 49 us in 2 parts, 42 in 4; 40 sequences 78 us in 1 part, 65 in 4. At
-        least 8 key blocks of 32 a part (4 each measured 2 % slower over a batch-1 decode step at
-        2,048 keys), at most 64 parts (what the merge kernel reads with every load in flight)."""
+        least 8 key blocks of 32 a part, at most 64 parts (what the merge kernel reads with every
+        load in flight); but up to 16 parts may have 2 key blocks each: a compute unit pulls no more
+        than some 34 GB/s however many waves it runs, so few sequences of short contexts want many
+        units (attention and merge, us: 320 keys, 6 sequences 14.1 in 1 or 2 parts, 11.5 in 4, 12.0 in 5; one
+        sequence of 640 keys 15.1 in 2 parts, 10.5 in 10, of 1,025 keys 14.8 in 4, 11.1 in 16; 32 sequences of
+        320 keys 16.2 in 1 part, 19.9 in 2, which the model knows)."""
         work = num_tiles * nkv
         blocks = (max_kv + 31) // 32
         cost = 0.06 * 2100 / max(max_kv, 1)
         best, best_time = 1, None
-        for parts in range(1, max(1, min(blocks // 8, 64)) + 1):
+        for parts in range(1, max(1, min(blocks // 8, 64), min(blocks // 2, 16)) + 1):
             time = -(-work * parts // 256) * (1.0 / parts + cost)
             if best_time is None or time < best_time * 0.999:
                 best, best_time = parts, time
