@@ -1,0 +1,101 @@
+"""Row passes that load whole pieces of a row: the norm behind a sub-layer with the sum and the next norm, the
+router's choice with a lane per expert, rotation by pieces, the squared relu; against the plain forms, at widths and
+numbers of rows on both sides of every choice between their variants."""
+
+import pytest
+import torch
+
+from plain import ops_ref as R
+from test_kernels_gpu import DEV, close, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    return HipOps()
+
+
+@pytest.mark.parametrize("t,h", [(3, 4), (5, 1020), (511, 2048), (512, 2052), (513, 3072), (600, 3076), (7, 4096), (4, 4100), (3, 37)])
+@pytest.mark.parametrize("planes,dtype", [(1, torch.bfloat16), (2, torch.float32), (5, torch.float32)])
+def test_norm_add_rmsnorm(ops, t, h, planes, dtype):
+    y = rnd(*((t, h) if planes == 1 else (planes, t, h)), dtype=dtype, seed=1)
+    residual, after, weight = rnd(t, h, seed=2), rnd(h, seed=3), rnd(h, seed=4)
+    rows = torch.tensor([t - 1, 0], dtype=torch.int32, device=DEV)
+    for picked in (rows, None):
+        got_r, want_r = residual.clone(), residual.double()
+        got = ops.add_rmsnorm(got_r, y, weight, 1e-5, torch.float32, rows=picked, delta_norm=(after, 1e-6))
+        d = y.double().sum(0) if y.dim() == 3 else y.double()
+        d = d * torch.rsqrt(d.square().mean(-1, keepdim=True) + 1e-6) * after.double()
+        x = want_r + d
+        want = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5) * weight.double()
+        # elements of a few units, float32 sums of up to 4,100 squares: relative errors of 1e-6 or so
+        close(got, (want if picked is None else want[picked.long()]).float(), 2e-5, 2e-5)
+        close(got_r, (x if picked is None else want_r).float(), 1e-5, 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("t,h,n,top,how", [
+    (1, 64, 3, 2, {}),
+    (255, 260, 16, 2, {"scoring": "softmax_all", "groups": 4, "keep": 2, "group_score": "max"}),
+    (256, 260, 16, 2, {"scoring": "softmax_all", "groups": 4, "keep": 2, "group_score": "max"}),
+    (300, 2560, 16, 2, {}),
+    (263, 128, 64, 8, {"scoring": "sigmoid", "groups": 8, "keep": 3}),
+    (9, 128, 64, 64, {"scoring": "sigmoid"}),
+    (257, 96, 20, 3, {"scoring": "softmax_all", "renormalise": True, "weight_scale": 2.5, "corrected": True}),
+    (4, 128, 65, 4, {}),                              # beyond the lanes of a wave: the other kernel
+    (258, 64, 1, 1, {"gate_row": True}),
+    (2, 64, 6, 2, {"gate_row": True}),
+])
+def test_route_top(ops, dtype, t, h, n, top, how):
+    how = dict(how)
+    x = rnd(t, h, dtype=dtype, seed=1)
+    router = rnd(n + int(how.get("gate_row", False)), h, seed=2, scale=2.0 * h ** -0.5)
+    bias = rnd(n, seed=3)
+    if how.pop("corrected", False):
+        how["correction"] = 0.1 * rnd(n, seed=5)
+    got = ops.route_top(x, router, bias, top, **how)
+    want = R.route_top(x.double().float(), router, bias, top, **how)
+    # scores of this size differ between two orders of float32 sums by 1e-6: where two lie closer the choice may differ
+    same = (got[0].long() == want[0].long().to(DEV)).all(-1)
+    assert same.float().mean() > 0.99
+    close(got[1][same], want[1][same], 2e-5, 2e-5)
+    assert (got[0].sort(-1).values.diff(dim=-1) > 0).all()   # an expert is chosen once
+    if len(got) == 3:
+        close(got[2], want[2], 2e-5, 2e-5)
+
+
+def test_route_top_of_scores_that_are_no_numbers_stays_within_the_experts(ops):
+    x = rnd(300, 64, seed=1)
+    x[::3] = float("nan")
+    x[1::7, 5] = float("inf")
+    for n, top, how in ((16, 4, {}), (16, 2, {"scoring": "sigmoid", "groups": 4, "keep": 1}), (64, 64, {"scoring": "softmax_all"})):
+        for rows in (x, x[:4].contiguous()):
+            index, _ = ops.route_top(rows, rnd(n, 64, seed=2), None, top, **how)
+            assert index.min() >= 0 and index.max() < n
+            assert (index.sort(-1).values.diff(dim=-1) > 0).all()
+
+
+@pytest.mark.parametrize("t", [3, 600])
+@pytest.mark.parametrize("heads,width,pairs,in_stride,in_offset,out_stride,out_offset", [
+    (4, 128, 64, 128, 0, 128, 0), (3, 64, 8, 192, 128, 96, 16), (2, 40, 0, 40, 0, 48, 8), (5, 24, 12, 24, 0, 24, 0),
+])
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+def test_rotate_half(ops, t, heads, width, pairs, in_stride, in_offset, out_stride, out_offset, dtype, out_dtype):
+    x = rnd(t, heads * in_stride, dtype=dtype, seed=1)
+    freq = (1e4 ** -(torch.arange(pairs, dtype=torch.float32) / max(pairs, 1))).to(DEV) if pairs else None
+    positions = (torch.arange(t, dtype=torch.int32, device=DEV) * 37 + 5)
+    outs = [torch.full((t, heads * out_stride), 7.0, dtype=out_dtype, device=DEV) for _ in range(2)]
+    ops.rotate_half(x, in_stride, in_offset, outs[0], out_stride, out_offset, heads, width, positions, freq, magnitude=1.25)
+    R.rotate_half_copy(x, in_stride, in_offset, outs[1], out_stride, out_offset, heads, width, positions, freq, magnitude=1.25)
+    tol = 1e-2 if out_dtype == torch.bfloat16 else 2e-5
+    close(outs[0], outs[1], tol, tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 8), (3, 37), (1500, 1024)])
+def test_squared_relu(ops, dtype, shape):
+    x = rnd(*shape, dtype=dtype, seed=1)
+    assert torch.equal(ops.unary_act(x, "relu2"), x.float().clamp(min=0).square().to(dtype))
