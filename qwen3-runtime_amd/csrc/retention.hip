@@ -23,6 +23,7 @@
 // does not depend on how the tokens are cut into steps, tiles or batches.
 #include "common.h"
 #include <math.h>
+#include <type_traits>
 
 struct RetentionArgs {
   const void* qkv;        // [T, channels] float32, or (STEP) bfloat16
@@ -189,6 +190,272 @@ __global__ __launch_bounds__(256) void retention_kernel(RetentionArgs a) {
   }
 }
 
+// Prompts under a constant decay, in chunks of 32 tokens on float32 MFMA. With S the state in front of the
+// chunk, i and j tokens of the chunk and n how many it has:
+//
+//   o_i = d^(i+1) S^T q_i + sum over j <= i of d^(i-j) (k_j . q_i) v_j
+//   S  <- d^n S + sum over j of d^(n-1-j) k_j v_j^T
+//
+// Walked token by token the recurrence was bound by its chain: one wave a SIMD, 187 ns a token (32 heads of 128 x
+// 128, 2,047 tokens: 383 us). In chunks that case takes 160 us, 2.5 us a chunk, of which 1.1 are matrix products and the
+// rest the way from LDS through them and back to it (3 heads of 32: 314 -> 117; 16 of 256: 590 -> 273).
+// Error against 64 bits of the same case: 1.1e-7 to 1.4e-7 by the head's decay, walked 1.1e-7 to 3.9e-7.
+// A block owns 16 columns of one head's state, as above; each of its NW waves owns 16 G of the state's rows
+// in accumulators, and because all of o is linear in the sums over rows, a wave carries its share of both terms
+// through to the end (its scores are its rows' part of k . q), so that the waves meet once a chunk, in LDS. Operands
+// need no rearrangement: register r of an accumulator holds rows 4 (lane / 16) + r at column lane % 16, which as an operand is
+// the k-slice {r, 4 + r, 8 + r, 12 + r}; whoever meets it takes the same slice. Scores are formed as
+// K Q^T for that reason. Rows of 128 are 132 apart in LDS: 16-byte reads of 16 neighbouring rows and
+// 4-byte reads of 16 neighbouring elements of every fourth row both meet the banks evenly.
+// A sum that is masked must not meet an infinity of a later token (0 x inf): a chunk with a value that is not finite,
+// or so large that a score could overflow, goes through the same products one token at a time.
+// Powers are products of repeated squares, so any decay goes (negative, none at all), in double and kept in two
+// floats: a rounded d^32 would be off by the same part every chunk, which over a memory of 500 tokens made ten
+// times the error of the walk (3e-6 against 4e-7).
+constexpr int RC_TOKENS = 32, RC_VROW = 20;
+
+template <int G, int NW>
+__global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs a) {
+  constexpr int DP = 16 * G * NW, ROW = DP + 4, THREADS = 64 * NW;
+  constexpr int PIECES = RC_TOKENS * DP / 4 / THREADS;       // 16-byte pieces of q, and of k, a thread
+  constexpr int OWN = RC_TOKENS * RT_COLS / THREADS;         // values, and read-outs, a thread
+  __shared__ __attribute__((aligned(16))) float qs[RC_TOKENS * ROW];
+  __shared__ __attribute__((aligned(16))) float ks[RC_TOKENS * ROW];
+  __shared__ __attribute__((aligned(16))) float vs[RC_TOKENS * RC_VROW];
+  __shared__ __attribute__((aligned(16))) float red[NW][2][64 * 4];
+  __shared__ float powers[RC_TOKENS + 1], powers_rest[RC_TOKENS + 1];
+  __shared__ int odd[2];  // whether the chunk (of even, of odd number) holds a value for single tokens
+  const int seq = a.seq_ids ? a.seq_ids[blockIdx.x] : blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * RT_COLS;
+  const int t0 = a.cu_q[seq], t1 = a.cu_q[seq + 1];
+  if (t1 <= t0) return;
+  const int dim = a.dim, vdim = a.vdim, qk_head = head / a.share;
+  const int lane = threadIdx.x & 63, wave = uniform_wave_number(), r16 = lane & 15, quad = lane >> 4;
+  const float* qkv = (const float*)a.qkv;
+  if (threadIdx.x <= RC_TOKENS) {
+    double by = a.decay[head], p = 1.0;
+    for (int e = threadIdx.x; e; e >>= 1, by *= by)
+      if (e & 1) p *= by;
+    powers[threadIdx.x] = (float)p;
+    powers_rest[threadIdx.x] = (float)(p - (double)(float)p);
+  }
+  if (threadIdx.x < 2) odd[threadIdx.x] = 0;
+  float* st = a.state + (((size_t)a.state_slots[seq] * a.heads + head) * vdim + min(col0 + r16, vdim - 1)) * dim;
+  const bool col_ok = col0 + r16 < vdim;
+  f32x4_t s[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int d = 16 * (G * wave + g) + 4 * quad;
+    s[g] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    if (d < dim && col_ok) s[g] = *(const f32x4_t*)(st + d);
+  }
+  // the pieces of the next two chunks, on their way while one is walked (1.7 us a chunk; a load takes about one); what lies beyond the head or the tokens becomes
+  // zero only on its way to LDS: a choice here would wait for the loads
+  struct Ahead {
+    f32x4_t q[PIECES], k[PIECES];
+    float v[OWN];
+  };
+  auto fetch = [&](Ahead& to, int base) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int e = threadIdx.x + THREADS * i, tok = e / (DP / 4), d = 4 * (e % (DP / 4));
+      const float* row = qkv + (size_t)min(base + tok, t1 - 1) * a.channels + qk_head * dim + min(d, dim - 4);
+      to.q[i] = *(const f32x4_t*)(row + a.q_first);
+      to.k[i] = *(const f32x4_t*)(row + a.k_first);
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int e = threadIdx.x + THREADS * i, tok = e >> 4, c = col0 + (e & 15);
+      to.v[i] = qkv[(size_t)min(base + tok, t1 - 1) * a.channels + a.v_first + head * vdim + min(c, vdim - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // asked for here, not where they are used
+  };
+  __syncthreads();
+  float to_row[2][4], to_row_rest[2][4], back[2][4], back_rest[2][4], to_end[2][4], to_end_rest[2][4];  // d^(i+1); d^(i-j) by how many tiles apart; d^(n-1-j)
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * i + 4 * quad + r, diff = 16 * i + r16 - 4 * quad - r;
+      to_row[i][r] = powers[row + 1];
+      to_row_rest[i][r] = powers_rest[row + 1];
+      back[i][r] = powers[max(diff, 0)];
+      back_rest[i][r] = powers_rest[max(diff, 0)];
+    }
+  auto ends = [&](int n) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        to_end[i][r] = powers[max(n - 1 - (16 * i + 4 * quad + r), 0)];
+        to_end_rest[i][r] = powers_rest[max(n - 1 - (16 * i + 4 * quad + r), 0)];
+      }
+  };
+  ends(RC_TOKENS);
+  auto times = [](float x, float by, float rest) { return fmaf(x, by, x * rest); };
+  // one chunk from LDS: rows off .. off + n - 1; SINGLE: one row (n = 1), the others taken as zeros
+  f32x4_t o[2];
+  auto walk = [&](auto single, int off, int n) {
+    constexpr bool SINGLE = decltype(single)::value;
+    constexpr int TILES = SINGLE ? 1 : 2;
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    // all of the wave's operands first, and no further apart than that: left alone the compiler waits for LDS 14 times
+    f32x4_t q[TILES][G], k[TILES][G], kt[TILES][G], v[TILES], scores[TILES][TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int at = (off + (SINGLE ? 0 : 16 * j + r16)) * ROW + 16 * (G * wave + g) + 4 * quad;
+        q[j][g] = *(const f32x4_t*)(qs + at);
+        k[j][g] = *(const f32x4_t*)(ks + at);
+      }
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = off + (SINGLE ? 0 : 16 * j + 4 * quad + r);
+        v[j][r] = vs[row * RC_VROW + r16];
+#pragma unroll
+        for (int g = 0; g < G; ++g) kt[j][g][r] = ks[row * ROW + 16 * (G * wave + g) + r16];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (SINGLE) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (r16) q[0][g] = k[0][g] = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (quad || r) kt[0][g][r] = 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (quad || r) v[0][r] = 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {  // scores[i][j]: rows are keys, columns queries
+#pragma unroll
+      for (int i = j; i < TILES; ++i) {
+        f32x4_t sum = zero;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          f32x4_t acc = zero;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j][g][r], q[i][g][r], acc, 0, 0, 0);
+          sum = g ? sum + acc : acc;
+        }
+        scores[i][j] = sum;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        f32x4_t acc = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i][g][r], s[g][r], acc, 0, 0, 0);
+        o[i] = g ? o[i] + acc : acc;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] = times(o[i][r], to_row[i][r], to_row_rest[i][r]);
+    }
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+      for (int j = 0; j <= i; ++j) {
+        f32x4_t acc = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = i == j && r16 < 4 * quad + r ? 0.f : times(scores[i][j][r], back[i - j][r], back_rest[i - j][r]);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p, v[j][r], acc, 0, 0, 0);
+        }
+        o[i] += acc;
+      }
+    const float all = powers[n], rest = powers_rest[n];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[j][r] = times(v[j][r], to_end[j][r], to_end_rest[j][r]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      f32x4_t add[TILES];
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) {
+        add[j] = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) add[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[j][g][r], v[j][r], add[j], 0, 0, 0);
+      }
+      if (!SINGLE) add[0] += add[TILES - 1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[g][r] = fmaf(s[g][r], all, fmaf(s[g][r], rest, add[0][r]));
+    }
+  };
+  auto leave = [&](int base, int n) {  // the waves' sums meet, and the read-outs leave
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *(f32x4_t*)(red[wave][i] + lane * 4) = o[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      // token tok, column c: register tok % 4 of lane 16 (tok % 16 / 4) + c in tile tok / 16
+      const int e = threadIdx.x + THREADS * i, tok = e >> 4, c = e & 15, at = (16 * ((tok & 15) >> 2) + c) * 4 + (tok & 3);
+      double sum = 0.0;  // rounded once
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sum += red[w][tok >> 4][at];
+      if (tok < n && col0 + c < vdim) a.out[((size_t)(base + tok) * a.heads + head) * vdim + col0 + c] = (float)sum;
+    }
+  };
+  auto chunk = [&](Ahead& from, int base, int turn) {
+    const int n = min(RC_TOKENS, t1 - base);
+    bool large = false;
+    auto look = [&](float x) { large |= !(fabsf(x) < 1e12f); };
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int e = threadIdx.x + THREADS * i, tok = e / (DP / 4), d = 4 * (e % (DP / 4));
+      if (tok >= n || d >= dim) from.q[i] = from.k[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      *(f32x4_t*)(qs + tok * ROW + d) = from.q[i];
+      *(f32x4_t*)(ks + tok * ROW + d) = from.k[i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) look(from.q[i][r]), look(from.k[i][r]);
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int e = threadIdx.x + THREADS * i;
+      if ((e >> 4) >= n || col0 + (e & 15) >= vdim) from.v[i] = 0.f;
+      vs[(e >> 4) * RC_VROW + (e & 15)] = from.v[i];
+      look(from.v[i]);
+    }
+    if (large) odd[turn] = 1;
+    __syncthreads();
+    const bool one_by_one = odd[turn];
+    if (threadIdx.x == 0) odd[turn ^ 1] = 0;  // read last before the barrier in `leave` of the chunk before
+    if (base + 2 * RC_TOKENS < t1) fetch(from, base + 2 * RC_TOKENS);
+    if (!one_by_one) {
+      if (n < RC_TOKENS) ends(n);  // the last chunk
+      walk(std::false_type{}, 0, n);
+      leave(base, n);
+    } else {
+      ends(1);
+      for (int i = 0; i < n; ++i) {
+        o[1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        walk(std::true_type{}, i, 1);
+        leave(base + i, 1);
+        __syncthreads();
+      }
+      ends(RC_TOKENS);
+    }
+  };
+  Ahead first, second;
+  fetch(first, t0);
+  if (t0 + RC_TOKENS < t1) fetch(second, t0 + RC_TOKENS);
+  for (int base = t0; base < t1; base += 2 * RC_TOKENS) {
+    chunk(first, base, 0);
+    if (base + RC_TOKENS < t1) chunk(second, base + RC_TOKENS, 1);
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int d = 16 * (G * wave + g) + 4 * quad;
+    if (d < dim && col_ok) *(f32x4_t*)(st + d) = s[g];
+  }
+}
+
 extern "C" int qrt_retention(const RetentionArgs* args, int num_tokens, int num_seqs, int num_slots, hipStream_t stream) {
   RetentionArgs a = *args;
   QRT_CHECK(num_tokens >= 0 && num_seqs >= 0 && num_slots > 0, "retention: bad counts");
@@ -203,6 +470,18 @@ extern "C" int qrt_retention(const RetentionArgs* args, int num_tokens, int num_
   if (num_tokens == 0 || num_seqs == 0) return 0;
   const dim3 grid(num_seqs, a.heads, (a.vdim + (a.gates ? 1 : 0) + RT_COLS - 1) / RT_COLS);
   const int groups = (a.dim + 63) / 64;
+  // Prompts under a constant decay by chunks where a head's rows are whole pieces of 16 bytes (in `qkv` and in the
+  // state) and fit the waves' accumulators; steps of single tokens are one chunk each and gain nothing
+  // (8 sequences of one token: 10.0 us walked).
+  const bool pieces = a.dim % 4 == 0 && a.channels % 4 == 0 && a.q_first % 4 == 0 && a.k_first % 4 == 0 &&
+                      ((uintptr_t)a.qkv | (uintptr_t)a.state) % 16 == 0;
+  if (!a.gates && !a.step && groups <= 4 && pieces && num_tokens > 2 * num_seqs) {
+    if (groups == 1) retention_chunk_kernel<1, 4><<<grid, 256, 0, stream>>>(a);
+    else if (groups == 2) retention_chunk_kernel<1, 8><<<grid, 512, 0, stream>>>(a);
+    else retention_chunk_kernel<2, 8><<<grid, 512, 0, stream>>>(a);
+    QRT_LAUNCH_CHECK("retention (chunks)");
+    return 0;
+  }
 #define GO(G, TILE)                                                                 \
   do {                                                                              \
     if (a.gates && a.qkv_code == QRT_BF16) retention_kernel<G, TILE, RT_GATES, bf16_t><<<grid, 256, 0, stream>>>(a); \

@@ -1,0 +1,77 @@
+"""Retention over prompts by chunks of tokens: against the recurrence in float64, at the edges of chunks, heads and columns."""
+
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qwen3_runtime_amd.ops.hip import HipOps
+    return HipOps()
+
+
+def _draw(lengths, heads, dim, vdim, decay, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    t = sum(lengths)
+    qkv = torch.randn((t, 2 * heads * dim + heads * vdim), generator=g)
+    slots = torch.randperm(len(lengths) + 2, generator=g)[:len(lengths)].to(torch.int32)
+    state = torch.randn((len(lengths) + 2, heads, vdim, dim), generator=g)
+    return qkv, torch.tensor([decay[h % len(decay)] for h in range(heads)]), state, slots
+
+
+def _recurrence(lengths, qkv, decay, state, slots, heads, dim, vdim):
+    """Read-outs and states in float64, and for both the same sums over sizes (what rounding is relative to)."""
+    t = qkv.shape[0]
+    q, k, v = (x.double() for x in qkv.split([heads * dim, heads * dim, heads * vdim], 1))
+    q, k, v = q.view(t, heads, dim), k.view(t, heads, dim), v.view(t, heads, vdim)
+    state, out = state.double().clone(), torch.empty((t, heads, vdim), dtype=torch.float64)
+    sizes, out_sizes = state.abs(), torch.empty_like(out)
+    d, at = decay.double()[:, None, None], 0
+    for n, slot in zip(lengths, slots.tolist()):
+        for i in range(at, at + n):
+            state[slot] = d * state[slot] + v[i][:, :, None] * k[i][:, None, :]
+            sizes[slot] = d.abs() * sizes[slot] + v[i].abs()[:, :, None] * k[i].abs()[:, None, :]
+            out[i] = (state[slot] * q[i][:, None, :]).sum(-1)
+            out_sizes[i] = (sizes[slot] * q[i].abs()[:, None, :]).sum(-1)
+        at += n
+    return out, out_sizes, state, sizes
+
+
+def _run(ops, lengths, qkv, decay, state, slots, heads, dim, vdim):
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    ctx = types.SimpleNamespace(num_tokens=sum(lengths), num_seqs=len(lengths), cu_q=cu.cuda(), state_slots=slots.cuda())
+    state = state.cuda()
+    return ops.retention_rule(ctx, qkv.cuda(), decay.cuda(), state, heads, dim, vdim).cpu(), state.cpu()
+
+
+@pytest.mark.parametrize("dim,vdim,heads", [(4, 1, 2), (60, 16, 3), (64, 40, 2), (68, 17, 2), (128, 128, 4), (132, 16, 1), (256, 33, 2)])
+@pytest.mark.parametrize("lengths", [(3,), (31,), (32,), (33, 1, 64), (100, 7)])
+@pytest.mark.parametrize("decay", [(0.9, 0.5), (1.0, 0.0), (-0.7, 0.999)])
+def test_chunks_match_the_recurrence(ops, dim, vdim, heads, lengths, decay):
+    qkv, d, state, slots = _draw(lengths, heads, dim, vdim, decay)
+    out, out_sizes, states, sizes = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
+    got, after = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    # a term takes part in at most `longest` + dim additions and passes `longest` decays, each one rounding
+    steps = 2 * max(lengths) + dim + 8
+    assert ((got.double() - out).abs() <= steps * EPS * out_sizes).all()
+    assert ((after.double() - states).abs() <= steps * EPS * sizes).all()
+
+
+@pytest.mark.parametrize("which", ["k", "v", "q"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 1e30])
+def test_a_value_that_is_not_finite_stays_behind_its_token(ops, which, value):
+    heads, dim, vdim, lengths, at = 2, 64, 32, (70,), 41
+    qkv, d, state, slots = _draw(lengths, heads, dim, vdim, (0.9, 0.5))
+    qkv[at, {"q": 3, "k": heads * dim + 3, "v": 2 * heads * dim + 3}[which]] = value
+    out, out_sizes, _, _ = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
+    got, _ = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    steps = 2 * max(lengths) + dim + 8
+    assert ((got.double() - out).abs() <= steps * EPS * out_sizes)[:at].all()
+    fine = torch.isfinite(out) & (out.abs() < 3e38)
+    assert (torch.isfinite(got) == fine).all()
+    assert ((got.double() - out).abs() <= steps * EPS * out_sizes)[fine].all()
