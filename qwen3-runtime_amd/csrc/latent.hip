@@ -13,6 +13,7 @@
 //   takes the same two options;
 // * a product per head, out[t, h, :] = W[h] x[t, h, :], on strided rows: W [heads, N, K].
 #include "common.h"
+#include "direct.h"
 #include <math.h>
 
 // Element i of a vector whose first 2 `pairs` elements turn: its partner and the pair's number.
@@ -246,7 +247,7 @@ extern "C" int qrt_rotate_half(const RotateArgs* args, int in_dtype, int out_dty
 // ---------------------------------------------------------------- a product per head
 // One block of four waves per (token, head): the head's input in LDS as float32, each wave takes
 // outputs wave, wave + 4, ...; an output is one wave's sum over K in a fixed order, whatever else is
-// in the batch. For few tokens and for float32; many tokens in bfloat16 go to a batched library product.
+// in the batch. For float32 (few tokens: the kernel below).
 template <typename T>
 __global__ __launch_bounds__(256) void heads_linear_kernel(const T* __restrict__ x, long x_row, int in_stride, int in_offset,
                                                            const T* __restrict__ w, int n, int k, T* __restrict__ out,
@@ -329,13 +330,114 @@ __global__ __launch_bounds__(256) void heads_linear_rows_kernel(const T* __restr
   }
 }
 
+// bfloat16 with K a multiple of 64 and rows in whole pieces of 16 bytes: tiles of 128 tokens x BN outputs of a head on
+// MFMA, four waves, 64 k at a time in two LDS stages filled by direct loads of whole cache lines (piece c of row r at
+// 128 r + 16 (c ^ (r & 7)), as in the other tile kernels). K is one head's width, so a tile is two to six stages and
+// the pass is bound by its rows' way in and out: strided rows are read and written in place. A batched library
+// product on transposed weights and a copy of its result into the strided rows took 61 and 33 us for 32 heads of
+// 128 -> 384 and 384 -> 128 at 2,047 tokens; this kernel 26 and 16 (67 MB: 14 at the rate of a copy).
+// Neighbouring blocks of an XCD share a head's weights and a stretch of tokens.
+template <int BN>
+__global__ __launch_bounds__(256, 2) void heads_linear_tile_kernel(const bf16_t* __restrict__ x, long x_row, int in_stride, int in_offset,
+                                                                   const bf16_t* __restrict__ w, int heads, int n, int k,
+                                                                   bf16_t* __restrict__ out, long out_row, int out_stride, int out_offset,
+                                                                   int num_tokens) {
+  constexpr int STAGE = (128 + BN) * 128, LOADS = (128 + BN) / 32, WN = BN / 2, JT = BN / 32;
+  extern __shared__ __align__(16) unsigned char lds[];  // [2][128 tokens | BN weight rows] x 128 bytes
+  const int col_tiles = (n + BN - 1) / BN, row_tiles = (num_tokens + 127) / 128;
+  const int total = heads * col_tiles * row_tiles, per = (total + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
+  const int h = tile / (col_tiles * row_tiles), rest = tile % (col_tiles * row_tiles);
+  const int t0 = rest / col_tiles * 128, n0 = rest % col_tiles * BN;
+  const int lane = threadIdx.x & 63, wave = uniform_wave_number();
+  const int r16 = lane & 15, quad = lane >> 4, wm = (wave >> 1) * 64, wn = (wave & 1) * WN;
+  const int sub = lane >> 3, piece = (lane & 7) ^ sub;
+  // a wave's loads of a stage, 8 rows x 128 bytes each; rows past the end repeat the last and are not stored
+  const bf16_t* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = (wave * LOADS + i) * 8 + sub;
+    src[i] = r < 128 ? x + (size_t)min(t0 + r, num_tokens - 1) * x_row + (size_t)h * in_stride + in_offset + 8 * piece
+                     : w + ((size_t)h * n + min(n0 + r - 128, n - 1)) * k + 8 * piece;
+  }
+  unsigned char* dst = lds + wave * LOADS * 1024;
+  auto fetch = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[i] + (size_t)s * 64), (lds_ptr_t)(dst + (s & 1) * STAGE + i * 1024), 16, 0, 0);
+  };
+  f32x4_t acc[4][JT];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < JT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const int stages = k >> 6;
+  fetch(0);
+  for (int s = 0; s < stages; ++s) {
+    if (s + 1 < stages) {
+      fetch(s + 1);
+      QRT_WAIT_LOADS(LOADS);
+    } else {
+      QRT_WAIT_LOADS(0);
+    }
+    QRT_BARRIER();
+    const unsigned char* at = lds + (s & 1) * STAGE;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int col = 16 * ((4 * e + quad) ^ (r16 & 7));
+      bf16x8_t xv[4], wv[JT];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xv[i] = *(const bf16x8_t*)(at + (wm + 16 * i + r16) * 128 + col);
+#pragma unroll
+      for (int j = 0; j < JT; ++j) wv[j] = *(const bf16x8_t*)(at + (128 + wn + 16 * j + r16) * 128 + col);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < JT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], xv[i], acc[i][j], 0, 0, 0);
+    }
+    QRT_WAIT_LDS();  // read before the barrier behind which the stage may be overwritten
+    QRT_BARRIER();
+  }
+  // acc[i][j]: token t0 + wm + 16 i + r16, four outputs from n0 + wn + 16 j + 4 quad on
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = t0 + wm + 16 * i + r16;
+    if (t >= num_tokens) continue;
+    bf16_t* o = out + (size_t)t * out_row + (size_t)h * out_stride + out_offset;
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      const int c = n0 + wn + 16 * j + 4 * quad;
+      if (c >= n) continue;  // n is a multiple of 4: four or none
+      bf16x4_t v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = from_f32<bf16_t>(acc[i][j][r]);
+      *(bf16x4_t*)(o + c) = v;
+    }
+  }
+}
+
 extern "C" int qrt_heads_linear(const void* x, long x_row, int in_stride, int in_offset, const void* w, int heads, int n, int k,
-                                void* out, long out_row, int out_stride, int out_offset, int dtype, int num_tokens,
+                                void* out, long out_row, int out_stride, int out_offset, int dtype, int num_tokens, int tiles,
                                 hipStream_t stream) {
   QRT_CHECK(num_tokens >= 0 && heads > 0 && heads <= 65535 && n > 0 && k > 0 && k <= 16384, "heads_linear: bad sizes");
   QRT_CHECK(in_offset >= 0 && in_offset + k <= in_stride && (long)heads * in_stride <= x_row && out_offset >= 0 &&
             out_offset + n <= out_stride && (long)heads * out_stride <= out_row, "heads_linear: heads do not fit their rows");
   if (num_tokens == 0) return 0;
+  if (tiles) {
+    QRT_CHECK(dtype == QRT_BF16 && k % 64 == 0 && n % 4 == 0 && (x_row | in_stride | in_offset) % 8 == 0 &&
+                  (out_row | out_stride | out_offset) % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0 && (uintptr_t)out % 8 == 0,
+              "heads_linear: rows of the tile kernel are whole pieces of 16 bytes");
+    const bool narrow = n <= 64;
+    const long blocks = (long)heads * ((n + (narrow ? 63 : 127)) / (narrow ? 64 : 128)) * ((num_tokens + 127) / 128);
+    QRT_CHECK(blocks < (1l << 30), "heads_linear: too many tiles");
+    const unsigned grid = (unsigned)((blocks + 7) / 8 * 8);
+    auto kernel = narrow ? heads_linear_tile_kernel<64> : heads_linear_tile_kernel<128>;
+    kernel<<<grid, 256, narrow ? 48 * 1024 : 64 * 1024, stream>>>((const bf16_t*)x, x_row, in_stride, in_offset, (const bf16_t*)w, heads, n, k,
+                                                                  (bf16_t*)out, out_row, out_stride, out_offset, num_tokens);
+    QRT_LAUNCH_CHECK("heads_linear_tile");
+    return 0;
+  }
   if (num_tokens <= 64 && k <= 1024) {  // the head's weights once a step
     const dim3 rows_grid((n + 63) / 64, heads);
     const size_t rows_lds = (size_t)(HL_TOKENS * k + 4 * HL_TOKENS * 64) * sizeof(float);

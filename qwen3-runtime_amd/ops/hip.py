@@ -508,7 +508,10 @@ class HipOps:
         self._check(self.lib, self.lib.qrt_rotate_half(byref(a), _CODE[x.dtype], _CODE[out.dtype], c_int(t), _stream()))
         return out
 
-    # bfloat16 steps with more tokens than this take the per-head products to the vendor library
+    # bfloat16 steps with more tokens than this whose rows are no whole pieces of 16 bytes take the per-head products
+    # to the vendor library (its right operand copied: transposed views of batches have faulted there); rows that
+    # are take the tile kernel at any number of tokens, which is faster than both (at 1 to 16 tokens 4.4 and
+    # 6.7 us against 5.1 to 8.4 and 9.0 to 18.3 of the kernel for few rows; at 33, 4.8 and 7.1 against 10.3 and 11.6)
     heads_linear_own_max_rows = 16
 
     def heads_linear(self, x, in_stride, in_offset, w, out, out_stride, out_offset):
@@ -522,15 +525,18 @@ class HipOps:
         if (heads * in_stride > x.shape[1] or in_offset + k > in_stride or heads * out_stride > out.shape[1]
                 or out_offset + n > out_stride):
             raise OpsError(f"heads_linear: {heads} heads of {in_stride} in rows of {x.shape[1]}, of {out_stride} in rows of {out.shape[1]}")
-        if x.dtype == torch.bfloat16 and t > self.heads_linear_own_max_rows:
+        tiles = (x.dtype == torch.bfloat16 and k % 64 == 0 and n % 4 == 0 and (x.shape[1] | in_stride | in_offset) % 8 == 0
+                 and (out.shape[1] | out_stride | out_offset) % 4 == 0
+                 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0)
+        if not tiles and x.dtype == torch.bfloat16 and t > self.heads_linear_own_max_rows:
             src = x.view(t, -1)[:, : heads * in_stride].view(t, heads, in_stride)[:, :, in_offset: in_offset + k]
-            res = torch.bmm(src.transpose(0, 1), w.transpose(1, 2))  # [heads, T, N]
+            res = torch.bmm(src.transpose(0, 1), w.transpose(1, 2).contiguous())  # [heads, T, N]
             out.view(t, -1)[:, : heads * out_stride].view(t, heads, out_stride)[:, :, out_offset: out_offset + n] = \
                 res.transpose(0, 1)
             return out
         self._check(self.lib, self.lib.qrt_heads_linear(
             _ptr(x), c_long(x.shape[1]), c_int(in_stride), c_int(in_offset), _ptr(w), c_int(heads), c_int(n), c_int(k),
-            _ptr(out), c_long(out.shape[1]), c_int(out_stride), c_int(out_offset), _CODE[x.dtype], c_int(t), _stream()))
+            _ptr(out), c_long(out.shape[1]), c_int(out_stride), c_int(out_offset), _CODE[x.dtype], c_int(t), c_int(tiles), _stream()))
         return out
 
     def retention_prepare(self, y, heads, dim, vdim, positions, freq, k_scale):

@@ -99,3 +99,25 @@ def test_rotate_half(ops, t, heads, width, pairs, in_stride, in_offset, out_stri
 def test_squared_relu(ops, dtype, shape):
     x = rnd(*shape, dtype=dtype, seed=1)
     assert torch.equal(ops.unary_act(x, "relu2"), x.float().clamp(min=0).square().to(dtype))
+
+
+@pytest.mark.parametrize("tokens", [1, 16, 17, 128, 129, 300])
+@pytest.mark.parametrize("heads,n,k,in_stride,in_offset,out_stride,out_offset",
+                         [(3, 4, 64, 64, 0, 4, 0), (2, 60, 128, 160, 24, 72, 8), (4, 384, 128, 192, 0, 448, 0),
+                          (2, 132, 64, 72, 8, 136, 4), (5, 128, 384, 448, 64, 128, 0), (2, 64, 100, 104, 0, 64, 0), (2, 30, 64, 64, 0, 33, 3)])
+def test_heads_linear_by_tiles(ops, tokens, heads, n, k, in_stride, in_offset, out_stride, out_offset):
+    g = torch.Generator().manual_seed(tokens + n + k)
+    x = torch.randn((tokens, heads * in_stride), generator=g).bfloat16()
+    w = torch.randn((heads, n, k), generator=g).bfloat16()
+    out = torch.full((tokens, heads * out_stride), 7.0).bfloat16()
+    got = ops.heads_linear(x.cuda(), in_stride, in_offset, w.cuda(), out.cuda(), out_stride, out_offset).cpu().double()
+    part = x.double().view(tokens, heads, in_stride)[:, :, in_offset: in_offset + k]
+    want = torch.einsum("thk,hnk->thn", part, w.double())
+    sizes = torch.einsum("thk,hnk->thn", part.abs(), w.double().abs())
+    got = got.view(tokens, heads, out_stride)
+    # k rounded additions in float32 and one rounding to bfloat16
+    here = got[:, :, out_offset: out_offset + n]
+    assert ((here - want).abs() <= k * 2.0 ** -24 * sizes + 2.0 ** -8 * want.abs() + 1e-30).all()
+    outside = torch.ones(out_stride, dtype=torch.bool)
+    outside[out_offset: out_offset + n] = False
+    assert (got[:, :, outside] == 7.0).all()
