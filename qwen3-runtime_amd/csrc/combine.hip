@@ -200,8 +200,9 @@ __global__ __launch_bounds__(1024) void norm_add_rmsnorm_kernel(float* __restric
   }
 }
 
-// VEC neighbouring elements of a sub-layer output, float32
-template <int VEC>
+// VEC neighbouring elements of a sub-layer output, float32. TWO: two planes have a way of their own (the routed
+// experts' outputs), where a kernel takes one output alone: with several, the branches' masks spill.
+template <int VEC, bool TWO = false>
 __device__ __forceinline__ void planes_piece(const Planes& y, size_t i, float* v) {
   typedef float fvec_t __attribute__((ext_vector_type(VEC)));
   typedef bf16_t bvec_t __attribute__((ext_vector_type(VEC)));
@@ -218,7 +219,7 @@ __device__ __forceinline__ void planes_piece(const Planes& y, size_t i, float* v
     for (int e = 0; e < VEC; ++e) v[e] = x[e];
     return;
   }
-  if (y.planes == 2) {
+  if (TWO && y.planes == 2) {
     const fvec_t a = *(const fvec_t*)(p + i), b = *(const fvec_t*)(p + y.plane_stride + i);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) v[e] = a[e] + b[e];
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(THREADS) void norm_add_rmsnorm_wide_kernel(float* _
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     const int i = min((int)threadIdx.x * 4 + j * STRIDE, hidden - 4);  // beyond the row: its last piece, dropped below
-    planes_piece<4>(y, row + i, vy[j]);
+    planes_piece<4, true>(y, row + i, vy[j]);
     vx[j] = *(const f32x4_t*)(residual + row + i);
     wa[j] = *(const f32x4_t*)(w_after + i);
     wn[j] = *(const f32x4_t*)(weight + i);
