@@ -121,3 +121,29 @@ def test_heads_linear_by_tiles(ops, tokens, heads, n, k, in_stride, in_offset, o
     outside = torch.ones(out_stride, dtype=torch.bool)
     outside[out_offset: out_offset + n] = False
     assert (got[:, :, outside] == 7.0).all()
+
+
+@pytest.mark.parametrize("tokens,heads,vdim", [(1, 1, 8), (3, 5, 24), (7, 3, 128), (33, 2, 512), (5, 2, 520), (65, 3, 40)])
+@pytest.mark.parametrize("gate_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("kind", ["silu", "sigmoid"])
+def test_read_out_norm_and_gate_in_pieces(ops, tokens, heads, vdim, gate_dtype, out_dtype, kind):
+    g = torch.Generator().manual_seed(tokens + vdim)
+    o, w = torch.randn((tokens, heads, vdim), generator=g), torch.randn(vdim, generator=g)
+    wide = torch.randn((tokens, heads * vdim + 16), generator=g).to(gate_dtype)
+    got = ops.delta_out(o.cuda(), w.cuda(), wide.cuda()[:, 8: 8 + heads * vdim], 1e-5, kind, out_dtype).double().cpu()
+    z = wide[:, 8: 8 + heads * vdim].double().view(tokens, heads, vdim)
+    act = torch.sigmoid(z) * (z if kind == "silu" else 1.0)
+    want = (o.double() / (o.double().pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double() * act).reshape(tokens, -1)
+    # float32 on the way: a dozen roundings, the exponential of an argument up to 6; bfloat16: half of 2^-7
+    rel = 40 * 2.0 ** -24 + (2.0 ** -8 if out_dtype == torch.bfloat16 else 0.0)
+    assert ((got - want).abs() <= rel * want.abs() * 1.01 + 1e-30).all()
+
+
+@pytest.mark.parametrize("tokens,width,first", [(1, 8, 8), (3, 40, 16), (65, 4096, 8), (5, 24, 4), (4, 30, 8)])
+def test_sigmoid_gate_in_pieces(ops, tokens, width, first):
+    g = torch.Generator().manual_seed(width)
+    out = torch.randn((tokens, width), generator=g).bfloat16()
+    wide = (3 * torch.randn((tokens, width + 24), generator=g)).bfloat16()
+    got = ops.sigmoid_gate(out.cuda(), wide.cuda()[:, first: first + width]).double().cpu()
+    want = out.double() * torch.sigmoid(wide[:, first: first + width].double())
+    assert ((got - want).abs() <= (2.0 ** -8 * 1.01 + 40 * 2.0 ** -24) * want.abs()).all()
