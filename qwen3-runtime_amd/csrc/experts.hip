@@ -16,7 +16,7 @@
 //   puts the pairs in their experts' order and lists the tiles.
 //
 // What they replace (MI355X, 16 experts of 2,560 x 1,536, 2 a token; us): a kernel of scalar products on LDS
-// copies of a few rows, 58 + 27 and a grouping and a combining kernel of 4.5 + 8.9 for 8 tokens; one library
+// copies of a few rows, 58 + 27 and a grouping and a combining kernel of 4.5 + 8.9 for 8 tokens (now 28 + 17); one library
 // product per expert and matrix behind a wait of the host, about 430 for 2,041 tokens, with the device idle for a
 // sixth of the step.
 #include "common.h"
@@ -50,7 +50,12 @@ __device__ __forceinline__ float expert_value(const ExpertArgs& a, float g, floa
 }
 
 // ------------------------------------------------------------------ few pairs an expert
-// blockIdx.x: the expert, or (BY_PAIR: fewer pairs than experts) the pair that is its expert's first.
+// blockIdx.y: the expert, or (BY_PAIR: fewer pairs than experts) the pair that is its expert's first. The weight rows are
+// blockIdx.x: blocks go to the eight XCDs in turn, and with the experts there an XCD had the work of experts e and e + 8
+// (of 16), two, one or none of which are chosen (16 x 2,560 x 1,536, 8 tokens, some 10 of 16 chosen: 34.9 + 22.2 us, now 31.0 +
+// 19.6). The weights are loaded as data used once, as in the few-row dense products (27.7 + 16.6 with that and the smallest rings:
+// 16 rows and two pieces in flight a wave, three or four blocks a compute unit; 80 tokens, where an expert's weights come
+// again from the caches: 49.1 + 29.4 -> 42.5 + 26.9).
 template <int NW, int NT, int U, int MODE, bool BY_PAIR>
 __global__ __launch_bounds__(64 * NW) void experts_rows_kernel(ExpertArgs a) {
   constexpr bool GATED = MODE == EXPERTS_GATED;
@@ -60,7 +65,7 @@ __global__ __launch_bounds__(64 * NW) void experts_rows_kernel(ExpertArgs a) {
   int* list = (int*)(lds + NW * U * SLOT);
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int pairs = a.tokens * a.top, K = a.K, N = a.N;
-  const int e = BY_PAIR ? a.index[blockIdx.x] : blockIdx.x;
+  const int e = BY_PAIR ? a.index[blockIdx.y] : blockIdx.y;
   // the expert's pairs in ascending order; every wave writes the same list
   int count = 0;
   for (int p0 = 0; p0 < pairs; p0 += 64) {
@@ -72,8 +77,8 @@ __global__ __launch_bounds__(64 * NW) void experts_rows_kernel(ExpertArgs a) {
   }
   __syncthreads();
   count = __builtin_amdgcn_readfirstlane(count);
-  if (count == 0 || (BY_PAIR && list[0] != (int)blockIdx.x)) return;  // the whole block alike
-  const int r16 = lane & 15, quad = lane >> 4, n0 = blockIdx.y * 16 * NT;
+  if (count == 0 || (BY_PAIR && list[0] != (int)blockIdx.y)) return;  // the whole block alike
+  const int r16 = lane & 15, quad = lane >> 4, n0 = blockIdx.x * 16 * NT;
   unsigned char* ring = lds + (size_t)wave * U * SLOT;
   const int sub = lane >> 3, piece = (lane & 7) ^ sub;
   const bf16_t* we = a.w + (size_t)e * (GATED ? 2 : 1) * N * K;
@@ -98,8 +103,12 @@ __global__ __launch_bounds__(64 * NW) void experts_rows_kernel(ExpertArgs a) {
 #pragma unroll
       for (int un = 0; un < UNITS; ++un)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          __builtin_amdgcn_global_load_lds((global_ptr_t)(src[un][j] + at), (lds_ptr_t)(dst + un * 2048 + j * 1024), 16, 0, 0);
+        for (int j = 0; j < 2; ++j) {
+          if (un < WT)
+            __builtin_amdgcn_global_load_lds((global_ptr_t)(src[un][j] + at), (lds_ptr_t)(dst + un * 2048 + j * 1024), 16, 0, 2);
+          else
+            __builtin_amdgcn_global_load_lds((global_ptr_t)(src[un][j] + at), (lds_ptr_t)(dst + un * 2048 + j * 1024), 16, 0, 0);
+        }
     };
     f32x4_t acc[WT];
 #pragma unroll
@@ -302,7 +311,7 @@ static int experts_rows_launch(const ExpertArgs& a, hipStream_t stream) {
   static bool allowed = false;  // once per kernel: not inside a stream capture again and again
   if (!allowed && !lds_allowed((const void*)kernel, 160 * 1024)) return qrt_fail("experts: cannot get 160 KB of LDS");
   allowed = true;
-  kernel<<<dim3(BY_PAIR ? pairs : a.experts, (a.N + 16 * NT - 1) / (16 * NT)), 64 * NW, smem, stream>>>(a);
+  kernel<<<dim3((a.N + 16 * NT - 1) / (16 * NT), BY_PAIR ? pairs : a.experts), 64 * NW, smem, stream>>>(a);
   return 0;
 }
 template <int NT, int U, int MODE>
@@ -351,11 +360,11 @@ extern "C" int qrt_experts(const void* x, const void* gate_up, const void* down,
   a.K = hidden; a.N = inter;
   int rc;
   if (act_kind == QRT_ACT_RELU2) rc = scratch ? experts_tile_launch<EXPERTS_RELU2>(a, stream) : experts_rows<2, 3, EXPERTS_RELU2>(a, stream);
-  else rc = scratch ? experts_tile_launch<EXPERTS_GATED>(a, stream) : experts_rows<1, 3, EXPERTS_GATED>(a, stream);
+  else rc = scratch ? experts_tile_launch<EXPERTS_GATED>(a, stream) : experts_rows<1, 2, EXPERTS_GATED>(a, stream);
   if (rc != 0) return rc;
   a.in = (const bf16_t*)act; a.w = (const bf16_t*)down; a.weight = weight_on_input ? nullptr : weight; a.out = out;
   a.K = inter; a.N = hidden;
-  rc = scratch ? experts_tile_launch<EXPERTS_DOWN>(a, stream) : experts_rows<2, 2, EXPERTS_DOWN>(a, stream);
+  rc = scratch ? experts_tile_launch<EXPERTS_DOWN>(a, stream) : experts_rows<1, 2, EXPERTS_DOWN>(a, stream);
   if (rc != 0) return rc;
   QRT_LAUNCH_CHECK("experts");
   return 0;
