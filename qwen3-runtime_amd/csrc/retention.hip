@@ -20,7 +20,8 @@
 // of 16 lanes. Tokens are staged through LDS 16 at a time; the next tile's global loads are in
 // flight while a tile is walked, the walk has no global access and no branch between tokens, and
 // the tile's read-outs leave together afterwards. The order of the float32 operations per token
-// does not depend on how the tokens are cut into steps, tiles or batches.
+// does not depend on how the tokens are cut into steps, tiles or batches. (Retention over prompts goes by
+// chunks instead: see retention_chunk_kernel.)
 #include "common.h"
 #include <math.h>
 #include <type_traits>

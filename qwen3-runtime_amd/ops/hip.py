@@ -6,7 +6,7 @@ current stream through ``ctypes``. There is no other implementation: if the
 library cannot be built or loaded, construction fails. Tensors are torch
 tensors on the GPU; outputs are allocated with torch's caching allocator.
 
-Matrix products: float32 goes to the library's own fused-multiply-add kernel
+Matrix products: float32 goes to the library's own float32 MFMA kernels
 (true 32-bit). bfloat16 with up to 64 rows (128 for the gated product and for
 products cut along K) goes to the library's MFMA kernels, which stream the
 weights; bfloat16 with more rows goes to the vendor BLAS through
