@@ -37,6 +37,7 @@ struct AttnArgs {
   const float* turn;  // [T, Dv] or null: cosines of the token's Dv / 2 angles, then their sines; the output is turned back by them
   const int* cu_q;    // [S + 1] or null: first token of every sequence (the tile kernel goes by it)
   int num_seqs, max_q_len;  // sequences, and the most tokens one brings
+  int min_q_len;            // the fewest (0: not known)
 };
 
 #define MAX_D 1024
@@ -146,7 +147,13 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
 // the row's maximum. The kernel before it (a wave per token and head, a key's dot product per lane,
 // uncoalesced) is bound by load latency: 354 tokens of 2 sequences with 32 heads of 128 took 798 us, two
 // decoded tokens behind 267 keys 170 us; this one 43 and 25 us.
+// A sequence of few rows has eight waves a tile (its keys are what there is to share: a token behind 2,049 keys with
+// 32 heads of 128 on 8 takes 78 us, with four 161), any other four (16 prompts of 64 tokens 60 us, with eight 105); heads wider than
+// 128 always eight (2,048 tokens, 16 heads of 256 on 4: 910 us, with four 1,440). That goes by
+// the sequence's own rows, and a block of keys goes to the wave of its number in the sequence, so that neither what shares
+// a step nor a tile changes a sum's order.
 // Head sizes in multiples of 16 up to 256, pages of a multiple of 4 keys; other sizes keep the kernel above.
+#define F32_FEW_ROWS 64
 template <int ND, int W>
 __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) {
   __shared__ __align__(16) f32x4_t hand[W > 1 ? W / 2 : 1][ND * 64];  // accumulators on their way from wave to wave
@@ -155,7 +162,7 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   const int r = lane & 15, q = lane >> 4;
   const int s = blockIdx.z, kvh = blockIdx.y, g = a.nq / a.nkv;
   const int t0 = a.cu_q[s], rows = (a.cu_q[s + 1] - t0) * g, row0 = blockIdx.x * 16;
-  if (row0 >= rows) return;  // the whole block alike
+  if (row0 >= rows || (ND < 16 && (rows <= F32_FEW_ROWS) != (W == 8))) return;  // the whole block alike
   const int D = a.head_dim, Dv = a.value_dim, ps = a.page_size, nd = D >> 4, nv = Dv >> 4;
   const int last_row = min(row0 + 15, rows - 1), rr = min(row0 + r, last_row);
   const int t = t0 + rr / g, h = kvh * g + rr % g;
@@ -165,8 +172,8 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   const int lo0 = a.window > 0 ? max(0, pos0 - a.window + 1) : (a.chunk > 0 ? pos0 - pos0 % a.chunk : 0);
   const int keep = a.window > 0 ? a.keep_first : 0;
   // blocks of 16 keys: the kept first ones that lie before the window's, then from the first row's first key on
-  const int main0 = lo0 >> 4, kept = min((keep + 15) >> 4, main0);
-  const int blocks = __builtin_amdgcn_readfirstlane(kept + (hi >> 4) - main0 + 1);
+  const int main0 = __builtin_amdgcn_readfirstlane(lo0 >> 4), kept = min((keep + 15) >> 4, main0);
+  const int last_block = __builtin_amdgcn_readfirstlane(hi >> 4);
 
   f32x4_t qv[ND], acc[ND];
   const float* qr = (const float*)a.q + ((size_t)t * a.nq + h) * D + 4 * q;
@@ -178,8 +185,10 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   float m = -INFINITY, l = 0.f;
   const float* kc = (const float*)a.k_cache;
   const float* vc = (const float*)a.v_cache;
-  for (int i = wave; i < blocks; i += W) {
-    const int j0 = 16 * (i < kept ? i : main0 + i - kept);
+  // a wave's blocks are those of its number modulo W
+  for (int b = wave < kept ? wave : main0 + ((wave - main0) & (W - 1)); b <= last_block;
+       b = b + W < kept || b >= main0 ? b + W : main0 + ((wave - main0) & (W - 1))) {
+    const int j0 = 16 * b;
     // K: the lane's key j0 + r; V: its keys j0 + 4 q .. + 3 (one page). Places after the last key, and pages
     // that were given back, are read as the sequence's last key (its page is there) and count for nothing
     const int kj = min(j0 + r, hi), vj = j0 + 4 * q;
@@ -292,13 +301,16 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   }
 }
 
-// Eight waves a row tile where tiles are few (decoding: the keys are what there is to share), four otherwise.
 template <int ND>
 static void attention_f32_tiles(const AttnArgs& a, hipStream_t stream) {
-  const int tiles = (int)(((long)a.max_q_len * (a.nq / a.nkv) + 15) / 16);
-  dim3 grid(tiles, a.nkv, a.num_seqs);
-  if ((long)tiles * a.nkv * a.num_seqs <= 512) attention_f32_tile_kernel<ND, 8><<<grid, 512, 0, stream>>>(a);
-  else attention_f32_tile_kernel<ND, 4><<<grid, 256, 0, stream>>>(a);
+  const long g = a.nq / a.nkv;
+  const auto grid = [&](long rows) { return dim3((unsigned)((rows + 15) / 16), a.nkv, a.num_seqs); };
+  if constexpr (ND >= 16) {
+    attention_f32_tile_kernel<ND, 8><<<grid(a.max_q_len * g), 512, 0, stream>>>(a);
+  } else {  // sequences of both kinds: both kernels, each leaves the other's alone
+    if (a.min_q_len * g <= F32_FEW_ROWS) attention_f32_tile_kernel<ND, 8><<<grid(min(a.max_q_len * g, (long)F32_FEW_ROWS)), 512, 0, stream>>>(a);
+    if (a.max_q_len * g > F32_FEW_ROWS) attention_f32_tile_kernel<ND, 4><<<grid(a.max_q_len * g), 256, 0, stream>>>(a);
+  }
 }
 
 extern "C" int qrt_attention_f32(const AttnArgs* args, int dtype, hipStream_t stream) {

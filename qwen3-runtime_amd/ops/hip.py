@@ -56,7 +56,7 @@ class _AttnArgs(Structure):
         ("head_dim", c_int), ("page_size", c_int), ("window", c_int), ("scale", c_float),
         ("chunk", c_int), ("softcap", c_float), ("value_dim", c_int), ("gate", c_void_p), ("gate_stride", c_long),
         ("keep_first", c_int), ("sink", c_int), ("turn", c_void_p),
-        ("cu_q", c_void_p), ("num_seqs", c_int), ("max_q_len", c_int),
+        ("cu_q", c_void_p), ("num_seqs", c_int), ("max_q_len", c_int), ("min_q_len", c_int),
     ]
 
 
@@ -1547,7 +1547,7 @@ class HipOps:
             a.keep_first, a.sink = int(keep_first), int(bool(sink))
             a.turn = _addr(self._turn_table(ctx, value_turn, dv))
             a.cu_q = _need(ctx.cu_q, "cu_q", torch.int32, (ctx.num_seqs + 1,)).data_ptr()
-            a.num_seqs, a.max_q_len = ctx.num_seqs, ctx.max_q_len
+            a.num_seqs, a.max_q_len, a.min_q_len = ctx.num_seqs, ctx.max_q_len, min(ctx.q_lens_host, default=0)
             self._check(self.lib, self.lib.qrt_attention_f32(byref(a), _CODE[q.dtype], _stream()))
         return out
 
