@@ -42,24 +42,30 @@ struct AttnArgs {
 
 #define MAX_D 1024
 
-template <typename T>
-__global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
-  __shared__ float qs[MAX_D];
-  const int lane = threadIdx.x;
-  const int t = blockIdx.x, h = blockIdx.y;
+// What a wave wrote to its own LDS is there for all of its lanes.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One token's head, by one wave; `qs`: MD floats of LDS of its own (heads and values of up to MD elements).
+template <typename T, int MD>
+__device__ __forceinline__ void attend_row(const AttnArgs& a, int t, int h, float* qs) {
+  const int lane = threadIdx.x & 63;
   const int D = a.head_dim, ps = a.page_size, Dv = a.value_dim;
   const int kvh = h / (a.nq / a.nkv);
   const int pos = a.positions[t];
   const int* table = a.block_table + (size_t)a.seq_of_token[t] * a.table_width;
   const T* q = (const T*)a.q + ((size_t)t * a.nq + h) * D;
   for (int i = lane; i < D; i += 64) qs[i] = to_f32<T>(q[i]);
-  __syncthreads();
+  wave_lds_fence();
 
   const int lo = a.window > 0 ? max(0, pos - a.window + 1) : (a.chunk > 0 ? pos - pos % a.chunk : 0);
   float m = -INFINITY, l = 0.f;
-  float acc[MAX_D / 64];
+  float acc[(MD + 63) / 64];
 #pragma unroll
-  for (int i = 0; i < MAX_D / 64; ++i) acc[i] = 0.f;
+  for (int i = 0; i < (MD + 63) / 64; ++i) acc[i] = 0.f;
 
   const T* kc = (const T*)a.k_cache;
   const T* vc = (const T*)a.v_cache;
@@ -87,7 +93,7 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
     l = l * corr + wave_sum(p);
     m = m_new;
 #pragma unroll
-    for (int i = 0; i < MAX_D / 64; ++i) acc[i] *= corr;
+    for (int i = 0; i < (MD + 63) / 64; ++i) acc[i] *= corr;
     const int n = min(64, seg_last - j0 + 1);
     for (int jj = 0; jj < n; ++jj) {
       const float pj = __shfl(p, jj, 64);
@@ -95,7 +101,7 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
       const int of = __shfl(off, jj, 64);
       const T* vr = vc + ((size_t)pg * a.nkv + kvh) * Dv * ps + of;
 #pragma unroll
-      for (int i = 0; i < MAX_D / 64; ++i) {
+      for (int i = 0; i < (MD + 63) / 64; ++i) {
         const int d = lane + 64 * i;
         if (d < Dv) acc[i] = fmaf(pj, to_f32<T>(vr[(size_t)d * ps]), acc[i]);
       }
@@ -107,21 +113,21 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
     const float corr = expf(m - m_new);
     l = l * corr + expf(-m_new);
 #pragma unroll
-    for (int i = 0; i < MAX_D / 64; ++i) acc[i] *= corr;
+    for (int i = 0; i < (MD + 63) / 64; ++i) acc[i] *= corr;
   }
   T* o = (T*)a.out + ((size_t)t * a.nq + h) * Dv;
   const T* gate = a.gate ? (const T*)a.gate + (size_t)t * a.gate_stride + (size_t)h * Dv : nullptr;
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   const float* angles = a.turn ? a.turn + (size_t)t * Dv : nullptr;
   if (angles) {  // partners meet in LDS, which the queries no longer need
-    __syncthreads();
+    wave_lds_fence();
 #pragma unroll
-    for (int i = 0; i < MAX_D / 64; ++i)
+    for (int i = 0; i < (MD + 63) / 64; ++i)
       if (lane + 64 * i < Dv) qs[lane + 64 * i] = acc[i];
-    __syncthreads();
+    wave_lds_fence();
   }
 #pragma unroll
-  for (int i = 0; i < MAX_D / 64; ++i) {
+  for (int i = 0; i < (MD + 63) / 64; ++i) {
     const int d = lane + 64 * i;
     if (d < Dv) {
       float v = acc[i] * inv;
@@ -138,6 +144,12 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
   }
 }
 
+template <typename T>
+__global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
+  __shared__ float qs[MAX_D];
+  attend_row<T, MAX_D>(a, blockIdx.x, blockIdx.y, qs);
+}
+
 // ---------------------------------------------------------------- float32 by tiles
 // A block takes 16 rows (token * g + head in group) of one sequence and key head, its W waves the
 // sequence's blocks of 16 keys in turn, each with a maximum, a sum and an accumulator of its own, which
@@ -152,12 +164,15 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
 // 128 always eight (2,048 tokens, 16 heads of 256 on 4: 910 us, with four 1,440). That goes by
 // the sequence's own rows, and a block of keys goes to the wave of its number in the sequence, so that neither what shares
 // a step nor a tile changes a sum's order.
+// A row takes nothing from keys it does not see, whatever they hold; but 0 times an infinity is no number, and the tile's rows
+// share the products. A tile with a result that is not finite is therefore made again row by row, as in the kernel above.
 // Head sizes in multiples of 16 up to 256, pages of a multiple of 4 keys; other sizes keep the kernel above.
 #define F32_FEW_ROWS 64
 template <int ND, int W>
 __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) {
   __shared__ __align__(16) f32x4_t hand[W > 1 ? W / 2 : 1][ND * 64];  // accumulators on their way from wave to wave
   __shared__ float hand_m[W][16], hand_l[W][16];
+  __shared__ int odd;  // whether a result is not finite
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r = lane & 15, q = lane >> 4;
   const int s = blockIdx.z, kvh = blockIdx.y, g = a.nq / a.nkv;
@@ -280,6 +295,7 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   }
   // rows into LDS in order, then out with the block's threads (a turned value's partner lies half a row away)
   float* out_rows = (float*)hand;
+  if (threadIdx.x == 0) odd = 0;
   if (wave == 0) {
     const float inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
@@ -287,6 +303,13 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
       if (j < nv) *(f32x4_t*)(out_rows + r * Dv + 16 * j + 4 * q) = acc[j] * inv;
   }
   __syncthreads();
+  for (int i = threadIdx.x; i < (last_row - row0 + 1) * Dv; i += 64 * W)
+    if (!(fabsf(out_rows[i]) < INFINITY)) odd = 1;
+  __syncthreads();
+  if (odd) {
+    for (int i = row0 + wave; i <= last_row; i += W) attend_row<float, 16 * ND>(a, t0 + i / g, kvh * g + i % g, out_rows + 16 * ND * wave);
+    return;
+  }
   for (int i = threadIdx.x; i < (last_row - row0 + 1) * Dv; i += 64 * W) {
     const int ri = row0 + i / Dv, d = i % Dv, ti = t0 + ri / g, hq = kvh * g + ri % g;
     float v = out_rows[i];

@@ -1,6 +1,7 @@
 """The float32 kernels at the edges of their tiles: products against float64 within the bound of a
 float32 sum, equal bits however many rows share a launch; attention by tiles against the plain one."""
 
+import copy
 import math
 
 import pytest
@@ -61,3 +62,47 @@ def test_attention_by_tiles(ops, seqs, nq, nkv, d, dv, ps, more):
     got = ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window, value_dim=dv, **more)
     # scores of size 3 * sqrt(d) * scale and values of size 3: sums of up to 300 float32 terms
     close(got, want.float(), 2e-5, 2e-5)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("nq,nkv,d,more", [(4, 2, 128, {}), (8, 8, 32, {"window": 23}), (6, 1, 256, {"window": 40, "keep_first": 5}), (4, 4, 64, {"chunk": 32})])
+def test_attention_takes_nothing_from_keys_a_token_does_not_see(ops, value, nq, nkv, d, more):
+    """A value and a key of one token that are not finite: tokens that do not see it are as they are without it (but for the
+    order of their sums)."""
+    n = 75
+    q, cache, ctx = build_attention_case([(n, n), (1, n)], nq, nkv, d, 16, torch.float32)
+    attend = lambda cache: ops.paged_attention(q, cache, ctx, nq, nkv, d, d ** -0.5, more.get("window"), chunk=more.get("chunk"),  # noqa: E731
+                                               keep_first=more.get("keep_first", 0))
+    want, pos = attend(cache), torch.arange(n, device=DEV)
+    for at in (0, 3, 16, 37, 74):
+        sees = pos >= at
+        if "window" in more:
+            sees &= (pos - at < more["window"]) | (at < more.get("keep_first", 0))
+        if "chunk" in more:
+            sees &= pos // 32 == at // 32
+        for stream in ("v", "k"):
+            odd = copy.copy(cache)
+            odd.k, odd.v = k, v = cache.k.clone(), cache.v.clone()
+            for s in (0, 1):
+                page, off = int(cache.group.block_table[s, at // 16]), at % 16
+                if stream == "v":
+                    v[page, :, d - 1, off] = value
+                else:
+                    k[page, :, off, 0] = value
+            got = attend(odd)
+            close(got[:n][~sees], want[:n][~sees], 2e-5, 2e-5)
+            if not bool(sees[n - 1]):
+                close(got[n], want[n], 2e-5, 2e-5)
+
+
+def test_a_first_key_of_no_weight_leaves_a_token_its_other_keys(ops):
+    """Token 16 alone sees key 16, whose score is minus infinity for all heads: its other sixteen keys count as ever."""
+    q, cache, ctx = build_attention_case([(17, 17)], 2, 2, 32, 16, torch.float32)
+    q.view(17, 2, 32)[16] = q.view(17, 2, 32)[16].abs()
+    page = int(cache.group.block_table[0, 1])
+    cache.k[page, :, 0, :] = float("-inf")
+    got = ops.paged_attention(q, cache, ctx, 2, 2, 32, 0.2, None).view(17, 2, 32)[16]
+    page = int(cache.group.block_table[0, 0])
+    k, v = cache.k[page].cpu().double(), cache.v[page].cpu().double()
+    p = torch.softmax((q.view(17, 2, 32)[16].cpu().double()[:, None, :] * k).sum(-1) * 0.2, -1)
+    close(got, (p[:, None, :] * v).sum(-1).float(), 2e-5, 2e-5)
