@@ -208,8 +208,9 @@ __global__ __launch_bounds__(256) void retention_kernel(RetentionArgs a) {
 // the k-slice {r, 4 + r, 8 + r, 12 + r}; whoever meets it takes the same slice. Scores are formed as
 // K Q^T for that reason. Rows of 128 are 132 apart in LDS: 16-byte reads of 16 neighbouring rows and
 // 4-byte reads of 16 neighbouring elements of every fourth row both meet the banks evenly.
-// A sum that is masked must not meet an infinity of a later token (0 x inf): a chunk with a value that is not finite,
-// or so large that a score could overflow, goes through the same products one token at a time.
+// A sum that is masked must not meet an infinity of a later token (0 x inf), nor a sum overflow whose decay, taken
+// afterwards here, would have kept it finite: a chunk with a value that is not finite or over 10^12, or with a state over 10^24
+// in front of it, goes through the same products one token at a time, each read out of the state after it.
 // Powers are products of repeated squares, so any decay goes (negative, none at all), in double and kept in two
 // floats: a rounded d^32 would be off by the same part every chunk, which over a memory of 500 tokens made ten
 // times the error of the walk (3e-6 against 4e-7).
@@ -319,17 +320,19 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
         for (int g = 0; g < G; ++g) kt[j][g][r] = ks[row * ROW + 16 * (G * wave + g) + r16];
       }
     __builtin_amdgcn_sched_barrier(0);
-    if (SINGLE) {
+    if (SINGLE) {  // S <- d S + k v^T, o = S^T q: nothing is multiplied that the recurrence does not multiply
+      const bool first = quad == 0;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        if (r16) q[0][g] = k[0][g] = zero;
+        f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x4f32(first ? kt[0][g][0] : 0.f, first ? v[0][0] : 0.f, zero, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (quad || r) kt[0][g][r] = 0.f;
+        for (int r = 0; r < 4; ++r) s[g][r] = fmaf(s[g][r], powers[1], acc[r]);
+        acc = zero;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(r16 ? 0.f : q[0][g][r], s[g][r], acc, 0, 0, 0);
+        o[0] = g ? o[0] + acc : acc;
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (quad || r) v[0][r] = 0.f;
+      return;
     }
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {  // scores[i][j]: rows are keys, columns queries
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
 #pragma unroll
         for (int r = 0; r < 4; ++r) add[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[j][g][r], v[j][r], add[j], 0, 0, 0);
       }
-      if (!SINGLE) add[0] += add[TILES - 1];
+      add[0] += add[TILES - 1];
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[g][r] = fmaf(s[g][r], all, fmaf(s[g][r], rest, add[0][r]));
     }
@@ -423,6 +426,10 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
       vs[(e >> 4) * RC_VROW + (e & 15)] = from.v[i];
       look(from.v[i]);
     }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) large |= !(fabsf(s[g][r]) < 1e24f);
     if (large) odd[turn] = 1;
     __syncthreads();
     const bool one_by_one = odd[turn];
@@ -433,14 +440,12 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
       walk(std::false_type{}, 0, n);
       leave(base, n);
     } else {
-      ends(1);
       for (int i = 0; i < n; ++i) {
         o[1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
         walk(std::true_type{}, i, 1);
         leave(base + i, 1);
         __syncthreads();
       }
-      ends(RC_TOKENS);
     }
   };
   Ahead first, second;

@@ -1,5 +1,6 @@
 """Retention over prompts by chunks of tokens: against the recurrence in float64, at the edges of chunks, heads and columns."""
 
+import math
 import types
 
 import pytest
@@ -75,3 +76,30 @@ def test_a_value_that_is_not_finite_stays_behind_its_token(ops, which, value):
     fine = torch.isfinite(out) & (out.abs() < 3e38)
     assert (torch.isfinite(got) == fine).all()
     assert ((got.double() - out).abs() <= steps * EPS * out_sizes)[fine].all()
+
+
+@pytest.mark.parametrize("size", [1e30, 3e37, float("inf")])
+@pytest.mark.parametrize("where", ["state", "k", "v"])
+def test_what_a_large_state_holds_decays_as_in_the_recurrence(ops, size, where):
+    """Read-outs and states that the recurrence keeps finite are finite and right, and one that became infinite stays so."""
+    heads, dim, vdim, lengths = 4, 64, 20, (80,)
+    qkv, d, state, slots = _draw(lengths, heads, dim, vdim, (0.0, 0.1, 0.5, 0.999))
+    qkv[:, : heads * dim] *= 100.0
+    if where == "state":
+        state[:, :, :, 2] *= size
+    else:
+        qkv[9, {"k": slice(heads * dim + 2, 2 * heads * dim, dim), "v": slice(2 * heads * dim + 2, None, vdim)}[where]] *= size
+    out, out_sizes, _, _ = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
+    got, after = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    steps = 2 * max(lengths) + dim + 8
+    fine = torch.isfinite(out) & (out_sizes < 1e37)
+    if not math.isinf(size):
+        assert fine.float().mean() > 0.5
+    assert ((got.double() - out).abs() <= steps * EPS * out_sizes + 1e-30)[fine].all()
+    walked = state[slots.long()].clone()[0]
+    q, k, v = qkv.split([heads * dim, heads * dim, heads * vdim], 1)
+    for i in range(80):
+        walked = d[:, None, None] * walked + v[i].view(heads, vdim, 1) * k[i].view(heads, 1, dim)
+    last = after[int(slots[0])]
+    assert torch.equal(torch.isnan(last), torch.isnan(walked))
+    assert torch.equal(last[torch.isinf(walked)], walked[torch.isinf(walked)])
