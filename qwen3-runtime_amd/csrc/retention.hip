@@ -41,6 +41,10 @@ struct RetentionArgs {
   const int* seq_ids;     // the sequences of this launch; null: all of the step's
   const float* gates;     // [T, 3, heads] (GATES): log keep, log write (a third row is not read here)
   float* last_out;        // [T, heads] (GATES): the read-out of the state's last column
+  // Retention: sequences of at least `chunk_from` tokens go by chunks (0: none does). It goes by the sequence's own
+  // tokens, not the step's, so that a request's results do not depend on what shares its step. `shortest`, `longest`:
+  // bounds of the step's lengths, as the caller knows them, that say whether a form has any work.
+  int chunk_from, shortest, longest;
 };
 
 constexpr int RT_CONSTANT = 0, RT_STEP = 1, RT_GATES = 2;  // where decays and writes come from
@@ -75,7 +79,7 @@ __global__ __launch_bounds__(256) void retention_kernel(RetentionArgs a) {
   __shared__ float ds[RT_TILE], steps[RT_TILE];  // a token's decay and what its value is multiplied by (PER_TOKEN)
   const int seq = a.seq_ids ? a.seq_ids[blockIdx.x] : blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * RT_COLS;
   const int t0 = a.cu_q[seq], t1 = a.cu_q[seq + 1];
-  if (t1 <= t0) return;
+  if (t1 <= t0 || (!PER_TOKEN && a.chunk_from > 0 && t1 - t0 >= a.chunk_from)) return;
   const int dim = a.dim, vdim = a.vdim;
   const int cols = GATES ? vdim + 1 : vdim;  // columns of the state
   const TI* qkv = (const TI*)a.qkv;
@@ -214,11 +218,14 @@ __global__ __launch_bounds__(256) void retention_kernel(RetentionArgs a) {
 // Powers are products of repeated squares, so any decay goes (negative, none at all), in double and kept in two
 // floats: a rounded d^32 would be off by the same part every chunk, which over a memory of 500 tokens made ten
 // times the error of the walk (3e-6 against 4e-7).
+// LEAN: the same operations with a quarter fewer registers (one chunk on its way, powers read where they are used), so that
+// one more block shares a compute unit: for launches of more blocks than one (256 threads: three) a unit. 2 sequences of 1,000
+// tokens, 32 heads of 128: 157 -> 145 us, 8 of 128 103 -> 78 (walked 73); a lone one of 2,047 155 and 170.
 constexpr int RC_TOKENS = 32, RC_VROW = 20;
 
-template <int G, int NW>
-__global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs a) {
-  constexpr int DP = 16 * G * NW, ROW = DP + 4, THREADS = 64 * NW;
+template <int G, int NW, bool LEAN>
+__global__ __launch_bounds__(64 * NW, LEAN ? 4 : 1) void retention_chunk_kernel(RetentionArgs a) {
+  constexpr int DP = 16 * G * NW, ROW = DP + 4, THREADS = 64 * NW, AHEAD = LEAN ? 1 : 2;
   constexpr int PIECES = RC_TOKENS * DP / 4 / THREADS;       // 16-byte pieces of q, and of k, a thread
   constexpr int OWN = RC_TOKENS * RT_COLS / THREADS;         // values, and read-outs, a thread
   __shared__ __attribute__((aligned(16))) float qs[RC_TOKENS * ROW];
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
   __shared__ int odd[2];  // whether the chunk (of even, of odd number) holds a value for single tokens
   const int seq = a.seq_ids ? a.seq_ids[blockIdx.x] : blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * RT_COLS;
   const int t0 = a.cu_q[seq], t1 = a.cu_q[seq + 1];
-  if (t1 <= t0) return;
+  if (t1 - t0 < a.chunk_from) return;
   const int dim = a.dim, vdim = a.vdim, qk_head = head / a.share;
   const int lane = threadIdx.x & 63, wave = uniform_wave_number(), r16 = lane & 15, quad = lane >> 4;
   const float* qkv = (const float*)a.qkv;
@@ -272,28 +279,30 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
     __builtin_amdgcn_sched_barrier(0);  // asked for here, not where they are used
   };
   __syncthreads();
-  float to_row[2][4], to_row_rest[2][4], back[2][4], back_rest[2][4], to_end[2][4], to_end_rest[2][4];  // d^(i+1); d^(i-j) by how many tiles apart; d^(n-1-j)
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * i + 4 * quad + r, diff = 16 * i + r16 - 4 * quad - r;
-      to_row[i][r] = powers[row + 1];
-      to_row_rest[i][r] = powers_rest[row + 1];
-      back[i][r] = powers[max(diff, 0)];
-      back_rest[i][r] = powers_rest[max(diff, 0)];
-    }
-  auto ends = [&](int n) {
+  // d^(i+1); d^(i-j) by how many tiles apart; d^(n-1-j): kept in registers or (LEAN) read where they are used
+  struct Powers {
+    float by[2][4], rest[2][4];
+  };
+  auto load_powers = [&](Powers& to, auto exponent) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        to_end[i][r] = powers[max(n - 1 - (16 * i + 4 * quad + r), 0)];
-        to_end_rest[i][r] = powers_rest[max(n - 1 - (16 * i + 4 * quad + r), 0)];
+        const int e = max(exponent(i, 4 * quad + r), 0);
+        to.by[i][r] = powers[e];
+        to.rest[i][r] = powers_rest[e];
       }
   };
-  ends(RC_TOKENS);
-  auto times = [](float x, float by, float rest) { return fmaf(x, by, x * rest); };
+  Powers to_row, back, to_end;
+  auto rows_powers = [&] { load_powers(to_row, [](int i, int row) { return 16 * i + row + 1; }); };
+  auto back_powers = [&] { load_powers(back, [&](int i, int row) { return 16 * i + r16 - row; }); };
+  auto end_powers = [&](int n) { load_powers(to_end, [&](int i, int row) { return n - 1 - (16 * i + row); }); };
+  if (!LEAN) {
+    rows_powers();
+    back_powers();
+    end_powers(RC_TOKENS);
+  }
+  auto times = [](float x, const Powers& p, int i, int r) { return fmaf(x, p.by[i][r], x * p.rest[i][r]); };
   // one chunk from LDS: rows off .. off + n - 1; SINGLE: one row (n = 1), the others taken as zeros
   f32x4_t o[2];
   auto walk = [&](auto single, int off, int n) {
@@ -349,6 +358,7 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
         scores[i][j] = sum;
       }
     }
+    if (LEAN) rows_powers();
 #pragma unroll
     for (int i = 0; i < TILES; ++i) {
 #pragma unroll
@@ -359,8 +369,9 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
         o[i] = g ? o[i] + acc : acc;
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[i][r] = times(o[i][r], to_row[i][r], to_row_rest[i][r]);
+      for (int r = 0; r < 4; ++r) o[i][r] = times(o[i][r], to_row, i, r);
     }
+    if (LEAN) back_powers();
 #pragma unroll
     for (int i = 0; i < TILES; ++i)
 #pragma unroll
@@ -368,16 +379,17 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
         f32x4_t acc = zero;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = i == j && r16 < 4 * quad + r ? 0.f : times(scores[i][j][r], back[i - j][r], back_rest[i - j][r]);
+          const float p = i == j && r16 < 4 * quad + r ? 0.f : times(scores[i][j][r], back, i - j, r);
           acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p, v[j][r], acc, 0, 0, 0);
         }
         o[i] += acc;
       }
     const float all = powers[n], rest = powers_rest[n];
+    if (LEAN) end_powers(n);
 #pragma unroll
     for (int j = 0; j < TILES; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[j][r] = times(v[j][r], to_end[j][r], to_end_rest[j][r]);
+      for (int r = 0; r < 4; ++r) v[j][r] = times(v[j][r], to_end, j, r);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       f32x4_t add[TILES];
@@ -434,9 +446,9 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
     __syncthreads();
     const bool one_by_one = odd[turn];
     if (threadIdx.x == 0) odd[turn ^ 1] = 0;  // read last before the barrier in `leave` of the chunk before
-    if (base + 2 * RC_TOKENS < t1) fetch(from, base + 2 * RC_TOKENS);
+    if (base + AHEAD * RC_TOKENS < t1) fetch(from, base + AHEAD * RC_TOKENS);
     if (!one_by_one) {
-      if (n < RC_TOKENS) ends(n);  // the last chunk
+      if (!LEAN && n < RC_TOKENS) end_powers(n);  // the last chunk
       walk(std::false_type{}, 0, n);
       leave(base, n);
     } else {
@@ -448,12 +460,17 @@ __global__ __launch_bounds__(64 * NW) void retention_chunk_kernel(RetentionArgs 
       }
     }
   };
-  Ahead first, second;
+  Ahead first;
   fetch(first, t0);
-  if (t0 + RC_TOKENS < t1) fetch(second, t0 + RC_TOKENS);
-  for (int base = t0; base < t1; base += 2 * RC_TOKENS) {
-    chunk(first, base, 0);
-    if (base + RC_TOKENS < t1) chunk(second, base + RC_TOKENS, 1);
+  if (LEAN) {
+    for (int base = t0, turn = 0; base < t1; base += RC_TOKENS, turn ^= 1) chunk(first, base, turn);
+  } else {
+    Ahead second;
+    if (t0 + RC_TOKENS < t1) fetch(second, t0 + RC_TOKENS);
+    for (int base = t0; base < t1; base += 2 * RC_TOKENS) {
+      chunk(first, base, 0);
+      if (base + RC_TOKENS < t1) chunk(second, base + RC_TOKENS, 1);
+    }
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) {
@@ -476,17 +493,20 @@ extern "C" int qrt_retention(const RetentionArgs* args, int num_tokens, int num_
   if (num_tokens == 0 || num_seqs == 0) return 0;
   const dim3 grid(num_seqs, a.heads, (a.vdim + (a.gates ? 1 : 0) + RT_COLS - 1) / RT_COLS);
   const int groups = (a.dim + 63) / 64;
-  // Prompts under a constant decay by chunks where a head's rows are whole pieces of 16 bytes (in `qkv` and in the
-  // state) and fit the waves' accumulators; steps of single tokens are one chunk each and gain nothing
-  // (8 sequences of one token: 10.0 us walked).
-  const bool pieces = a.dim % 4 == 0 && a.channels % 4 == 0 && a.q_first % 4 == 0 && a.k_first % 4 == 0 &&
-                      ((uintptr_t)a.qkv | (uintptr_t)a.state) % 16 == 0;
-  if (!a.gates && !a.step && groups <= 4 && pieces && num_tokens > 2 * num_seqs) {
-    if (groups == 1) retention_chunk_kernel<1, 4><<<grid, 256, 0, stream>>>(a);
-    else if (groups == 2) retention_chunk_kernel<1, 8><<<grid, 512, 0, stream>>>(a);
-    else retention_chunk_kernel<2, 8><<<grid, 512, 0, stream>>>(a);
-    QRT_LAUNCH_CHECK("retention (chunks)");
-    return 0;
+  if (a.chunk_from > 0) {
+    QRT_CHECK(!a.gates && !a.step && groups <= 4 && a.dim % 4 == 0 && a.channels % 4 == 0 && a.q_first % 4 == 0 && a.k_first % 4 == 0 &&
+                  ((uintptr_t)a.qkv | (uintptr_t)a.state) % 16 == 0,
+              "retention: chunks go with constant decays and heads of up to 256 elements in whole pieces of 16 bytes");
+    if (a.longest >= a.chunk_from) {
+      const long blocks = (long)grid.x * grid.y * grid.z;
+      if (groups == 1 && blocks > 768) retention_chunk_kernel<1, 4, true><<<grid, 256, 0, stream>>>(a);
+      else if (groups == 1) retention_chunk_kernel<1, 4, false><<<grid, 256, 0, stream>>>(a);
+      else if (groups == 2 && blocks > 256) retention_chunk_kernel<1, 8, true><<<grid, 512, 0, stream>>>(a);
+      else if (groups == 2) retention_chunk_kernel<1, 8, false><<<grid, 512, 0, stream>>>(a);
+      else retention_chunk_kernel<2, 8, false><<<grid, 512, 0, stream>>>(a);
+      QRT_LAUNCH_CHECK("retention (chunks)");
+      if (a.shortest >= a.chunk_from) return 0;
+    }
   }
 #define GO(G, TILE)                                                                 \
   do {                                                                              \
@@ -496,7 +516,7 @@ extern "C" int qrt_retention(const RetentionArgs* args, int num_tokens, int num_
     else if (a.step) retention_kernel<G, TILE, RT_STEP, float><<<grid, 256, 0, stream>>>(a); \
     else retention_kernel<G, TILE, RT_CONSTANT, float><<<grid, 256, 0, stream>>>(a);      \
   } while (0)
-  if (num_tokens <= 2 * num_seqs) {  // decoded tokens, mostly
+  if (num_tokens <= 2 * num_seqs || (a.chunk_from > 0 && a.longest >= a.chunk_from && a.shortest <= 4)) {  // decoded tokens, mostly
     if (groups <= 1) GO(1, 4);
     else if (groups <= 2) GO(2, 4);
     else if (groups <= 4) GO(4, 4);

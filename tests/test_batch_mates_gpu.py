@@ -1,11 +1,12 @@
 """What a request gets does not depend on what else is in its step: equal bits alone and beside others."""
 
 import copy
+import types
 
 import pytest
 import torch
 
-from test_kernels_gpu import DEV, build_attention_case
+from test_kernels_gpu import DEV, build_attention_case, rnd
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +45,28 @@ def test_float32_attention(ops, nq, nkv, d, more):
     for s, skip in ((0, 0), (1, 0), (2, 0), (3, 0), (3, 7), (150, 0)):
         part, pages, rows = _part(ctx, cache, s, skip)
         assert torch.equal(attend(q[rows].contiguous(), pages, part), whole[rows]), (s, skip)
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 32), (128, 40), (200, 16)])
+@pytest.mark.parametrize("lengths", [(1, 1, 300, 1), (63, 64, 65, 127, 128, 1), (2,) * 40 + (133,), (70,) * 160])
+def test_retention(ops, dim, vdim, lengths):
+    heads, t = 3, sum(lengths)
+    qkv, state = rnd(t, 2 * heads * dim + heads * vdim, seed=1), rnd(len(lengths), heads, vdim, dim, seed=2)
+    decay = torch.tensor([0.9, 0.99, 0.5], device=DEV)
+
+    def run(lengths, qkv, slots, on_host):
+        cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+        ctx = types.SimpleNamespace(num_tokens=sum(lengths), num_seqs=len(lengths), cu_q=cu,
+                                    state_slots=torch.tensor(slots, dtype=torch.int32, device=DEV))
+        if on_host:  # without its lengths on the host a step launches both forms
+            ctx.q_lens_host = list(lengths)
+        after = state.clone()
+        return ops.retention_rule(ctx, qkv, decay, after, heads, dim, vdim), after
+
+    whole, after = run(lengths, qkv, range(len(lengths)), True)
+    assert all(torch.equal(a, b) for a, b in zip(run(lengths, qkv, range(len(lengths)), False), (whole, after)))
+    at = 0
+    for s, n in enumerate(lengths[:6]):
+        got, own = run((n,), qkv[at: at + n].contiguous(), [s], True)
+        assert torch.equal(got, whole[at: at + n]) and torch.equal(own[s], after[s]), (s, n)
+        at += n

@@ -63,6 +63,21 @@ def test_chunks_match_the_recurrence(ops, dim, vdim, heads, lengths, decay):
     assert ((after.double() - states).abs() <= steps * EPS * sizes).all()
 
 
+@pytest.mark.parametrize("lengths,heads,dim,vdim", [((1,), 1, 4, 1), ((31,), 3, 60, 16), ((32, 33, 2), 2, 68, 17), ((65, 3), 2, 256, 33),
+                                                    ((33, 1, 64, 97) * 3, 4, 68, 128), ((33, 1, 64, 97) * 3, 9, 60, 128)])
+def test_every_form_of_the_chunks_matches_the_recurrence(ops, lengths, heads, dim, vdim):
+    """Spans of any length by chunks, in launches of few blocks and of many (the last two)."""
+    decay = (0.9, -0.7, 1.0, 0.5)
+    qkv, d, state, slots = _draw(lengths, heads, dim, vdim, decay)
+    out, out_sizes, states, sizes = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
+    ops = type(ops)()
+    ops.retention_chunk_min_tokens = (1, 1)
+    got, after = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    steps = 2 * max(lengths) + dim + 8
+    assert ((got.double() - out).abs() <= steps * EPS * out_sizes).all()
+    assert ((after.double() - states).abs() <= steps * EPS * sizes).all()
+
+
 @pytest.mark.parametrize("which", ["k", "v", "q"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 1e30])
 def test_a_value_that_is_not_finite_stays_behind_its_token(ops, which, value):
