@@ -216,10 +216,9 @@ __global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restri
   typedef T xvec_t __attribute__((ext_vector_type(4)));
   extern __shared__ __align__(16) unsigned char route_lds[];
   T* xs = (T*)route_lds;  // [TB][hidden] for TB > 1
-  __shared__ float logit[TB][65];
-  __shared__ float gate_part[16];
+  __shared__ float logit[TB][64];
+  __shared__ float gate_part[TB][16];
   const int t0 = blockIdx.x * TB, lane = threadIdx.x & 63, wave = uniform_wave_number();
-  float gate_acc = 0.f;
   if (TB > 1) {
     const int pieces = hidden / 4;
     for (int i = threadIdx.x; i < TB * pieces; i += 1024) {
@@ -227,17 +226,23 @@ __global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restri
       *(xvec_t*)(xs + (size_t)t * hidden + c) = *(const xvec_t*)(x + (size_t)min(t0 + t, num_tokens - 1) * hidden + c);
     }
     __syncthreads();
-  } else if (gate) {  // one token: the gate's row is shared by the block, on its way beside the waves' own rows
+  }
+  float gate_acc[TB];
+#pragma unroll
+  for (int t = 0; t < TB; ++t) gate_acc[t] = 0.f;
+  if (gate) {  // the gate's row is shared by the block, on its way beside the waves' own rows, for one token and for many alike
     const float* wr = router + (size_t)experts * hidden;
     for (int c = threadIdx.x * 4; c < hidden; c += 4096) {
       const f32x4_t wv = *(const f32x4_t*)(wr + c);
-      const xvec_t xv = *(const xvec_t*)(x + (size_t)t0 * hidden + c);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) gate_acc = fmaf(to_f32<T>(xv[k]), wv[k], gate_acc);
+      for (int t = 0; t < TB; ++t) {
+        const xvec_t xv = TB > 1 ? *(const xvec_t*)(xs + (size_t)t * hidden + c) : *(const xvec_t*)(x + (size_t)t0 * hidden + c);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gate_acc[t] = fmaf(to_f32<T>(xv[k]), wv[k], gate_acc[t]);
+      }
     }
   }
-  const int rows = experts + (TB > 1 && gate ? 1 : 0);
-  for (int e = wave; e < rows; e += 16) {
+  for (int e = wave; e < experts; e += 16) {
     const float* wr = router + (size_t)e * hidden;
     float acc[TB];
 #pragma unroll
@@ -255,20 +260,22 @@ __global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restri
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
       const float z = wave_sum(acc[t]);
-      if (lane == 0) logit[t][e] = z + (e < experts && bias ? bias[e] : 0.f);
+      if (lane == 0) logit[t][e] = z + (bias ? bias[e] : 0.f);
     }
   }
-  if (TB == 1 && gate) {
-    gate_acc = wave_sum(gate_acc);
-    if (lane == 0) gate_part[wave] = gate_acc;
+  if (gate) {
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+      const float z = wave_sum(gate_acc[t]);
+      if (lane == 0) gate_part[t][wave] = z;
+    }
   }
   __syncthreads();
   const int t = t0 + wave;
   if (wave >= TB || t >= num_tokens) return;
   if (gate && lane == 0) {
-    float z = TB > 1 ? logit[wave][experts] : 0.f;
-    if (TB == 1)
-      for (int i = 0; i < 16; ++i) z += gate_part[i];
+    float z = 0.f;
+    for (int i = 0; i < 16; ++i) z += gate_part[wave][i];
     gate[t] = 1.0f / (1.0f + expf(-z));
   }
   const bool mine = lane < experts;
