@@ -962,7 +962,7 @@ class HipOps:
         _need(weight, "expert weight", torch.float32, (t, top))
         if out is not None:  # the caller's own float32 rows
             _need(out, "experts' output", torch.float32, (t, h))
-        if t and self.experts_fit(x, h, inter):
+        if t and self.experts_fit(x, h, inter, gate_up, down):
             planes = self.moe_for_residual(x, gate_up, down, index, weight, activation, limit, weight_on_input)
             total = planes[0] if top == 1 else self.accumulate(planes[0], planes[1:])
             return total if out is None else out.copy_(total)
@@ -1006,9 +1006,10 @@ class HipOps:
     experts_rows_max_pairs = 8192  # the stream's blocks list their expert's pairs in LDS
 
     @staticmethod
-    def experts_fit(x, hidden, inter) -> bool:
-        """Whether the experts' MFMA kernels take these operands (rows of whole cache lines)."""
-        return x.dtype == torch.bfloat16 and hidden % 64 == 0 and inter % 64 == 0
+    def experts_fit(x, hidden, inter, *weights) -> bool:
+        """Whether the experts' MFMA kernels take these operands (rows of whole cache lines, 16 bytes a load)."""
+        return (x.dtype == torch.bfloat16 and hidden % 64 == 0 and inter % 64 == 0
+                and all(a.data_ptr() % 16 == 0 for a in (x, *weights)))
 
     def moe_for_residual(self, x, gate_up, down, index, weight, activation="swiglu", limit=0.0, weight_on_input=False,
                          out=None):
@@ -1019,7 +1020,7 @@ class HipOps:
         n, rows_e, _ = gate_up.shape
         inter = rows_e if activation == "relu2" else rows_e // 2
         top = index.shape[1]
-        if not self.experts_fit(x, h, inter):
+        if not self.experts_fit(x, h, inter, gate_up, down):
             return None
         if weight_on_input and activation == "relu2":
             raise OpsError("weights on the experts' input go with gated experts")

@@ -171,7 +171,7 @@ class RoutedSwiGLU(FeedForward):
         # few tokens: the shared expert's product leaves float32 planes with some to spare, the routed
         # experts write theirs into them, and the norm that comes next adds them all up
         fits = getattr(ops, "experts_fit", None)
-        if fits is not None and fits(x, self.hidden_size, self.intermediate_size):
+        if fits is not None and fits(x, self.hidden_size, self.intermediate_size, self.gate_up, self.down):
             planes = ops.linear_planes_with_spare(act, self.shared_down, self.top)
             if planes is not None:
                 ops.moe_for_residual(x, self.gate_up, self.down, index, weight, out=planes[-self.top:], **more)

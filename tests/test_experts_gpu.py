@@ -74,3 +74,22 @@ def test_widths_that_whole_lines_do_not_fit_keep_the_general_form(ops):
     assert ops.moe_for_residual(x, gate_up, down, index, weight) is None
     want = plain(x, gate_up, down, index, weight, "swiglu", 0.0, False).sum(0)
     close(ops.moe_swiglu(x, gate_up, down, index, weight), want.float(), 1e-3, 1e-3)
+
+
+@pytest.mark.parametrize("which,t", [("x", 3), ("x", 70), ("gate_up", 3), ("down", 3)])
+def test_operands_that_begin_between_16_bytes_keep_the_general_form(ops, which, t):
+    def at_8_bytes(a):
+        room = torch.empty(a.numel() + 4, dtype=a.dtype, device=DEV)
+        room[4:].copy_(a.reshape(-1))
+        return room[4:].view(a.shape)
+
+    x, gate_up, down = (rnd(*s, dtype=torch.bfloat16, scale=0.1) for s in ((t, 128), (4, 128, 128), (4, 128, 64)))
+    scores = rnd(t, 4, seed=4)
+    weight, index = scores.topk(2, -1)
+    weight, index = torch.softmax(weight, -1).contiguous(), index.int().contiguous()
+    want = plain(x, gate_up, down, index, weight, "swiglu", 0.0, False).sum(0)
+    moved = {"x": x, "gate_up": gate_up, "down": down}
+    moved[which] = at_8_bytes(moved[which])
+    assert moved[which].is_contiguous() and moved[which].data_ptr() % 16 == 8
+    assert ops.moe_for_residual(moved["x"], moved["gate_up"], moved["down"], index, weight) is None
+    close(ops.moe_swiglu(moved["x"], moved["gate_up"], moved["down"], index, weight), want.float(), 1e-3, 1e-3)
