@@ -170,7 +170,7 @@ class RoutedSwiGLU(FeedForward):
         act = ops.gated_linear(x, self.shared_gate_up, activation=self.activation, limit=self.shared_limit, **opened)
         # few tokens: the shared expert's product leaves float32 planes with some to spare, the routed
         # experts write theirs into them, and the norm that comes next adds them all up
-        fits = getattr(ops, "experts_fit", None)
+        fits = getattr(ops, "experts_fit", None) if self.top <= self.max_planes else None
         if fits is not None and fits(x, self.hidden_size, self.intermediate_size, self.gate_up, self.down):
             planes = ops.linear_planes_with_spare(act, self.shared_down, self.top)
             if planes is not None:
@@ -184,8 +184,12 @@ class RoutedSwiGLU(FeedForward):
         out = ops.moe_swiglu(x, self.gate_up, self.down, index, weight, **more)
         return ops.accumulate(out, ops.linear_for_residual(act, self.shared_down))
 
+    # experts a token, beyond which their outputs are added up first: the next norm would read a plane for each, and
+    # takes a limited number of planes
+    max_planes = 8
+
     def _routed(self, ops, x, index, weight, **more):
         """The routed experts' sum, as the norm that comes next may have it: in planes where the ops make them."""
-        planes = getattr(ops, "moe_for_residual", None) if self.top <= 8 else None
+        planes = getattr(ops, "moe_for_residual", None) if self.top <= self.max_planes else None
         out = None if planes is None else planes(x, self.gate_up, self.down, index, weight, **more)
         return ops.moe_swiglu(x, self.gate_up, self.down, index, weight, **more) if out is None else out
