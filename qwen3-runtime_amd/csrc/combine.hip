@@ -200,29 +200,35 @@ __global__ __launch_bounds__(1024) void norm_add_rmsnorm_kernel(float* __restric
   }
 }
 
-// VEC neighbouring elements of a sub-layer output, float32. TWO: two planes have a way of their own (the routed
-// experts' outputs), where a kernel takes one output alone: with several, the branches' masks spill.
-template <int VEC, bool TWO = false>
+// VEC neighbouring elements of a sub-layer output, float32. PLANES: how many planes it has, where that is known when
+// compiling (0: it may be any output).
+template <int VEC, int PLANES = 0>
 __device__ __forceinline__ void planes_piece(const Planes& y, size_t i, float* v) {
   typedef float fvec_t __attribute__((ext_vector_type(VEC)));
   typedef bf16_t bvec_t __attribute__((ext_vector_type(VEC)));
+  const float* p = (const float*)y.p;
+  if (PLANES > 0) {
+    fvec_t part[PLANES > 0 ? PLANES : 1];
+#pragma unroll
+    for (int k = 0; k < PLANES; ++k) part[k] = *(const fvec_t*)(p + (size_t)k * y.plane_stride + i);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      v[e] = part[0][e];
+#pragma unroll
+      for (int k = 1; k < PLANES; ++k) v[e] += part[k][e];
+    }
+    return;
+  }
   if (y.code == QRT_BF16) {
     const bvec_t x = *(const bvec_t*)((const bf16_t*)y.p + i);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) v[e] = (float)x[e];
     return;
   }
-  const float* p = (const float*)y.p;
   if (y.planes == 1) {
     const fvec_t x = *(const fvec_t*)(p + i);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) v[e] = x[e];
-    return;
-  }
-  if (TWO && y.planes == 2) {
-    const fvec_t a = *(const fvec_t*)(p + i), b = *(const fvec_t*)(p + y.plane_stride + i);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) v[e] = a[e] + b[e];
     return;
   }
   fvec_t part[8];
@@ -256,8 +262,9 @@ __device__ __forceinline__ float block_sum_once(float x, float* red) {
 // The same for widths in multiples of 4 up to what a block's registers hold: pieces of 4 neighbouring elements (a
 // lane of the kernel above loads 4 bytes at a time, and a block of 1,024 threads per row leaves a compute unit two
 // rows in flight), 256 threads a row where rows are many, and two barriers in place of six. 2,047 rows of 2,560:
-// 38 -> 15 us (63 MB); 8 rows, with the planes of products cut along K: 6.1 -> 4.7.
-template <typename TO, int THREADS, int KEEP>
+// 38 -> 15 us (63 MB); 8 rows, with the planes of products cut along K: 6.1 -> 4.7. Two planes, what two experts a token
+// leave, have instances of their own (PLANES): the general way asks for eight, the first one again for those not there.
+template <typename TO, int THREADS, int KEEP, int PLANES>
 __global__ __launch_bounds__(THREADS) void norm_add_rmsnorm_wide_kernel(float* __restrict__ residual, Planes y,
                                                                         const float* __restrict__ w_after, float eps_after,
                                                                         const float* __restrict__ weight, float eps,
@@ -273,7 +280,7 @@ __global__ __launch_bounds__(THREADS) void norm_add_rmsnorm_wide_kernel(float* _
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     const int i = min((int)threadIdx.x * 4 + j * STRIDE, hidden - 4);  // beyond the row: its last piece, dropped below
-    planes_piece<4, true>(y, row + i, vy[j]);
+    planes_piece<4, PLANES>(y, row + i, vy[j]);
     vx[j] = *(const f32x4_t*)(residual + row + i);
     wa[j] = *(const f32x4_t*)(w_after + i);
     wn[j] = *(const f32x4_t*)(weight + i);
@@ -316,14 +323,21 @@ static bool norm_add_wide(float* residual, const Planes& y, const float* w_after
                           const int* rows, TO* out, int num_out, int hidden, hipStream_t stream) {
   const uintptr_t at = (uintptr_t)residual | (uintptr_t)y.p | (uintptr_t)w_after | (uintptr_t)weight | (uintptr_t)out;
   if (hidden % 4 || hidden > 4096 || y.plane_stride % 4 || at % 16) return false;
-#define GO(THREADS, KEEP)                                                                                                  \
-  norm_add_rmsnorm_wide_kernel<TO, THREADS, KEEP><<<num_out, THREADS, 0, stream>>>(residual, y, w_after, eps_after, weight, \
-                                                                                  eps, rows, out, hidden)
+  const bool two = y.code == QRT_F32 && y.planes == 2;
+#define LAUNCH(THREADS, KEEP, PLANES)                                                                                     \
+  norm_add_rmsnorm_wide_kernel<TO, THREADS, KEEP, PLANES><<<num_out, THREADS, 0, stream>>>(residual, y, w_after, eps_after, \
+                                                                                          weight, eps, rows, out, hidden)
+#define GO(THREADS, KEEP)                    \
+  do {                                       \
+    if (two) LAUNCH(THREADS, KEEP, 2);       \
+    else LAUNCH(THREADS, KEEP, 0);           \
+  } while (0)
   if (num_out < 512) GO(1024, 1);  // few rows: a piece a thread, one trip to memory
   else if (hidden <= 2048) GO(256, 2);
   else if (hidden <= 3072) GO(256, 3);
   else GO(256, 4);
 #undef GO
+#undef LAUNCH
   return true;
 }
 
