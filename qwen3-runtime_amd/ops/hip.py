@@ -509,9 +509,10 @@ class HipOps:
         return out
 
     # bfloat16 steps with more tokens than this whose rows are no whole pieces of 16 bytes take the per-head products
-    # to the vendor library (its right operand copied: transposed views of batches have faulted there); rows that
-    # are take the tile kernel at any number of tokens, which is faster than both (at 1 to 16 tokens 4.4 and
-    # 6.7 us against 5.1 to 8.4 and 9.0 to 18.3 of the kernel for few rows; at 33, 4.8 and 7.1 against 10.3 and 11.6)
+    # to the vendor library; rows that are take the tile kernel at any number of tokens, which is faster than both
+    # (at 1 to 16 tokens 4.4 and 6.7 us against 5.1 to 8.4 and 9.0 to 18.3 of the kernel for few rows; at 33, 4.8 and 7.1
+    # against 10.3 and 11.6). The library gets whole matrices and no views of batches: nothing here depends on what its
+    # batched product makes of their strides
     heads_linear_own_max_rows = 16
 
     def heads_linear(self, x, in_stride, in_offset, w, out, out_stride, out_offset):
@@ -530,7 +531,7 @@ class HipOps:
                  and (x.data_ptr() | w.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0)
         if not tiles and x.dtype == torch.bfloat16 and t > self.heads_linear_own_max_rows:
             src = x.view(t, -1)[:, : heads * in_stride].view(t, heads, in_stride)[:, :, in_offset: in_offset + k]
-            res = torch.bmm(src.transpose(0, 1), w.transpose(1, 2).contiguous())  # [heads, T, N]
+            res = torch.bmm(src.transpose(0, 1).contiguous(), w.transpose(1, 2).contiguous())  # [heads, T, N]
             out.view(t, -1)[:, : heads * out_stride].view(t, heads, out_stride)[:, :, out_offset: out_offset + n] = \
                 res.transpose(0, 1)
             return out
