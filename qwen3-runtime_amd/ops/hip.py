@@ -1636,6 +1636,22 @@ class HipOps:
         return max(1, min((max_kv + 255) // 256, (1024 + work - 1) // work, 64))
 
     @staticmethod
+    def choose_wide_splits(walks, nkv: int, row_bytes: float) -> int:
+        """The same for the kernel whose eight waves share keys and values (one block a compute unit, tiles of 128 rows, longest
+        first): ``walks`` holds the blocks of 32 keys of every tile, ``row_bytes`` the float32 results of all rows. A block of keys
+        takes 1.7 us, so a launch takes as long as its longest walk or a compute unit's share of all of them, and each part
+        more is written and read once more (at 5.2 TB/s, after some 5 us for the merge). 32 heads of 448 on one, us in 1, 2, 3 and 4
+        parts: 3 prompts of 300 tokens 34, 91, 107, 120; one of 1,000 73, 116, 138, 155; 200 tokens behind
+        3,800 215, 132, 100, 87; 8 tokens behind 4,000 beside a prompt of 500 166, 120, 109, 99."""
+        longest, share = max(walks), sum(walks) * nkv / 256
+        best, best_time = 1, None
+        for parts in range(1, max(1, min((longest + 1) // 2, 64)) + 1):
+            time = 1.7 * max(-(-longest // parts), share) + (5 + 2 * parts * row_bytes / 5.2e6 if parts > 1 else 0)
+            if best_time is None or time < best_time:
+                best, best_time = parts, time
+        return best
+
+    @staticmethod
     def choose_decode_splits(num_tiles: int, nkv: int, max_kv: int) -> int:
         """Decoding: blocks of four waves, two to a compute unit. The parts are chosen by a small
         model of the launch's time that the measurements fit: the busiest compute unit gets
@@ -1749,6 +1765,7 @@ class HipOps:
         plan = ctx.scratch.get(key)
         if plan is None:  # the same for every layer of the step
             dev = out.device
+            wide_splits = None
             if decode:
                 tiles = None if subset is None else torch.tensor(subset, dtype=torch.int32, device=dev)
                 n_tiles = len(q_lens)
@@ -1759,6 +1776,13 @@ class HipOps:
                 if (waves == 4 and widest > 256 and d % 64 == 0 and dv % 64 == 0 and not keep_first
                         and self.prefill_through_lds):
                     groups = 3  # eight waves of one tile of 16 rows each share keys and values through LDS
+                    walks = []
+                    for n, kv in zip(q_lens, kv_lens):
+                        for r in range(0, n * g, 128):
+                            first, last = kv - n + r // g, kv - n + (min(n * g, r + 128) - 1) // g
+                            lo = max(0, first - window + 1) if window else first - first % chunk if chunk else 0
+                            walks.append((last >> 5) - (lo >> 5) + 1)
+                    wide_splits = self.choose_wide_splits(walks, nkv, 4.0 * sum(q_lens) * nq * dv)
                 host, n_tiles = self.plan_tiles(q_lens, kv_lens, g, 128 if groups == 3 else 16 * waves * row_tiles, nkv,
                                                 self.resident_blocks if waves == 4 and row_tiles >= 2 and groups < 2
                                                 else 0, subset)
@@ -1768,10 +1792,10 @@ class HipOps:
                 cu = np.concatenate([[0], np.cumsum(ctx.q_lens_host)])
                 tokens = torch.from_numpy(np.concatenate([np.arange(cu[s], cu[s + 1]) for s in subset])
                                           .astype(np.int32)).to(dev)
-            plan = (tiles, n_tiles, tokens, 0 if decode else groups)
+            plan = (tiles, n_tiles, tokens, 0 if decode else groups, wide_splits)
             ctx.scratch[key] = plan
-        tiles, n_tiles, tokens, groups = plan
-        splits = ctx.scratch.get("attn_splits") or (
+        tiles, n_tiles, tokens, groups, wide_splits = plan
+        splits = ctx.scratch.get("attn_splits") or wide_splits or (
             self.choose_decode_splits(n_tiles, nkv, seen_kv) if decode else self.choose_splits(n_tiles, nkv, seen_kv, widest))
         a = _AttnTileArgs()
         a.chunk = chunk
