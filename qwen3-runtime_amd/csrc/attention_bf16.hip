@@ -1094,7 +1094,8 @@ __global__ __launch_bounds__(512, 1) void attention_bf16_wide_kernel(AttnTileArg
       for (int e = 0; e < 2; ++e) in[n % (AHEAD + 1)][e] = *(const bf16x8_t*)(at + value_at + 256 * (2 * n + e));
     };
 #pragma unroll
-    for (int n = 0; n < AHEAD; ++n) keys(n);
+    for (int n = 0; n < AHEAD; ++n)
+      if (n < KFULL) keys(n);
 #pragma unroll
     for (int n = 0; n < KFULL; ++n) {
       if (n + AHEAD < KFULL) keys(n + AHEAD);
@@ -1103,7 +1104,8 @@ __global__ __launch_bounds__(512, 1) void attention_bf16_wide_kernel(AttnTileArg
       for (int e = 0; e < 2; ++e) sc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in[n % (AHEAD + 1)][e], qreg[n], sc[e], 0, 0, 0);
     }
 #pragma unroll
-    for (int n = 0; n < AHEAD; ++n) values(n);
+    for (int n = 0; n < AHEAD; ++n)
+      if (n < DB / 2) values(n);
     if (a.cap_in > 0.f) cap_scores(sc, a.cap_in, a.cap_out);  // the same for the whole launch
     const bool whole = base + 31 <= tile_pos_min && base >= tile_lo_max;
     float mx = lane_max(sc);

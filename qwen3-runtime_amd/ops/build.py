@@ -181,7 +181,7 @@ def build_library(name: str, force: bool = False) -> Path:
 
 
 def build_all(head_dims=(16, 32, 48, 64, 80, 96, 112, 128, 160, 176, 192, 208, 256, 320, 448, 512),
-              value_dims=((16, 48), (32, 16), (32, 80), (64, 16), (64, 32), (64, 128), (80, 48), (128, 64), (256, 16)),
+              value_dims=((16, 48), (32, 16), (32, 80), (64, 16), (64, 32), (64, 128), (80, 48), (128, 64), (256, 16), (320, 64), (64, 320)),
               force: bool = True) -> list[Path]:
     """Every library the tests, the smoke run and the measurements load (head sizes above 256 are
     those of latent rows: latent plus turned key part; ``value_dims``: sizes of keys and values where they

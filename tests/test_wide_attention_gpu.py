@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from plain import ops_ref as R
-from test_kernels_gpu import build_attention_case, close
+from test_kernels_gpu import DEV, build_attention_case, close, rnd
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +39,42 @@ def test_portions_with_wide_heads(d, seqs, nq, ps, window, splits):
         cache.group.block_table = table
     got = ops.paged_attention(q, cache, ctx, nq, 1, d, scale, window)
     # as for the other head sizes: probabilities rounded to bfloat16, values of size 3
+    close(got, want, 2e-2, 2e-2)
+
+
+@pytest.mark.parametrize("d,dv,nq,nkv,splits,more", [
+    (448, 448, 32, 1, None, {"softcap": 3.0}),
+    (448, 448, 16, 1, 3, {"softcap": 3.0, "sink": True}),
+    (320, 320, 16, 1, None, {"chunk": 40}),
+    (320, 320, 16, 1, 2, {"chunk": 40, "gate": True}),
+    (448, 448, 8, 1, None, {"sink": True, "gate": True}),
+    (448, 448, 8, 1, None, {"turn": True}),
+    (320, 320, 8, 1, 2, {"turn": True, "sink": True}),
+    (320, 64, 32, 1, None, {}),                       # values narrower than the loads asked for ahead
+    (320, 64, 12, 3, 2, {"window": 50, "gate": True}),
+    (64, 320, 16, 2, None, {"sink": True}),           # and keys
+    (64, 320, 16, 2, 2, {"turn": True}),
+])
+def test_options_of_portions_with_wide_heads(d, dv, nq, nkv, splits, more):
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops, more = HipOps(), dict(more)
+    window = more.pop("window", None)
+    q, cache, ctx = build_attention_case([(70, 97), (9, 9), (1, 130), (33, 64)], nq, nkv, d, 16, torch.bfloat16, window=window, poison=dv == d)
+    if dv != d:
+        cache.v = rnd(cache.v.shape[0], nkv, dv, 16, dtype=torch.bfloat16, seed=7)
+    if splits:
+        ctx.scratch["attn_splits"] = splits
+    if more.pop("gate", False):
+        more["gate"] = rnd(ctx.num_tokens, nq * dv, dtype=torch.bfloat16, seed=9)
+    if more.pop("turn", False):
+        more["value_turn"] = (1e3 ** -(torch.arange(dv // 2, dtype=torch.float32, device=DEV) / (dv // 2)), "turned")
+    scale = 1.0 / math.sqrt(d)
+    want = R.paged_attention(q, cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, 16, nq, nkv, d,
+                             scale, window, value_dim=dv, **more)
+    got = ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window, value_dim=dv, **more)
+    assert next(p for k, p in ctx.scratch.items() if k[0] == "attn_plan")[3] == 3   # by the kernel that this file is about
+    # as above; a turned output is made of two of them
     close(got, want, 2e-2, 2e-2)
 
 
