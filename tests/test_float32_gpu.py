@@ -106,3 +106,19 @@ def test_a_first_key_of_no_weight_leaves_a_token_its_other_keys(ops):
     k, v = cache.k[page].cpu().double(), cache.v[page].cpu().double()
     p = torch.softmax((q.view(17, 2, 32)[16].cpu().double()[:, None, :] * k).sum(-1) * 0.2, -1)
     close(got, (p[:, None, :] * v).sum(-1).float(), 2e-5, 2e-5)
+
+
+@pytest.mark.parametrize("nq,nkv,d,window,keep", [(4, 2, 128, 40, 0), (6, 1, 64, 33, 0), (2, 2, 256, 50, 21), (8, 8, 16, 17, 5)])
+def test_attention_where_pages_in_front_of_the_window_were_given_back(ops, nq, nkv, d, window, keep):
+    seqs = [(1, 200), (30, 150), (70, 300), (5, 20)]
+    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, 16, torch.float32, window=window, poison=True)
+    attend = lambda: ops.paged_attention(q, cache, ctx, nq, nkv, d, d ** -0.5, window, keep_first=keep)  # noqa: E731
+    want = R.paged_attention(q.double(), cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, 16,
+                             nq, nkv, d, d ** -0.5, window, torch.float64, keep_first=keep)
+    table = cache.group.block_table.clone()
+    for s, (n, kv) in enumerate(seqs):
+        for p in range(-(-keep // 16), max(0, kv - n - window + 1) // 16):
+            cache.k[int(table[s, p])] = cache.v[int(table[s, p])] = float("nan")   # its next holder's
+            table[s, p] = -1
+    cache.group.block_table = table
+    close(attend(), want.float(), 2e-5, 2e-5)
