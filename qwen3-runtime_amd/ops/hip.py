@@ -1000,11 +1000,19 @@ class HipOps:
                                                      _stream()))
         return out
 
-    # Pairs per expert from which the experts' products go by tiles and not as a stream of the weights: 16 experts
-    # of 2,560 x 1,536, 2 a token, both products, us by the stream and by tiles: 77 and 95 at 64 tokens (8 pairs
-    # an expert), 104 and 97 at 96 (12), 263 and 114 at 512
-    experts_tile_pairs_per_expert = 11
+    # Pairs per expert from which the experts' products go by tiles and not as a stream of the weights (None: as
+    # ``choose_experts_tile_pairs`` says)
+    experts_tile_pairs_per_expert = None
     experts_rows_max_pairs = 8192  # the stream's blocks list their expert's pairs in LDS
+
+    @staticmethod
+    def choose_experts_tile_pairs(experts: int, inter: int) -> int:
+        """Tiles take about as long at 4 pairs an expert as at 32, the stream reads an expert's weights once more for every
+        16 pairs; and the fewer blocks the experts' tiles are, the longer those take beside the stream. Both products, us by
+        the stream and by tiles: 16 experts of 2,560 x 1,536 (384 tiles), 2 a token, at 8 pairs an expert 64 and 90, at 15
+        91 and 94, at 16 107 and 94, at 64 326 and 111; 64 of 2,048 x 768 (768 tiles), 8 a token, at 8 132 and 138, at 10 146 and
+        140, at 16 196 and 145; 8 of 4,096 x 1,024 (128 tiles) at 16 56 and 72, at 24 71 and 73, at 32 87 and 75."""
+        return min(32, max(8, 6000 // max(1, experts * inter // 64)))
 
     @staticmethod
     def experts_fit(x, hidden, inter, *weights) -> bool:
@@ -1037,7 +1045,10 @@ class HipOps:
         pairs = t * top
         act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
         scratch = None
-        if pairs >= self.experts_tile_pairs_per_expert * n or pairs > self.experts_rows_max_pairs:
+        tile_pairs = self.experts_tile_pairs_per_expert
+        if tile_pairs is None:
+            tile_pairs = self.choose_experts_tile_pairs(n, inter)
+        if pairs >= tile_pairs * n or pairs > self.experts_rows_max_pairs:
             scratch = torch.empty(pairs + n + 2 + 2 * (pairs // 128 + n), dtype=torch.int32, device=x.device)
         self._check(self.lib, self.lib.qrt_experts(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(index), _ptr(weight), _ptr(act),
                                                    _ptr(out), _ptr(scratch), c_int(t), c_int(h), c_int(inter), c_int(n),
