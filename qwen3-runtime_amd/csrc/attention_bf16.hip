@@ -980,8 +980,8 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void attention_bf16_prefil
 // MFMAs. Here eight waves, 128 rows, share each block of 32 keys through LDS, two stages filled by direct
 // loads (no registers on the way) during the products of the block before, one barrier a block. The LDS
 // reads, 57 KB a wave and block at 220 B/clk, then take about as long as the products. 2,047 tokens with 32
-// heads of 448: 789 -> 225 us without history, 2,190 -> 438 us with 2,048 tokens of it (0.76 PFLOP/s); LDS and matrix pipes
-// are busy a quarter of the time each: what is left is a wave's own chain, which two waves a SIMD do not hide.
+// heads of 448: 783 -> 155 us without history (0.78 PFLOP/s), 2,189 -> 372 us with 2,048 tokens of it (0.97); matrix pipes and LDS are
+// busy a quarter of the time each: what is left is a wave's own chain, which two waves a SIMD do not hide.
 // A stage holds the keys group by group as they lie in the cache, 8 rows of 2 D bytes, the 16-byte pieces of
 // key k of group p permuted within every 128 bytes (piece c at place c ^ (2 p + k / 2 % 2)), and the values
 // group by group as [DV][8 keys]: neither operand read then meets a bank twice, and a load's source is

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
 // O^T = V^T P^T takes against one 16-byte read of the transposed value page, so nothing crosses lanes but
 // the row's maximum. The kernel before it (a wave per token and head, a key's dot product per lane,
 // uncoalesced) is bound by load latency: 354 tokens of 2 sequences with 32 heads of 128 took 798 us, two
-// decoded tokens behind 267 keys 170 us; this one 43 and 25 us.
+// decoded tokens behind 267 keys 170 us; this one 49 and 19 us.
 // A sequence of few rows has eight waves a tile (its keys are what there is to share: a token behind 2,049 keys with
 // 32 heads of 128 on 8 takes 78 us, with four 161), any other four (16 prompts of 64 tokens 60 us, with eight 105); heads wider than
 // 128 always eight (2,048 tokens, 16 heads of 256 on 4: 910 us, with four 1,440). That goes by

@@ -20,8 +20,8 @@
 // of 16 lanes. Tokens are staged through LDS 16 at a time; the next tile's global loads are in
 // flight while a tile is walked, the walk has no global access and no branch between tokens, and
 // the tile's read-outs leave together afterwards. The order of the float32 operations per token
-// does not depend on how the tokens are cut into steps, tiles or batches. (Retention over prompts goes by
-// chunks instead: see retention_chunk_kernel.)
+// does not depend on how the tokens are cut into steps, tiles or batches. (Retention over long spans goes
+// by chunks instead: see retention_chunk_kernel.)
 #include "common.h"
 #include <math.h>
 #include <type_traits>
@@ -202,8 +202,8 @@ __global__ __launch_bounds__(256) void retention_kernel(RetentionArgs a) {
 //   S  <- d^n S + sum over j of d^(n-1-j) k_j v_j^T
 //
 // Walked token by token the recurrence was bound by its chain: one wave a SIMD, 187 ns a token (32 heads of 128 x
-// 128, 2,047 tokens: 383 us). In chunks that case takes 160 us, 2.5 us a chunk, of which 1.1 are matrix products and the
-// rest the way from LDS through them and back to it (3 heads of 32: 314 -> 117; 16 of 256: 590 -> 273).
+// 128, 2,047 tokens: 386 us). In chunks that case takes 155 us, 2.4 us a chunk, of which 1.1 are matrix products and the
+// rest the way from LDS through them and back to it (4 heads of 32: 315 -> 116; 16 of 256: 590 -> 257).
 // Error against 64 bits of the same case: 1.1e-7 to 1.4e-7 by the head's decay, walked 1.1e-7 to 3.9e-7.
 // A block owns 16 columns of one head's state, as above; each of its NW waves owns 16 G of the state's rows
 // in accumulators, and because all of o is linear in the sums over rows, a wave carries its share of both terms
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64 * NW, LEAN ? 4 : 1) void retention_chunk_kernel(
     s[g] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     if (d < dim && col_ok) s[g] = *(const f32x4_t*)(st + d);
   }
-  // the pieces of the next two chunks, on their way while one is walked (1.7 us a chunk; a load takes about one); what lies beyond the head or the tokens becomes
+  // the pieces of the next two chunks (LEAN: of the next), on their way while one is walked (2.4 us a chunk; a load takes about one); what lies beyond the head or the tokens becomes
   // zero only on its way to LDS: a choice here would wait for the loads
   struct Ahead {
     f32x4_t q[PIECES], k[PIECES];
