@@ -1012,13 +1012,17 @@ class HipOps:
         the stream and by tiles: 16 experts of 2,560 x 1,536 (384 tiles), 2 a token, at 8 pairs an expert 64 and 90, at 15
         91 and 94, at 16 107 and 94, at 64 326 and 111; 64 of 2,048 x 768 (768 tiles), 8 a token, at 8 132 and 138, at 10 146 and
         140, at 16 196 and 145; 8 of 4,096 x 1,024 (128 tiles) at 16 56 and 72, at 24 71 and 73, at 32 87 and 75."""
-        return min(32, max(8, 6000 // max(1, experts * inter // 64)))
+        return min(32, max(9, 6000 // (experts * inter // 64 or 1)))
 
     @staticmethod
     def experts_fit(x, hidden, inter, *weights) -> bool:
         """Whether the experts' MFMA kernels take these operands (rows of whole cache lines, 16 bytes a load)."""
-        return (x.dtype == torch.bfloat16 and hidden % 64 == 0 and inter % 64 == 0
-                and all(a.data_ptr() % 16 == 0 for a in (x, *weights)))
+        if x.dtype != torch.bfloat16 or hidden % 64 or inter % 64:
+            return False
+        at = x.data_ptr()
+        for w in weights:
+            at |= w.data_ptr()
+        return at % 16 == 0
 
     def moe_for_residual(self, x, gate_up, down, index, weight, activation="swiglu", limit=0.0, weight_on_input=False,
                          out=None):

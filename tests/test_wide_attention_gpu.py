@@ -76,16 +76,3 @@ def test_options_of_portions_with_wide_heads(d, dv, nq, nkv, splits, more):
     assert next(p for k, p in ctx.scratch.items() if k[0] == "attn_plan")[3] == 3   # by the kernel that this file is about
     # as above; a turned output is made of two of them
     close(got, want, 2e-2, 2e-2)
-
-
-@pytest.mark.parametrize("d", [320, 448])
-def test_how_many_parts_the_keys_of_portions_with_wide_heads_are_cut_into(d):
-    from qwen3_runtime_amd.ops.hip import HipOps
-
-    def parts(*seqs):
-        walks = [((kv - n + (min(32 * n, r + 128) - 1) // 32) >> 5) + 1 for n, kv in seqs for r in range(0, 32 * n, 128)]
-        return HipOps.choose_wide_splits(walks, 1, 4.0 * sum(n for n, _ in seqs) * 32 * d)
-
-    assert parts((300, 300), (300, 300), (300, 300)) == parts((1000, 1000)) == parts(*[(150, 150)] * 5) == 1
-    assert parts((1000, 3000), *[(1, 200)] * 8) == 1
-    assert 3 <= parts((200, 4000)) <= 6 and parts((33, 8000)) >= 10
