@@ -1678,17 +1678,23 @@ class HipOps:
         least 8 key blocks of 32 a part, at most 64 parts (what the merge kernel reads with every
         load in flight); but up to 16 parts may have 2 key blocks each: a compute unit pulls no more
         than some 34 GB/s however many waves it runs, so few sequences of short contexts want many
-        units (attention and merge, us: 320 keys, 6 sequences 14.1 in 1 or 2 parts, 11.5 in 4, 12.0 in 5; one
-        sequence of 640 keys 15.1 in 2 parts, 10.5 in 10, of 1,025 keys 14.8 in 4, 11.1 in 16; 32 sequences of
-        320 keys 16.2 in 1 part, 19.9 in 2, which the model knows)."""
+        units (attention and merge, us: one sequence of 640 keys 12.0 in 2 parts, 8.1 in 10, of 1,025 keys 11.9 in 4, 9.2 in
+        16; 320 keys, 6 sequences 10.3 in 1 part, 8.7 in 5). Where one part was the choice before these, the merge is a launch
+        more, as long as a walk over 180 keys: 128 keys, any few sequences 6.6 in 1 part, 8.1 to 8.5 in 2; 48 sequences
+        of 320 keys 16.8 and 21.1; 16 of 200 8.8 and 9.8."""
         work = num_tiles * nkv
         blocks = (max_kv + 31) // 32
         cost = 0.06 * 2100 / max(max_kv, 1)
-        best, best_time = 1, None
-        for parts in range(1, max(1, min(blocks // 8, 64), min(blocks // 2, 16)) + 1):
-            time = -(-work * parts // 256) * (1.0 / parts + cost)
-            if best_time is None or time < best_time * 0.999:
-                best, best_time = parts, time
+        time = lambda parts: -(-work * parts // 256) * (1.0 / parts + cost)  # noqa: E731
+        best, long_parts = 1, max(1, min(blocks // 8, 64))
+        for parts in range(2, long_parts + 1):
+            if time(parts) < time(best) * 0.999:
+                best = parts
+        merge = 180.0 / max(max_kv, 1) if best == 1 else 0.0
+        best_time = time(best)
+        for parts in range(long_parts + 1, min(blocks // 2, 16) + 1):
+            if time(parts) + merge < best_time * 0.999:
+                best, best_time = parts, time(parts) + merge
         return best
 
     # decoding over unequal lengths: from this ratio of the longest to the mean length on, pieces

@@ -5,6 +5,15 @@ import pytest
 from qwen3_runtime_amd.ops.hip import HipOps
 
 
+@pytest.mark.parametrize("sequences,keys,parts", [
+    (1, 128, (1, 1)), (1, 200, (1, 1)), (8, 128, (1, 1)), (16, 200, (1, 1)), (48, 320, (1, 1)),     # the merge costs more than it saves
+    (1, 320, (4, 8)), (6, 320, (4, 5)), (1, 640, (8, 16)), (1, 1025, (16, 16)), (8, 1025, (4, 4)),  # few sequences: many units
+    (12, 2100, (2, 5)), (24, 2100, (4, 4)), (32, 2049, (1, 1)), (40, 2100, (4, 4)),
+])
+def test_parts_of_decoded_tokens_keys(sequences, keys, parts):
+    assert parts[0] <= HipOps.choose_decode_splits(sequences, 8, keys) <= parts[1]
+
+
 @pytest.mark.parametrize("experts,inter,pairs", [(16, 1536, 15), (64, 768, 9), (8, 1024, 32), (4, 512, 32), (1024, 64, 9), (1, 64, 32)])
 def test_pairs_an_expert_from_which_tiles_are_taken(experts, inter, pairs):
     assert HipOps.choose_experts_tile_pairs(experts, inter) == pairs
