@@ -577,17 +577,17 @@ class HipOps:
         a.cu_q = _need(ctx.cu_q, "cu_q", torch.int32, (ctx.num_seqs + 1,)).data_ptr()
         a.state_slots = _need(ctx.state_slots, "state_slots", torch.int32, (ctx.num_seqs,)).data_ptr()
         a.heads, a.dim, a.vdim = heads, dim, vdim
-        if dim % 4 == 0 and dim <= 256 and c % 4 == 0 and (a.qkv | a.state) % 16 == 0:
+        if t >= self.retention_chunk_min_tokens and dim % 4 == 0 and dim <= 256 and c % 4 == 0 and (a.qkv | a.state) % 16 == 0:
             # a context without its lengths on the host: both forms are launched where both may have work
             lens = getattr(ctx, "q_lens_host", None) or ([t] if ctx.num_seqs == 1 else [0, t])
-            a.chunk_from, a.shortest, a.longest = self.retention_chunk_min_tokens[dim > 128], min(lens), max(lens)
+            a.chunk_from, a.shortest, a.longest = self.retention_chunk_min_tokens, min(lens), max(lens)
         self._check(self.lib, self.lib.qrt_retention(byref(a), c_int(t), c_int(ctx.num_seqs), c_int(state.shape[0]), _stream()))
         return out
 
-    # spans of at least this many tokens run chunk by chunk (heads of up to 128 elements, wider ones). By the span alone, never
-    # by the step: 32 heads of 128, us token by token and by chunks, 1 sequence of 48 tokens 12.5 and 9.5, of 64 15.5 and 9.5,
-    # 8 of 48 31 and 42, of 64 39 and 42, of 500 288 and 281; 16 heads of 256, 1 of 64 23 and 12, 8 of 64 74 and 82
-    retention_chunk_min_tokens = (64, 128)
+    # spans of at least this many tokens run chunk by chunk: by the span alone, never by the step. us token by token and by chunks,
+    # 32 heads of 128, 1 sequence of 64 tokens 15.5 and 9.5, of 128 27 and 14, of 512 99 and 42; 8 sequences of 64 39 and 42, of 100
+    # 61 and 75, of 128 73 and 78, of 500 288 and 281; 16 heads of 256, 1 of 128 41 and 20, 8 of 128 139 and 154, of 500 528 and 530
+    retention_chunk_min_tokens = 128
 
     def state_space(self, ctx, xbc, step, step_bias, a_log, skip, state, heads, groups, n, vdim):
         """Per sequence and head from the slot's state (float32 [slots, heads, vdim, n], updated in place):

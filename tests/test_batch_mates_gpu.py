@@ -48,7 +48,7 @@ def test_float32_attention(ops, nq, nkv, d, more):
 
 
 @pytest.mark.parametrize("dim,vdim", [(64, 32), (128, 40), (200, 16)])
-@pytest.mark.parametrize("lengths", [(1, 1, 300, 1), (63, 64, 65, 127, 128, 1), (2,) * 40 + (133,), (70,) * 160])
+@pytest.mark.parametrize("lengths", [(1, 1, 300, 1), (63, 64, 65, 127, 128, 1), (2,) * 40 + (133,), (130,) * 160])
 def test_retention(ops, dim, vdim, lengths):
     heads, t = 3, sum(lengths)
     qkv, state = rnd(t, 2 * heads * dim + heads * vdim, seed=1), rnd(len(lengths), heads, vdim, dim, seed=2)

@@ -63,16 +63,24 @@ def test_chunks_match_the_recurrence(ops, dim, vdim, heads, lengths, decay):
     assert ((after.double() - states).abs() <= steps * EPS * sizes).all()
 
 
+@pytest.fixture(scope="module")
+def chunking():
+    """Spans of any length by chunks."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops = HipOps()
+    ops.retention_chunk_min_tokens = 1
+    return ops
+
+
 @pytest.mark.parametrize("lengths,heads,dim,vdim", [((1,), 1, 4, 1), ((31,), 3, 60, 16), ((32, 33, 2), 2, 68, 17), ((65, 3), 2, 256, 33),
                                                     ((33, 1, 64, 97) * 3, 4, 68, 128), ((33, 1, 64, 97) * 3, 9, 60, 128)])
-def test_every_form_of_the_chunks_matches_the_recurrence(ops, lengths, heads, dim, vdim):
+def test_every_form_of_the_chunks_matches_the_recurrence(chunking, lengths, heads, dim, vdim):
     """Spans of any length by chunks, in launches of few blocks and of many (the last two)."""
     decay = (0.9, -0.7, 1.0, 0.5)
     qkv, d, state, slots = _draw(lengths, heads, dim, vdim, decay)
     out, out_sizes, states, sizes = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
-    ops = type(ops)()
-    ops.retention_chunk_min_tokens = (1, 1)
-    got, after = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    got, after = _run(chunking, lengths, qkv, d, state, slots, heads, dim, vdim)
     steps = 2 * max(lengths) + dim + 8
     assert ((got.double() - out).abs() <= steps * EPS * out_sizes).all()
     assert ((after.double() - states).abs() <= steps * EPS * sizes).all()
@@ -95,7 +103,7 @@ def test_a_value_that_is_not_finite_stays_behind_its_token(ops, which, value):
 
 @pytest.mark.parametrize("size", [1e30, 3e37, float("inf")])
 @pytest.mark.parametrize("where", ["state", "k", "v"])
-def test_what_a_large_state_holds_decays_as_in_the_recurrence(ops, size, where):
+def test_what_a_large_state_holds_decays_as_in_the_recurrence(chunking, size, where):
     """Read-outs and states that the recurrence keeps finite are finite and right, and one that became infinite stays so."""
     heads, dim, vdim, lengths = 4, 64, 20, (80,)
     qkv, d, state, slots = _draw(lengths, heads, dim, vdim, (0.0, 0.1, 0.5, 0.999))
@@ -105,7 +113,7 @@ def test_what_a_large_state_holds_decays_as_in_the_recurrence(ops, size, where):
     else:
         qkv[9, {"k": slice(heads * dim + 2, 2 * heads * dim, dim), "v": slice(2 * heads * dim + 2, None, vdim)}[where]] *= size
     out, out_sizes, _, _ = _recurrence(lengths, qkv, d, state, slots, heads, dim, vdim)
-    got, after = _run(ops, lengths, qkv, d, state, slots, heads, dim, vdim)
+    got, after = _run(chunking, lengths, qkv, d, state, slots, heads, dim, vdim)
     steps = 2 * max(lengths) + dim + 8
     fine = torch.isfinite(out) & (out_sizes < 1e37)
     if not math.isinf(size):
@@ -118,3 +126,9 @@ def test_what_a_large_state_holds_decays_as_in_the_recurrence(ops, size, where):
     last = after[int(slots[0])]
     assert torch.equal(torch.isnan(last), torch.isnan(walked))
     assert torch.equal(last[torch.isinf(walked)], walked[torch.isinf(walked)])
+
+
+@pytest.mark.parametrize("which", ["k", "v", "q"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 1e30])
+def test_a_value_that_is_not_finite_stays_behind_its_token_in_chunks(chunking, which, value):
+    test_a_value_that_is_not_finite_stays_behind_its_token(chunking, which, value)
