@@ -169,7 +169,8 @@ __global__ __launch_bounds__(256) void rotate_half_kernel(RotateArgs a) {
 
 // The rotation of halves by pieces of 8 elements, a token's sines and cosines made once for all its heads (the kernel
 // above makes them for every element, in float64 up to the reduced angle, which is what it takes its time for): 2,047
-// tokens, 64 heads of 128 into float32 44 -> 19 us.
+// tokens, 64 heads of 128 into float32 44 -> 19 us. A few tokens of which little turns are spread wider by the kernel above
+// (8 tokens, 32 heads of 192, 64 of them turned: 2.5 us there, 3.1 here).
 #define ROTATE_MAX_PAIRS 512
 template <typename TI, typename TO>
 __global__ __launch_bounds__(256) void rotate_half_wide_kernel(RotateArgs a) {
@@ -228,7 +229,7 @@ extern "C" int qrt_rotate_half(const RotateArgs* args, int in_dtype, int out_dty
   if (num_tokens == 0) return 0;
   const int total = a.heads * a.width;
   const dim3 grid(num_tokens, num_tokens >= 512 ? 1 : min((total + 255) / 256, 64));
-  const bool pieces = !a.neighbours && a.pairs <= ROTATE_MAX_PAIRS &&
+  const bool pieces = !a.neighbours && a.pairs <= ROTATE_MAX_PAIRS && (num_tokens > 8 || 2 * a.pairs == a.width) &&
                       (a.pairs | a.width | a.in_stride | a.in_offset | a.out_stride | a.out_offset) % 8 == 0 &&
                       a.x_row % 8 == 0 && a.out_row % 8 == 0 && ((uintptr_t)a.x | (uintptr_t)a.out) % 16 == 0;
   if (pieces && in_dtype <= QRT_BF16 && out_dtype <= QRT_BF16 && !(in_dtype == QRT_F32 && out_dtype == QRT_BF16)) {
