@@ -73,11 +73,12 @@ def test_retention(ops, dim, vdim, lengths):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("hidden", [64, 1000, 5120])
-def test_router_and_its_gate(ops, dtype, hidden):
-    """Steps of 256 tokens and more share the router's rows among tokens; a token's choice, weights and gate are the same."""
-    x, router = rnd(270, hidden, dtype=dtype, seed=1), rnd(17, hidden, seed=2, scale=2.0 * hidden ** -0.5)
-    whole = ops.route_top(x, router, None, 3, scoring="sigmoid", gate_row=True)
-    for a, b in ((0, 1), (5, 13), (265, 270)):
-        part = ops.route_top(x[a:b].contiguous(), router, None, 3, scoring="sigmoid", gate_row=True)
+@pytest.mark.parametrize("hidden", [64, 1000, 2560, 5120])
+@pytest.mark.parametrize("how", [{"scoring": "sigmoid"}, {"scoring": "softmax_all", "groups": 4, "keep": 2, "group_score": "max"}, {}])
+def test_router_and_its_gate(ops, dtype, hidden, how):
+    """Steps of many tokens share the router's rows among eight; a token's choice, weights and gate are the same."""
+    x, router = rnd(805, hidden, dtype=dtype, seed=1), rnd(17, hidden, seed=2, scale=2.0 * hidden ** -0.5)
+    whole = ops.route_top(x, router, None, 3, gate_row=True, **how)
+    for a, b in ((0, 1), (5, 13), (300, 805)):
+        part = ops.route_top(x[a:b].contiguous(), router, None, 3, gate_row=True, **how)
         assert all(torch.equal(p, w[a:b]) for p, w in zip(part, whole))
