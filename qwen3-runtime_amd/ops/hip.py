@@ -511,7 +511,8 @@ class HipOps:
     # bfloat16 steps with more tokens than this whose rows are no whole pieces of 16 bytes take the per-head products
     # to the vendor library; rows that are take the tile kernel at any number of tokens, which is faster than both
     # (at 1 to 16 tokens 4.4 and 6.7 us against 5.1 to 8.4 and 9.0 to 18.3 of the kernel for few rows; at 33, 4.8 and 7.1
-    # against 10.3 and 11.6). The library gets whole matrices and no views of batches: nothing here depends on what its
+    # against 10.3 and 11.6), up to the 16,384 elements a head and 65,535 heads that the entry point of the own kernels
+    # takes. The library gets whole matrices and no views of batches: nothing here depends on what its
     # batched product makes of their strides
     heads_linear_own_max_rows = 16
 
@@ -526,7 +527,8 @@ class HipOps:
         if (heads * in_stride > x.shape[1] or in_offset + k > in_stride or heads * out_stride > out.shape[1]
                 or out_offset + n > out_stride):
             raise OpsError(f"heads_linear: {heads} heads of {in_stride} in rows of {x.shape[1]}, of {out_stride} in rows of {out.shape[1]}")
-        tiles = (x.dtype == torch.bfloat16 and k % 64 == 0 and n % 4 == 0 and (x.shape[1] | in_stride | in_offset) % 8 == 0
+        tiles = (x.dtype == torch.bfloat16 and k % 64 == 0 and k <= 16384 and heads <= 65535 and n % 4 == 0
+                 and (x.shape[1] | in_stride | in_offset) % 8 == 0
                  and (out.shape[1] | out_stride | out_offset) % 4 == 0
                  and (x.data_ptr() | w.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0)
         if not tiles and x.dtype == torch.bfloat16 and t > self.heads_linear_own_max_rows:

@@ -123,6 +123,10 @@ def test_heads_linear_by_tiles(ops, tokens, heads, n, k, in_stride, in_offset, o
     assert (got[:, :, outside] == 7.0).all()
 
 
+def test_heads_wider_than_the_own_kernels_take_are_still_multiplied(ops):
+    test_heads_linear_by_tiles(ops, 17, 1, 8, 16448, 16448, 0, 8, 0)
+
+
 @pytest.mark.parametrize("tokens,heads,vdim", [(1, 1, 8), (3, 5, 24), (7, 3, 128), (33, 2, 512), (5, 2, 520), (65, 3, 40)])
 @pytest.mark.parametrize("gate_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.float32, torch.bfloat16)])
 @pytest.mark.parametrize("kind", ["silu", "sigmoid"])
