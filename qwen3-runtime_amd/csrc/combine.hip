@@ -247,15 +247,37 @@ __device__ __forceinline__ void planes_piece(const Planes& y, size_t i, float* v
   }
 }
 
-// The sum over a block of THREADS threads with one barrier: every thread adds up the waves' sums, in order.
-template <int THREADS>
-__device__ __forceinline__ float block_sum_once(float x, float* red) {
-  x = wave_sum(x);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+// wave_sum with the same additions, lanes 32, 16, 8, 4, 2 and 1 apart, but by swaps and rotations of registers: after each of
+// them lanes that far apart hold the same, so a rotation within 16 lanes brings the partner's.
+__device__ __forceinline__ float wave_sum_in_registers(float x) {
+  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+  const unsigned int u = __float_as_uint(x);
+  const u32x2_t a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const unsigned int v = __float_as_uint(x);
+  const u32x2_t b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  x = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, true));  // row_ror:8
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, true));  // row_ror:4
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xF, 0xF, true));  // row_ror:2
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xF, 0xF, true));  // row_ror:1
+  return x;
+}
+
+// The sum of N values a thread over a block of THREADS threads, with one barrier. The parts are added in the order of the
+// elements, 64 threads' pieces of the row at a time, so that a block of a quarter of the threads with four pieces each sums as the whole one.
+template <int THREADS, int N>
+__device__ __forceinline__ float block_sum_once(const float* x, float* red) {
+  float z[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) z[j] = wave_sum_in_registers(x[j]);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int j = 0; j < N; ++j) red[j * (THREADS / 64) + (threadIdx.x >> 6)] = z[j];
   __syncthreads();
   float s = 0.f;
 #pragma unroll
-  for (int w = 0; w < THREADS / 64; ++w) s += red[w];
+  for (int w = 0; w < N * THREADS / 64; ++w) s += red[w];
   return s;
 }
 
@@ -271,7 +293,7 @@ __global__ __launch_bounds__(THREADS) void norm_add_rmsnorm_wide_kernel(float* _
                                                                         const int* __restrict__ rows, TO* __restrict__ out, int hidden) {
   typedef TO ovec_t __attribute__((ext_vector_type(4)));
   constexpr int STRIDE = THREADS * 4;
-  __shared__ float red[2][THREADS / 64];
+  __shared__ float red[2][KEEP * THREADS / 64];
   const int b = blockIdx.x;
   const int r = rows ? rows[b] : b;
   const size_t row = (size_t)r * hidden;
@@ -285,27 +307,29 @@ __global__ __launch_bounds__(THREADS) void norm_add_rmsnorm_wide_kernel(float* _
     wa[j] = *(const f32x4_t*)(w_after + i);
     wn[j] = *(const f32x4_t*)(weight + i);
   }
-  float sy = 0.f;
+  float sums[KEEP];
 #pragma unroll
-  for (int j = 0; j < KEEP; ++j)
+  for (int j = 0; j < KEEP; ++j) {
+    sums[j] = 0.f;
     if ((int)threadIdx.x * 4 + j * STRIDE < hidden)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sy += vy[j][e] * vy[j][e];
-  const float iy = 1.0f / sqrtf(block_sum_once<THREADS>(sy, red[0]) / (float)hidden + eps_after);
-  float sx = 0.f;
+      for (int e = 0; e < 4; ++e) sums[j] += vy[j][e] * vy[j][e];
+  }
+  const float iy = 1.0f / sqrtf(block_sum_once<THREADS, KEEP>(sums, red[0]) / (float)hidden + eps_after);
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     const int i = threadIdx.x * 4 + j * STRIDE;
+    sums[j] = 0.f;
     if (i < hidden) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         vx[j][e] += vy[j][e] * iy * wa[j][e];
-        sx += vx[j][e] * vx[j][e];
+        sums[j] += vx[j][e] * vx[j][e];
       }
       if (!rows) *(f32x4_t*)(residual + row + i) = vx[j];
     }
   }
-  const float ix = 1.0f / sqrtf(block_sum_once<THREADS>(sx, red[1]) / (float)hidden + eps);
+  const float ix = 1.0f / sqrtf(block_sum_once<THREADS, KEEP>(sums, red[1]) / (float)hidden + eps);
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     const int i = threadIdx.x * 4 + j * STRIDE;

@@ -82,3 +82,21 @@ def test_router_and_its_gate(ops, dtype, hidden, how):
     for a, b in ((0, 1), (5, 13), (300, 805)):
         part = ops.route_top(x[a:b].contiguous(), router, None, 3, gate_row=True, **how)
         assert all(torch.equal(p, w[a:b]) for p, w in zip(part, whole))
+
+
+@pytest.mark.parametrize("hidden", [64, 1000, 2048, 2560, 4096, 4100])
+@pytest.mark.parametrize("planes", [1, 2, 4])
+def test_norm_behind_a_sublayer(ops, hidden, planes):
+    """Steps of many tokens take a quarter of the threads a row; a token's sums are the same."""
+    t = 700
+    y = rnd(t, hidden, seed=1) if planes == 1 else rnd(planes, t, hidden, seed=1)
+    residual, after, weight = rnd(t, hidden, seed=2), rnd(hidden, seed=3), rnd(hidden, seed=4)
+    norm = lambda r, y, **more: ops.add_rmsnorm(r, y, weight, 1e-5, torch.float32, delta_norm=(after, 1e-6), **more)  # noqa: E731
+    whole_r = residual.clone()
+    whole = norm(whole_r, y)
+    for a, b in ((0, 1), (5, 13), (100, 600)):
+        part_r = residual[a:b].clone()
+        part = norm(part_r, y[..., a:b, :].contiguous())
+        assert torch.equal(part, whole[a:b]) and torch.equal(part_r, whole_r[a:b])
+    rows = torch.tensor([3, 699, 4], dtype=torch.int32, device=DEV)
+    assert torch.equal(norm(residual.clone(), y, rows=rows), whole[rows.long()])
