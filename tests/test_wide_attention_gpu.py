@@ -1,6 +1,7 @@
 """Prompt portions with heads wider than 256 (rows of a latent): the kernel whose eight waves share keys and
 values through LDS, at the edges of its tiles of 128 rows and blocks of 32 keys."""
 
+import copy
 import math
 
 import pytest
@@ -76,3 +77,43 @@ def test_options_of_portions_with_wide_heads(d, dv, nq, nkv, splits, more):
     assert next(p for k, p in ctx.scratch.items() if k[0] == "attn_plan")[3] == 3   # by the kernel that this file is about
     # as above; a turned output is made of two of them
     close(got, want, 2e-2, 2e-2)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("d,nq,splits,more", [(448, 32, None, {}), (448, 4, 3, {"window": 40}), (320, 16, 2, {"chunk": 32}),
+                                              (320, 5, None, {"window": 23, "turn": True, "sink": True, "softcap": 3.0, "gate": True}),
+                                              (512, 2, 2, {"turn": True, "sink": True})])
+def test_a_token_takes_nothing_from_keys_it_does_not_see(value, d, nq, splits, more):
+    """A value and a key of one token that are not finite: tokens that do not see it are as they are without it."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops, more, n = HipOps(), dict(more), 75
+    window = more.pop("window", None)
+    q, cache, ctx = build_attention_case([(n, n), (9, n)], nq, 1, d, 16, torch.bfloat16)
+    if splits:
+        ctx.scratch["attn_splits"] = splits
+    if more.pop("gate", False):
+        more["gate"] = rnd(ctx.num_tokens, nq * d, dtype=torch.bfloat16, seed=9)
+    if more.pop("turn", False):
+        more["value_turn"] = (1e3 ** -(torch.arange(d // 2, dtype=torch.float32, device=DEV) / (d // 2)), "turned")
+    attend = lambda cache: ops.paged_attention(q, cache, ctx, nq, 1, d, d ** -0.5, window, **more)  # noqa: E731
+    want, pos = attend(cache), torch.cat([torch.arange(n), torch.arange(n - 9, n)]).to(DEV)
+    assert next(p for k, p in ctx.scratch.items() if k[0] == "attn_plan")[3] == 3
+    assert torch.isfinite(want).all()
+    for at in (0, 3, 31, 37, 74):
+        sees = pos >= at
+        if window:
+            sees &= pos - at < window
+        if "chunk" in more:
+            sees &= pos // 32 == at // 32
+        for stream in ("v", "k"):
+            odd = copy.copy(cache)
+            odd.k, odd.v = cache.k.clone(), cache.v.clone()
+            for s in (0, 1):
+                page, off = int(cache.group.block_table[s, at // 16]), at % 16
+                if stream == "v":
+                    odd.v[page, :, d - 1, off] = value
+                else:
+                    odd.k[page, :, off, 0] = value
+            # one rounding to bfloat16 of results whose probabilities were rounded to it, or were not
+            close(attend(odd)[~sees], want[~sees], 2e-2, 2e-2)
