@@ -10,6 +10,7 @@
 // by side along N. Skinny M (decode) uses MT = 1.
 #include "common.h"
 #include "direct.h"
+#include "gemm_epilogue.h"
 #include <type_traits>
 
 template <bool ALIGNED>
@@ -27,21 +28,6 @@ __device__ __forceinline__ bf16x8_t load_k8(const bf16_t* __restrict__ row, int 
   }
   return v;
 }
-
-// What the gated products do with a gate and an up value (their template's GATED: 0 no gate, 1 SwiGLU and
-// nothing else, 2 what is given here): an activation of common.h, times a factor per row of the
-// activations (null: 1).
-struct GatedEpilogue {
-  int kind;
-  float limit;
-  const float* row_scale;
-  template <int GATED>
-  __device__ __forceinline__ float apply(float g, float u, int m) const {
-    if (GATED == 1) return gated_act(g, u, QRT_ACT_SWIGLU, 0.f);
-    const float v = gated_act(g, u, kind, limit);
-    return row_scale ? v * row_scale[m] : v;
-  }
-};
 
 template <int MT, int NT, bool ALIGNED, typename TO>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
@@ -421,14 +407,6 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
   if (tiles >= 384 && K <= 4096) return launch_rows<4, 2, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (tiles >= 384) return launch_rows<4, 1, 4, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   return launch_rows<4, 1, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-}
-
-__device__ __forceinline__ void store4(float* p, const float (&o)[4]) {
-  *(f32x4_t*)p = (f32x4_t){o[0], o[1], o[2], o[3]};
-}
-__device__ __forceinline__ void store4(bf16_t* p, const float (&o)[4]) {
-  typedef bf16_t bf16x4_t __attribute__((ext_vector_type(4)));
-  *(bf16x4_t*)p = (bf16x4_t){(bf16_t)o[0], (bf16_t)o[1], (bf16_t)o[2], (bf16_t)o[3]};
 }
 
 // A page of zeros for a wave that has no tile of its own: read at no cost in memory traffic.

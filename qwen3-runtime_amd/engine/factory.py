@@ -73,7 +73,7 @@ def load(model_dir: str | Path | None, engine: EngineConfig, *, source=None, raw
 
         if device.type != "cuda":
             raise RuntimeError("the engine runs on a GPU only; there is no CPU path")
-        ops = HipOps()
+        ops = HipOps(residual_planes=True)  # parts give its results to norms
     loader = load_model(model, source, device, dtype, where=f" in {model_dir}" if model_dir else "")
     num_pages = engine.num_pages or pages_for_memory(model, engine, dtype, device)
     cache = CacheManager(

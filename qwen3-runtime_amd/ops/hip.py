@@ -8,15 +8,17 @@ tensors on the GPU; outputs are allocated with torch's caching allocator.
 
 Matrix products: float32 goes to the library's own float32 MFMA kernels
 (true 32-bit). bfloat16 with up to 64 rows (128 for the gated product and for
-products cut along K) goes to the library's MFMA kernels, which stream the
-weights; bfloat16 with more rows goes to the vendor BLAS through
-``torch.matmul``, as the reference leaves its products to cuBLAS
-(qwen3_runtime/models/qwen3.py:76-77,134-135).
+products cut along K) goes to the library's MFMA kernels that stream the
+weights, bfloat16 with more rows to its tiles through LDS; what those do not
+take (K no multiple of 64, weight rows no multiple of 16, operands off 16
+bytes) goes to the vendor BLAS through ``torch.matmul``, as the reference
+leaves its products to cuBLAS (qwen3_runtime/models/qwen3.py:76-77,134-135).
 """
 
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from ctypes import POINTER, Structure, byref, c_float, c_int, c_long, c_void_p
 
@@ -250,8 +252,22 @@ def _need(t: torch.Tensor, name: str, dtype=None, shape=None) -> torch.Tensor:
 check_tensor = _need  # for parts that call a library of their own
 
 
+# The tiles of csrc/gemm_tiles.hip in the order of their numbers there: rows, columns, blocks a compute unit holds at
+# once, and what a launch takes, in microseconds: 3, and for every round of blocks over the compute units c, and for each
+# of its stages of 64 columns of K a, and b more where the round is full (fewer blocks share the caches and the clock).
+# Least squares over 3,600 launches: the q/k/v, output, gate/up and down sizes of the 4B, 8B and 32B models with 65 to
+# 4,096 rows, whole and in two to eight parts of K, weights of several layers in turn; single launches lie 4 to 10 % from it.
+TILES = (
+    (256, 192, 1, 1.014, 0.188, 7.734), (256, 160, 1, 0.590, 0.319, 8.114), (256, 128, 1, 0.519, 0.257, 6.862),
+    (192, 192, 1, 0.558, 0.275, 7.049), (192, 160, 1, 0.515, 0.229, 6.576), (192, 128, 1, 0.442, 0.190, 5.529),
+    (128, 160, 1, 0.500, 0.127, 4.733), (128, 128, 1, 0.430, 0.104, 3.965), (128, 96, 1, 0.371, 0.081, 2.902),
+    (96, 160, 1, 0.442, 0.062, 4.100), (96, 96, 1, 0.298, 0.062, 3.375), (128, 64, 1, 0.304, 0.062, 2.725),
+    (64, 64, 2, 0.168, 0.287, 1.183),
+)
+
+
 class HipOps:
-    # bfloat16 products with more rows than this go to the vendor BLAS
+    # bfloat16 products with more rows than this are made by tiles
     own_max_rows = 64
     # the same for the two forms in which a block fetches fewer activations than weights: the
     # gated product, and the product cut along K whose planes the residual's norm adds
@@ -275,8 +291,11 @@ class HipOps:
     # None where the longest tile's chain of rounds would otherwise set the kernel's time
     prefill_key_groups = None
 
-    def __init__(self):
+    def __init__(self, residual_planes=False):
+        """``residual_planes``: ``linear_for_residual`` may cut K into planes with any number of rows, and not
+        only with few; for callers that hand its result to nothing but the norms and ``accumulate``."""
         self.lib = core_library()
+        self.residual_planes = residual_planes
 
     def _check(self, lib, code: int) -> None:
         if code != 0:
@@ -1160,8 +1179,10 @@ class HipOps:
         if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
             raise OpsError(f"linear: no product of {x.dtype} activations with {w.dtype} weights")
         kernel = self._own_kernel(m, n, k, "whole")
+        if kernel is None and self._tiles_take(x, w):
+            return self._tile_product(x, w, self.choose_tile(m, n, k)[0], out_f32=out_f32)
         if kernel is None:
-            # many rows: the vendor library; both accumulate in float32
+            # the vendor library; all accumulate in float32
             if out_f32:
                 return torch.mm(x, w.t(), out_dtype=torch.float32)
             return self._library_product(x, w)
@@ -1169,6 +1190,51 @@ class HipOps:
         self._check(self.lib, self.lib.qrt_gemm_bf16(
             _ptr(x), _ptr(w), _ptr(out), F32 if out_f32 else BF16,
             c_int(m), c_int(n), c_int(k), c_int(0), c_int(kernel), c_int(1), _stream()))
+        return out
+
+    @staticmethod
+    def _tiles_take(x, w) -> bool:
+        """Whether the product by tiles takes these bfloat16 operands: whole stages of K and whole MFMA tiles of
+        weight rows, 16 bytes at a time, offsets in 32 bits."""
+        n, k = w.shape
+        return (x.shape[0] > 0 and k > 0 and n > 0 and k % 64 == 0 and n % 16 == 0 and x.data_ptr() % 16 == 0
+                and w.data_ptr() % 16 == 0 and x.numel() < 2**31 - 64 and w.numel() < 2**31 - 64)
+
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def choose_tile(m: int, n: int, k: int, form: str = "whole") -> tuple[int, int]:
+        """(tile, parts of K) for ``m`` rows by a weight [n, k] ("gated": [2n, k]): the least time by the model of
+        ``TILES``. ``form`` "planes": K may be cut into up to eight parts of at least eight stages each, for products
+        whose tiles do not fill the compute units; the norm that adds the planes reads them at some 5 TB/s. It is
+        within 3 % of the best choice on average over the launches the model is made from, 30 % at worst (256 rows
+        and fewer, where launches take 15 us). Follows from the sizes alone, so that equal inputs give equal bits."""
+        best = None
+        for number, (rows, columns, resident, a, b, c) in enumerate(TILES):
+            tiles = -(-m // rows) * -(-n // (columns // 2 if form == "gated" else columns))
+            for parts in range(1, 9 if form == "planes" else 2):
+                stages = -(-(k // 64) // parts)
+                if parts > 1 and (stages < 8 or stages * (parts - 1) >= k // 64):
+                    break
+                load = -(-tiles * parts // 256)  # blocks of the busiest compute unit
+                rounds = -(-load // resident)
+                full = load / (resident * rounds) if 1 < load and resident > 1 else tiles * parts / (256 * resident * rounds)
+                us = 3 + rounds * (c + stages * (a + b * full))
+                if form == "planes":
+                    us += m * n * (4 * parts if parts > 1 else 2) / 5e6
+                if best is None or us < best[0]:
+                    best = us, number, parts
+        return best[1:]
+
+    def _tile_product(self, x, w, tile, parts=1, out_f32=False, gate=None):
+        """``gate``: None, or (activation, limit, row_scale) with w [2I, K]."""
+        m, k = x.shape
+        n = w.shape[0] if gate is None else w.shape[0] // 2
+        out = torch.empty((parts, m, n) if parts > 1 else (m, n), device=x.device,
+                          dtype=torch.float32 if out_f32 or parts > 1 else torch.bfloat16)
+        act, limit, row_scale = (-1, 0.0, None) if gate is None else (ACTIVATIONS[gate[0]], gate[1], gate[2])
+        self._check(self.lib, self.lib.qrt_gemm_tiles(
+            _ptr(x), _ptr(w), _ptr(out), F32 if out.dtype == torch.float32 else BF16, c_int(m), c_int(n), c_int(k),
+            c_int(tile), c_int(parts), c_int(act), c_float(limit), _ptr(row_scale), _stream()))
         return out
 
     # rows from which a library product is made in two column chunks; False: never
@@ -1235,6 +1301,11 @@ class HipOps:
             kernel = self._own_kernel(m, n, k, "planes")
             if kernel is not None:
                 parts = self.choose_k_parts(n, k, m, kernel == 1)
+            elif self.residual_planes and w.shape == (n, k) and self._tiles_take(x, w):
+                _need(x, "x")
+                _need(w, "weight")
+                tile, parts = self.choose_tile(m, n, k, "planes")
+                return self._tile_product(x, w, tile, parts)
         if parts == 1:
             return self.linear(x, w)
         _need(x, "x", torch.bfloat16)
@@ -1309,6 +1380,11 @@ class HipOps:
                     _ptr(x), _ptr(w_gate_up), _ptr(out), BF16, c_int(m), c_int(two_i // 2), c_int(k), c_int(kernel),
                     c_int(ACTIVATIONS[activation]), c_float(limit), _ptr(row_scale), _stream()))
                 return out
+            if self._tiles_take(x, w_gate_up) and two_i % 32 == 0:
+                if row_scale is not None:
+                    _need(row_scale, "row factors", torch.float32, (m,))
+                return self._tile_product(x, w_gate_up, self.choose_tile(m, two_i // 2, k, "gated")[0],
+                                          gate=(activation, limit, row_scale))
         return self.gated_act(self.linear(x, w_gate_up), activation, limit, row_scale=row_scale)
 
     # ---- q/k norm, rotation, cache write ----------------------------------------

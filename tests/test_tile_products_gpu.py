@@ -1,0 +1,144 @@
+"""The product of many rows by tiles through LDS, tile by tile at its edges, and the calls that come to it."""
+
+from ctypes import c_float, c_int
+
+import pytest
+import torch
+
+from qwen3_runtime_amd.ops.hip import BF16, F32, TILES, HipOps, _ptr, _stream
+
+DEV = "cuda"
+STAGES = {0: 2, 1: 3, 2: 3, 3: 3, 4: 3, 5: 3, 6: 4, 7: 4, 8: 4, 9: 4, 10: 6, 11: 6, 12: 4}  # in flight
+
+
+def rnd(*shape, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (scale * torch.randn(*shape, generator=g)).to(torch.bfloat16).to(DEV)
+
+
+def close(got, want, k, rounded):
+    """Sums of k products in float32: each addition errs by 2^-24 of the sum so far, at most k of them in a row, and
+    a bfloat16 result by 2^-9 of itself (and of what lies nearest to a tie, so 2^-8)."""
+    err = (got.double() - want).abs()
+    size = want.abs().max()
+    assert torch.isfinite(got).all()
+    bound = k * 2.0 ** -24 * size + (2.0 ** -8 * want.abs() if rounded else 0.0)
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+def launch(ops, x, w, out, tile, parts=1, act=-1, limit=0.0, row_scale=None):
+    m, k = x.shape
+    n = w.shape[0] // (2 if act >= 0 else 1)
+    ops._check(ops.lib, ops.lib.qrt_gemm_tiles(_ptr(x), _ptr(w), _ptr(out), F32 if out.dtype == torch.float32 else BF16,
+                                               c_int(m), c_int(n), c_int(k), c_int(tile), c_int(parts), c_int(act),
+                                               c_float(limit), _ptr(row_scale), _stream()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_every_tile_at_its_edges(tile):
+    """One row and one past the tile, a column tile and a single MFMA tile more, bands of row tiles, and as many stages
+    as fit the ring, one fewer and one more; every result in both types, in planes (some empty) and gated."""
+    ops = HipOps()
+    rows, columns, s = *TILES[tile][:2], STAGES[tile]
+    for m, n, k in [(1, 16, 64), (rows - 1, columns, 64 * (s - 1)), (rows, columns + 16, 64 * s), (rows + 1, 2 * columns - 16, 64 * (s + 1)),
+                    (17, 3 * columns, 64 * (2 * s + 1)), (2048 + rows + 5, columns + 48, 64)]:
+        x, w = rnd(m, k, seed=1), rnd(n, k, seed=2, scale=0.05)
+        want = x.double() @ w.double().T
+        for dtype in (torch.bfloat16, torch.float32):
+            out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+            launch(ops, x, w, out, tile)
+            close(out, want, k, dtype == torch.bfloat16)
+        for parts in (2, 3, 8):
+            out = torch.full((parts, m, n), float("nan"), device=DEV)
+            launch(ops, x, w, out, tile, parts)
+            close(out.double().sum(0), want, k, False)
+        wg = rnd(2 * n, k, seed=3, scale=0.05)
+        g, u = (x.double() @ wg.double().T).split(n, 1)
+        gate = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        launch(ops, x, wg, gate, tile, act=0)
+        # gate and up value are rounded to bfloat16 first (2^-8 of each), the result again; silu's slope is below 1.1
+        assert bool(((gate.double() - torch.sigmoid(g) * g * u).abs() <= 2.0 ** -8 * ((1.1 * g.abs() + 2 * (torch.sigmoid(g) * g).abs()) * u.abs()) + 1e-4).all())
+        scale = torch.rand(m, device=DEV)
+        launch(ops, x, wg, gate, tile, act=1, limit=0.5, row_scale=scale)
+        both = ops.linear(x, wg) if m <= 64 else torch.cat([x.float() @ wg.float().T]).to(torch.bfloat16)
+        same = ops.gated_act(both, "clamped", 0.5, row_scale=scale).double()
+        assert bool(((gate.double() - same).abs() <= 2.0 ** -5 * same.abs() + 2.0 ** -7).all())
+
+
+@pytest.mark.gpu
+def test_bits_depend_on_neither_rows_nor_tile():
+    """Every output is one sum in the order of k: the same in every tile, beside any other rows; and a row that is not
+    finite changes no other row, a weight row that is not finite no other column."""
+    ops = HipOps()
+    x, w = rnd(300, 640, seed=4), rnd(336, 640, seed=5, scale=0.05)
+    x[7, 3], w[9, 5] = float("nan"), float("inf")
+    outs = []
+    for tile in range(len(TILES)):
+        for rows in (300, 131):
+            out = torch.empty((rows, 336), device=DEV)
+            launch(ops, x[:rows], w, out, tile)
+            outs.append(out)
+    for out in outs:
+        assert torch.equal(out[:131].nan_to_num(0.0, 1.0, -1.0), outs[0][:131].nan_to_num(0.0, 1.0, -1.0))
+    bad = ~torch.isfinite(outs[0])
+    assert bad[7].all() and bad[:, 9].all() and int(bad.sum()) == 336 + 300 - 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [65, 129, 257, 700])
+@pytest.mark.parametrize("n,k", [(96, 2048), (2560, 4096), (512, 64), (1040, 448)])
+def test_calls_that_come_to_tiles(m, n, k):
+    """linear, gated_linear and linear_for_residual with more rows than the streams of weights take, and the same with
+    operands that tiles do not take (8 bytes off, K or weight rows of other sizes): the general ways, the same values."""
+    ops, planes = HipOps(), HipOps(residual_planes=True)
+    x, w = rnd(m, k, seed=6), rnd(2 * n, k, seed=7, scale=0.05)
+    want = x.double() @ w.double().T
+    assert ops._tiles_take(x, w)
+    close(ops.linear(x, w), want, k, True)
+    close(ops.linear(x, w, out_f32=True), want, k, False)
+    for form, one in ((ops, 2), (planes, None)):
+        got = form.linear_for_residual(x, w)
+        assert got.dim() == one or (m <= 128 or one is None)
+        close(got if got.dim() == 2 else got.double().sum(0), want, k, got.dim() == 2)
+        assert torch.equal(got, form.linear_for_residual(x, w))
+    scale = torch.rand(m, device=DEV)
+    for act, limit, rs in (("swiglu", 0.0, None), ("clamped", 0.7, None), ("swiglu", 0.0, scale)):
+        got = ops.gated_linear(x, w, act, limit, row_scale=rs).double()
+        same = ops.gated_act(want.to(torch.bfloat16), act, limit, row_scale=rs).double()
+        # both round gate and up value to bfloat16: where sums lie at a tie, one step of 2^-8 of either
+        assert bool(((got - same).abs() <= 2.0 ** -6 * same.abs() + 2.0 ** -7 * want.abs().max()).all())
+    off = torch.empty(m * k + 4, dtype=torch.bfloat16, device=DEV)[4:].view(m, k)
+    off.copy_(x)
+    assert not ops._tiles_take(off, w)
+    close(ops.linear(off, w), want, k, True)
+    thin = w[: 2 * n - 8]
+    assert not ops._tiles_take(x, thin)
+    close(ops.linear(x, thin), want[:, : 2 * n - 8], k, True)
+
+
+@pytest.mark.gpu
+def test_what_tiles_refuse():
+    ops = HipOps()
+    x, w, out = rnd(70, 128, seed=1), rnd(64, 128, seed=2), torch.empty((2, 70, 64), device=DEV)
+    for bad in (dict(tile=len(TILES)), dict(tile=-1), dict(tile=3, parts=0), dict(tile=3, parts=2, act=0), dict(tile=3, act=2)):
+        with pytest.raises(Exception, match="gemm_tiles"):
+            launch(ops, x, w, out, **bad)
+    for a, b in ((x[:, :96].contiguous(), w[:, :96].contiguous()), (x, w[:40])):
+        with pytest.raises(Exception, match="gemm_tiles"):
+            launch(ops, a, b, out, tile=3)
+
+
+def test_choice_of_tile():
+    """By the sizes alone; K is cut only for planes, in parts of eight stages and more, none of them empty."""
+    assert HipOps.choose_tile(2048, 6144, 2560) == (0, 1)                     # 256 tiles of 256 x 192: one round
+    assert HipOps.choose_tile(512, 9728, 2560, "gated") == (1, 1)             # 244 of 256 x 160
+    tile, parts = HipOps.choose_tile(2048, 2560, 9728, "planes")
+    assert TILES[tile][:2] == (256, 160) and parts == 2                       # 128 tiles in two parts
+    for m in (1, 65, 129, 300, 1000, 2047, 8192, 100_000):
+        for n, k in ((16, 64), (2560, 4096), (5120, 25600), (151936, 2560), (1024, 512)):
+            assert HipOps.choose_tile(m, n, k)[1] == HipOps.choose_tile(m, n, k, "gated")[1] == 1
+            tile, parts = HipOps.choose_tile(m, n, k, "planes")
+            stages = k // 64
+            each = -(-stages // parts)
+            assert 0 <= tile < len(TILES) and 1 <= parts <= 8 and (parts == 1 or (each >= 8 and each * (parts - 1) < stages))
