@@ -12,8 +12,8 @@
 //   ballots: no grouping kernel, no count that reaches the host. Weights and tokens come to LDS by direct
 //   loads of whole cache lines, as in the few-row dense products. More than 16 pairs of an expert are taken 16 at a
 //   time, the weights coming again from the caches.
-// * many: `experts_tile_kernel`, tiles of 128 pairs x 128 weight rows through LDS; `experts_group_kernel`
-//   puts the pairs in their experts' order and lists the tiles.
+// * many: `experts_tile_kernel`, tiles of the products of many rows (tiles.h) over an expert's pairs;
+//   `experts_group_kernel` puts the pairs in their experts' order and lists the tiles.
 //
 // What they replace (MI355X, 16 experts of 2,560 x 1,536, 2 a token; us): a kernel of scalar products on LDS
 // copies of a few rows, 58 + 27 and a grouping and a combining kernel of 4.5 + 8.9 for 8 tokens (now 28 + 17); one library
@@ -21,6 +21,7 @@
 // sixth of the step.
 #include "common.h"
 #include "direct.h"
+#include "tiles.h"
 
 #define EXPERTS_DOWN 0   // second product: input rows by place, weighted float32 planes out
 #define EXPERTS_GATED 1  // first product with a gate
@@ -197,105 +198,97 @@ __global__ __launch_bounds__(1024) void experts_group_kernel(const int* __restri
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) order[atomicAdd(&at[index[p]], 1)] = p;
 }
 
-// 128 places x 128 weight rows (GATED: 64 gate rows and the 64 up rows that go with them, 32 and 32 in turn, so that
-// a wave holds both halves of its outputs), four waves of 64 x 64, 64 k at a time in two LDS stages filled
-// by direct loads of whole cache lines (piece c of row r at 128 r + 16 (c ^ (r & 7)): operand reads meet
-// no bank twice); 64 KB, so two blocks share a compute unit and one's products cover the other's waits.
-template <int MODE>
-__global__ __launch_bounds__(256, 2) void experts_tile_kernel(ExpertArgs a) {
+// BM places of one expert x BN weight rows (GATED: 8 gate rows and the 8 up rows that go with them in turn, BN / 2
+// outputs). What bounds it is what bounds the dense products, and the places that an expert's last tile leaves empty:
+// which tile is the best goes by how many pairs an expert has (HipOps.choose_experts_tiles). With one loop of 128 x 128
+// tiles behind two barriers a stage, as it was, 2,041 tokens took 125 + 75 us in a prompt step of 16 experts of 2,560 x
+// 1,536 with 2 a token.
+template <int BM, int BN, int WM, int WN, int S, int MODE>
+__global__ __launch_bounds__(64 * WM * WN, 2) void experts_tile_kernel(ExpertArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host's compiler knows no buffer resources
+  typedef Tile<BM, BN, WM, WN, S> T;
   constexpr bool GATED = MODE == EXPERTS_GATED;
-  constexpr int STAGE = 256 * 128, BN = GATED ? 64 : 128;
-  extern __shared__ __align__(16) unsigned char lds[];  // [2][rows of the input 128 | rows of the weights 128] x 128 bytes
-  const int K = a.K, N = a.N, row_tiles = a.tiles[0], col_tiles = (N + BN - 1) / BN;
+  constexpr int TM = T::TM, TN = T::TN, WIDTH = GATED ? BN / 2 : BN;
+  extern __shared__ __align__(16) unsigned char lds[];  // [S] stages, then the result
+  const int K = a.K, N = a.N, row_tiles = a.tiles[0], col_tiles = (N + WIDTH - 1) / WIDTH;
   // blocks go to the eight XCDs in turn: each takes a stretch of neighbouring tiles, an expert's row tiles
   // of the same weight rows first
   const int total = row_tiles * col_tiles, per = (total + 7) >> 3;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
-  const int row_tile = tile % row_tiles, n0 = tile / row_tiles * BN;
-  const int e = a.tiles[1 + 2 * row_tile], first = a.tiles[2 + 2 * row_tile];
-  const int rows = min(128, a.offsets[e + 1] - first);
+  const int row_tile = tile % row_tiles, n0 = tile / row_tiles * WIDTH;
+  const int e = __builtin_amdgcn_readfirstlane(a.tiles[1 + 2 * row_tile]);
+  const int first = __builtin_amdgcn_readfirstlane(a.tiles[2 + 2 * row_tile]);
+  const int rows = min(BM, __builtin_amdgcn_readfirstlane(a.offsets[e + 1]) - first);
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
-  const int r16 = lane & 15, quad = lane >> 4, wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const int sub = lane >> 3, piece = (lane & 7) ^ sub;
-  // eight loads a wave and stage, 8 rows x 128 bytes each: waves 0, 1 the input's rows, 2, 3 the weights'
-  const bf16_t* src[8];
+  const int r16 = lane & 15, quad = lane >> 4, wm = wave / WN, wn = wave % WN;
+  unsigned aoff[T::AL], woff[T::WL];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = (wave & 1) * 64 + 8 * i + sub;
-    if (wave < 2) {
-      const int place = first + min(r, rows - 1);  // beyond the expert's last pair: that one again, not stored
-      src[i] = a.in + (size_t)(MODE ? a.order[place] / a.top : place) * K + 8 * piece;
-    } else {
-      const int n = min(GATED ? n0 + (r >> 6) * 32 + (r & 31) : n0 + r, N - 1);
-      src[i] = a.w + ((size_t)e * (GATED ? 2 : 1) * N + (GATED && (r & 32) ? N : 0) + n) * K + 8 * piece;
-    }
+  for (int j = 0; j < T::AL; ++j) {
+    const int r = min(T::row_of(j, T::AU, wave, lane), rows - 1);  // beyond the expert's last pair: that one again, not stored
+    aoff[j] = (unsigned)(MODE ? a.order[first + r] / a.top : r) * (unsigned)(2 * K) + T::piece_of(lane);
   }
-  unsigned char* dst = lds + wave * 8192;
-  auto fetch = [&](int s) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[i] + (size_t)s * 64), (lds_ptr_t)(dst + (s & 1) * STAGE + i * 1024), 16, 0, 0);
-  };
-  f32x4_t acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  const int stages = K >> 6;
-  fetch(0);
-  for (int s = 0; s < stages; ++s) {
-    if (s + 1 < stages) {
-      fetch(s + 1);
-      QRT_WAIT_LOADS(8);
-    } else {
-      QRT_WAIT_LOADS(0);
-    }
-    QRT_BARRIER();
-    const unsigned char* at = lds + (s & 1) * STAGE;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int col = 16 * ((4 * h + quad) ^ (r16 & 7));
-      bf16x8_t x[4], w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        x[i] = *(const bf16x8_t*)(at + (wm + 16 * i + r16) * 128 + col);
-        w[i] = *(const bf16x8_t*)(at + (128 + wn + 16 * i + r16) * 128 + col);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], x[i], acc[i][j], 0, 0, 0);
-    }
-    QRT_WAIT_LDS();  // read before the barrier behind which the stage may be overwritten
-    QRT_BARRIER();
+  for (int j = 0; j < T::WL; ++j) {
+    const int r = T::row_of(j, T::WU, wave, lane);
+    const int row = GATED ? min(n0 + 8 * (r >> 4) + (r & 7), N - 1) + ((r & 8) ? N : 0) : min(n0 + r, N - 1);
+    woff[j] = (unsigned)row * (unsigned)(2 * K) + T::piece_of(lane);
   }
-  // acc[i][j]: place first + wm + 16 i + r16, four weight rows from wn + 16 j + 4 quad on
+  const bf16_t* in = MODE ? a.in : a.in + (size_t)first * K;  // by token, or by place
+  const size_t matrix = (size_t)(GATED ? 2 : 1) * N * K;
+  f32x4_t acc[TM][TN];
+  T::products(T::buffer(in, (size_t)(MODE ? a.tokens : rows) * K * 2), T::buffer(a.w + e * matrix, matrix * 2), aoff, woff, 0, K >> 6,
+              lds, acc);
+  // acc[i][j][r]: place first + m + 16 i + r16, row 16 j + 4 quad + r of the wave's weights
+  constexpr int ROWS = BM / WM, COLS = (GATED ? 8 : 16) * TN;
+  const int mw = wm * ROWS, nw = n0 + wn * COLS;
+  if (MODE == EXPERTS_DOWN) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = wm + 16 * i + r16;
-    if (m >= rows) continue;
-    const int p = a.order[first + m];
-    const float by = a.weight ? a.weight[p] : 1.0f;
-    if (MODE) {
-#pragma unroll
-      for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-        const int n = n0 + (GATED ? wn / 2 : wn) + 16 * j + 4 * quad;
-        if (n >= N) continue;  // N is a multiple of 4: four or none
-        bf16x4_t v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = from_f32<bf16_t>(expert_value<MODE>(a, acc[i][j][r] * by, GATED ? acc[i][j + 2][r] * by : 0.f));
-        *(bf16x4_t*)((bf16_t*)a.out + (size_t)(first + m) * N + n) = v;
-      }
-    } else {
+    for (int i = 0; i < TM; ++i) {
+      const int m = mw + 16 * i + r16;
+      if (m >= rows) continue;
+      const int p = a.order[first + m];
+      const float by = a.weight ? a.weight[p] : 1.0f;
       float* out = (float*)a.out + ((size_t)(p % a.top) * a.tokens + p / a.top) * N;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = n0 + wn + 16 * j + 4 * quad;
+      for (int j = 0; j < TN; ++j) {
+        const int n = nw + 16 * j + 4 * quad;
         if (n < N) *(f32x4_t*)(out + n) = acc[i][j] * by;
       }
     }
+    return;
   }
+  // through LDS, so that rows are stored in whole lines
+  constexpr int PITCH = 2 * COLS + 16, PIECES = COLS / 8;
+  __syncthreads();  // nobody reads the ring any more
+  unsigned char* own = lds + wave * ROWS * PITCH;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    unsigned char* row = own + (16 * i + r16) * PITCH;
+    const float by = a.weight ? a.weight[a.order[first + min(mw + 16 * i + r16, rows - 1)]] : 1.0f;
+#pragma unroll
+    for (int j = 0; j < TN; j += GATED ? 2 : 1) {
+      const bool pair = j + 1 < TN;  // GATED: two tiles change halves, a last single one leaves the upper half idle
+      bf16x4_t v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float g = acc[i][j][r], u = GATED ? acc[i][pair ? j + 1 : j][r] : 0.f;
+        if (GATED) swap_halves(g, u);
+        v[r] = from_f32<bf16_t>(expert_value<MODE>(a, g * by, u * by));
+      }
+      if (!GATED) *(bf16x4_t*)(row + 32 * j + 8 * quad) = v;
+      else if (pair || quad < 2) *(bf16x4_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)) = v;
+    }
+  }
+#pragma unroll
+  for (int c0 = 0; c0 < ROWS * PIECES; c0 += 64) {
+    const int c = c0 + lane, row = c / PIECES, at = c % PIECES;
+    if (ROWS * PIECES % 64 && c >= ROWS * PIECES) break;
+    const u32x4_t v = *(const u32x4_t*)(own + row * PITCH + 16 * at);
+    const int m = mw + row, n = nw + 8 * at;  // N is a multiple of 8: all or none
+    if (m < rows && n < N) *(u32x4_t*)((bf16_t*)a.out + (size_t)(first + m) * N + n) = v;
+  }
+#endif
 }
 
 static bool lds_allowed(const void* kernel, size_t bytes) {
@@ -319,25 +312,50 @@ static int experts_rows(const ExpertArgs& a, hipStream_t stream) {
   return a.tokens * a.top < a.experts ? experts_rows_launch<NT, U, MODE, true>(a, stream) : experts_rows_launch<NT, U, MODE, false>(a, stream);
 }
 
-template <int MODE>
+template <int BM, int BN, int WM, int WN, int S, int MODE>
 static int experts_tile_launch(const ExpertArgs& a, hipStream_t stream) {
-  auto kernel = experts_tile_kernel<MODE>;
+  constexpr size_t ring = Tile<BM, BN, WM, WN, S>::RING;
+  constexpr size_t result = MODE == EXPERTS_DOWN ? 0 : (size_t)BM * ((MODE == EXPERTS_GATED ? BN : 2 * BN) + 16 * WN);
+  constexpr size_t smem = ring > result ? ring : result;
+  static_assert(smem <= 160 * 1024, "the result of this tile does not fit LDS");
+  auto kernel = experts_tile_kernel<BM, BN, WM, WN, S, MODE>;
   static bool allowed = false;
-  if (!allowed && !lds_allowed((const void*)kernel, 64 * 1024)) return qrt_fail("experts: cannot get 64 KB of LDS");
+  if (!allowed && !lds_allowed((const void*)kernel, smem)) return qrt_fail("experts: cannot get %zu bytes of LDS", smem);
   allowed = true;
-  const int pairs = a.tokens * a.top, bn = MODE == EXPERTS_GATED ? 64 : 128;
-  const long row_tiles = pairs / 128 + (pairs < a.experts ? pairs : a.experts);  // at most: one ragged tile an expert
+  const int pairs = a.tokens * a.top, bn = MODE == EXPERTS_GATED ? BN / 2 : BN;
+  const long row_tiles = pairs / BM + (pairs < a.experts ? pairs : a.experts);  // at most: one ragged tile an expert
   const long blocks = (row_tiles * ((a.N + bn - 1) / bn) + 7) / 8 * 8;
   QRT_CHECK(blocks < (1l << 31), "experts: too many tiles");
-  kernel<<<(unsigned)blocks, 256, 64 * 1024, stream>>>(a);
+  kernel<<<(unsigned)blocks, 64 * WM * WN, smem, stream>>>(a);
   return 0;
 }
 
+// The tiles that experts take, by their numbers in TILES of ops/hip.py; rows of each, or 0.
+static int experts_tile_rows(int tile) {
+  switch (tile) {
+    case 3: case 4: case 5: return 192;
+    case 12: case 13: return 64;
+    default: return 0;
+  }
+}
+template <int MODE>
+static int experts_tile(const ExpertArgs& a, int tile, hipStream_t stream) {
+  switch (tile) {
+    case 3: return experts_tile_launch<192, 192, 4, 2, 3, MODE>(a, stream);
+    case 4: return experts_tile_launch<192, 160, 4, 2, 3, MODE>(a, stream);
+    case 5: return experts_tile_launch<192, 128, 4, 2, 3, MODE>(a, stream);
+    case 12: return experts_tile_launch<64, 64, 1, 4, 4, MODE>(a, stream);
+    case 13: return experts_tile_launch<64, 128, 1, 4, 3, MODE>(a, stream);
+    default: return qrt_fail("experts: no tile %d", tile);
+  }
+}
+
 // x [T, H], gate_up [E, 2I or I, H], down [E, H, I], index and weight [T, top] -> act [pairs, I] (scratch), out [top, T, H]
-// float32 planes. `scratch`: null for the few-pairs form; else int32 [pairs + E + 1 + 1 + 2 (pairs / 128 + E)].
+// float32 planes. `scratch`: null for the few-pairs form; else int32 [pairs + E + 1 + 1 + 2 (pairs / BM + E)], and `tile` and
+// `tile_down` the two products' tiles, both of BM rows.
 extern "C" int qrt_experts(const void* x, const void* gate_up, const void* down, const int* index, const float* weight,
                            void* act, float* out, int* scratch, int tokens, int hidden, int inter, int experts, int top,
-                           int act_kind, float limit, int weight_on_input, hipStream_t stream) {
+                           int act_kind, float limit, int weight_on_input, int tile, int tile_down, hipStream_t stream) {
   QRT_CHECK(tokens >= 0 && hidden > 0 && inter > 0 && experts >= 1 && experts <= 1024 && top >= 1, "experts: bad sizes");
   QRT_CHECK(hidden % 64 == 0 && inter % 64 == 0, "experts: widths %d and %d are no multiples of 64", hidden, inter);
   QRT_CHECK(act_kind == QRT_ACT_SWIGLU || act_kind == QRT_ACT_CLAMPED || act_kind == QRT_ACT_RELU2, "experts: unknown activation %d", act_kind);
@@ -347,24 +365,29 @@ extern "C" int qrt_experts(const void* x, const void* gate_up, const void* down,
   if (tokens == 0) return 0;
   const int pairs = tokens * top;
   QRT_CHECK(scratch || (size_t)pairs * 4 <= 32 * 1024, "experts: %d pairs are too many for the form of few", pairs);
+  const uint64_t limit_bytes = (1ull << 32) - 128;  // tiles' offsets are 32 bits
+  const int bm = experts_tile_rows(tile);
+  QRT_CHECK(!scratch || (bm > 0 && bm == experts_tile_rows(tile_down)), "experts: no two tiles %d and %d of as many rows", tile, tile_down);
+  QRT_CHECK(!scratch || ((uint64_t)tokens * hidden * 2 <= limit_bytes && (uint64_t)4 * inter * hidden <= limit_bytes),
+            "experts: tiles take operands of less than 4 GiB (%d tokens of %d, %d wide)", tokens, hidden, inter);
   ExpertArgs a{};
   a.index = index; a.tokens = tokens; a.top = top; a.experts = experts; a.act_kind = act_kind; a.limit = limit;
   if (scratch) {
     int* order = scratch;
     int* offsets = order + pairs;
     int* tiles = offsets + experts + 1;
-    experts_group_kernel<<<1, 1024, (size_t)experts * 8, stream>>>(index, order, offsets, tiles, pairs, experts, 128);
+    experts_group_kernel<<<1, 1024, (size_t)experts * 8, stream>>>(index, order, offsets, tiles, pairs, experts, bm);
     a.order = order; a.offsets = offsets; a.tiles = tiles;
   }
   a.in = (const bf16_t*)x; a.w = (const bf16_t*)gate_up; a.weight = weight_on_input ? weight : nullptr; a.out = act;
   a.K = hidden; a.N = inter;
   int rc;
-  if (act_kind == QRT_ACT_RELU2) rc = scratch ? experts_tile_launch<EXPERTS_RELU2>(a, stream) : experts_rows<2, 3, EXPERTS_RELU2>(a, stream);
-  else rc = scratch ? experts_tile_launch<EXPERTS_GATED>(a, stream) : experts_rows<1, 2, EXPERTS_GATED>(a, stream);
+  if (act_kind == QRT_ACT_RELU2) rc = scratch ? experts_tile<EXPERTS_RELU2>(a, tile, stream) : experts_rows<2, 3, EXPERTS_RELU2>(a, stream);
+  else rc = scratch ? experts_tile<EXPERTS_GATED>(a, tile, stream) : experts_rows<1, 2, EXPERTS_GATED>(a, stream);
   if (rc != 0) return rc;
   a.in = (const bf16_t*)act; a.w = (const bf16_t*)down; a.weight = weight_on_input ? nullptr : weight; a.out = out;
   a.K = inter; a.N = hidden;
-  rc = scratch ? experts_tile_launch<EXPERTS_DOWN>(a, stream) : experts_rows<1, 2, EXPERTS_DOWN>(a, stream);
+  rc = scratch ? experts_tile<EXPERTS_DOWN>(a, tile_down, stream) : experts_rows<1, 2, EXPERTS_DOWN>(a, stream);
   if (rc != 0) return rc;
   QRT_LAUNCH_CHECK("experts");
   return 0;

@@ -190,6 +190,7 @@ extern "C" int qrt_gemm_tiles(const void* a, const void* w, void* c, int out_dty
     case 10: return by_result<96, 96, 2, 2, 6>(p, out_dtype, mode, stream);
     case 11: return by_result<128, 64, 2, 2, 6>(p, out_dtype, mode, stream);
     case 12: return by_result<64, 64, 1, 4, 4>(p, out_dtype, mode, stream);
+    case 13: return by_result<64, 128, 1, 4, 3>(p, out_dtype, mode, stream);
     default: return qrt_fail("gemm_tiles: no tile %d", tile);
   }
 }

@@ -262,7 +262,7 @@ TILES = (
     (192, 192, 1, 0.558, 0.275, 7.049), (192, 160, 1, 0.515, 0.229, 6.576), (192, 128, 1, 0.442, 0.190, 5.529),
     (128, 160, 1, 0.500, 0.127, 4.733), (128, 128, 1, 0.430, 0.104, 3.965), (128, 96, 1, 0.371, 0.081, 2.902),
     (96, 160, 1, 0.442, 0.062, 4.100), (96, 96, 1, 0.298, 0.062, 3.375), (128, 64, 1, 0.304, 0.062, 2.725),
-    (64, 64, 2, 0.168, 0.287, 1.183),
+    (64, 64, 2, 0.168, 0.287, 1.183), (64, 128, 2, 0.258, 0.391, 1.737),
 )
 
 
@@ -1035,10 +1035,49 @@ class HipOps:
         140, at 16 196 and 145; 8 of 4,096 x 1,024 (128 tiles) at 16 56 and 72, at 24 71 and 73, at 32 87 and 75."""
         return min(32, max(9, 6000 // (experts * inter // 64 or 1)))
 
+    # tiles that the experts' kernel knows: 64 and 192 rows
+    EXPERT_TILES = (3, 4, 5, 12, 13)
+
+    @classmethod
+    @functools.lru_cache(maxsize=4096)
+    def choose_experts_tiles(cls, pairs: int, experts: int, hidden: int, inter: int, gated: bool) -> tuple[int, int, int]:
+        """(rows, first product's tile, second's) for experts by tiles: the least time of both by the model of ``TILES``,
+        for as many row tiles as experts have on average whose pairs are dealt out evenly (normal, with the
+        deviation of equal chances). Experts with more pairs than 1.7 short tiles hold take the long ones. Both
+        products, us, with 128 x 128 tiles of the former loop and now, at 16, 64, 128, 256 and 700 pairs an expert: 16 of 2,560 x
+        1,536, 2 a token, 97, 113, 155, 203, 430 and 87, 104, 103, 167, 347; 64 of 2,048 x 768, 8 a token, 154, 175, 235, 350, 735
+        and 148, 185, 214, 318, 640 (the one place where the former loop was faster, from 64 to 96 pairs); 8 of 4,096 x 1,024
+        57, 84, 97, 136, 236 and 56, 74, 82, 97, 204. 128 x 128 with two blocks a unit was tried beside these: no better."""
+        per = pairs / experts
+        width = math.sqrt(2 * per)
+
+        def row_tiles(rows):
+            more = sum(0.5 * math.erfc((i * rows - per) / width) for i in range(1, int((per + 4 * width) / rows) + 1))
+            return min(pairs, experts * (1.0 + more))
+
+        def us(number, n, k, halved):
+            rows, columns, resident, a, b, c = TILES[number]
+            tiles = max(1, round(row_tiles(rows) * -(-n // (columns // 2 if halved else columns))))
+            rounds = -(-(-(-tiles // 256)) // resident)
+            return 3 + rounds * (c + k // 64 * (a + b * min(1.0, tiles / (256 * resident * rounds))))
+
+        best = None
+        longest = max(TILES[i][0] for i in cls.EXPERT_TILES)
+        for rows in sorted({TILES[i][0] for i in cls.EXPERT_TILES}):
+            if rows < longest and 1.7 * rows < per:
+                continue
+            same = [i for i in cls.EXPERT_TILES if TILES[i][0] == rows]
+            first = min((us(i, inter, hidden, gated), i) for i in same)
+            second = min((us(i, hidden, inter, False), i) for i in same)
+            if best is None or first[0] + second[0] < best[0]:
+                best = first[0] + second[0], rows, first[1], second[1]
+        return best[1:]
+
     @staticmethod
     def experts_fit(x, hidden, inter, *weights) -> bool:
-        """Whether the experts' MFMA kernels take these operands (rows of whole cache lines, 16 bytes a load)."""
-        if x.dtype != torch.bfloat16 or hidden % 64 or inter % 64:
+        """Whether the experts' MFMA kernels take these operands (rows of whole cache lines, 16 bytes a load, an
+        expert's matrices of less than 4 GiB)."""
+        if x.dtype != torch.bfloat16 or hidden % 64 or inter % 64 or 2 * inter * hidden >= 2**31 - 64:
             return False
         at = x.data_ptr()
         for w in weights:
@@ -1069,16 +1108,22 @@ class HipOps:
             _need(out, "experts' planes", torch.float32, (top, t, h))
         pairs = t * top
         act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
-        scratch = None
+        scratch, tile, tile_down = None, 0, 0
         tile_pairs = self.experts_tile_pairs_per_expert
         if tile_pairs is None:
             tile_pairs = self.choose_experts_tile_pairs(n, inter)
         if pairs >= tile_pairs * n or pairs > self.experts_rows_max_pairs:
-            scratch = torch.empty(pairs + n + 2 + 2 * (pairs // 128 + n), dtype=torch.int32, device=x.device)
+            if x.numel() >= 2**31 - 64:  # tiles' offsets are 32 bits: the tokens in two goes
+                for part in (slice(0, t // 2), slice(t // 2, t)):
+                    out[:, part] = self.moe_for_residual(x[part], gate_up, down, index[part], weight[part], activation, limit,
+                                                         weight_on_input)
+                return out
+            rows, tile, tile_down = self.choose_experts_tiles(pairs, n, h, inter, activation != "relu2")
+            scratch = torch.empty(pairs + n + 2 + 2 * (pairs // rows + n), dtype=torch.int32, device=x.device)
         self._check(self.lib, self.lib.qrt_experts(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(index), _ptr(weight), _ptr(act),
                                                    _ptr(out), _ptr(scratch), c_int(t), c_int(h), c_int(inter), c_int(n),
                                                    c_int(top), c_int(ACTIVATIONS[activation]), c_float(limit),
-                                                   c_int(bool(weight_on_input)), _stream()))
+                                                   c_int(bool(weight_on_input)), c_int(tile), c_int(tile_down), _stream()))
         return out
 
     # Steps of many tokens run the experts one by one, each on the rows of its own tokens, with

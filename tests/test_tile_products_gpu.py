@@ -8,7 +8,7 @@ import torch
 from qwen3_runtime_amd.ops.hip import BF16, F32, TILES, HipOps, _ptr, _stream
 
 DEV = "cuda"
-STAGES = {0: 2, 1: 3, 2: 3, 3: 3, 4: 3, 5: 3, 6: 4, 7: 4, 8: 4, 9: 4, 10: 6, 11: 6, 12: 4}  # in flight
+STAGES = {0: 2, 1: 3, 2: 3, 3: 3, 4: 3, 5: 3, 6: 4, 7: 4, 8: 4, 9: 4, 10: 6, 11: 6, 12: 4, 13: 3}  # in flight
 
 
 def rnd(*shape, seed, scale=1.0):
@@ -118,6 +118,31 @@ def test_calls_that_come_to_tiles(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("first,second", [(i, j) for i in HipOps.EXPERT_TILES for j in HipOps.EXPERT_TILES
+                                          if TILES[i][0] == TILES[j][0]])
+@pytest.mark.parametrize("activation", ["swiglu", "relu2"])
+def test_experts_by_every_tile(first, second, activation):
+    """Experts with one pair past a tile, one that fills a tile, one with a single pair and one without any; widths of
+    a part of a tile, over more stages than the ring holds."""
+    from test_experts_gpu import close as near
+    from test_experts_gpu import plain
+
+    ops = HipOps()
+    rows = TILES[first][0]
+    ops.experts_tile_pairs_per_expert = 0
+    ops.choose_experts_tiles = lambda *sizes: (rows, first, second)
+    counts, h, inter = [rows + 1, rows, 1, 0], 448, 320
+    index = torch.cat([torch.full((c, 1), e) for e, c in enumerate(counts)])
+    index = index[torch.randperm(len(index), generator=torch.Generator().manual_seed(1))].int().to(DEV)
+    t = index.shape[0]
+    x = rnd(t, h, seed=1)
+    up, down = rnd(4, (2 if activation == "swiglu" else 1) * inter, h, seed=2, scale=h ** -0.5), rnd(4, h, inter, seed=3, scale=inter ** -0.5)
+    weight = torch.rand(t, 1, device=DEV)
+    got = ops.moe_for_residual(x, up, down, index, weight, activation, 0.0)
+    near(got, plain(x, up, down, index, weight, activation, 0.0, False).float(), 4e-3, 4e-3)
+
+
+@pytest.mark.gpu
 def test_what_tiles_refuse():
     ops = HipOps()
     x, w, out = rnd(70, 128, seed=1), rnd(64, 128, seed=2), torch.empty((2, 70, 64), device=DEV)
@@ -127,6 +152,15 @@ def test_what_tiles_refuse():
     for a, b in ((x[:, :96].contiguous(), w[:, :96].contiguous()), (x, w[:40])):
         with pytest.raises(Exception, match="gemm_tiles"):
             launch(ops, a, b, out, tile=3)
+
+
+def test_choice_of_experts_tiles():
+    """Both products' tiles have as many rows; one row tile an expert where a tile holds all that it may have."""
+    for pairs, experts, hidden, inter in ((1, 16, 2560, 1536), (4082, 16, 2560, 1536), (512, 64, 2048, 768), (100_000, 8, 4096, 1024)):
+        for gated in (True, False):
+            rows, first, second = HipOps.choose_experts_tiles(pairs, experts, hidden, inter, gated)
+            assert TILES[first][0] == TILES[second][0] == rows and {first, second} <= set(HipOps.EXPERT_TILES)
+    assert HipOps.choose_experts_tiles(16 * 128, 16, 2560, 1536, True)[0] == 192
 
 
 def test_choice_of_tile():
