@@ -10,7 +10,10 @@
 // arithmetic is float32; a row's sums are taken in a fixed order, whatever else is in the batch.
 // One block per token; a thread owns VEC neighbouring columns at tid, tid + BT, ... (VEC = 4
 // where rows allow 16-byte accesses) and keeps them in registers between the passes (KEEP
-// vectors: rows up to 8,192 wide).
+// vectors: rows up to 8,192 wide). Rows of up to 4,096 have a thread for every vector, however many
+// tokens there are, so that a token's sums are the same in steps of few and of many. Bound by memory
+// where tokens are many (2,041 tokens of four streams of 2,560: 219 MB with two planes:
+// 56 -> 41 us against blocks of 256 threads with three vectors each and planes in a loop; 8 tokens, four planes: 6.4 -> 5.7).
 #include "common.h"
 #include <math.h>
 
@@ -33,11 +36,11 @@ struct MixNormArgs {
 };
 
 // PL: the number of planes of the pending output where it is known when compiling (0: nothing
-// pending; 4 and 8: float32 planes, as the products cut along K leave them), -1: any number, in a
+// pending; 2 to 8: float32 planes, as the products cut along K leave them), -1: any number, in a
 // loop. With PL >= 0 every load of the row (streams, planes, norm weights, coefficients) stands
-// in one stretch of code ahead of the first use, so a token costs one round of memory latency;
-// steps of few tokens run blocks of 1,024 threads (BT) so that a thread owns one vector of the row.
-template <int KEEP, int VEC, int BT, int PL>
+// in one stretch of code ahead of the first use, so a token costs one round of memory latency.
+// MS: at most so many streams; four take half the registers of eight.
+template <int KEEP, int VEC, int BT, int PL, int MS>
 __global__ __launch_bounds__(BT) void mix_norm_kernel(MixNormArgs a) {
   typedef float fvec_t __attribute__((ext_vector_type(VEC)));
   typedef bf16_t bvec_t __attribute__((ext_vector_type(VEC)));
@@ -62,12 +65,12 @@ __global__ __launch_bounds__(BT) void mix_norm_kernel(MixNormArgs a) {
   const bool copy_through = xout && (a.s_in != S || xout != xin);  // nothing pending, but streams to write
   const bool y_f32 = a.y_dtype == QRT_F32;
 
-  fvec_t old[KEEP][MAX_STREAMS], y[KEEP], w[KEEP], bias[KEEP];
+  fvec_t old[KEEP][MS], y[KEEP], w[KEEP], bias[KEEP];
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     const int c = min((int)(threadIdx.x + BT * j) * VEC, H - VEC);  // beyond the row: its last vector, dropped below
 #pragma unroll
-    for (int s = 0; s < MAX_STREAMS; ++s)
+    for (int s = 0; s < MS; ++s)
       if (s < S) old[j][s] = *(const fvec_t*)(xin + (size_t)(a.s_in == 1 ? 0 : s) * H + c);
     w[j] = *(const fvec_t*)(a.weight + c);
     if (a.bias) bias[j] = *(const fvec_t*)(a.bias + c);
@@ -122,14 +125,14 @@ __global__ __launch_bounds__(BT) void mix_norm_kernel(MixNormArgs a) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
 #pragma unroll
-      for (int t = 0; t < MAX_STREAMS; ++t) {
+      for (int t = 0; t < MS; ++t) {
         if (t < S) {
           fvec_t v;
           if (PL != 0) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) v[e] = 0.f;
 #pragma unroll
-            for (int s = 0; s < MAX_STREAMS; ++s)
+            for (int s = 0; s < MS; ++s)
               if (s < S) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) v[e] = fmaf(cmix[s * MAX_STREAMS + t], old[j][s][e], v[e]);
@@ -186,28 +189,34 @@ __global__ __launch_bounds__(BT) void mix_norm_kernel(MixNormArgs a) {
   }
 }
 
-template <int VEC, int BT, int PL>
-static void mix_norm_keep(const MixNormArgs& a, hipStream_t stream) {
-  dim3 grid(a.num_out), block(BT);
-  const int keep = (a.hidden + BT * VEC - 1) / (BT * VEC);  // vectors a thread keeps: at most 8 (see the launch)
-  // what a thread holds must fit its registers (128 of them in a block of 1,024 threads): two vectors
-  // there, and with eight planes known when compiling only one
-  constexpr bool SMALL = BT == 1024 && VEC == 4;
-  if (keep <= 1) mix_norm_kernel<1, VEC, BT, PL><<<grid, block, 0, stream>>>(a);
-  else if (keep <= 2 && SMALL && PL == 8) mix_norm_kernel<2, VEC, BT, (SMALL && PL == 8 ? -1 : PL)><<<grid, block, 0, stream>>>(a);
-  else if (keep <= 2) mix_norm_kernel<2, VEC, BT, (SMALL && PL == 8 ? -1 : PL)><<<grid, block, 0, stream>>>(a);
-  else if (keep <= 4 && !SMALL) mix_norm_kernel<(SMALL ? 2 : 4), VEC, BT, (SMALL ? -1 : PL)><<<grid, block, 0, stream>>>(a);
-  else if (VEC == 1) mix_norm_kernel<(VEC == 1 ? 8 : 2), VEC, BT, (VEC == 1 ? PL : -1)><<<grid, block, 0, stream>>>(a);
+// Rows of up to 4,096 that allow 16-byte accesses: a vector a thread.
+template <int PL>
+static void mix_norm_one(const MixNormArgs& a, hipStream_t stream) {
+  const int threads = (a.hidden / 4 + 63) / 64 * 64;
+  if (a.streams <= 4) mix_norm_kernel<1, 4, 1024, PL, 4><<<a.num_out, threads, 0, stream>>>(a);
+  else mix_norm_kernel<1, 4, 1024, PL, MAX_STREAMS><<<a.num_out, threads, 0, stream>>>(a);
+}
+static void mix_norm_one_planes(const MixNormArgs& a, hipStream_t stream) {
+  if (!a.y) return mix_norm_one<0>(a, stream);
+  if (a.planes == 1) return mix_norm_one<1>(a, stream);
+  if (a.y_dtype == QRT_F32) switch (a.planes) {
+    case 2: return mix_norm_one<2>(a, stream);
+    case 3: return mix_norm_one<3>(a, stream);
+    case 4: return mix_norm_one<4>(a, stream);
+    case 5: return mix_norm_one<5>(a, stream);
+    case 6: return mix_norm_one<6>(a, stream);
+    case 7: return mix_norm_one<7>(a, stream);
+    case 8: return mix_norm_one<8>(a, stream);
+  }
+  mix_norm_one<-1>(a, stream);
 }
 
-template <int VEC, int BT>
-static void mix_norm_planes(const MixNormArgs& a, hipStream_t stream) {
-  const bool f32 = a.y_dtype == QRT_F32;
-  if (!a.y) mix_norm_keep<VEC, BT, 0>(a, stream);
-  else if (a.planes == 1) mix_norm_keep<VEC, BT, 1>(a, stream);
-  else if (VEC == 4 && f32 && a.planes == 4) mix_norm_keep<VEC, BT, (VEC == 4 ? 4 : -1)>(a, stream);
-  else if (VEC == 4 && f32 && a.planes == 8) mix_norm_keep<VEC, BT, (VEC == 4 ? 8 : -1)>(a, stream);
-  else mix_norm_keep<VEC, BT, -1>(a, stream);
+// Any other row: 1,024 threads with two vectors of four elements each, or with eight single elements.
+template <int VEC, int KEEP>
+static void mix_norm_any(const MixNormArgs& a, hipStream_t stream) {
+  if (!a.y) mix_norm_kernel<KEEP, VEC, 1024, 0, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
+  else if (a.planes == 1) mix_norm_kernel<KEEP, VEC, 1024, 1, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
+  else mix_norm_kernel<KEEP, VEC, 1024, -1, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
 }
 
 extern "C" int qrt_mix_norm(const MixNormArgs* args, hipStream_t stream) {
@@ -226,12 +235,12 @@ extern "C" int qrt_mix_norm(const MixNormArgs* args, hipStream_t stream) {
   auto lined_up = [](const void* p, size_t n) { return ((uintptr_t)p % n) == 0; };
   const bool wide = a.hidden % 4 == 0 && lined_up(a.x_in, 16) && lined_up(a.x_out, 16) && lined_up(a.weight, 16) &&
                     lined_up(a.bias, 16) && lined_up(a.out, 16) && lined_up(a.y, 16) && a.plane_stride % 4 == 0;
-  // few tokens: the launch is one round of memory latency, taken by as many threads as the row has vectors
-  // (blocks of 256 threads keep up to four vectors a thread, which is rows of 4,096; wider rows
-  // and rows without 16-byte accesses take 1,024 threads as well)
-  if (wide && a.num_out > 512 && a.hidden <= 4096) mix_norm_planes<4, 256>(a, stream);
-  else if (wide) mix_norm_planes<4, 1024>(a, stream);
-  else mix_norm_planes<1, 1024>(a, stream);
+  if (wide && a.hidden <= 4096) mix_norm_one_planes(a, stream);
+  else if (wide) mix_norm_any<4, 2>(a, stream);
+  else if (a.hidden <= 1024) mix_norm_any<1, 1>(a, stream);
+  else if (a.hidden <= 2048) mix_norm_any<1, 2>(a, stream);
+  else if (a.hidden <= 4096) mix_norm_any<1, 4>(a, stream);
+  else mix_norm_any<1, 8>(a, stream);
   QRT_LAUNCH_CHECK("mix_norm");
   return 0;
 }
