@@ -274,7 +274,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void experts_tile_kernel(ExpertArg
       for (int r = 0; r < 4; ++r) {
         float g = acc[i][j][r], u = GATED ? acc[i][pair ? j + 1 : j][r] : 0.f;
         if (GATED) swap_halves(g, u);
-        v[r] = from_f32<bf16_t>(expert_value<MODE>(a, g * by, u * by));
+        v[r] = from_f32<bf16_t>(GATED ? gated_act_rounded(g * by, u * by, a.act_kind, a.limit) : expert_value<MODE>(a, g * by, u * by));
       }
       if (!GATED) *(bf16x4_t*)(row + 32 * j + 8 * quad) = v;
       else if (pair || quad < 2) *(bf16x4_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)) = v;

@@ -101,7 +101,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
             float g = acc[i][j][r], u = acc[i][pair ? j + 1 : j][r];
             swap_halves(g, u);
             // both rounded to bfloat16 first, as the unfused kernels see them
-            o[r] = p.ep.template apply<GATED>((float)(bf16_t)g, (float)(bf16_t)u, m);
+            o[r] = gated_act_rounded((float)(bf16_t)g, (float)(bf16_t)u, GATED == 1 ? QRT_ACT_SWIGLU : p.ep.kind, p.ep.limit);
+            if (GATED == 2 && p.ep.row_scale) o[r] *= p.ep.row_scale[m];
           }
           if (pair || quad < 2) store4((bf16_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)), o);
         }

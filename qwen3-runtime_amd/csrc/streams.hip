@@ -12,7 +12,7 @@
 // where rows allow 16-byte accesses) and keeps them in registers between the passes (KEEP
 // vectors: rows up to 8,192 wide). Rows of up to 4,096 have a thread for every vector, however many
 // tokens there are, so that a token's sums are the same in steps of few and of many. Bound by memory
-// where tokens are many (2,041 tokens of four streams of 2,560: 219 MB with two planes:
+// where tokens are many (2,041 tokens of four streams of 2,560: 219 MB with two planes;
 // 56 -> 41 us against blocks of 256 threads with three vectors each and planes in a loop; 8 tokens, four planes: 6.4 -> 5.7).
 #include "common.h"
 #include <math.h>
