@@ -11,8 +11,9 @@ Matrix products: float32 goes to the library's own float32 MFMA kernels
 products cut along K) goes to the library's MFMA kernels that stream the
 weights, bfloat16 with more rows to its tiles through LDS; what those do not
 take (K no multiple of 64, weight rows no multiple of 16, operands off 16
-bytes) goes to the vendor BLAS through ``torch.matmul``, as the reference
-leaves its products to cuBLAS (qwen3_runtime/models/qwen3.py:76-77,134-135).
+bytes), and beyond 2,048 rows what fills the vendor BLAS's own tiles, goes
+to that through ``torch.matmul``, as the reference leaves its products to
+cuBLAS (qwen3_runtime/models/qwen3.py:76-77,134-135).
 """
 
 from __future__ import annotations
@@ -264,6 +265,8 @@ TILES = (
     (96, 160, 1, 0.442, 0.062, 4.100), (96, 96, 1, 0.298, 0.062, 3.375), (128, 64, 1, 0.304, 0.062, 2.725),
     (64, 64, 2, 0.168, 0.287, 1.183), (64, 128, 2, 0.258, 0.391, 1.737),
 )
+
+SHORT_TILE = 12
 
 
 class HipOps:
@@ -1224,7 +1227,7 @@ class HipOps:
         if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
             raise OpsError(f"linear: no product of {x.dtype} activations with {w.dtype} weights")
         kernel = self._own_kernel(m, n, k, "whole")
-        if kernel is None and self._tiles_take(x, w):
+        if kernel is None and self._tiles_take(x, w) and not self.library_takes(m, n, k):
             return self._tile_product(x, w, self.choose_tile(m, n, k)[0], out_f32=out_f32)
         if kernel is None:
             # the vendor library; all accumulate in float32
@@ -1244,6 +1247,19 @@ class HipOps:
         n, k = w.shape
         return (x.shape[0] > 0 and k > 0 and n > 0 and k % 64 == 0 and n % 16 == 0 and x.data_ptr() % 16 == 0
                 and w.data_ptr() % 16 == 0 and x.numel() < 2**31 - 64 and w.numel() < 2**31 - 64)
+
+    @staticmethod
+    def library_takes(m: int, n: int, k: int, form: str = "whole") -> bool:
+        """Whether the vendor library makes a product that the tiles could make as well: with more than 2,048 rows those
+        whose 256 x 256 tiles fill the compute units to 0.62 or more in whole rounds, and gated ones from 4,096 rows on, or
+        from 4,096 columns of K and 1,537 rows on. Library and tiles in turn, us, at 1,536, 2,048, 2,500 and 3,500 rows: 4B q/k/v 50, 59, 64, 100
+        and 43, 52, 71, 104; 4B down 97, 115, 137, 166 and 74, 92, 116, 151; 8B output 56, 66, 76, 95 and 48, 62, 76, 110; 8B down 148, 187, 199, 270
+        and 140, 171, 234, 311; gate/up and SwiGLU, 4B 158, 197, 241, 324 and 144, 189, 227, 317, 8B 269, 317, 405, 557 and 262, 349, 445, 602;
+        at 4,096 and 8,192: 4B 362, 693 and 370, 719, 8B 608, 1,191 and 678, 1,335."""
+        if form == "gated":
+            return m >= 4096 or (k >= 4096 and m > 1536)
+        tiles = -(-m // 256) * -(-n // 256)
+        return m > 2048 and tiles >= 0.62 * 256 * -(-tiles // 256)
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
@@ -1269,6 +1285,19 @@ class HipOps:
                 if best is None or us < best[0]:
                     best = us, number, parts
         return best[1:]
+
+    @staticmethod
+    def choose_short_parts(m: int, n: int, k: int) -> int:
+        """Parts of K in which 17 to 128 rows go by tiles of 64 x 64, a block a compute unit (0: by the kernel that shares
+        the activations). Four stages of 16 KB in flight bring a compute unit its 200 KB of a weight sooner than that
+        kernel's two chunks; larger weights, which it streams at 5 TB/s, it brings sooner. Product and the norm's read of
+        the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6 and 6.9, 7.4, 7.8, 10.4;
+        2,560 x 9,728 13.3, 15.0, 16.1, 21.3 and 12.5, 13.6, 14.7, 20.5; 2,048 x 2,048 6.7, 6.8, 8.3, 10.4 and 5.2, 5.6, 5.9, 6.7;
+        4,096 x 4,096 9.3, 10.6, 12.0, 16.7 and 9.3, 10.3, 11.1, 15.4; 4,096 x 12,288 19.3, 22.7, 22.9, 30.6 and 21.9, 23.5, 24.7, 31.5."""
+        if not 17 <= m <= 128 or n * k > 26 << 20:
+            return 0
+        parts = min(8, 256 // (-(-m // 64) * -(-n // 64)), k // 64 // 8)
+        return parts if parts > 1 and -(-(k // 64) // parts) * (parts - 1) < k // 64 else 0
 
     def _tile_product(self, x, w, tile, parts=1, out_f32=False, gate=None):
         """``gate``: None, or (activation, limit, row_scale) with w [2I, K]."""
@@ -1344,13 +1373,14 @@ class HipOps:
         kernel, parts = None, 1
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % 64 == 0:
             kernel = self._own_kernel(m, n, k, "planes")
+            if self.residual_planes and w.shape == (n, k) and self._tiles_take(x, w) and not self.library_takes(m, n, k, "planes"):
+                tile, parts = self.choose_tile(m, n, k, "planes") if kernel is None else (SHORT_TILE, self.choose_short_parts(m, n, k))
+                if parts:
+                    _need(x, "x")
+                    _need(w, "weight")
+                    return self._tile_product(x, w, tile, parts)
             if kernel is not None:
                 parts = self.choose_k_parts(n, k, m, kernel == 1)
-            elif self.residual_planes and w.shape == (n, k) and self._tiles_take(x, w):
-                _need(x, "x")
-                _need(w, "weight")
-                tile, parts = self.choose_tile(m, n, k, "planes")
-                return self._tile_product(x, w, tile, parts)
         if parts == 1:
             return self.linear(x, w)
         _need(x, "x", torch.bfloat16)
@@ -1425,7 +1455,7 @@ class HipOps:
                     _ptr(x), _ptr(w_gate_up), _ptr(out), BF16, c_int(m), c_int(two_i // 2), c_int(k), c_int(kernel),
                     c_int(ACTIVATIONS[activation]), c_float(limit), _ptr(row_scale), _stream()))
                 return out
-            if self._tiles_take(x, w_gate_up) and two_i % 32 == 0:
+            if self._tiles_take(x, w_gate_up) and two_i % 32 == 0 and not self.library_takes(m, two_i // 2, k, "gated"):
                 if row_scale is not None:
                     _need(row_scale, "row factors", torch.float32, (m,))
                 return self._tile_product(x, w_gate_up, self.choose_tile(m, two_i // 2, k, "gated")[0],

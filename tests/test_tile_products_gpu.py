@@ -86,7 +86,7 @@ def test_bits_depend_on_neither_rows_nor_tile():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m", [65, 129, 257, 700])
+@pytest.mark.parametrize("m", [17, 64, 65, 128, 129, 257, 700])
 @pytest.mark.parametrize("n,k", [(96, 2048), (2560, 4096), (512, 64), (1040, 448)])
 def test_calls_that_come_to_tiles(m, n, k):
     """linear, gated_linear and linear_for_residual with more rows than the streams of weights take, and the same with
@@ -97,9 +97,9 @@ def test_calls_that_come_to_tiles(m, n, k):
     assert ops._tiles_take(x, w)
     close(ops.linear(x, w), want, k, True)
     close(ops.linear(x, w, out_f32=True), want, k, False)
-    for form, one in ((ops, 2), (planes, None)):
+    for form in (ops, planes):
         got = form.linear_for_residual(x, w)
-        assert got.dim() == one or (m <= 128 or one is None)
+        assert got.dim() == 2 or m <= 128 or form is planes
         close(got if got.dim() == 2 else got.double().sum(0), want, k, got.dim() == 2)
         assert torch.equal(got, form.linear_for_residual(x, w))
     scale = torch.rand(m, device=DEV)
@@ -108,6 +108,8 @@ def test_calls_that_come_to_tiles(m, n, k):
         same = ops.gated_act(want.to(torch.bfloat16), act, limit, row_scale=rs).double()
         # both round gate and up value to bfloat16: where sums lie at a tie, one step of 2^-8 of either
         assert bool(((got - same).abs() <= 2.0 ** -6 * same.abs() + 2.0 ** -7 * want.abs().max()).all())
+    if m <= 64:  # streams of the weights, which refuse such operands
+        return
     off = torch.empty(m * k + 4, dtype=torch.bfloat16, device=DEV)[4:].view(m, k)
     off.copy_(x)
     assert not ops._tiles_take(off, w)
@@ -152,6 +154,26 @@ def test_what_tiles_refuse():
     for a, b in ((x[:, :96].contiguous(), w[:, :96].contiguous()), (x, w[:40])):
         with pytest.raises(Exception, match="gemm_tiles"):
             launch(ops, a, b, out, tile=3)
+
+
+def test_what_the_library_keeps():
+    takes = HipOps.library_takes
+    assert not any(takes(m, n, k, form) for m in (65, 2048) for n in (256, 6144, 9728) for k, form in ((4096, "whole"), (9728, "planes"), (2560, "gated")))
+    assert takes(1537, 12288, 4096, "gated") and not takes(1536, 12288, 4096, "gated")
+    assert takes(4096, 12288, 2560, "gated") and takes(2500, 12288, 4096, "gated") and not takes(2500, 9728, 2560, "gated")
+    assert takes(8192, 6144, 2560) and takes(2500, 4096, 12288, "planes") and takes(16384, 2560, 9728, "planes")
+    assert not takes(2500, 2560, 9728, "planes") and not takes(3500, 2560, 4096, "planes")
+
+
+def test_parts_of_few_rows():
+    """Between the few-row kernel and the tiles of many rows, where the weight is small: a block a compute unit."""
+    parts = HipOps.choose_short_parts
+    assert [parts(m, 2560, 4096) for m in (16, 17, 64, 65, 128, 129)] == [0, 6, 6, 3, 3, 0]
+    assert parts(48, 2560, 9728) == 6 and parts(48, 4096, 4096) == 4 and parts(48, 2048, 2048) == 4
+    assert parts(48, 4096, 12288) == parts(48, 64, 64) == parts(100, 16384, 1024) == 0
+    for n, k in ((16, 1024), (2560, 4096), (2064, 1600), (1040, 5888)):
+        p = parts(40, n, k)
+        assert p == 0 or (-(-(k // 64) // p) * (p - 1) < k // 64 and k // 64 >= 8 * p)
 
 
 def test_choice_of_experts_tiles():
