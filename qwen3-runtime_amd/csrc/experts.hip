@@ -238,7 +238,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void experts_tile_kernel(ExpertArg
   const size_t matrix = (size_t)(GATED ? 2 : 1) * N * K;
   f32x4_t acc[TM][TN];
   T::products(T::buffer(in, (size_t)(MODE ? a.tokens : rows) * K * 2), T::buffer(a.w + e * matrix, matrix * 2), aoff, woff, 0, K >> 6,
-              lds, acc);
+              lds, 0, acc);
   // acc[i][j][r]: place first + m + 16 i + r16, row 16 j + 4 quad + r of the wave's weights
   constexpr int ROWS = BM / WM, COLS = (GATED ? 8 : 16) * TN;
   const int mw = wm * ROWS, nw = n0 + wn * COLS;

@@ -4,11 +4,12 @@
 // caller adds. tiles.h has the loop over K and what bounds it.
 //
 // The result goes through LDS so that rows are stored in whole lines: 64 -> 59 us for 2,048 x 6,144
-// x 2,560, whose blocks all end at once. Every output is a sum over K in the order of k, so its bits
+// x 2,560, whose blocks all end at once. Blocks that make several tiles ask for the next one's first
+// stages before they store the last one's result: 186 -> 179 us for gate/up at 2,048 rows, 976 tiles. Every output is a sum over K in the order of k, so its bits
 // depend neither on M nor on the tile, only on the number of planes.
 // Against the library's product (and gated_act behind it) at the 4B sizes, weights of several layers
-// in turn, q/k/v, output, gate/up and down at 512 rows: 27 (29), 19 (25), 53 (67) and 33 us (53);
-// at 2,048 rows: 59 (58), 44 (52), 191 (209) and 79 us (117). See HipOps.choose_tile for which
+// in turn, q/k/v, output, gate/up and down at 512 rows: 27 (29), 19 (25), 52 (67) and 34 us (53);
+// at 2,048 rows: 58 (58), 41 (50), 179 (209) and 82 us (117). See HipOps.choose_tile for which
 // tile is taken.
 #include "common.h"
 #include "direct.h"
@@ -24,6 +25,21 @@ struct TileArgs {
   GatedEpilogue ep;
 };
 
+// Bytes of LDS that a tile's bfloat16 result passes through, and of LDS in all: the ring, and one stage more than the result
+// where both fit (the first stage of the next tile has then a place beside it).
+template <int BM, int BN, int WN, int GATED, typename TO>
+constexpr int tile_result_bytes() {
+  return sizeof(TO) == 4 ? 0 : BM * ((GATED ? BN : 2 * BN) + 16 * WN);
+}
+template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO>
+constexpr size_t tile_lds_bytes() {
+  typedef Tile<BM, BN, WM, WN, S> T;
+  constexpr size_t result = tile_result_bytes<BM, BN, WN, GATED, TO>(), both = result + T::STAGE;
+  constexpr size_t least = T::RING > result ? T::RING : result;
+  static_assert(least <= 160 * 1024, "the result of this tile does not fit LDS");
+  return result > 0 && both > least && both <= 160 * 1024 ? both : least;
+}
+
 // WM x WN waves, each with BM / WM rows and BN / WN columns of the tile. GATED: 16 rows of the tile's
 // weights are 8 gate rows and the 8 up rows that belong to them, so any BN makes BN / 2 columns.
 template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO>
@@ -37,102 +53,125 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
   const int r16 = lane & 15, quad = lane >> 4;
   const int K = p.K;
 
-  // Blocks reach the XCDs in turn: each gets a run of neighbouring tiles, so that its L2 holds the rows
-  // they share. Runs go down bands of some 2,048 rows, column by column.
-  const int total = gridDim.x, xcd = blockIdx.x & 7;
-  int id = xcd * (total >> 3) + min(xcd, total & 7) + (int)(blockIdx.x >> 3);
-  const int part = id / (p.mtiles * p.ntiles);
-  id -= part * p.mtiles * p.ntiles;
-  constexpr int BAND = 2048 / BM;
-  const int band = id / (BAND * p.ntiles), in_band = id - band * BAND * p.ntiles;
-  const int high = min(BAND, p.mtiles - band * BAND);
-  const int m0 = (band * BAND + in_band % high) * BM, n0 = in_band / high * (GATED ? BN / 2 : BN);
-
-  const int all = K >> 6, each = (all + p.parts - 1) / p.parts;
-  const int s0 = min(all, part * each), stages = min(all, s0 + each) - s0;
-
+  // A tile of the launch by its number. Blocks reach the XCDs in turn: each gets a run of neighbouring tiles, so that its
+  // L2 holds the rows they share. Runs go down bands of some 2,048 rows, column by column.
+  const int total = p.mtiles * p.ntiles * p.parts;
+  int part, m0, n0, s0, stages;
   unsigned aoff[T::AL], woff[T::WL];  // rows past the end repeat the last one and are not stored
+  auto locate = [&](int tile) {
+    const int xcd = tile & 7;
+    int id = xcd * (total >> 3) + min(xcd, total & 7) + (tile >> 3);
+    part = id / (p.mtiles * p.ntiles);
+    id -= part * p.mtiles * p.ntiles;
+    constexpr int BAND = 2048 / BM;
+    const int band = id / (BAND * p.ntiles), in_band = id - band * BAND * p.ntiles;
+    const int high = min(BAND, p.mtiles - band * BAND);
+    m0 = (band * BAND + in_band % high) * BM;
+    n0 = in_band / high * (GATED ? BN / 2 : BN);
+    const int all = K >> 6, each = (all + p.parts - 1) / p.parts;
+    s0 = min(all, part * each);
+    stages = min(all, s0 + each) - s0;
 #pragma unroll
-  for (int j = 0; j < T::AL; ++j)
-    aoff[j] = (unsigned)min(m0 + T::row_of(j, T::AU, wave, lane), p.M - 1) * (unsigned)(2 * K) + T::piece_of(lane);
+    for (int j = 0; j < T::AL; ++j)
+      aoff[j] = (unsigned)min(m0 + T::row_of(j, T::AU, wave, lane), p.M - 1) * (unsigned)(2 * K) + T::piece_of(lane);
 #pragma unroll
-  for (int j = 0; j < T::WL; ++j) {
-    const int in_tile = T::row_of(j, T::WU, wave, lane);
-    const int row = GATED ? min(n0 + 8 * (in_tile >> 4) + (in_tile & 7), p.N - 1) + ((in_tile & 8) ? p.N : 0)
-                          : min(n0 + in_tile, p.N - 1);
-    woff[j] = (unsigned)row * (unsigned)(2 * K) + T::piece_of(lane);
-  }
-  f32x4_t acc[TM][TN];
-  T::products(T::buffer(p.A, (size_t)p.M * K * 2), T::buffer(p.W, (size_t)(GATED ? 2 : 1) * p.N * K * 2), aoff, woff, s0, stages,
-              tiles_lds, acc);
-
-  // acc[i][j][r]: row 16 i + r16 of the wave's result, row 16 j + 4 quad + r of its weights
-  TO* C = (TO*)p.C + (size_t)part * p.M * p.N;
-  constexpr int ROWS = BM / WM, COLS = (GATED ? 8 : 16) * TN;
-  const int mw = m0 + wm * ROWS, nw = n0 + wn * COLS;
-  if constexpr (sizeof(TO) == 4) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = mw + 16 * i + r16;
-      if (m >= p.M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = nw + 16 * j + 4 * quad;
-        if (n < p.N) *(f32x4_t*)(C + (size_t)m * p.N + n) = acc[i][j];
-      }
+    for (int j = 0; j < T::WL; ++j) {
+      const int in_tile = T::row_of(j, T::WU, wave, lane);
+      const int row = GATED ? min(n0 + 8 * (in_tile >> 4) + (in_tile & 7), p.N - 1) + ((in_tile & 8) ? p.N : 0)
+                            : min(n0 + in_tile, p.N - 1);
+      woff[j] = (unsigned)row * (unsigned)(2 * K) + T::piece_of(lane);
     }
-  } else {
-    constexpr int PITCH = 2 * COLS + 16;
-    __syncthreads();  // nobody reads the ring any more
-    unsigned char* own = tiles_lds + wave * ROWS * PITCH;
+  };
+  const __amdgpu_buffer_rsrc_t a_buf = T::buffer(p.A, (size_t)p.M * K * 2);
+  const __amdgpu_buffer_rsrc_t w_buf = T::buffer(p.W, (size_t)(GATED ? 2 : 1) * p.N * K * 2);
+
+  // Where tiles are more than the compute units hold, a block makes several, gridDim.x apart (a multiple of 8: of the same
+  // XCD), and asks for the first stages of the next one before it stores the last one's result: the stages whose
+  // slots the result leaves free (FIRST of them; it lies at the end of LDS).
+  constexpr int RESULT = tile_result_bytes<BM, BN, WN, GATED, TO>();
+  constexpr int FIRST = RESULT == 0 ? S : ((int)tile_lds_bytes<BM, BN, WM, WN, S, GATED, TO>() - RESULT) / T::STAGE;
+  unsigned char* const result = tiles_lds + tile_lds_bytes<BM, BN, WM, WN, S, GATED, TO>() - RESULT;
+  int tile = blockIdx.x, fetched = 0;
+  locate(tile);
+  while (true) {
+    f32x4_t acc[TM][TN];
+    T::products(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, fetched, acc);
+    QRT_WAIT_LDS();
+    QRT_BARRIER();  // nobody reads the ring any more
+    // acc[i][j][r]: row 16 i + r16 of the wave's result, row 16 j + 4 quad + r of its weights
+    TO* C = (TO*)p.C + (size_t)part * p.M * p.N;
+    constexpr int ROWS = BM / WM, COLS = (GATED ? 8 : 16) * TN;
+    const int mw = m0 + wm * ROWS, nw = n0 + wn * COLS;
+    const bool more = tile + (int)gridDim.x < total;
+    tile += gridDim.x;
+    if (more) {
+      locate(tile);
+      T::fetch_first(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, 0, FIRST);
+    }
+    if constexpr (sizeof(TO) == 4) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      unsigned char* row = own + (16 * i + r16) * PITCH;
-      if constexpr (GATED) {
-        // the lower half of the lanes holds gate values and the upper half the up values that belong to
-        // them: two tiles change halves, and every lane has a gate and an up value
-        const int m = min(mw + 16 * i + r16, p.M - 1);
-#pragma unroll
-        for (int j = 0; j < TN; j += 2) {
-          const bool pair = j + 1 < TN;  // a last single tile leaves the upper half idle
-          float o[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float g = acc[i][j][r], u = acc[i][pair ? j + 1 : j][r];
-            swap_halves(g, u);
-            // both rounded to bfloat16 first, as the unfused kernels see them
-            o[r] = gated_act_rounded((float)(bf16_t)g, (float)(bf16_t)u, GATED == 1 ? QRT_ACT_SWIGLU : p.ep.kind, p.ep.limit);
-            if (GATED == 2 && p.ep.row_scale) o[r] *= p.ep.row_scale[m];
-          }
-          if (pair || quad < 2) store4((bf16_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)), o);
-        }
-      } else {
+      for (int i = 0; i < TM; ++i) {
+        const int m = mw + 16 * i + r16;
+        if (m >= p.M) continue;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const float o[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-          store4((bf16_t*)(row + 32 * j + 8 * quad), o);
+          const int n = nw + 16 * j + 4 * quad;
+          if (n < p.N) *(f32x4_t*)(C + (size_t)m * p.N + n) = acc[i][j];
         }
       }
-    }
-    constexpr int PIECES = COLS / 8;  // of 16 bytes in a row
+    } else {
+      constexpr int PITCH = 2 * COLS + 16;
+      unsigned char* own = result + wave * ROWS * PITCH;
 #pragma unroll
-    for (int c0 = 0; c0 < ROWS * PIECES; c0 += 64) {
-      const int c = c0 + lane, row = c / PIECES, at = c % PIECES;
-      if (ROWS * PIECES % 64 && c >= ROWS * PIECES) break;
-      const u32x4_t v = *(const u32x4_t*)(own + row * PITCH + 16 * at);
-      const int m = mw + row, n = nw + 8 * at;
-      if (m < p.M && n < p.N) *(u32x4_t*)(C + (size_t)m * p.N + n) = v;
+      for (int i = 0; i < TM; ++i) {
+        unsigned char* row = own + (16 * i + r16) * PITCH;
+        if constexpr (GATED) {
+          // the lower half of the lanes holds gate values and the upper half the up values that belong to
+          // them: two tiles change halves, and every lane has a gate and an up value
+          const int m = min(mw + 16 * i + r16, p.M - 1);
+#pragma unroll
+          for (int j = 0; j < TN; j += 2) {
+            const bool pair = j + 1 < TN;  // a last single tile leaves the upper half idle
+            float o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float g = acc[i][j][r], u = acc[i][pair ? j + 1 : j][r];
+              swap_halves(g, u);
+              // both rounded to bfloat16 first, as the unfused kernels see them
+              o[r] = gated_act_rounded((float)(bf16_t)g, (float)(bf16_t)u, GATED == 1 ? QRT_ACT_SWIGLU : p.ep.kind, p.ep.limit);
+              if (GATED == 2 && p.ep.row_scale) o[r] *= p.ep.row_scale[m];
+            }
+            if (pair || quad < 2) store4((bf16_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)), o);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const float o[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            store4((bf16_t*)(row + 32 * j + 8 * quad), o);
+          }
+        }
+      }
+      constexpr int PIECES = COLS / 8;  // of 16 bytes in a row
+#pragma unroll
+      for (int c0 = 0; c0 < ROWS * PIECES; c0 += 64) {
+        const int c = c0 + lane, row = c / PIECES, at = c % PIECES;
+        if (ROWS * PIECES % 64 && c >= ROWS * PIECES) break;
+        const u32x4_t v = *(const u32x4_t*)(own + row * PITCH + 16 * at);
+        const int m = mw + row, n = nw + 8 * at;
+        if (m < p.M && n < p.N) *(u32x4_t*)(C + (size_t)m * p.N + n) = v;
+      }
     }
+    if (!more) break;
+    fetched = FIRST < S ? FIRST : S;
+    QRT_WAIT_LDS();
+    QRT_BARRIER();  // the result's room is the ring's again
   }
 #endif
 }
 
 template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO>
 static int launch_tiles(TileArgs p, hipStream_t stream) {
-  constexpr size_t ring = Tile<BM, BN, WM, WN, S>::RING;
-  constexpr size_t result = sizeof(TO) == 4 ? 0 : (size_t)BM * ((GATED ? BN : 2 * BN) + 16 * WN);
-  constexpr size_t smem = ring > result ? ring : result;
-  static_assert(smem <= 160 * 1024, "the result of this tile does not fit LDS");
+  constexpr size_t smem = tile_lds_bytes<BM, BN, WM, WN, S, GATED, TO>();
   const int width = GATED ? BN / 2 : BN;
   p.mtiles = (p.M + BM - 1) / BM;
   p.ntiles = (p.N + width - 1) / width;
@@ -145,7 +184,8 @@ static int launch_tiles(TileArgs p, hipStream_t stream) {
       return qrt_fail("gemm_tiles: cannot get %zu bytes of LDS", smem);
     allowed = true;
   }
-  kernel<<<(unsigned)blocks, 64 * WM * WN, smem, stream>>>(p);
+  constexpr int64_t resident = 256 * (160 * 1024 / smem);  // blocks that the compute units hold
+  kernel<<<(unsigned)(blocks < resident ? blocks : resident), 64 * WM * WN, smem, stream>>>(p);
   QRT_LAUNCH_CHECK("gemm_tiles");
   return 0;
 }

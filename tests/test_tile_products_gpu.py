@@ -42,7 +42,8 @@ def test_every_tile_at_its_edges(tile):
     ops = HipOps()
     rows, columns, s = *TILES[tile][:2], STAGES[tile]
     for m, n, k in [(1, 16, 64), (rows - 1, columns, 64 * (s - 1)), (rows, columns + 16, 64 * s), (rows + 1, 2 * columns - 16, 64 * (s + 1)),
-                    (17, 3 * columns, 64 * (2 * s + 1)), (2048 + rows + 5, columns + 48, 64)]:
+                    (17, 3 * columns, 64 * (2 * s + 1)), (2048 + rows + 5, columns + 48, 64),
+                    (2100, 5776, 64 * s + 64)]:  # the last: more tiles than the compute units hold, a block makes several
         x, w = rnd(m, k, seed=1), rnd(n, k, seed=2, scale=0.05)
         want = x.double() @ w.double().T
         for dtype in (torch.bfloat16, torch.float32):
@@ -158,7 +159,8 @@ def test_what_tiles_refuse():
 
 def test_what_the_library_keeps():
     takes = HipOps.library_takes
-    assert not any(takes(m, n, k, form) for m in (65, 2048) for n in (256, 6144, 9728) for k, form in ((4096, "whole"), (9728, "planes"), (2560, "gated")))
+    assert not any(takes(m, n, k, form) for m in (65, 2048) for n in (256, 6144, 9728) for k, form in ((2560, "whole"), (9728, "planes"), (2560, "gated")))
+    assert takes(2048, 6144, 4096) and not takes(1536, 6144, 4096) and not takes(2048, 10240, 5120)
     assert takes(1537, 12288, 4096, "gated") and not takes(1536, 12288, 4096, "gated")
     assert takes(4096, 12288, 2560, "gated") and takes(2500, 12288, 4096, "gated") and not takes(2500, 9728, 2560, "gated")
     assert takes(8192, 6144, 2560) and takes(2500, 4096, 12288, "planes") and takes(16384, 2560, 9728, "planes")
@@ -169,8 +171,8 @@ def test_parts_of_few_rows():
     """Between the few-row kernel and the tiles of many rows, where the weight is small: a block a compute unit."""
     parts = HipOps.choose_short_parts
     assert [parts(m, 2560, 4096) for m in (16, 17, 64, 65, 128, 129)] == [0, 6, 6, 3, 3, 0]
-    assert parts(48, 2560, 9728) == 6 and parts(48, 4096, 4096) == 4 and parts(48, 2048, 2048) == 4
-    assert parts(48, 4096, 12288) == parts(48, 64, 64) == parts(100, 16384, 1024) == 0
+    assert parts(48, 2560, 9728) == 6 and parts(48, 2048, 2048) == 4
+    assert parts(48, 4096, 4096) == parts(48, 4096, 12288) == parts(48, 64, 64) == parts(100, 16384, 1024) == 0
     for n, k in ((16, 1024), (2560, 4096), (2064, 1600), (1040, 5888)):
         p = parts(40, n, k)
         assert p == 0 or (-(-(k // 64) // p) * (p - 1) < k // 64 and k // 64 >= 8 * p)
