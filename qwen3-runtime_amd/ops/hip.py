@@ -1252,14 +1252,18 @@ class HipOps:
     def library_takes(m: int, n: int, k: int, form: str = "whole") -> bool:
         """Whether the vendor library makes a product that the tiles could make as well: with more than 2,048 rows those
         whose 256 x 256 tiles fill the compute units to 0.62 or more in whole rounds, and gated ones from 4,096 rows on, or
-        from 4,096 columns of K and 1,537 rows on. Library and tiles in turn, us, at 1,536, 2,048, 2,500 and 3,500 rows: 4B q/k/v 50, 59, 64, 100
+        from 4,096 columns of K and 1,537 rows on. So do whole ones of such rows that fill 0.7 (a 2,048-token prompt of the 8B
+        size: 26.5 ms with q/k/v and gate/up by the library and the rest by tiles, 28.1 with q/k/v by tiles as well, 27.0 with
+        everything by either). Library and tiles in turn, us, at 1,536, 2,048, 2,500 and 3,500 rows: 4B q/k/v 50, 59, 64, 100
         and 43, 52, 71, 104; 4B down 97, 115, 137, 166 and 74, 92, 116, 151; 8B output 56, 66, 76, 95 and 48, 62, 76, 110; 8B down 148, 187, 199, 270
         and 140, 171, 234, 311; gate/up and SwiGLU, 4B 158, 197, 241, 324 and 144, 189, 227, 317, 8B 269, 317, 405, 557 and 262, 349, 445, 602;
         at 4,096 and 8,192: 4B 362, 693 and 370, 719, 8B 608, 1,191 and 678, 1,335."""
+        long_rows = k >= 4096 and m > 1536
         if form == "gated":
-            return m >= 4096 or (k >= 4096 and m > 1536)
+            return m >= 4096 or long_rows
         tiles = -(-m // 256) * -(-n // 256)
-        return m > 2048 and tiles >= 0.62 * 256 * -(-tiles // 256)
+        full = tiles / (256 * -(-tiles // 256))
+        return full >= 0.62 if m > 2048 else form == "whole" and long_rows and full >= 0.7
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
@@ -1289,12 +1293,13 @@ class HipOps:
     @staticmethod
     def choose_short_parts(m: int, n: int, k: int) -> int:
         """Parts of K in which 17 to 128 rows go by tiles of 64 x 64, a block a compute unit (0: by the kernel that shares
-        the activations). Four stages of 16 KB in flight bring a compute unit its 200 KB of a weight sooner than that
-        kernel's two chunks; larger weights, which it streams at 5 TB/s, it brings sooner. Product and the norm's read of
-        the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6 and 6.9, 7.4, 7.8, 10.4;
-        2,560 x 9,728 13.3, 15.0, 16.1, 21.3 and 12.5, 13.6, 14.7, 20.5; 2,048 x 2,048 6.7, 6.8, 8.3, 10.4 and 5.2, 5.6, 5.9, 6.7;
-        4,096 x 4,096 9.3, 10.6, 12.0, 16.7 and 9.3, 10.3, 11.1, 15.4; 4,096 x 12,288 19.3, 22.7, 22.9, 30.6 and 21.9, 23.5, 24.7, 31.5."""
-        if not 17 <= m <= 128 or n * k > 26 << 20:
+        the activations). Four stages of 16 KB in flight bring a compute unit its 200 KB of a small weight sooner than that
+        kernel does, whose blocks of eight row tiles then leave compute units idle: 2,560 weight rows in eight parts are 160
+        blocks. 4,096 weight rows are 256, and it keeps them (64 requests of the 8B size 7.66 ms a step, by tiles 7.73). Product
+        and the norm's read of the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6
+        and 6.9, 7.4, 7.8, 10.4; 2,560 x 9,728 13.3, 15.0, 16.1, 21.3 and 12.5, 13.6, 14.7, 20.5; 2,048 x 2,048 6.7, 6.8, 8.3, 10.4 and
+        5.2, 5.6, 5.9, 6.7; 4,096 x 12,288 19.3, 22.7, 22.9, 30.6 and 21.9, 23.5, 24.7, 31.5."""
+        if not 17 <= m <= 128 or n * k > 26 << 20 or -(-n // 128) * HipOps.choose_k_parts(n, k, m, True) >= 224:
             return 0
         parts = min(8, 256 // (-(-m // 64) * -(-n // 64)), k // 64 // 8)
         return parts if parts > 1 and -(-(k // 64) // parts) * (parts - 1) < k // 64 else 0
