@@ -1295,8 +1295,10 @@ class HipOps:
         """Parts of K in which 17 to 128 rows go by tiles of 64 x 64, a block a compute unit (0: by the kernel that shares
         the activations). Four stages of 16 KB in flight bring a compute unit its 200 KB of a small weight sooner than that
         kernel does, whose blocks of eight row tiles then leave compute units idle: 2,560 weight rows in eight parts are 160
-        blocks. 4,096 weight rows are 256, and it keeps them (64 requests of the 8B size 7.66 ms a step, by tiles 7.73). Product
-        and the norm's read of the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6
+        blocks. 4,096 weight rows are 256, and it keeps them: decoding 64 requests of the 8B size from 256 tokens on takes 4.55 ms
+        a step with its output projection, 4.64 with tiles for that one product (32 requests 3.91 and 3.98; three runs of each in
+        turn, 0.01 apart), though by itself, called again and again, tiles are level or ahead (4,096 x 4,096 at 24, 48 and 64 rows 9.3,
+        10.6, 12.0 and 9.3, 10.3, 11.1 us). Product and the norm's read of the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6
         and 6.9, 7.4, 7.8, 10.4; 2,560 x 9,728 13.3, 15.0, 16.1, 21.3 and 12.5, 13.6, 14.7, 20.5; 2,048 x 2,048 6.7, 6.8, 8.3, 10.4 and
         5.2, 5.6, 5.9, 6.7; 4,096 x 12,288 19.3, 22.7, 22.9, 30.6 and 21.9, 23.5, 24.7, 31.5."""
         if not 17 <= m <= 128 or n * k > 26 << 20 or -(-n // 128) * HipOps.choose_k_parts(n, k, m, True) >= 224:
