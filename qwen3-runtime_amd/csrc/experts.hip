@@ -269,13 +269,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void experts_tile_kernel(ExpertArg
 #pragma unroll
     for (int j = 0; j < TN; j += GATED ? 2 : 1) {
       const bool pair = j + 1 < TN;  // GATED: two tiles change halves, a last single one leaves the upper half idle
+      float g[4], u[4], o[4];
       bf16x4_t v;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float g = acc[i][j][r], u = GATED ? acc[i][pair ? j + 1 : j][r] : 0.f;
-        if (GATED) swap_halves(g, u);
-        v[r] = from_f32<bf16_t>(GATED ? gated_act_rounded(g * by, u * by, a.act_kind, a.limit) : expert_value<MODE>(a, g * by, u * by));
+        g[r] = acc[i][j][r], u[r] = GATED ? acc[i][pair ? j + 1 : j][r] : 0.f;
+        if (GATED) swap_halves(g[r], u[r]);
+        g[r] *= by, u[r] *= by;
       }
+      if (GATED) gated_act4(g, u, a.act_kind, a.limit, o);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = from_f32<bf16_t>(GATED ? o[r] : expert_value<MODE>(a, g[r], u[r]));
       if (!GATED) *(bf16x4_t*)(row + 32 * j + 8 * quad) = v;
       else if (pair || quad < 2) *(bf16x4_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)) = v;
     }

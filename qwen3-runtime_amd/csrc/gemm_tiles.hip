@@ -132,14 +132,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
 #pragma unroll
           for (int j = 0; j < TN; j += 2) {
             const bool pair = j + 1 < TN;  // a last single tile leaves the upper half idle
-            float o[4];
+            float g[4], u[4], o[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              float g = acc[i][j][r], u = acc[i][pair ? j + 1 : j][r];
-              swap_halves(g, u);
+              g[r] = acc[i][j][r], u[r] = acc[i][pair ? j + 1 : j][r];
+              swap_halves(g[r], u[r]);
               // both rounded to bfloat16 first, as the unfused kernels see them
-              o[r] = gated_act_rounded((float)(bf16_t)g, (float)(bf16_t)u, GATED == 1 ? QRT_ACT_SWIGLU : p.ep.kind, p.ep.limit);
-              if (GATED == 2 && p.ep.row_scale) o[r] *= p.ep.row_scale[m];
+              g[r] = (float)(bf16_t)g[r], u[r] = (float)(bf16_t)u[r];
+            }
+            gated_act4(g, u, GATED == 1 ? QRT_ACT_SWIGLU : p.ep.kind, p.ep.limit, o);
+            if (GATED == 2 && p.ep.row_scale) {
+              const float by = p.ep.row_scale[m];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[r] *= by;
             }
             if (pair || quad < 2) store4((bf16_t*)(row + 16 * (j + (quad >> 1)) + 8 * (quad & 1)), o);
           }

@@ -200,3 +200,58 @@ def test_choice_of_tile():
             stages = k // 64
             each = -(-stages // parts)
             assert 0 <= tile < len(TILES) and 1 <= parts <= 8 and (parts == 1 or (each >= 8 and each * (parts - 1) < stages))
+
+
+GATES = [0.0, -0.0, 1e-30, -1e-30, 1e-3, -1e-3, 1.0, -1.0, 20.0, -20.0, 51.0, -51.0, 51.25, -51.25, 87.0, -87.0, 87.5, -87.5, 88.0, -88.0,
+         88.5, -88.5, -89.0, -100.0, -104.0, 1e4, -1e4, 1e30, -1e30, float("inf"), -float("inf"), float("nan")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act,limit", [("swiglu", 0.0), ("clamped", 0.7), ("clamped", 1e4)])
+@pytest.mark.parametrize("way,up", [(way, up) for way in ("dense", "experts") for up in (2.0, -1e30, 0.0)] + [("dense", float("inf"))])
+def test_gates_of_every_size(act, limit, up, way):
+    """One column of K is not zero, so gate and up values are exact: small ones, those around the end of what the exponential
+    and the quotient hold, infinite ones and NaN, beside ordinary ones in the same wave. Both forms of the activation
+    err by a few 2^-24 before they round to bfloat16, half a step of 2^-8 each; zeros, infinities and NaN are the same. What
+    stands beside them changes no result."""
+    ops, n = HipOps(), 128
+    gates = torch.tensor(GATES).to(torch.bfloat16)
+    values = rnd(n, seed=9, scale=3.0).cpu()
+    values[5: 5 + 2 * len(GATES): 2] = gates
+    if way == "experts":  # the second product would carry what is not finite to every column
+        bad = ~torch.isfinite(ops.gated_act(torch.cat([values, torch.full_like(values, up)])[None].to(DEV), act, limit)[0]).cpu()
+        values[bad] = 1.0
+    tame = torch.where(torch.isfinite(values) & (values.abs() < 50), values, torch.ones(()).to(values))
+
+    def run(gate):
+        w = torch.zeros(2 * n, 128)
+        w[:n, 3], w[n:, 3] = gate, up
+        w, x = w.to(torch.bfloat16).to(DEV), torch.zeros(200, 128, dtype=torch.bfloat16, device=DEV)
+        x[:, 3] = 1.0
+        if way == "dense":
+            assert ops._tiles_take(x, w) and not ops.library_takes(200, n, 128, "gated")
+            got = ops.gated_linear(x, w, act, limit)
+        else:  # the second product takes each value to a column of its own
+            ops.experts_tile_pairs_per_expert = 0
+            one = torch.eye(n, dtype=torch.bfloat16, device=DEV)[None]
+            assert ops.experts_fit(x, 128, n, w, one)
+            act_of = ops.moe_for_residual(x, w[None].contiguous(), one, torch.zeros(200, 1, dtype=torch.int32, device=DEV),
+                                          torch.ones(200, 1, device=DEV), act, limit)
+            got = act_of[0]
+        assert torch.equal(got.nan_to_num(7.0), got[:1].nan_to_num(7.0).expand_as(got))
+        return got[0], ops.gated_act(w[:, 3].float().to(torch.bfloat16)[None].contiguous(), act, limit)[0]
+
+    got, want = run(values)
+    got, want = got.double(), want.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    known = torch.isfinite(want)
+    assert torch.equal(got[~known].nan_to_num(7.0), want[~known].nan_to_num(7.0))
+    assert torch.equal(got[known] == 0, want[known] == 0)
+    assert bool(((got - want)[known].abs() <= 2.0 ** -7 * want[known].abs()).all())
+    if act == "swiglu" and up == 2.0:
+        g = values.to(DEV).double()
+        exact = g / (1 + torch.exp(-g)) * up
+        near = known & (g.abs() <= 87)
+        assert bool(((got - exact)[near].abs() <= 2.0 ** -8 * exact[near].abs()).all())
+    same = (tame == values).to(DEV)
+    assert torch.equal(run(tame)[0].double()[same].nan_to_num(7.0), got[same].nan_to_num(7.0))
