@@ -211,11 +211,13 @@ static void mix_norm_one_planes(const MixNormArgs& a, hipStream_t stream) {
   mix_norm_one<-1>(a, stream);
 }
 
-// Any other row: 1,024 threads with two vectors of four elements each, or with eight single elements.
+// Any other row: 1,024 threads with two vectors of four elements each, or with eight single elements. Two vectors leave registers for
+// four planes known when compiling, not for eight.
 template <int VEC, int KEEP>
 static void mix_norm_any(const MixNormArgs& a, hipStream_t stream) {
   if (!a.y) mix_norm_kernel<KEEP, VEC, 1024, 0, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
   else if (a.planes == 1) mix_norm_kernel<KEEP, VEC, 1024, 1, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
+  else if (VEC == 4 && a.planes == 4 && a.y_dtype == QRT_F32) mix_norm_kernel<KEEP, VEC, 1024, (VEC == 4 ? 4 : -1), MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
   else mix_norm_kernel<KEEP, VEC, 1024, -1, MAX_STREAMS><<<a.num_out, 1024, 0, stream>>>(a);
 }
 
