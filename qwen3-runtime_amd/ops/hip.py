@@ -1076,6 +1076,9 @@ class HipOps:
                 best = first[0] + second[0], rows, first[1], second[1]
         return best[1:]
 
+    # elements of the tokens that one launch of the experts' tiles takes: their offsets are 32 bits
+    experts_tile_max_elements = 2**31 - 64
+
     @staticmethod
     def experts_fit(x, hidden, inter, *weights) -> bool:
         """Whether the experts' MFMA kernels take these operands (rows of whole cache lines, 16 bytes a load, an
@@ -1110,19 +1113,19 @@ class HipOps:
         else:
             _need(out, "experts' planes", torch.float32, (top, t, h))
         pairs = t * top
-        act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
         scratch, tile, tile_down = None, 0, 0
         tile_pairs = self.experts_tile_pairs_per_expert
         if tile_pairs is None:
             tile_pairs = self.choose_experts_tile_pairs(n, inter)
         if pairs >= tile_pairs * n or pairs > self.experts_rows_max_pairs:
-            if x.numel() >= 2**31 - 64:  # tiles' offsets are 32 bits: the tokens in two goes
+            if x.numel() >= self.experts_tile_max_elements:  # the tokens in two goes
                 for part in (slice(0, t // 2), slice(t // 2, t)):
                     out[:, part] = self.moe_for_residual(x[part], gate_up, down, index[part], weight[part], activation, limit,
                                                          weight_on_input)
                 return out
             rows, tile, tile_down = self.choose_experts_tiles(pairs, n, h, inter, activation != "relu2")
             scratch = torch.empty(pairs + n + 2 + 2 * (pairs // rows + n), dtype=torch.int32, device=x.device)
+        act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
         self._check(self.lib, self.lib.qrt_experts(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(index), _ptr(weight), _ptr(act),
                                                    _ptr(out), _ptr(scratch), c_int(t), c_int(h), c_int(inter), c_int(n),
                                                    c_int(top), c_int(ACTIVATIONS[activation]), c_float(limit),

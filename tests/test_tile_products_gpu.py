@@ -255,3 +255,20 @@ def test_gates_of_every_size(act, limit, up, way):
         assert bool(((got - exact)[near].abs() <= 2.0 ** -8 * exact[near].abs()).all())
     same = (tame == values).to(DEV)
     assert torch.equal(run(tame)[0].double()[same].nan_to_num(7.0), got[same].nan_to_num(7.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("activation", ["swiglu", "relu2"])
+@pytest.mark.parametrize("given", [False, True])
+def test_experts_tokens_in_several_goes(activation, given):
+    """Tokens whose offsets would not fit 32 bits are taken in halves, here forced for an odd number of them: the same bits."""
+    ops, (t, n, h, inter, top) = HipOps(), (77, 5, 192, 128, 3)
+    ops.experts_tile_pairs_per_expert = 0
+    x, weight = rnd(t, h, seed=1), torch.rand(t, top, device=DEV)
+    up, down = rnd(n, (2 if activation == "swiglu" else 1) * inter, h, seed=2, scale=0.1), rnd(n, h, inter, seed=3, scale=0.1)
+    index = torch.rand(t, n, generator=torch.Generator().manual_seed(4)).topk(top, -1).indices.int().to(DEV).contiguous()
+    whole = ops.moe_for_residual(x, up, down, index, weight, activation, 0.0)
+    ops.experts_tile_max_elements = 20 * h
+    out = torch.full_like(whole, float("nan")) if given else None
+    got = ops.moe_for_residual(x, up, down, index, weight, activation, 0.0, out=out)
+    assert torch.equal(got, whole) and (out is None or got is out)
