@@ -334,10 +334,13 @@ static int experts_tile_launch(const ExpertArgs& a, hipStream_t stream) {
   return 0;
 }
 
-// The tiles that experts take, by their numbers in TILES of ops/hip.py; rows of each, or 0.
+// The tiles that experts take, by their numbers in TILES of ops/hip.py (plus EXPERTS_TWO_BLOCKS: with half the stages, so that
+// two blocks share a compute unit); rows of each, or 0.
+#define EXPERTS_TWO_BLOCKS 16
 static int experts_tile_rows(int tile) {
   switch (tile) {
     case 3: case 4: case 5: return 192;
+    case 7: case 7 + EXPERTS_TWO_BLOCKS: return 128;
     case 12: case 13: return 64;
     default: return 0;
   }
@@ -348,6 +351,8 @@ static int experts_tile(const ExpertArgs& a, int tile, hipStream_t stream) {
     case 3: return experts_tile_launch<192, 192, 4, 2, 3, MODE>(a, stream);
     case 4: return experts_tile_launch<192, 160, 4, 2, 3, MODE>(a, stream);
     case 5: return experts_tile_launch<192, 128, 4, 2, 3, MODE>(a, stream);
+    case 7: return experts_tile_launch<128, 128, 2, 2, 4, MODE>(a, stream);
+    case 7 + EXPERTS_TWO_BLOCKS: return experts_tile_launch<128, 128, 2, 2, 2, MODE>(a, stream);
     case 12: return experts_tile_launch<64, 64, 1, 4, 4, MODE>(a, stream);
     case 13: return experts_tile_launch<64, 128, 1, 4, 3, MODE>(a, stream);
     default: return qrt_fail("experts: no tile %d", tile);

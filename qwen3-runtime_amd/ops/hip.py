@@ -1038,42 +1038,55 @@ class HipOps:
         140, at 16 196 and 145; 8 of 4,096 x 1,024 (128 tiles) at 16 56 and 72, at 24 71 and 73, at 32 87 and 75."""
         return min(32, max(9, 6000 // (experts * inter // 64 or 1)))
 
-    # tiles that the experts' kernel knows: 64 and 192 rows
-    EXPERT_TILES = (3, 4, 5, 12, 13)
+    # Tiles that the experts' kernel knows, by their numbers in ``TILES``, and what a product of one takes, in microseconds, as
+    # there but with one tile a block: c for every round of blocks over the compute units, a for each of its stages, b more
+    # where the round is full, and w for every megabyte of weights. 128 x 128 has a second form with half the stages, two blocks
+    # a compute unit. Least squares over the launches within 1.25 of the best of each of 90: 8 to 128 experts of 2,048 x 768 to
+    # 4,096 x 1,024, 12 to 700 pairs an expert, weights of several layers in turn.
+    EXPERT_COSTS = {3: (1, 0.333, 0.363, 13.802, 0.046), 4: (1, 0.419, 0.226, 13.148, 0.017), 5: (1, 0.253, 0.272, 12.431, 0.011),
+                    7: (1, 0.244, 0.140, 11.070, 0.032), 12: (2, 0.028, 0.274, 5.871, 0.083), 13: (2, 0.105, 0.381, 7.739, 0.100)}
+    EXPERT_COSTS_TWO_BLOCKS = {7: (2, 0.407, 0.321, 16.214, 0.043)}
+    EXPERT_TILES = tuple(EXPERT_COSTS)
+    experts_two_blocks = 16  # what csrc/experts.hip adds to the number of that form
+
+    @classmethod
+    @functools.lru_cache(maxsize=4096)
+    def experts_product(cls, tile: int, pairs: int, experts: int, n: int, k: int, halved: bool) -> tuple[float, int, int]:
+        """(microseconds by the model of ``EXPERT_COSTS``, number of the tile's better form, tiles) for as many row tiles
+        as experts have on average whose pairs are dealt out evenly (normal, with the deviation of equal chances)."""
+        rows, columns = TILES[tile][:2]
+        per = pairs / experts
+        width = math.sqrt(2 * per)
+        more = sum(0.5 * math.erfc((i * rows - per) / width) for i in range(1, int((per + 4 * width) / rows) + 1))
+        tiles = max(1, round(min(pairs, experts * (1.0 + more)) * -(-n // (columns // 2 if halved else columns))))
+        forms = []
+        for number, costs in ((tile, cls.EXPERT_COSTS), (tile + cls.experts_two_blocks, cls.EXPERT_COSTS_TWO_BLOCKS)):
+            if tile in costs:
+                resident, a, b, c, w = costs[tile]
+                rounds = -(-(-(-tiles // 256)) // resident)
+                full = min(1.0, tiles / (256 * resident * rounds))
+                forms.append((rounds * (c + k // 64 * (a + b * full)) + w * experts * n * k * (4e-6 if halved else 2e-6), number, tiles))
+        return min(forms)
 
     @classmethod
     @functools.lru_cache(maxsize=4096)
     def choose_experts_tiles(cls, pairs: int, experts: int, hidden: int, inter: int, gated: bool) -> tuple[int, int, int]:
-        """(rows, first product's tile, second's) for experts by tiles: the least time of both by the model of ``TILES``,
-        for as many row tiles as experts have on average whose pairs are dealt out evenly (normal, with the
-        deviation of equal chances). Experts with more pairs than 1.7 short tiles hold take the long ones. Both
-        products, us, with 128 x 128 tiles of the former loop and now, at 16, 64, 128, 256 and 700 pairs an expert: 16 of 2,560 x
-        1,536, 2 a token, 97, 113, 155, 203, 430 and 87, 104, 103, 167, 347; 64 of 2,048 x 768, 8 a token, 154, 175, 235, 350, 735
-        and 148, 185, 214, 318, 640 (the one place where the former loop was faster, from 64 to 96 pairs); 8 of 4,096 x 1,024
-        57, 84, 97, 136, 236 and 56, 74, 82, 97, 204. 128 x 128 with two blocks a unit was tried beside these: no better."""
-        per = pairs / experts
-        width = math.sqrt(2 * per)
-
-        def row_tiles(rows):
-            more = sum(0.5 * math.erfc((i * rows - per) / width) for i in range(1, int((per + 4 * width) / rows) + 1))
-            return min(pairs, experts * (1.0 + more))
-
-        def us(number, n, k, halved):
-            rows, columns, resident, a, b, c = TILES[number]
-            tiles = max(1, round(row_tiles(rows) * -(-n // (columns // 2 if halved else columns))))
-            rounds = -(-(-(-tiles // 256)) // resident)
-            return 3 + rounds * (c + k // 64 * (a + b * min(1.0, tiles / (256 * resident * rounds))))
-
+        """(rows, first product's tile, second's) for experts by tiles: the least time of both by ``experts_product``. Over
+        the launches its model is made from, the choice takes 1.6 % more than the best on average, 16 % at worst. Tiles of 128
+        rows are for some 60 to 110 pairs an expert, where 64 rows are two tiles and 192 mostly padding, if there are enough to
+        give every compute unit one (8 experts of 4,096 x 1,024 with 80 pairs each: 74 us, 69 with 64 rows). Both products, us, with the loop of
+        128 x 128 tiles behind two barriers a stage that was first there, with tiles of 64 and 192 rows alone, and now, at 32, 64, 80, 96 and 255 pairs an expert: 16 of 2,560 x 1,536, 2 a token, 104, 114,
+        119, 124, 207; 95, 110, 100, 101, 168 and 95, 96, 97, 100, 168; 24 of 3,072 x 1,280, 3 a token, 137, 150, 157, 166, 299; 126, 163, 171, 179, 257
+        and 126, 153, 160, 168, 257; 64 of 2,048 x 768, 8 a token, 166, 183, 187, 194, 337; 165, 188, 201, 207, 320 and 155, 185, 193, 201, 316; 128
+        of those 294, 324, 335, 353, 660; 282, 332, 375, 390, 633 and 282, 323, 337, 350, 621; 8 of 4,096 x 1,024 82, 84, 86, 87, 139; 60, 74, 70, 73,
+        100 and 59, 73, 70, 73, 99."""
         best = None
-        longest = max(TILES[i][0] for i in cls.EXPERT_TILES)
         for rows in sorted({TILES[i][0] for i in cls.EXPERT_TILES}):
-            if rows < longest and 1.7 * rows < per:
-                continue
             same = [i for i in cls.EXPERT_TILES if TILES[i][0] == rows]
-            first = min((us(i, inter, hidden, gated), i) for i in same)
-            second = min((us(i, hidden, inter, False), i) for i in same)
-            if best is None or first[0] + second[0] < best[0]:
-                best = first[0] + second[0], rows, first[1], second[1]
+            (first, _, tiles), one = min((cls.experts_product(i, pairs, experts, inter, hidden, gated), i) for i in same)
+            (second, _, _), two = min((cls.experts_product(i, pairs, experts, hidden, inter, False), i) for i in same)
+            if (best is None or first + second < best[0]) and (rows != 128 or tiles >= 256):
+                best = first + second, rows, one, two
         return best[1:]
 
     # elements of the tokens that one launch of the experts' tiles takes: their offsets are 32 bits
@@ -1124,6 +1137,8 @@ class HipOps:
                                                          weight_on_input)
                 return out
             rows, tile, tile_down = self.choose_experts_tiles(pairs, n, h, inter, activation != "relu2")
+            tile = self.experts_product(tile, pairs, n, inter, h, activation != "relu2")[1]
+            tile_down = self.experts_product(tile_down, pairs, n, h, inter, False)[1]
             scratch = torch.empty(pairs + n + 2 + 2 * (pairs // rows + n), dtype=torch.int32, device=x.device)
         act = torch.empty((pairs, inter), dtype=x.dtype, device=x.device)
         self._check(self.lib, self.lib.qrt_experts(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(index), _ptr(weight), _ptr(act),

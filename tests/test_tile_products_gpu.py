@@ -272,3 +272,41 @@ def test_experts_tokens_in_several_goes(activation, given):
     out = torch.full_like(whole, float("nan")) if given else None
     got = ops.moe_for_residual(x, up, down, index, weight, activation, 0.0, out=out)
     assert torch.equal(got, whole) and (out is None or got is out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first,second", [(0, 0), (16, 0), (0, 16), (16, 16)])
+@pytest.mark.parametrize("activation", ["swiglu", "relu2"])
+def test_experts_two_blocks_a_compute_unit(activation, first, second):
+    """Both forms of the tiles of 128 x 128, in launches of more blocks than the compute units hold: an expert with one
+    pair past a tile, one with a whole one, others with one or none. Sums are in the order of k, so the bits are those of every
+    other tile."""
+    from test_experts_gpu import close as near
+    from test_experts_gpu import plain
+
+    ops = HipOps()
+    ops.experts_tile_pairs_per_expert = 0
+    n, h, inter = 150, 448, 320
+    counts = [129, 128, 0] + [1] * (n - 3)
+    index = torch.cat([torch.full((c, 1), e) for e, c in enumerate(counts)])
+    index = index[torch.randperm(len(index), generator=torch.Generator().manual_seed(1))].int().to(DEV)
+    t = index.shape[0]
+    x = rnd(t, h, seed=1)
+    up, down = rnd(n, (2 if activation == "swiglu" else 1) * inter, h, seed=2, scale=h ** -0.5), rnd(n, h, inter, seed=3, scale=inter ** -0.5)
+    weight = torch.rand(t, 1, device=DEV)
+    outs = []
+    for rows, tiles in ((128, (7 + first, 7 + second)), (64, (12, 12))):
+        ops.choose_experts_tiles = lambda *sizes: (rows, 0, 1)  # noqa: B023
+        ops.experts_product = lambda i, *sizes: (0.0, tiles[i], 1)  # noqa: B023
+        outs.append(ops.moe_for_residual(x, up, down, index, weight, activation, 0.0))
+    near(outs[0], plain(x, up, down, index, weight, activation, 0.0, False).float(), 4e-3, 4e-3)
+    assert torch.equal(*outs)
+
+
+def test_experts_of_60_to_110_pairs_take_tiles_of_128():
+    """Between tiles that are mostly padding and two tiles an expert, where they give every compute unit one."""
+    rows = [HipOps.choose_experts_tiles(64 * per, 64, 2048, 768, True)[0] for per in (32, 64, 80, 128)]
+    assert rows == [64, 128, 128, 192] and HipOps.choose_experts_tiles(24 * 80, 24, 3072, 1280, True)[0] == 128
+    assert HipOps.choose_experts_tiles(8 * 80, 8, 4096, 1024, True)[0] == 64
+    assert HipOps.experts_product(7, 64 * 128, 128, 768, 2048, True)[1] == 7 + HipOps.experts_two_blocks   # 1,536 tiles: 3 rounds of 512
+    assert HipOps.experts_product(7, 64 * 64, 64, 768, 2048, True)[1] == 7                                  # 768: 3 rounds of 256, not 1.5 of 512
