@@ -1288,24 +1288,31 @@ class HipOps:
     def choose_tile(m: int, n: int, k: int, form: str = "whole") -> tuple[int, int]:
         """(tile, parts of K) for ``m`` rows by a weight [n, k] ("gated": [2n, k]): the least time by the model of
         ``TILES``. ``form`` "planes": K may be cut into up to eight parts of at least eight stages each, for products
-        whose tiles do not fill the compute units; the norm that adds the planes reads them at some 5 TB/s. It is
-        within 3 % of the best choice on average over the launches the model is made from, 30 % at worst (256 rows
-        and fewer, where launches take 15 us). Follows from the sizes alone, so that equal inputs give equal bits."""
-        best = None
+        whose tiles do not fill the compute units; the norm that adds the planes reads them at some 5 TB/s. Follows from
+        the sizes alone, so that equal inputs give equal bits.
+
+        Tiles are looked at in the order of a bound that no number of parts undercuts, until the bound is above the
+        best found: 33 us of the host for a size that it has not seen, 64 where every choice is tried."""
+        stages = k // 64
+        most, read = (9, m * n / 5e6) if form == "planes" else (2, 0.0)
+        order = []
         for number, (rows, columns, resident, a, b, c) in enumerate(TILES):
             tiles = -(-m // rows) * -(-n // (columns // 2 if form == "gated" else columns))
-            for parts in range(1, 9 if form == "planes" else 2):
-                stages = -(-(k // 64) // parts)
-                if parts > 1 and (stages < 8 or stages * (parts - 1) >= k // 64):
+            order.append((3 + c + stages * (a + b) * tiles / (256 * resident) + 2 * read, number, tiles))
+        best = math.inf, 0, 0
+        for bound, number, tiles in sorted(order):
+            if bound > best[0] * (1 + 1e-9):  # by more than rounding, so that no equal time is missed
+                break
+            _, _, resident, a, b, c = TILES[number]
+            for parts in range(1, most):
+                part = -(-stages // parts)
+                if parts > 1 and (part < 8 or part * (parts - 1) >= stages):
                     break
                 load = -(-tiles * parts // 256)  # blocks of the busiest compute unit
                 rounds = -(-load // resident)
                 full = load / (resident * rounds) if 1 < load and resident > 1 else tiles * parts / (256 * resident * rounds)
-                us = 3 + rounds * (c + stages * (a + b * full))
-                if form == "planes":
-                    us += m * n * (4 * parts if parts > 1 else 2) / 5e6
-                if best is None or us < best[0]:
-                    best = us, number, parts
+                us = 3 + rounds * (c + part * (a + b * full)) + read * (4 * parts if parts > 1 else 2)
+                best = min(best, (us, number, parts))
         return best[1:]
 
     @staticmethod

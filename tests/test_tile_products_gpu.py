@@ -310,3 +310,33 @@ def test_experts_of_60_to_110_pairs_take_tiles_of_128():
     assert HipOps.choose_experts_tiles(8 * 80, 8, 4096, 1024, True)[0] == 64
     assert HipOps.experts_product(7, 64 * 128, 128, 768, 2048, True)[1] == 7 + HipOps.experts_two_blocks   # 1,536 tiles: 3 rounds of 512
     assert HipOps.experts_product(7, 64 * 64, 64, 768, 2048, True)[1] == 7                                  # 768: 3 rounds of 256, not 1.5 of 512
+
+
+def test_choice_of_tile_misses_none():
+    """The search that leaves out what its bound excludes finds what trying everything finds."""
+    import random
+
+    def every(m, n, k, form):
+        best = None
+        for number, (rows, columns, resident, a, b, c) in enumerate(TILES):
+            tiles = -(-m // rows) * -(-n // (columns // 2 if form == "gated" else columns))
+            for parts in range(1, 9 if form == "planes" else 2):
+                stages = -(-(k // 64) // parts)
+                if parts > 1 and (stages < 8 or stages * (parts - 1) >= k // 64):
+                    break
+                load = -(-tiles * parts // 256)
+                rounds = -(-load // resident)
+                full = load / (resident * rounds) if 1 < load and resident > 1 else tiles * parts / (256 * resident * rounds)
+                us = 3 + rounds * (c + stages * (a + b * full))
+                if form == "planes":
+                    us += m * n * (4 * parts if parts > 1 else 2) / 5e6
+                if best is None or us < best[0]:
+                    best = us, number, parts
+        return best[1:]
+
+    draw = random.Random(5)
+    sizes = [(m, n, k) for m in (65, 129, 512, 2048, 8191) for n, k in ((16, 64), (2560, 9728), (6144, 2560), (5120, 25600))]
+    sizes += [(draw.randint(1, 9000), 16 * draw.randint(1, 2000), 64 * draw.randint(1, 450)) for _ in range(1500)]
+    for m, n, k in sizes:
+        for form in ("whole", "gated", "planes"):
+            assert HipOps.choose_tile(m, n, k, form) == every(m, n, k, form), (m, n, k, form)
