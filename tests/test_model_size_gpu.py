@@ -169,6 +169,29 @@ def test_long_context_decode_beside_a_prompt_portion(sized, monkeypatch):
     check_rounding_noise(got, {k: want[k] for k in got})
 
 
+@pytest.mark.parametrize("name", ["qwen3_4b", "qwen3_8b"])
+def test_a_prompt_of_two_thousand_tokens(sized, name):
+    """2,041 tokens in one step, then one by one: products by tiles in several rounds of blocks, planes of K cut in two,
+    ragged last tiles. Logits all over the prompt against the plain implementation."""
+    from qwen3_runtime_amd.ops.hip import TILES, HipOps
+
+    cfg, folder = sized[name]
+    tile, _ = HipOps.choose_tile(2041, cfg.intermediate_size, cfg.hidden_size, "gated")
+    if name == "qwen3_4b":  # more tiles than the compute units hold: blocks make several
+        assert not HipOps.library_takes(2041, cfg.intermediate_size, cfg.hidden_size, "gated")
+        assert -(-2041 // TILES[tile][0]) * -(-cfg.intermediate_size // (TILES[tile][1] // 2)) > 256
+        assert HipOps.choose_tile(2041, cfg.hidden_size, cfg.intermediate_size, "planes")[1] > 1
+    at = sorted({0, 1, 63, 64, 191, 192, 255, 256, 1023, 1024, 1791, 1792, 1919, 1920, 2040, 2043, *range(7, 2041, 97)})
+    reqs, want = sized.plain_logits(name, [2044], seed=71, positions={"r0": at})
+    first = [p for p in at if p < 2041]
+    steps = [{"entries": [{"id": "r0", "tokens": reqs["r0"][:2041], "want": first}], "end": []}]
+    steps += [{"entries": [{"id": "r0", "tokens": reqs["r0"][p: p + 1], "want": [0] if p in at else []}], "end": ["r0"] if p == 2043 else []}
+              for p in range(2041, 2044)]
+    got = traces.replay(load_sized(folder, traces._number(steps), "bfloat16"), steps)
+    assert set(got) == set(want)
+    check_rounding_noise(got, want)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_six_layers_deep(sized, dtype):
     """The 4B width six layers deep, the last 32 tokens of each request decoded one by one from
