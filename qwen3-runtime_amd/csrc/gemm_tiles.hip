@@ -42,7 +42,7 @@ constexpr size_t tile_lds_bytes() {
 
 // WM x WN waves, each with BM / WM rows and BN / WN columns of the tile. GATED: 16 rows of the tile's
 // weights are 8 gate rows and the 8 up rows that belong to them, so any BN makes BN / 2 columns.
-template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO>
+template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO, int POLICY = 0>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileArgs p) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host's compiler knows no buffer resources
   typedef Tile<BM, BN, WM, WN, S> T;
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
   locate(tile);
   while (true) {
     f32x4_t acc[TM][TN];
-    T::products(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, fetched, acc);
+    T::template products<POLICY>(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, fetched, acc);
     QRT_WAIT_LDS();
     QRT_BARRIER();  // nobody reads the ring any more
     // acc[i][j][r]: row 16 i + r16 of the wave's result, row 16 j + 4 quad + r of its weights
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
     tile += gridDim.x;
     if (more) {
       locate(tile);
-      T::fetch_first(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, 0, FIRST);
+      T::template fetch_first<POLICY>(a_buf, w_buf, aoff, woff, s0, stages, tiles_lds, 0, FIRST);
     }
     if constexpr (sizeof(TO) == 4) {
 #pragma unroll
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
 #endif
 }
 
-template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO>
+template <int BM, int BN, int WM, int WN, int S, int GATED, typename TO, int POLICY = 0>
 static int launch_tiles(TileArgs p, hipStream_t stream) {
   constexpr size_t smem = tile_lds_bytes<BM, BN, WM, WN, S, GATED, TO>();
   const int width = GATED ? BN / 2 : BN;
@@ -182,7 +182,7 @@ static int launch_tiles(TileArgs p, hipStream_t stream) {
   p.ntiles = (p.N + width - 1) / width;
   const int64_t blocks = (int64_t)p.mtiles * p.ntiles * p.parts;
   QRT_CHECK(blocks < (1 << 30), "gemm_tiles: too many tiles for one launch (M=%d N=%d)", p.M, p.N);
-  auto kernel = gemm_bf16_tiles_kernel<BM, BN, WM, WN, S, GATED, TO>;
+  auto kernel = gemm_bf16_tiles_kernel<BM, BN, WM, WN, S, GATED, TO, POLICY>;
   static bool allowed = false;  // once per kernel: not inside a stream capture again and again
   if (smem > 64 * 1024 && !allowed) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
@@ -235,7 +235,13 @@ extern "C" int qrt_gemm_tiles(const void* a, const void* w, void* c, int out_dty
     case 9: return by_result<96, 160, 2, 2, 4>(p, out_dtype, mode, stream);
     case 10: return by_result<96, 96, 2, 2, 6>(p, out_dtype, mode, stream);
     case 11: return by_result<128, 64, 2, 2, 6>(p, out_dtype, mode, stream);
-    case 12: return by_result<64, 64, 1, 4, 4>(p, out_dtype, mode, stream);
+    case 12:
+      // One row tile: no block reads another's weights, so they come as data used once. As plain loads they put out of the L2s what the
+      // kernels around the product read again, and every one of those took longer (the router of a 2,048-wide model 6.6 -> 8.1 us): decoding
+      // 48 requests of the 2B size with latent attention took 2.52 ms a step with the kernel that shares the activations, 2.61 with
+      // plain tiles and 2.50 so; the 4B size 3.71, 3.65 and 3.56.
+      if (M <= 64 && mode == 0 && out_dtype == QRT_F32) return launch_tiles<64, 64, 1, 4, 4, 0, float, 2>(p, stream);
+      return by_result<64, 64, 1, 4, 4>(p, out_dtype, mode, stream);
     case 13: return by_result<64, 128, 1, 4, 3>(p, out_dtype, mode, stream);
     default: return qrt_fail("gemm_tiles: no tile %d", tile);
   }

@@ -92,8 +92,10 @@ struct Tile {
     return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, RAW);
   }
 
-  // load j of the stage that begins at byte `at` of every row, into the slot that begins at `dst`. aoff, woff: where each
+  // POLICY: the cache policy of the weights' loads (2: non-temporal, for weights that no other block reads).
+  // Load j of the stage that begins at byte `at` of every row, into the slot that begins at `dst`. aoff, woff: where each
   // load of this lane begins, in bytes from its buffer, without the stage's.
+  template <int POLICY>
   static __device__ __forceinline__ void fetch_one(const __amdgpu_buffer_rsrc_t a_buf, const __amdgpu_buffer_rsrc_t w_buf,
                                                    const unsigned (&aoff)[AL], const unsigned (&woff)[WL], int at,
                                                    unsigned char* dst, int j, int wave) {
@@ -102,10 +104,11 @@ struct Tile {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buf, (lds_ptr_t)(dst + unit * 1024), 16, aoff[j], at, 0, 0);
     } else {
       const int unit = WU % WAVES && j == LOADS - 1 ? min(wave + WAVES * (j - AL), WU - 1) : wave + WAVES * (j - AL);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf, (lds_ptr_t)(dst + (AU + unit) * 1024), 16, woff[j - AL], at, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf, (lds_ptr_t)(dst + (AU + unit) * 1024), 16, woff[j - AL], at, 0, POLICY);
     }
   }
   // stages `from` to `to` - 1 of a tile of `stages`, each into the slot of its number
+  template <int POLICY = 0>
   static __device__ __forceinline__ void fetch_first(const __amdgpu_buffer_rsrc_t a_buf, const __amdgpu_buffer_rsrc_t w_buf,
                                                      const unsigned (&aoff)[AL], const unsigned (&woff)[WL], int s0, int stages,
                                                      unsigned char* lds, int from, int to) {
@@ -114,13 +117,14 @@ struct Tile {
     for (int s = 0; s < S; ++s)
       if (s >= from && s < to && s < stages) {
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j) fetch_one(a_buf, w_buf, aoff, woff, (s0 + s) * 128, lds + s * STAGE, j, wave);
+        for (int j = 0; j < LOADS; ++j) fetch_one<POLICY>(a_buf, w_buf, aoff, woff, (s0 + s) * 128, lds + s * STAGE, j, wave);
       }
   }
 
   // acc[i][j] of a wave, from zero: row 16 i + (lane & 15) of its rows, rows 16 j + 4 (lane / 16) + 0..3 of its
   // weights. `fetched`: how many first stages have been asked for already; whatever else the wave has on its way to memory
   // since (stores) only makes the waits longer, since loads land in order.
+  template <int POLICY = 0>
   static __device__ __forceinline__ void products(const __amdgpu_buffer_rsrc_t a_buf, const __amdgpu_buffer_rsrc_t w_buf,
                                                   const unsigned (&aoff)[AL], const unsigned (&woff)[WL], int s0, int stages,
                                                   unsigned char* lds, int fetched, f32x4_t (&acc)[TM][TN]) {
@@ -167,7 +171,7 @@ struct Tile {
         if (owed) {
 #pragma unroll
           for (int j = i * LATE_A_ROW; j < (i + 1) * LATE_A_ROW && j < LATE; ++j)
-            fetch_one(a_buf, w_buf, aoff, woff, stage_at(it - 1 + S), lds + before * STAGE, SOON + j, wave);
+            fetch_one<POLICY>(a_buf, w_buf, aoff, woff, stage_at(it - 1 + S), lds + before * STAGE, SOON + j, wave);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -185,14 +189,14 @@ struct Tile {
         if (MORE) {
 #pragma unroll
           for (int j = i * SOON_A_ROW; j < (i + 1) * SOON_A_ROW && j < SOON; ++j)
-            fetch_one(a_buf, w_buf, aoff, woff, stage_at(it + S), lds + slot * STAGE, j, wave);
+            fetch_one<POLICY>(a_buf, w_buf, aoff, woff, stage_at(it + S), lds + slot * STAGE, j, wave);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     };
 
     if (stages > 0) {  // the same in every wave of the block
-      fetch_first(a_buf, w_buf, aoff, woff, s0, stages, lds, fetched, S);
+      fetch_first<POLICY>(a_buf, w_buf, aoff, woff, s0, stages, lds, fetched, S);
       if (stages >= S) QRT_WAIT_LOADS((S - 1) * LOADS);
       else QRT_WAIT_LOADS(0);
       QRT_BARRIER();

@@ -1320,12 +1320,14 @@ class HipOps:
         """Parts of K in which 17 to 128 rows go by tiles of 64 x 64, a block a compute unit (0: by the kernel that shares
         the activations). Four stages of 16 KB in flight bring a compute unit its 200 KB of a small weight sooner than that
         kernel does, whose blocks of eight row tiles then leave compute units idle: 2,560 weight rows in eight parts are 160
-        blocks. 4,096 weight rows are 256, and it keeps them: decoding 64 requests of the 8B size from 256 tokens on takes 4.55 ms
-        a step with its output projection, 4.64 with tiles for that one product (32 requests 3.91 and 3.98; three runs of each in
-        turn, 0.01 apart), though by itself, called again and again, tiles are level or ahead (4,096 x 4,096 at 24, 48 and 64 rows 9.3,
-        10.6, 12.0 and 9.3, 10.3, 11.1 us). Product and the norm's read of the planes, us, that kernel and tiles at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.0, 9.3, 9.9, 13.6
-        and 6.9, 7.4, 7.8, 10.4; 2,560 x 9,728 13.3, 15.0, 16.1, 21.3 and 12.5, 13.6, 14.7, 20.5; 2,048 x 2,048 6.7, 6.8, 8.3, 10.4 and
-        5.2, 5.6, 5.9, 6.7; 4,096 x 12,288 19.3, 22.7, 22.9, 30.6 and 21.9, 23.5, 24.7, 31.5."""
+        blocks. Product and the norm's read of the planes, us, that kernel and tiles in turn at 24, 48, 64 and 128 rows: 2,560 x 4,096 8.8, 9.9, 10.5,
+        13.4 and 7.9, 8.7, 9.3, 12.0; 2,560 x 9,728 14.3, 14.9, 16.2, 22.5 and 12.9, 13.4, 14.4, 22.3 (19.4 and 20.6 at 96 rows, the weight
+        then comes twice); 2,048 x 2,048 6.9, 6.8, 8.2, 10.1 and 5.9, 6.4, 6.9, 7.1; sizes not looked at when the lines were drawn: 2,048 x 6,144 10.2, 9.4, 11.3,
+        14.5 and 8.4, 8.8, 9.6, 13.4; 3,072 x 8,192 13.1, 15.2, 15.8, 20.9 and 12.8, 13.8, 14.9, 24.6. A decoding step of the 4B size, 20, 48 and 100
+        requests of 256 tokens, 2.84, 3.71, 4.94 and 2.74, 3.56, 4.91 ms. Larger weights, and those that give the sharing kernel 224 blocks or
+        more, are level: 4,096 x 4,096 9.4, 11.3, 12.0, 17.0 and 9.8, 10.8, 11.6, 18.3; 5,120 x 8,192 18.3, 19.5, 20.3, 29.3 and 19.2, 19.3, 21.0, 29.4;
+        steps of the 8B size with 20, 32, 48 and 64 requests 3.78, 3.86, 4.62, 4.52 and 3.76, 3.87, 4.58, 4.56 ms, of the 32B size 14.2, 14.8, 16.7, 17.4 and
+        14.3, 14.9, 16.8, 17.7."""
         if not 17 <= m <= 128 or n * k > 26 << 20 or -(-n // 128) * HipOps.choose_k_parts(n, k, m, True) >= 224:
             return 0
         parts = min(8, 256 // (-(-m // 64) * -(-n // 64)), k // 64 // 8)

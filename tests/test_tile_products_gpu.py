@@ -340,3 +340,18 @@ def test_choice_of_tile_misses_none():
     for m, n, k in sizes:
         for form in ("whole", "gated", "planes"):
             assert HipOps.choose_tile(m, n, k, form) == every(m, n, k, form), (m, n, k, form)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 17, 48, 64])
+def test_weights_used_once(m):
+    """Up to 64 rows tiles of 64 x 64 load the weights as data used once, beyond as any other: the same bits."""
+    ops, n, k = HipOps(), 1040, 1600
+    x, w = rnd(65, k, seed=1), rnd(n, k, seed=2, scale=0.05)
+    for parts in (1, 3, 8):
+        outs = []
+        for rows in (m, 65):
+            out = torch.full((parts, rows, n) if parts > 1 else (rows, n), float("nan"), device=DEV)
+            launch(ops, x[:rows], w, out, 12, parts)
+            outs.append(out)
+        assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1][..., :m, :])
