@@ -1038,14 +1038,15 @@ class HipOps:
         140, at 16 196 and 145; 8 of 4,096 x 1,024 (128 tiles) at 16 56 and 72, at 24 71 and 73, at 32 87 and 75."""
         return min(32, max(9, 6000 // (experts * inter // 64 or 1)))
 
-    # Tiles that the experts' kernel knows, by their numbers in ``TILES``, and what a product of one takes, in microseconds, as
-    # there but with one tile a block: c for every round of blocks over the compute units, a for each of its stages, b more
-    # where the round is full, and w for every megabyte of weights. 128 x 128 has a second form with half the stages, two blocks
-    # a compute unit. Least squares over the launches within 1.25 of the best of each of 90: 8 to 128 experts of 2,048 x 768 to
-    # 4,096 x 1,024, 12 to 700 pairs an expert, weights of several layers in turn.
-    EXPERT_COSTS = {3: (1, 0.333, 0.363, 13.802, 0.046), 4: (1, 0.419, 0.226, 13.148, 0.017), 5: (1, 0.253, 0.272, 12.431, 0.011),
-                    7: (1, 0.244, 0.140, 11.070, 0.032), 12: (2, 0.028, 0.274, 5.871, 0.083), 13: (2, 0.105, 0.381, 7.739, 0.100)}
-    EXPERT_COSTS_TWO_BLOCKS = {7: (2, 0.407, 0.321, 16.214, 0.043)}
+    # Tiles that the experts' kernel knows, by their numbers in ``TILES``, and what a product of one takes, in microseconds, with one
+    # tile a block: the root of the squares' sum of c for every round of blocks over the compute units, a for each of its stages and b more
+    # where the round is full, and of w for every megabyte of weights (they come while others compute, in part). 128 x 128 has a
+    # second form with half the stages, two blocks a compute unit. Least squares over the launches within 1.25 of the best of each of 155: 8
+    # to 128 experts of 2,048 x 768 to 4,096 x 2,048, 8 to 700 pairs an expert, weights of several layers in turn; 6 % off on average.
+    # Those of 64 rows are 4 % below their fit, with which the fewest launches take a slower tile than before.
+    EXPERT_COSTS = {3: (1, 0.472, 0.453, 10.603, 0.117), 4: (1, 0.422, 0.409, 9.058, 0.104), 5: (1, 0.166, 0.518, 9.078, 0.082),
+                    7: (1, 0.191, 0.376, 6.826, 0.140), 12: (2, 0.057, 0.371, 5.003, 0.146), 13: (2, 0.181, 0.506, 5.810, 0.168)}
+    EXPERT_COSTS_TWO_BLOCKS = {7: (2, 0.420, 0.685, 9.124, 0.142)}
     EXPERT_TILES = tuple(EXPERT_COSTS)
     experts_two_blocks = 16  # what csrc/experts.hip adds to the number of that form
 
@@ -1065,21 +1066,23 @@ class HipOps:
                 resident, a, b, c, w = costs[tile]
                 rounds = -(-(-(-tiles // 256)) // resident)
                 full = min(1.0, tiles / (256 * resident * rounds))
-                forms.append((rounds * (c + k // 64 * (a + b * full)) + w * experts * n * k * (4e-6 if halved else 2e-6), number, tiles))
+                arrive = w * experts * n * k * (4e-6 if halved else 2e-6)
+                forms.append((math.hypot(rounds * (c + k // 64 * (a + b * full)), arrive), number, tiles))
         return min(forms)
 
     @classmethod
     @functools.lru_cache(maxsize=4096)
     def choose_experts_tiles(cls, pairs: int, experts: int, hidden: int, inter: int, gated: bool) -> tuple[int, int, int]:
         """(rows, first product's tile, second's) for experts by tiles: the least time of both by ``experts_product``. Over
-        the launches its model is made from, the choice takes 1.6 % more than the best on average, 16 % at worst. Tiles of 128
-        rows are for some 60 to 110 pairs an expert, where 64 rows are two tiles and 192 mostly padding, if there are enough to
+        the launches its model is made from, the choice takes 2.1 % more than the best on average, 20 % at worst. Tiles of 128
+        rows are for some 50 to 110 pairs an expert, where 64 rows are two tiles and 192 mostly padding, if there are enough to
         give every compute unit one (8 experts of 4,096 x 1,024 with 80 pairs each: 74 us, 69 with 64 rows). Both products, us, with the loop of
-        128 x 128 tiles behind two barriers a stage that was first there, with tiles of 64 and 192 rows alone, and now, at 32, 64, 80, 96 and 255 pairs an expert: 16 of 2,560 x 1,536, 2 a token, 104, 114,
-        119, 124, 207; 95, 110, 100, 101, 168 and 95, 96, 97, 100, 168; 24 of 3,072 x 1,280, 3 a token, 137, 150, 157, 166, 299; 126, 163, 171, 179, 257
-        and 126, 153, 160, 168, 257; 64 of 2,048 x 768, 8 a token, 166, 183, 187, 194, 337; 165, 188, 201, 207, 320 and 155, 185, 193, 201, 316; 128
-        of those 294, 324, 335, 353, 660; 282, 332, 375, 390, 633 and 282, 323, 337, 350, 621; 8 of 4,096 x 1,024 82, 84, 86, 87, 139; 60, 74, 70, 73,
-        100 and 59, 73, 70, 73, 99."""
+        128 x 128 tiles behind two barriers a stage that was first there, with tiles of 64 and 192 rows alone, and now, at 32, 64, 80, 96 and 255 pairs an
+        expert: 16 of 2,560 x 1,536, 2 a token, 107, 117, 122, 128, 207; 98, 114, 102, 101, 174 and 98, 96, 98, 100, 166; 24 of 3,072 x 1,280, 3 a
+        token, 137, 151, 158, 166, 301; 126, 166, 174, 182, 262 and 125, 152, 160, 169, 253; 64 of 2,048 x 768, 8 a token, 159, 176, 182, 188, 336;
+        154, 181, 195, 201, 314 and 155, 174, 181, 190, 320; 128 of those 293, 328, 334, 351, 646; 274, 328, 365, 386, 627 and 274, 316, 329, 342,
+        615; 16 of 4,096 x 2,048, 2 a token, 197, 203, 205, 211, 405; 199, 226, 221, 231, 362 and 187, 222, 223, 225, 362 (from 64 to 96 pairs
+        the former loop is still 7 to 10 % ahead there, the only size measured where it is)."""
         best = None
         for rows in sorted({TILES[i][0] for i in cls.EXPERT_TILES}):
             same = [i for i in cls.EXPERT_TILES if TILES[i][0] == rows]
