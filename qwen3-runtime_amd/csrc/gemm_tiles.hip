@@ -5,12 +5,12 @@
 //
 // The result goes through LDS so that rows are stored in whole lines: 64 -> 59 us for 2,048 x 6,144
 // x 2,560, whose blocks all end at once. Blocks that make several tiles ask for the next one's first
-// stages before they store the last one's result: 186 -> 179 us for gate/up at 2,048 rows, 976 tiles. Every output is a sum over K in the order of k, so its bits
-// depend neither on M nor on the tile, only on the number of planes.
-// Against the library's product (and gated_act behind it) at the 4B sizes, weights of several layers
-// in turn, q/k/v, output, gate/up and down at 512 rows: 27 (29), 19 (25), 52 (67) and 34 us (53);
-// at 2,048 rows: 58 (58), 41 (50), 179 (209) and 82 us (117). See HipOps.choose_tile for which
-// tile is taken.
+// stages before they store the last one's result: 186 -> 179 us for gate/up at 2,048 rows, 976 tiles.
+// Every output is a sum over K in the order of k, so its bits depend neither on M nor on the tile,
+// only on the number of planes.
+// Against the library's product (and gated_act behind it) at the 4B sizes, called in turn with it, weights of several
+// layers, q/k/v, output, gate/up and down at 512 rows: 27 (27), 19 (24), 52 (69) and 34 us (51); at 2,048
+// rows: 60 (58), 43 (51), 183 (195) and 85 us (107), output and down as float32 planes. See HipOps.choose_tile for which tile is taken.
 #include "common.h"
 #include "direct.h"
 #include "gemm_epilogue.h"

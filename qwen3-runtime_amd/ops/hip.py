@@ -11,8 +11,8 @@ Matrix products: float32 goes to the library's own float32 MFMA kernels
 products cut along K) goes to the library's MFMA kernels that stream the
 weights, bfloat16 with more rows to its tiles through LDS; what those do not
 take (K no multiple of 64, weight rows no multiple of 16, operands off 16
-bytes), and beyond 2,048 rows what fills the vendor BLAS's own tiles, goes
-to that through ``torch.matmul``, as the reference leaves its products to
+bytes), and what fills the vendor BLAS's own tiles beyond 2,048 rows (with
+4,096 columns of K beyond 1,536), goes to that through ``torch.matmul``, as the reference leaves its products to
 cuBLAS (qwen3_runtime/models/qwen3.py:76-77,134-135).
 """
 
@@ -257,7 +257,10 @@ check_tensor = _need  # for parts that call a library of their own
 # once, and what a launch takes, in microseconds: 3, and for every round of blocks over the compute units c, and for each
 # of its stages of 64 columns of K a, and b more where the round is full (fewer blocks share the caches and the clock).
 # Least squares over 3,600 launches: the q/k/v, output, gate/up and down sizes of the 4B, 8B and 32B models with 65 to
-# 4,096 rows, whole and in two to eight parts of K, weights of several layers in turn; single launches lie 4 to 10 % from it.
+# 4,096 rows, whole and in two to eight parts of K, weights of several layers in turn, when a block made one tile. Blocks that make
+# several hide the start of further rounds, which c still counts; checked over 24,000 launches of that kernel, 37 weights of the 1.7B to 32B
+# sizes and of seven designs, single launches lie 8 to 15 % from it, and the tile it chooses takes 2.3 % more than the best on average, 31 % at
+# worst. Constants of the same kind for the first and for further rounds, fitted to those launches, choose 1.7 % above the best: not worth other sums.
 TILES = (
     (256, 192, 1, 1.014, 0.188, 7.734), (256, 160, 1, 0.590, 0.319, 8.114), (256, 128, 1, 0.519, 0.257, 6.862),
     (192, 192, 1, 0.558, 0.275, 7.049), (192, 160, 1, 0.515, 0.229, 6.576), (192, 128, 1, 0.442, 0.190, 5.529),
@@ -270,7 +273,7 @@ SHORT_TILE = 12
 
 
 class HipOps:
-    # bfloat16 products with more rows than this are made by tiles
+    # bfloat16 products with more rows than this are made by tiles or the vendor library
     own_max_rows = 64
     # the same for the two forms in which a block fetches fewer activations than weights: the
     # gated product, and the product cut along K whose planes the residual's norm adds
@@ -1275,10 +1278,18 @@ class HipOps:
         whose 256 x 256 tiles fill the compute units to 0.62 or more in whole rounds, and gated ones from 4,096 rows on, or
         from 4,096 columns of K and 1,537 rows on. So do whole ones of such rows that fill 0.7 (a 2,048-token prompt of the 8B
         size: 26.5 ms with q/k/v and gate/up by the library and the rest by tiles, 28.1 with q/k/v by tiles as well, 27.0 with
-        everything by either). Library and tiles in turn, us, at 1,536, 2,048, 2,500 and 3,500 rows: 4B q/k/v 50, 59, 64, 100
-        and 43, 52, 71, 104; 4B down 97, 115, 137, 166 and 74, 92, 116, 151; 8B output 56, 66, 76, 95 and 48, 62, 76, 110; 8B down 148, 187, 199, 270
-        and 140, 171, 234, 311; gate/up and SwiGLU, 4B 158, 197, 241, 324 and 144, 189, 227, 317, 8B 269, 317, 405, 557 and 262, 349, 445, 602;
-        at 4,096 and 8,192: 4B 362, 693 and 370, 719, 8B 608, 1,191 and 678, 1,335."""
+        everything by either). Library and tiles (for the residual with the norm's read of the planes) in turn with one another, weights of several layers, us, at 1,536, 2,048, 2,500
+        and 3,500 rows: 4B q/k/v 54, 58, 63, 97 and 45, 60, 76, 108; 4B down 92, 111, 138, 162 and 73, 93, 125, 149; 8B output 56, 68, 75, 95 and 50, 64, 86, 111; 8B
+        down 146, 196, 196, 278 and 143, 172, 245, 316; gate/up and SwiGLU, 4B 153, 195, 234, 314 and 139, 183, 223, 311, 8B 273, 313, 418, 572 and 261, 344,
+        439, 605; at 4,096 and 8,192: 4B 353, 677 and 353, 703, 8B 625, 1,211 and 672, 1,341.
+
+        On 37 weights, 25 of which were not looked at when the lines were drawn, at 65 to 8,192 rows, what they choose takes
+        1.6 % (gated) and 3.3 % (for the residual) more than the best of library and tiles on average. Whole products called alone are
+        10 % off, narrow ones above all: 16 or 32 weight rows of 2,560 take 10.5 us by tiles and 6.3 by the library, 448 at 200 rows 11.2 and 7.4;
+        12,368 and 16,384 at 2,048 rows 119 and 159, by the library 124 and 130. In whole prompt steps it is the tiles that are ahead: ten models of seven designs at
+        100, 200, 400, 700, 1,024, 1,500 and 2,048 tokens take up to 6 % less with these lines than with all whole products by
+        the library, 1 % more where a joint projection has 16,384 rows (700, 1,024 and 2,048 tokens); with
+        narrow ones alone by the library they take 0.9 % less to 7 % more."""
         long_rows = k >= 4096 and m > 1536
         if form == "gated":
             return m >= 4096 or long_rows
@@ -1386,7 +1397,7 @@ class HipOps:
     def _own_kernel(self, m: int, n: int, k: int, form: str) -> int | None:
         """Which of the library's kernels multiplies ``m`` rows by a weight [n, k]: 0 the few-row
         kernel (up to 16 rows), 1 the kernel that shares the activations through LDS (K a
-        multiple of 64 and at least 128, n a multiple of 16), None the vendor library. Both read
+        multiple of 64 and at least 128, n a multiple of 16), None neither (tiles or the vendor library). Both read
         the weight as stored. ``form``: "whole", "gated", or "planes" (cut along K). Measured at
         the 4B shapes against the vendor library: 28 to 32 % less time over the four products of
         a layer at 32 and 64 rows; at 128 rows 71 us against 116 for the gated product and the
