@@ -121,3 +121,45 @@ def test_the_route_of_the_engine(n, k):
         assert (y.shape[0] if y.dim() == 3 else 1) == parts and (y.dim() == 3) == (parts > 1)
         want = x.double() @ w.double().T
         near(y.sum(0) if parts > 1 else y, want, 2.0 ** -24 * k, 0.0 if parts > 1 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("name", ["qwen3_4b", "deginex_4b_moe", "roserax_2b", "zisedra_2b", "zuvasun_2b", "sarudra_2b", "dekinex_2b"])
+def test_whole_models_with_and_without(name):
+    """A few layers of every design at the sizes it is run at, a prompt of 333 tokens and portions behind it: with the engine's ops
+    and with those that hand products of many rows over as one bfloat16 matrix, both beside the same engine in float32. Planes round
+    less, so their error is no larger but for chance (a rounding that moves a token to another expert moves its logits in
+    either): the middle token's by a quarter. A plane lost or added twice would move every token by a sizeable part of its logits."""
+    from qwen3_runtime_amd.engine.batch import StepEntry
+    from qwen3_runtime_amd.llm import build_engine
+    from qwen3_runtime_amd.registry import preset_config
+
+    raw = dict(preset_config(name))
+    if isinstance(raw.get("layers"), list):
+        raw["layers"] = raw["layers"][:4]
+    else:
+        raw["num_hidden_layers"] = 3
+    ids = torch.randint(0, 2000, (500,), generator=torch.Generator().manual_seed(2)).tolist()
+
+    def logits(engine):
+        engine.cache.admit("a")
+        rows = [engine.runner.step([StepEntry("a", ids[p:q], list(range(0, q - p, 7)))]) for p, q in ((0, 333), (333, 463), (463, 500))]
+        engine.cache.release("a")
+        return torch.cat([r.float() if isinstance(r, torch.Tensor) else torch.stack(list(r.values())).float() for r in rows])
+
+    got = {}
+    for dtype in ("float32", "bfloat16"):
+        engine = build_engine(None, config=raw, seed=5, dtype=dtype, block_size=16, num_kv_blocks=80, max_num_seqs=2,
+                              max_num_batched_tokens=512, max_model_len=1024, cuda_graph=False)
+        ops, made = engine.runner.ops, []
+        assert ops.residual_planes
+        inner = ops.linear_for_residual
+        ops.linear_for_residual = lambda x, w: (made.append(inner(x, w)), made[-1])[1]  # noqa: B023
+        for planes in (True, False) if dtype == "bfloat16" else (None,):
+            ops.residual_planes = bool(planes)
+            made.clear()
+            got[planes] = logits(engine)
+            assert (3 in [y.dim() for y in made if y.shape[-2] > 128]) == bool(planes)
+    want = got.pop(None)
+    err = {planes: float(((rows - want).square().mean(-1).sqrt() / want.std(-1)).median()) for planes, rows in got.items()}
+    print(name, err)
+    assert torch.isfinite(got[True]).all() and err[True] <= 1.25 * err[False], err
