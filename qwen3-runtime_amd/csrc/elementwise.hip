@@ -114,6 +114,19 @@ extern "C" int qrt_rope_table(const int* positions, const float* inv_freq, float
 // residual, planes and weights are then all loaded at once, unconditionally (clamped index), so
 // that a row costs one round of memory latency instead of one per plane and one for the weights;
 // PL = -1 loops over any number of planes.
+// In the 32-bit mode (float32 rows out) the planes' sum joins the stream with one rounding, as a product that comes whole
+// does; beside bfloat16 rows each plane joins by itself.
+template <typename TD, typename VEC_T, int VEC>
+__device__ __forceinline__ VEC_T sum_of_planes(const TD* __restrict__ d, int planes, size_t plane_stride) {
+  typedef TD dvec_t __attribute__((ext_vector_type(VEC)));
+  VEC_T sum;
+  for (int p = 0; p < planes; ++p) {
+    const dvec_t v = *(const dvec_t*)(d + p * plane_stride);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) sum[e] = p ? sum[e] + to_f32<TD>(v[e]) : to_f32<TD>(v[e]);
+  }
+  return sum;
+}
 template <typename TD, typename TO, int VEC, int KEEP, int PL>
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ residual, const TD* __restrict__ delta,
                                                           const float* __restrict__ weight,
@@ -130,10 +143,25 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ re
   const TD* del = delta ? delta + (size_t)r * hidden : nullptr;
   const bool write_back = del && !rows;
   constexpr int STRIDE = 256 * VEC;
+  constexpr bool SUM_FIRST = sizeof(TO) == 4;
   const int i0 = threadIdx.x * VEC;
 
   fvec_t x[KEEP], w[KEEP];
   float ss = 0.f;
+  auto join = [&](fvec_t v, int i) {  // the planes' elements from i on joined to v
+    if (SUM_FIRST) {
+      const fvec_t sum = sum_of_planes<TD, fvec_t, VEC>(del + i, planes, plane_stride);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = fmaf(dscale, sum[e], v[e]);
+      return v;
+    }
+    for (int p = 0; p < planes; ++p) {
+      const dvec_t d = *(const dvec_t*)(del + p * plane_stride + i);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = fmaf(dscale, to_f32<TD>(d[e]), v[e]);
+    }
+    return v;
+  };
   if (PL >= 0) {
     dvec_t d[PL > 0 ? PL : 1][KEEP];
 #pragma unroll
@@ -144,12 +172,24 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ re
 #pragma unroll
       for (int p = 0; p < PL; ++p) d[p][j] = *(const dvec_t*)(del + p * plane_stride + ic);
     }
-#pragma unroll
-    for (int p = 0; p < PL; ++p)
+    if (SUM_FIRST && PL > 1) {
 #pragma unroll
       for (int j = 0; j < KEEP; ++j)
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) x[j][e] = fmaf(dscale, to_f32<TD>(d[p][j][e]), x[j][e]);
+        for (int e = 0; e < VEC; ++e) {
+          float sum = to_f32<TD>(d[0][j][e]);
+#pragma unroll
+          for (int p = 1; p < PL; ++p) sum += to_f32<TD>(d[p][j][e]);
+          x[j][e] = fmaf(dscale, sum, x[j][e]);
+        }
+    } else {
+#pragma unroll
+      for (int p = 0; p < PL; ++p)
+#pragma unroll
+        for (int j = 0; j < KEEP; ++j)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) x[j][e] = fmaf(dscale, to_f32<TD>(d[p][j][e]), x[j][e]);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < KEEP; ++j) {
@@ -157,7 +197,10 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ re
       x[j] = *(const fvec_t*)(res + ic);
       w[j] = *(const fvec_t*)(weight + ic);
     }
-    if (del) {
+    if (del && SUM_FIRST) {
+#pragma unroll
+      for (int j = 0; j < KEEP; ++j) x[j] = join(x[j], min(i0 + j * STRIDE, hidden - VEC));
+    } else if (del) {
       for (int p = 0; p < planes; ++p) {
 #pragma unroll
         for (int j = 0; j < KEEP; ++j) {
@@ -182,11 +225,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ re
   for (int i = i0 + KEEP * STRIDE; i < hidden; i += STRIDE) {
     fvec_t v = *(const fvec_t*)(res + i);
     if (del) {
-      for (int p = 0; p < planes; ++p) {
-        const dvec_t d = *(const dvec_t*)(del + p * plane_stride + i);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) v[e] = fmaf(dscale, to_f32<TD>(d[e]), v[e]);
-      }
+      v = join(v, i);
       if (write_back) *(fvec_t*)(res + i) = v;
     }
 #pragma unroll
@@ -206,13 +245,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ re
   }
   for (int i = i0 + KEEP * STRIDE; i < hidden; i += STRIDE) {
     fvec_t v = *(const fvec_t*)(res + i);  // already summed if written back
-    if (del && !write_back) {
-      for (int p = 0; p < planes; ++p) {
-        const dvec_t d = *(const dvec_t*)(del + p * plane_stride + i);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) v[e] = fmaf(dscale, to_f32<TD>(d[e]), v[e]);
-      }
-    }
+    if (del && !write_back) v = join(v, i);
     const fvec_t wv = *(const fvec_t*)(weight + i);
     ovec_t y;
 #pragma unroll

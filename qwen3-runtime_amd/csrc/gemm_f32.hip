@@ -6,7 +6,7 @@
 // of K alone), within a part 16 k at a time by four MFMAs (MFMA c multiplies k = 4 q + c for q = 0 .. 3),
 // and the parts' sums are added from the first to the last.
 //
-// * few rows (up to 64): `gemm_f32_rows_kernel` streams the weights. A block owns 16 weight rows, each
+// * few rows (up to 32, or 64): `gemm_f32_rows_kernel` streams the weights. A block owns 16 weight rows, each
 //   wave one part of K, and the parts meet in LDS. Bound by the weights' bytes.
 // * more rows: `gemm_f32_tile_kernel`, tiles through LDS, bound by the float32 MFMA rate. A wave adds
 //   its accumulators into a second set where a part ends.
@@ -14,11 +14,10 @@
 //   of fused multiply-adds per output, as every product had before: 64 x 64 outputs a block, one block per
 //   64 weight rows however few the rows of A.
 //
-// Measured (MI355X, us; the 4B products q/k/v, output, gate/up, down; weights of six layers in turn). One row: 22, 14,
-// 49, 36 (2.8 to 4.1 TB/s) against 262, 409, 326, 994 by the sequential kernel. 354 rows: 151, 98, 392, 235 (74 to 90
-// TFLOP/s of 157) against 472, 443, 1,112, 1,080. Error against float64, relative: 3.3e-7 (K 2,560), 4.5e-7 (9,728); the
-// sequential sums': 9.0e-7 and 1.8e-6.
+// Either MFMA kernel may leave a product for the residual in four planes, the sums of groups of neighbouring parts.
+// Error against float64, relative: 3.3e-7 (K 2,560), 4.5e-7 (9,728); the sequential sums': 9.0e-7 and 1.8e-6.
 #include "common.h"
+#include "direct.h"
 
 #define TM 64
 #define TN 64
@@ -80,106 +79,165 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // chain and 1.1e-7 in four parts at K 128, 4.1e-7 and 1.6e-7 at 512 (equal up to 32, where there is one part).
 static inline int f32_parts(int K) { return K >= 8192 ? 16 : K >= 256 ? 8 : K > 64 ? 4 : K > 32 ? 2 : 1; }
 static inline int f32_part_len(int K, int parts) { return ((K + parts - 1) / parts + 31) / 32 * 32; }
+// For the residual a product may leave four planes that its reader adds, each the sum of a group of
+// neighbouring parts (8 or 16 parts, from K 256 on), so that blocks can share K whatever the number of rows.
+#define F32_GROUPS 4
 
 __device__ __forceinline__ f32x4_t load_f32x4_below(const float* __restrict__ row, int k, int end) {
   const f32x4_t v = *(const f32x4_t*)(row + (k < end ? k : 0));
   return k < end ? v : f32x4_t{0.f, 0.f, 0.f, 0.f};  // K is a multiple of 4: all four or none
 }
 
-// 16 weight rows a block, PARTS waves of one part of K each, MB blocks of 16 rows of A. A lane holds
-// weight row lane & 15 and, of 16 k, the four from 4 (lane >> 4) on: one 16-byte load feeds four MFMAs,
-// and 64 k of a row are two whole cache lines.
-template <int MB, int PARTS>
+// Few rows (up to 64), a stream of the weights. A block owns 16 weight rows (GATED: 8 gate rows and the 8 up rows that
+// go with them), each wave one part of K, MB blocks of 16 rows of A. Operands reach LDS by direct loads of 8 rows x 128
+// bytes, whole cache lines: lane l fetches piece (l & 7) ^ (l / 8) of row l / 8, so piece c of row r lies at
+// 128 r + 16 (c ^ (r & 7)) and the operand reads (row lane & 15, piece 4 h + lane / 16 for the h-th 16 k) touch every bank
+// once. A slot of the wave's ring holds 32 k of all units (16 rows x 32 k, 2 KB), U slots are in flight, and the waits on the
+// loads' counter are counted by hand. Weights are loaded as data used once. FEW: up to 8 rows of A, whose unit is half as
+// long (operand rows 8 to 15 repeat them, and are not stored).
+// Loads straight to registers (a lane 16 bytes of its row, sixteen half lines an instruction) made the same products at one row
+// in 22, 14, 49, 36 us (4B q/k/v, output, gate/up, down, weights of six layers in turn); this takes 13.8, 9.7, 31.4, 19.9 (4.4 to
+// 6.4 TB/s), and at 16 rows 17, 12, 40, 28 instead of 29, 18, 71, 51.
+template <int MB, int PARTS, int U, bool FEW, int GATED>
 __global__ __launch_bounds__(64 * PARTS) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                                   float* __restrict__ C, int M, int N, int K, int part_len) {
-  extern __shared__ __align__(16) float sums[];  // [PARTS][MB][64 lanes][4]
+                                                                   float* __restrict__ C, int M, int N, int K, int part_len, float limit) {
+  constexpr int SLOT = (1 + MB) * 2048 - (FEW ? 1024 : 0), LOADS = 2 + (FEW ? 1 : 2 * MB);
+  constexpr int ONCE = 2;  // the cache policy of a non-temporal load
+  static_assert(!FEW || MB == 1, "up to 8 rows are one block of rows");
+  static_assert((U - 1) * LOADS < 64, "the loads' counter holds 63");
+  extern __shared__ __align__(16) unsigned char f32_lds[];  // [PARTS][U] slots, then the parts' sums
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
-  const int r = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16;
-  const int begin = wave * part_len, end = min(K, begin + part_len);
-  const float* w = W + (size_t)min(n0 + r, N - 1) * K;  // rows beyond the matrix: its last one, dropped below
-  const float* a[MB];
+  const int r = lane & 15, q = lane >> 4, n0 = blockIdx.x * (GATED ? 8 : 16);
+  const int begin = (blockIdx.y * PARTS + wave) * part_len, end = min(K, begin + part_len);
+  C += (size_t)blockIdx.y * M * N;
+  const int mine = max(0, (end - begin + 31) >> 5);  // slots of this wave
+  unsigned char* ring = f32_lds + (size_t)wave * U * SLOT;
+  const int sub = lane >> 3, col = 4 * ((lane & 7) ^ sub);
+  const float* src[1 + MB][2];
 #pragma unroll
-  for (int b = 0; b < MB; ++b) a[b] = A + (size_t)min(16 * b + r, M - 1) * K;
+  for (int j = 0; j < 2; ++j) {
+    // rows beyond the matrix: its last one, dropped below
+    src[0][j] = W + ((size_t)(GATED ? j * N : 0) + min(n0 + (GATED ? 0 : 8 * j) + sub, N - 1)) * K;
+#pragma unroll
+    for (int b = 0; b < MB; ++b) src[1 + b][j] = A + (size_t)min(16 * b + 8 * j + sub, M - 1) * K;
+  }
+  auto fetch = [&](int i, int slot) {
+    const int k = begin + 32 * i + col, at = k < end ? k : 0;  // K is a multiple of 4: all four or none
+    unsigned char* dst = ring + slot * SLOT;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[0][j] + at), (lds_ptr_t)(dst + j * 1024), 16, 0, ONCE);
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int j = 0; j < (FEW ? 1 : 2); ++j)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(src[1 + b][j] + at), (lds_ptr_t)(dst + (1 + b) * 2048 + j * 1024), 16, 0, 0);
+  };
   f32x4_t acc[MB];
 #pragma unroll
   for (int b = 0; b < MB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // 64 k a round, all of its loads asked for at once; what hides their latency is the number of waves (asking
-  // for the next round's before this one's are multiplied costs as many registers and gains nothing:
-  // 26.7 us against 21.6 for the 4B q/k/v weights and one row)
-  auto round = [&](int at, bool whole) {
-    f32x4_t wv[4], av[4][MB];
+  int fetched = 0;
+  for (; fetched < U && fetched < mine; ++fetched) fetch(fetched, fetched);
+  const int read_at[2] = {r * 128 + 16 * (q ^ (r & 7)), r * 128 + 16 * ((4 + q) ^ (r & 7))};
+  const int ra = FEW ? r & 7 : r, a_at[2] = {2048 + ra * 128 + 16 * (q ^ (r & 7)), 2048 + ra * 128 + 16 * ((4 + q) ^ (r & 7))};
+  int slot = 0;
+  for (int i = 0; i < mine; ++i) {
+    // slot i has landed when at most the U - 1 fetched after it are on their way; near the end the wave waits for all
+    if (fetched - i == U) QRT_WAIT_LOADS((U - 1) * LOADS);
+    else QRT_WAIT_LOADS(0);
+    const unsigned char* at = ring + slot * SLOT;
+    f32x4_t w[2], a[MB][2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = at + 16 * u + 4 * q, from = whole || k < end ? k : 0;  // K is a multiple of 4: all four or none
-      wv[u] = __builtin_nontemporal_load((const f32x4_t*)(w + from));
+    for (int h = 0; h < 2; ++h) {
+      w[h] = *(const f32x4_t*)(at + read_at[h]);
 #pragma unroll
-      for (int b = 0; b < MB; ++b) av[u][b] = *(const f32x4_t*)(a[b] + from);
+      for (int b = 0; b < MB; ++b) a[b][h] = *(const f32x4_t*)(at + b * 2048 + a_at[h]);
     }
+    QRT_WAIT_LDS();  // the slot is in registers: the next one may overwrite it
+    if (fetched < mine) {
+      fetch(fetched, slot);
+      ++fetched;
+    }
+    const int k = begin + 32 * i + 4 * q;
+    if (begin + 32 * i + 32 > end)  // the end of K inside a slot: what lies beyond counts as zero
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const bool there = whole || at + 16 * u + 4 * q < end;
+      for (int h = 0; h < 2; ++h) {
+        const bool there = k + 16 * h < end;
+        w[h] = there ? w[h] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < MB; ++b) a[b][h] = there ? a[b][h] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int b = 0; b < MB; ++b)
-          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? wv[u][c] : 0.f, there ? av[u][b][c] : 0.f, acc[b], 0, 0, 0);
-    }
-  };
-  int at = begin;
-  for (; at + 64 <= end; at += 64) round(at, true);
-  if (at < end) round(at, false);
-  f32x4_t* mine = (f32x4_t*)sums + ((size_t)wave * MB) * 64 + lane;
+        for (int b = 0; b < MB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][c], a[b][h][c], acc[b], 0, 0, 0);
+    slot = slot + 1 == U ? 0 : slot + 1;
+  }
+  __syncthreads();  // every wave has read its last slot: the rings' room now takes the parts' sums
+  f32x4_t* sums = (f32x4_t*)f32_lds;  // [PARTS][MB][64 lanes]
 #pragma unroll
-  for (int b = 0; b < MB; ++b) mine[b * 64] = acc[b];
+  for (int b = 0; b < MB; ++b) sums[(wave * MB + b) * 64 + lane] = acc[b];
   __syncthreads();
-  for (int i = threadIdx.x; i < MB * 64; i += 64 * PARTS) {
-    f32x4_t s = ((const f32x4_t*)sums)[i];
+  auto total = [&](int i) {
+    f32x4_t s = sums[i];
 #pragma unroll
-    for (int p = 1; p < PARTS; ++p) s += ((const f32x4_t*)sums)[p * MB * 64 + i];
-    const int m = 16 * (i >> 6) + (i & 15), n = n0 + 4 * ((i & 63) >> 4);  // an accumulator: rows 4 q .., column r
-    if (m >= M) continue;
+    for (int p = 1; p < PARTS; ++p) s += sums[p * MB * 64 + i];
+    return s;
+  };
+  // an accumulator: rows 4 q .., column r; gated: the gate rows' in lanes 0 to 31, their up rows' in the others
+  for (int i = threadIdx.x; i < MB * 64; i += 64 * PARTS) {
+    const int m = 16 * (i >> 6) + (i & 15), n = n0 + 4 * ((i & 63) >> 4);
+    if (m >= M || (GATED && (i & 32))) continue;
+    f32x4_t s = total(i);
+    if (GATED) {
+      const f32x4_t up = total(i + 32);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = gated_act(s[e], up[e], GATED - 1, limit);
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (n + e < N) C[(size_t)m * N + n + e] = s[e];
   }
 }
 
-// Tiles of T x T outputs, four waves of (T / 2) x (T / 2). 32 k of both operands at a time through LDS,
+// Tiles of TM x TN outputs, four waves of (TM / 2) x (TN / 2). 32 k of both operands at a time through LDS,
 // two stages; the 32 k after the next come into registers during the products. Rows of 40 floats: 32 bytes
-// modulo 64, with which operand reads meet no bank twice.
+// modulo 64, with which operand reads meet no bank twice. PLANES: the block makes plane blockIdx.z of the result, the sum
+// of that group of parts; else all parts, from the first to the last.
 #define F32_LD 40
-template <int T>
+template <int TM_, int TN_, bool PLANES>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                            float* __restrict__ C, int M, int N, int K, int part_len) {
-  constexpr int B = T / 32;   // 16 x 16 blocks a wave and direction
-  constexpr int L = T / 32;   // 16-byte pieces a thread brings per operand and stage
-  __shared__ __align__(16) float as[2][T * F32_LD];
-  __shared__ __align__(16) float ws[2][T * F32_LD];
+                                                            float* __restrict__ C, int M, int N, int K, int part_len, int group) {
+  constexpr int BI = TM_ / 32, BJ = TN_ / 32;  // 16 x 16 blocks a wave, rows of A by rows of W
+  __shared__ __align__(16) float as[2][TM_ * F32_LD];
+  __shared__ __align__(16) float ws[2][TN_ * F32_LD];
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r = lane & 15, q = lane >> 4;
-  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
-  const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+  const int m0 = blockIdx.y * TM_, n0 = blockIdx.x * TN_;
+  const int wm = (wave >> 1) * (TM_ / 2), wn = (wave & 1) * (TN_ / 2);
   const int lrow = threadIdx.x >> 3, lk = (threadIdx.x & 7) * 4;
-  const float* ar[L];
-  const float* wr[L];
+  // BI (BJ) pieces of 16 bytes a thread brings per operand and stage
+  const float* ar[BI];
+  const float* wr[BJ];
 #pragma unroll
-  for (int i = 0; i < L; ++i) {
-    ar[i] = A + (size_t)min(m0 + lrow + 32 * i, M - 1) * K;
-    wr[i] = W + (size_t)min(n0 + lrow + 32 * i, N - 1) * K;
-  }
-  f32x4_t acc[B][B], total[B][B];
+  for (int i = 0; i < BI; ++i) ar[i] = A + (size_t)min(m0 + lrow + 32 * i, M - 1) * K;
 #pragma unroll
-  for (int i = 0; i < B; ++i)
+  for (int i = 0; i < BJ; ++i) wr[i] = W + (size_t)min(n0 + lrow + 32 * i, N - 1) * K;
+  f32x4_t acc[BI][BJ], total[BI][BJ];
 #pragma unroll
-    for (int j = 0; j < B; ++j) acc[i][j] = total[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  f32x4_t ga[2][L], gw[2][L];
-  const int stages = (K + 31) / 32, per_part = part_len / 32;
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) acc[i][j] = total[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t ga[2][BI], gw[2][BJ];
+  const int per_part = part_len / 32, all = (K + 31) / 32;
+  const int s_first = PLANES ? blockIdx.z * group * per_part : 0, stages = PLANES ? min(all, s_first + group * per_part) : all;
   auto fetch = [&](int buf, int s) {
 #pragma unroll
-    for (int i = 0; i < L; ++i) {
-      ga[buf][i] = load_f32x4_below(ar[i], 32 * s + lk, K);
-      gw[buf][i] = load_f32x4_below(wr[i], 32 * s + lk, K);
-    }
+    for (int i = 0; i < BI; ++i) ga[buf][i] = load_f32x4_below(ar[i], 32 * s + lk, K);
+#pragma unroll
+    for (int i = 0; i < BJ; ++i) gw[buf][i] = load_f32x4_below(wr[i], 32 * s + lk, K);
   };
   int left = per_part;
   bool first = true;
@@ -187,10 +245,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     float* da = as[buf];
     float* dw = ws[buf];
 #pragma unroll
-    for (int i = 0; i < L; ++i) {
-      *(f32x4_t*)(da + (lrow + 32 * i) * F32_LD + lk) = ga[buf][i];
-      *(f32x4_t*)(dw + (lrow + 32 * i) * F32_LD + lk) = gw[buf][i];
-    }
+    for (int i = 0; i < BI; ++i) *(f32x4_t*)(da + (lrow + 32 * i) * F32_LD + lk) = ga[buf][i];
+#pragma unroll
+    for (int i = 0; i < BJ; ++i) *(f32x4_t*)(dw + (lrow + 32 * i) * F32_LD + lk) = gw[buf][i];
     __syncthreads();  // the stage before last was read before the barrier of the last one: two stages suffice
     // unconditional (under a branch the compiler loses count of the loads in flight and waits for all of
     // them), and held up here (it would move them down to their use): 448 -> 234 us for 354 x 2,560 x 9,728
@@ -198,43 +255,45 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      f32x4_t av[B], wv[B];
+      f32x4_t av[BI], wv[BJ];
 #pragma unroll
-      for (int i = 0; i < B; ++i) {
-        av[i] = *(const f32x4_t*)(da + (wm + 16 * i + r) * F32_LD + 16 * h + 4 * q);
-        wv[i] = *(const f32x4_t*)(dw + (wn + 16 * i + r) * F32_LD + 16 * h + 4 * q);
-      }
+      for (int i = 0; i < BI; ++i) av[i] = *(const f32x4_t*)(da + (wm + 16 * i + r) * F32_LD + 16 * h + 4 * q);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) wv[j] = *(const f32x4_t*)(dw + (wn + 16 * j + r) * F32_LD + 16 * h + 4 * q);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int i = 0; i < B; ++i)
+        for (int i = 0; i < BI; ++i)
 #pragma unroll
-          for (int j = 0; j < B; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][c], av[i][c], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < BJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][c], av[i][c], acc[i][j], 0, 0, 0);
     }
-    if (--left == 0 || s + 1 == stages) {  // a part of K ends (sums of nothing but zeros may follow the last)
+    // a part of K ends. An odd number of stages is followed by one that counts for nothing (zeros, or the next group's
+    // first, whose products are dropped)
+    if (--left == 0 || s + 1 >= stages) {
 #pragma unroll
-      for (int i = 0; i < B; ++i)
+      for (int i = 0; i < BI; ++i)
 #pragma unroll
-        for (int j = 0; j < B; ++j) {
-          total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
+        for (int j = 0; j < BJ; ++j) {
+          if (s < stages) total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
           acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
       first = false;
       left = per_part;
     }
   };
-  fetch(0, 0);
-  fetch(1, 1);
-  for (int s = 0; s < stages; s += 2) {  // an odd number of stages ends with one of zeros
+  fetch(0, s_first);
+  fetch(1, s_first + 1);
+  for (int s = s_first; s < stages; s += 2) {
     stage(0, s);
     stage(1, s + 1);
   }
+  if (PLANES) C += (size_t)blockIdx.z * M * N;
 #pragma unroll
-  for (int i = 0; i < B; ++i) {
+  for (int i = 0; i < BI; ++i) {
     const int m = m0 + wm + 16 * i + r;
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < B; ++j) {
+    for (int j = 0; j < BJ; ++j) {
       const int n = n0 + wn + 16 * j + 4 * q;
       float* c = C + (size_t)m * N + n;
       if (N % 4 == 0 && n < N) *(f32x4_t*)c = total[i][j];
@@ -246,19 +305,70 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
   }
 }
 
-template <int MB, int PARTS>
-static void f32_rows(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
-  gemm_f32_rows_kernel<MB, PARTS><<<(N + 15) / 16, 64 * PARTS, (size_t)PARTS * MB * 64 * 16, stream>>>(a, w, c, M, N, K, f32_part_len(K, PARTS));
-}
-template <int MB>
-static void f32_rows_parts(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
-  switch (f32_parts(K)) {
-    case 16: return f32_rows<MB, 16>(a, w, c, M, N, K, stream);
-    case 8: return f32_rows<MB, 8>(a, w, c, M, N, K, stream);
-    case 4: return f32_rows<MB, 4>(a, w, c, M, N, K, stream);
-    case 2: return f32_rows<MB, 2>(a, w, c, M, N, K, stream);
-    default: return f32_rows<MB, 1>(a, w, c, M, N, K, stream);
+// A block's waves: all parts of K, or those of one group (gridDim.y of them, each a plane of the result).
+template <int MB, int PARTS, int U, bool FEW, int GATED>
+static int f32_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, int groups = 1) {
+  constexpr size_t smem = (size_t)PARTS * U * ((1 + MB) * 2048 - (FEW ? 1024 : 0));  // the parts' sums fit in it
+  static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
+  auto kernel = gemm_f32_rows_kernel<MB, PARTS, U, FEW, GATED>;
+  static bool allowed = false;  // once per kernel: not inside a stream capture again and again
+  if (smem > 64 * 1024 && !allowed) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      return qrt_fail("gemm_f32: cannot get %zu bytes of LDS", smem);
+    allowed = true;
   }
+  kernel<<<dim3(GATED ? (N + 7) / 8 : (N + 15) / 16, groups), 64 * PARTS, smem, stream>>>(a, w, c, M, N, K, f32_part_len(K, PARTS * groups), limit);
+  return 0;
+}
+template <int MB, bool FEW, int GATED>
+static int f32_rows_parts(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream) {
+  constexpr int MANY = MB > 1 ? 1 : 2;  // sixteen rings and their slots have to fit LDS
+  switch (f32_parts(K)) {
+    case 16: return f32_rows<MB, 16, MANY, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+    case 8: return f32_rows<MB, 8, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+    case 4: return f32_rows<MB, 4, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+    case 2: return f32_rows<MB, 2, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+    default: return f32_rows<MB, 1, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+  }
+}
+template <int MB, bool FEW>
+static int f32_rows_planes(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+  return f32_parts(K) == 16 ? f32_rows<MB, 4, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, F32_GROUPS)
+                            : f32_rows<MB, 2, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, F32_GROUPS);
+}
+template <int GATED>
+static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream) {
+  if constexpr (!GATED)
+    if (M > 32) return f32_rows_parts<4, false, 0>(a, w, c, M, N, K, limit, stream);
+  if (M <= 8) return f32_rows_parts<1, true, GATED>(a, w, c, M, N, K, limit, stream);
+  if (M <= 16) return f32_rows_parts<1, false, GATED>(a, w, c, M, N, K, limit, stream);
+  return f32_rows_parts<2, false, GATED>(a, w, c, M, N, K, limit, stream);
+}
+
+// Which tile: the fewest rounds of blocks over the 256 compute units times what a round takes, us for 32 k: a unit's blocks
+// share its matrix cores, so a tile costs its area and little more (113, 107, 98 TFLOP/s of the 157 where rounds are whole, 24,
+// 12 and 6 of them), but alone on its unit a block waits for its own loads: no fewer than 1.3, 1.8 and 2.5 rounds' time.
+// 4B sizes, us, by 64 x 64, 64 x 32, 32 x 32: q/k/v at 64, 180, 354, 1,024 rows 62 47 42, 101 81 76, 146 131 144, 291 309 340;
+// down in planes at 64, 180, 354, 1,024 rows 62 59 49, 97 101 108, 189 195 203, 455 478 521 (whole: 230, 224, 223, 543 by
+// 64 x 64). Larger tiles are slower: 2,048 x 19,456 x 2,560 1,792 us, 1,940 by 128 x 128, 1,854 by 96 x 64.
+static int f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
+  const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
+  const long cost = rounds * 100 * round;
+  return (int)min(max(cost, (long)least * round), 0x7fffffffL);
+}
+template <bool PLANES>
+static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+  const int parts = f32_parts(K), part_len = f32_part_len(K, parts), groups = PLANES ? F32_GROUPS : 1;
+  const int c64 = f32_tile_cost(M, N, groups, 64, 64, 606, 130), c32 = f32_tile_cost(M, N, groups, 64, 32, 329, 180),
+            c16 = f32_tile_cost(M, N, groups, 32, 32, 190, 250);
+  QRT_CHECK((M + 63) / 64 <= 65535, "gemm_f32: M=%d is too large for one launch", M);
+  if (c64 <= c32 && c64 <= c16)
+    gemm_f32_tile_kernel<64, 64, PLANES><<<dim3((N + 63) / 64, (M + 63) / 64, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
+  else if (c32 <= c16 || (M + 31) / 32 > 65535)
+    gemm_f32_tile_kernel<64, 32, PLANES><<<dim3((N + 31) / 32, (M + 63) / 64, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
+  else
+    gemm_f32_tile_kernel<32, 32, PLANES><<<dim3((N + 31) / 32, (M + 31) / 32, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
+  return 0;
 }
 
 extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
@@ -269,22 +379,44 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
     dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM), block(256);
     QRT_CHECK(grid.y <= 65535, "gemm_f32: M=%d is too large for one launch", M);
     gemm_f32_kernel<<<grid, block, 0, stream>>>(a, w, c, M, N, K);
-  } else if (M <= 16) {
-    f32_rows_parts<1>(a, w, c, M, N, K, stream);
-  } else if (M <= 32) {
-    f32_rows_parts<2>(a, w, c, M, N, K, stream);
-  } else if (M <= 64) {
-    f32_rows_parts<4>(a, w, c, M, N, K, stream);
   } else {
-    // tiles of 128 only where they fill the 256 compute units several times: 2,048 x 2,560 x 9,728 is 320 of them, two
-    // rounds for 1.25, 2,090 us; in 1,280 tiles of 64 it takes 946
-    const int part_len = f32_part_len(K, f32_parts(K));
-    const int t = (long)((N + 127) / 128) * ((M + 127) / 128) >= 1024 ? 128 : 64;
-    dim3 grid((N + t - 1) / t, (M + t - 1) / t);
-    QRT_CHECK(grid.y <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-    if (t == 128) gemm_f32_tile_kernel<128><<<grid, 256, 0, stream>>>(a, w, c, M, N, K, part_len);
-    else gemm_f32_tile_kernel<64><<<grid, 256, 0, stream>>>(a, w, c, M, N, K, part_len);
+    // 33 to 64 rows: tiles of 32 x 32 where they give every compute unit one and a half (4B gate/up 85 us, as a stream 100;
+    // q/k/v 42 either way)
+    const bool few = M <= 32 || (M <= 64 && (long)((M + 31) / 32) * ((N + 31) / 32) < 384);
+    if (const int rc = few ? f32_few_rows<0>(a, w, c, M, N, K, 0.f, stream) : f32_tiles<false>(a, w, c, M, N, K, stream)) return rc;
   }
   QRT_LAUNCH_CHECK("gemm_f32");
+  return 0;
+}
+
+// The product in planes [4, M, N] whose sum, from the first to the last, it is (K in multiples of 4 from 256 on): the groups
+// of K's parts, the same whatever the number of rows. Blocks of their own make each, which fills the chip where the weight
+// has few rows. Up to 32 rows as a stream (4B output and down projections at 1, 16, 32 rows 9.5, 10.4, 14.7 and 18.1, 22.9, 31.5 us;
+// all parts in a block 9.7, 12.3, 17.2 and 19.9, 28.1, 40.6), beyond by tiles.
+extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+  QRT_CHECK(M >= 0 && N > 0 && K >= 256 && K % 4 == 0, "gemm_f32_planes: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0, "gemm_f32_planes: operands are read 16 bytes at a time");
+  if (M == 0) return 0;
+  if (const int rc = M <= 8    ? f32_rows_planes<1, true>(a, w, c, M, N, K, stream)
+                     : M <= 16 ? f32_rows_planes<1, false>(a, w, c, M, N, K, stream)
+                     : M <= 32 ? f32_rows_planes<2, false>(a, w, c, M, N, K, stream)
+                               : f32_tiles<true>(a, w, c, M, N, K, stream))
+    return rc;
+  QRT_LAUNCH_CHECK("gemm_f32_planes");
+  return 0;
+}
+
+// The gated product of few rows: W is [2N, K] (gate rows, then up rows), C[M, N] = act(A Wg^T, A Wu^T) as gated_act makes it
+// of the product's columns, with the same bits.
+extern "C" int qrt_gated_gemm_f32(const float* a, const float* w, float* c, int M, int N, int K, int act_kind, float limit,
+                                  hipStream_t stream) {
+  QRT_CHECK(M >= 0 && M <= 32 && N > 0 && N <= 1 << 30 && K > 0, "gated_gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(act_kind == QRT_ACT_SWIGLU || act_kind == QRT_ACT_CLAMPED, "gated_gemm_f32: unknown activation %d", act_kind);
+  QRT_CHECK(K % 4 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0, "gated_gemm_f32: operands are read 16 bytes at a time (K=%d)", K);
+  if (M == 0) return 0;
+  const int rc = act_kind == QRT_ACT_SWIGLU ? f32_few_rows<1 + QRT_ACT_SWIGLU>(a, w, c, M, N, K, limit, stream)
+                                            : f32_few_rows<1 + QRT_ACT_CLAMPED>(a, w, c, M, N, K, limit, stream);
+  if (rc) return rc;
+  QRT_LAUNCH_CHECK("gated_gemm_f32");
   return 0;
 }

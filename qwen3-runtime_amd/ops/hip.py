@@ -1418,6 +1418,13 @@ class HipOps:
         per row tile, which fills the chip (160 row tiles for 256 compute units at the 4B size)."""
         m, k = x.shape
         n = w.shape[0]
+        if (self.residual_planes and x.dtype == torch.float32 and w.dtype == torch.float32 and w.shape == (n, k)
+                and k >= 256 and k % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
+            _need(x, "x")
+            _need(w, "weight")
+            out = torch.empty((4, m, n), dtype=torch.float32, device=x.device)
+            self._check(self.lib, self.lib.qrt_gemm_f32_planes(_ptr(x), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), _stream()))
+            return out
         kernel, parts = None, 1
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and k % 64 == 0:
             kernel = self._own_kernel(m, n, k, "planes")
@@ -1485,7 +1492,7 @@ class HipOps:
 
     def gated_linear(self, x, w_gate_up, activation="swiglu", limit=0.0, row_scale=None):
         """``gated_act(linear(x, w_gate_up), ...)`` with ``w_gate_up`` [2I, K], gate rows first. With few
-        rows in bfloat16 one kernel forms both halves and applies the activation in its epilogue,
+        rows one kernel forms both halves and applies the activation in its epilogue,
         so the [T, 2I] intermediate never reaches memory."""
         m, k = x.shape
         two_i, kw = w_gate_up.shape
@@ -1508,6 +1515,16 @@ class HipOps:
                     _need(row_scale, "row factors", torch.float32, (m,))
                 return self._tile_product(x, w_gate_up, self.choose_tile(m, two_i // 2, k, "gated")[0],
                                           gate=(activation, limit, row_scale))
+        if (x.dtype == torch.float32 and w_gate_up.dtype == torch.float32 and row_scale is None and 0 < m <= 32
+                and two_i > 0 and k > 0 and k % 4 == 0 and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0):
+            # the same bits as the two kernels (2 rows of the 4B size: 32 us against 31 and 6)
+            _need(x, "x")
+            _need(w_gate_up, "weight")
+            out = torch.empty((m, two_i // 2), dtype=torch.float32, device=x.device)
+            self._check(self.lib, self.lib.qrt_gated_gemm_f32(
+                _ptr(x), _ptr(w_gate_up), _ptr(out), c_int(m), c_int(two_i // 2), c_int(k),
+                c_int(ACTIVATIONS[activation]), c_float(limit), _stream()))
+            return out
         return self.gated_act(self.linear(x, w_gate_up), activation, limit, row_scale=row_scale)
 
     # ---- q/k norm, rotation, cache write ----------------------------------------

@@ -29,8 +29,39 @@ def test_product_against_float64_and_equal_bits_for_any_number_of_rows(ops, n, k
     # a sum of k products in any order, each rounded: at most k units of 2^-24 of the sum of magnitudes
     bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert ((whole.double() - want).abs() <= bound).all()
-    for m in (1, 16, 17, 32, 33, 64, 65, 129):
+    for m in (1, 8, 9, 16, 17, 32, 33, 64, 65, 129):
         assert torch.equal(ops.linear(x[70: 70 + m].contiguous(), w), whole[70: 70 + m]), m
+
+
+# rows: one unit of 8, its edges, the blocks of 16 and 64; weight rows: none, one and part of a block of 8; K: an end inside a slot of 32
+@pytest.mark.parametrize("activation,limit", [("swiglu", 0.0), ("clamped", 0.7)])
+@pytest.mark.parametrize("inter,k", [(1, 4), (12, 68), (40, 2560), (24, 8228)])
+def test_gated_product_of_few_rows_has_the_bits_of_product_and_activation(ops, inter, k, activation, limit):
+    x, w = rnd(33, k, seed=5), rnd(2 * inter, k, seed=6, scale=0.1)
+    for m in (1, 8, 9, 16, 17, 32, 33):
+        both = ops.linear(x[:m], w)
+        assert torch.equal(ops.gated_linear(x[:m], w, activation, limit), ops.gated_act(both, activation, limit)), m
+
+
+# weight rows: a remainder of every tile; K: groups of two and of four parts, one that K ends before, an end inside a slot of 32
+@pytest.mark.parametrize("n,k", [(1, 260), (65, 1028), (2560, 264), (52, 8196)])
+def test_product_in_planes_is_the_same_for_any_number_of_rows(ops, n, k):
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    planes = HipOps(residual_planes=True)
+    x, w = rnd(300, k, seed=11), rnd(n, k, seed=12, scale=0.05)
+    whole = planes.linear_for_residual(x, w)
+    assert whole.shape == (4, 300, n)
+    want = x.double() @ w.double().T
+    assert ((whole.double().sum(0) - want).abs() <= k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
+    for m in (1, 8, 9, 16, 17, 32, 33, 64, 65, 129):
+        assert torch.equal(planes.linear_for_residual(x[70: 70 + m].contiguous(), w), whole[:, 70: 70 + m]), m
+    # the norm adds the planes' sum with one rounding
+    res, weight = rnd(300, n, seed=13), torch.ones(n, device=DEV)
+    total = ((whole[0] + whole[1]) + whole[2]) + whole[3]
+    a, b = res.clone(), res.clone()
+    assert torch.equal(ops.add_rmsnorm(a, whole, weight, 1e-6, torch.float32), ops.add_rmsnorm(b, total, weight, 1e-6, torch.float32))
+    assert torch.equal(a, b)
 
 
 def test_product_of_many_rows_in_large_tiles(ops):
