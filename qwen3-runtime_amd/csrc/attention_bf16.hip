@@ -91,13 +91,14 @@ struct AttnTileArgs {
   const int* slots;        // [T]: place of the token in the cache, page * page_size + offset
   float eps;
   // Decoding over sequences of very different lengths: instead of num_splits equal parts of every
-  // sequence, pieces of split_blocks 32-key blocks, as many as a sequence has (at most num_splits),
-  // listed in `items` as (sequence, piece), whole pieces first and the sequences' last, shorter
-  // pieces after them, then (-1, 0) up to max_items. The launch is (key head, item): blocks of
-  // equal work, the heavy ones next to each other in launch order, which spreads them evenly over
-  // the compute units. qrt_attention_work_list fills the list from the step's lengths.
+  // sequence, pieces of at most split_blocks 32-key blocks, of one length within a sequence (at most num_splits),
+  // listed in `items` as (sequence, piece), those of more than three quarters of that first, then the
+  // others, then (-1, 0) up to max_items. The launch is (key head, item): blocks of
+  // like work, the heavy ones next to each other in launch order, which spreads them evenly over
+  // the compute units. With split_most > split_blocks the list's kernel looks for the best length of that range by the step's
+  // lengths as they are, which a captured launch's host does not know; items[2 max_items] is the one it took. qrt_attention_work_list fills the list from the step's lengths.
   int split_blocks, max_items;
-  int* items;              // [max_items][2] or null
+  int* items;              // [max_items][2] and the length taken, or null
   int chunk;               // > 0: a query sees the keys of its own chunk of this many positions (no window then)
   float cap_in, cap_out;   // score cap c > 0: cap_in = scale / c, cap_out = c / scale; 0: no cap
   // An output gate: the result at (token, head, element) is multiplied by the sigmoid of
@@ -119,6 +120,7 @@ struct AttnTileArgs {
   // are. The cached values are turned by their own positions, element j against j + DV / 2, and a row's
   // output is turned back by its token's angles where it is written (here, or in the merge).
   const float* turn;
+  int split_most;
 };
 
 // The first key position that the query at position p sees. It does not fall as p grows, so for a
@@ -1406,22 +1408,66 @@ __device__ __forceinline__ void decode_key_blocks(int kv_len, int q_len, int win
   end = any_cached ? (pos_max >> 5) + 1 : begin;
 }
 
+// Blocks of keys in the pieces of a sequence of `blocks`: as few pieces as have at most `most` each, of one length (a last
+// piece of a few keys costs a block's start like any other: 16 sequences of 290 to 2,600 keys, at most 512 a piece, 29.8 us
+// with whole pieces and rests, 27.5 so; 48 of 136 to 2,606, at most 1,024, 47.4 and 45.4).
+__device__ __forceinline__ int piece_blocks(int blocks, int most) {
+  const int pieces = max(1, (blocks + most - 1) / most);
+  return max(1, (blocks + pieces - 1) / pieces);
+}
+
 // The work list of a decode launch in pieces (AttnTileArgs::items). One block; up to LIST_TILES
 // sequences. Every sequence has at least one piece (its last piece also takes the token's own key
-// in the fused form), at most ceil(blocks / split_blocks).
-constexpr int LIST_TILES = 1024;
-__global__ __launch_bounds__(256) void attention_work_list_kernel(AttnTileArgs a, int fused) {
+// in the fused form), at most ceil(blocks / split_blocks). Sequences with long pieces come first.
+// Which length: the least of 5 us for every round of blocks (two to each of 256 compute units), of what the longest piece
+// takes times the blocks of the busiest unit (0.6 us for 100 keys of 512 bytes), and of the merge of more than four parts. On 15 sets
+// of 3 to 64 sequences of 60 to 16,000 keys, timed at every multiple of 32 from 128 to 512 and ten lengths beyond, it takes 1.2 %
+// more than the best on average, 5 % at worst; one length for some 1,536 blocks took 13 and 36 %.
+constexpr int LIST_TILES = 1024, LIST_LENGTHS = 32;
+__global__ __launch_bounds__(8 * LIST_LENGTHS) void attention_work_list_kernel(AttnTileArgs a, int fused) {
   __shared__ int whole[LIST_TILES + 1], rest[LIST_TILES + 1];  // pieces of each tile, then where they begin
+  __shared__ int blocks_of[LIST_TILES];
+  __shared__ float cost_of[LIST_LENGTHS];
   for (int t = threadIdx.x; t < a.num_tiles; t += blockDim.x) {
     const int seq = a.tile_seq ? a.tile_seq[t] : t;
     int begin, end;
     decode_key_blocks(a.kv_lens[seq], a.cu_q[seq + 1] - a.cu_q[seq], a.window, a.chunk, fused != 0, begin, end);
-    const int blocks = end - begin;
-    whole[t] = blocks / a.split_blocks;
-    rest[t] = blocks % a.split_blocks != 0 || blocks == 0 ? 1 : 0;
+    blocks_of[t] = end - begin;
+  }
+  __syncthreads();
+  const int range = max(0, a.split_most - a.split_blocks);
+  auto length = [&](int c) { return a.split_blocks + c * range / (LIST_LENGTHS - 1); };
+  {  // eight lanes a length
+    const int most = length(threadIdx.x >> 3);
+    int count = 0, longest = 0, parts = 0;
+    for (int t = threadIdx.x & 7; t < a.num_tiles; t += 8) {
+      const int blocks = blocks_of[t], per = piece_blocks(blocks, most), pieces = max(1, (blocks + per - 1) / per);
+      count += pieces;
+      longest = max(longest, per);
+      parts = max(parts, pieces);
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      count += __shfl_xor(count, o, 64);
+      longest = max(longest, __shfl_xor(longest, o, 64));
+      parts = max(parts, __shfl_xor(parts, o, 64));
+    }
+    const int units = (count * a.nkv + 255) / 256;
+    cost_of[threadIdx.x >> 3] = 5.0f * ((units + 1) / 2) + 0.192f * (D + DV) / 256.0f * longest * units + 0.05f * max(parts - 4, 0);
+  }
+  __syncthreads();
+  int best = 0;
+  for (int c = 1; c < LIST_LENGTHS; ++c) best = cost_of[c] < cost_of[best] ? c : best;
+  const int most = length(best);
+  for (int t = threadIdx.x; t < a.num_tiles; t += blockDim.x) {
+    const int blocks = blocks_of[t], per = piece_blocks(blocks, most), pieces = max(1, (blocks + per - 1) / per);
+    const bool heavy = 4 * per > 3 * most;
+    whole[t] = heavy ? pieces : 0;
+    rest[t] = heavy ? 0 : pieces;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    a.items[2 * a.max_items] = most;
     int at = 0;
     for (int t = 0; t < a.num_tiles; ++t) { const int n = whole[t]; whole[t] = at; at += n; }
     whole[a.num_tiles] = at;
@@ -1431,12 +1477,11 @@ __global__ __launch_bounds__(256) void attention_work_list_kernel(AttnTileArgs a
   __syncthreads();
   for (int t = threadIdx.x; t < a.num_tiles; t += blockDim.x) {
     const int seq = a.tile_seq ? a.tile_seq[t] : t;
-    const int n_whole = whole[t + 1] - whole[t];
-    for (int p = 0; p < n_whole; ++p) {
-      const int at = whole[t] + p;
+    const int* from = whole[t + 1] > whole[t] ? whole : rest;
+    for (int p = 0; p < from[t + 1] - from[t]; ++p) {
+      const int at = from[t] + p;
       if (at < a.max_items) { a.items[2 * at] = seq; a.items[2 * at + 1] = p; }
     }
-    if (rest[t + 1] > rest[t] && rest[t] < a.max_items) { a.items[2 * rest[t]] = seq; a.items[2 * rest[t] + 1] = n_whole; }
   }
   for (int i = rest[a.num_tiles] + threadIdx.x; i < a.max_items; i += blockDim.x) { a.items[2 * i] = -1; a.items[2 * i + 1] = 0; }
 }
@@ -1536,8 +1581,9 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   // every sequence is one tile here, so without a list the block's number is the sequence's: one
   // dependent load less before the first key arrives. A list names the sequences of a launch
   // that covers only some of the step's.
-  int seq, kvh, split;
+  int seq, kvh, split, longest_piece = 0;
   if (a.items) {  // pieces from the work list: (key head, item)
+    longest_piece = a.items[2 * a.max_items];
     seq = a.items[2 * blockIdx.y];
     if (seq < 0) return;  // past the end of the list
     split = a.items[2 * blockIdx.y + 1];
@@ -1575,8 +1621,8 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   const int lo = max(0, first_seen(first_pos, a.window, a.chunk));
   int blk_begin, blk_end;
   decode_key_blocks(kv_len, q_len, a.window, a.chunk, FUSED, blk_begin, blk_end);
-  // equal parts of the sequence's blocks, or pieces of a fixed length, as many as it has
-  const int per = a.items ? a.split_blocks : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
+  // equal parts of the sequence's blocks: as many as all sequences have, or as pieces of at most a given length make
+  const int per = a.items ? piece_blocks(blk_end - blk_begin, longest_piece) : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
   const int last_split = a.items ? max(1, (blk_end - blk_begin + per - 1) / per) - 1 : (int)gridDim.z - 1;
   const int b0 = blk_begin + split * per;
   const int b1 = min(blk_end, b0 + per);
@@ -1772,7 +1818,7 @@ extern "C" int qrt_attention_work_list(const AttnTileArgs* args, int fused, hipS
             "attention work list: %d sequences (at most %d), %d items, pieces of %d blocks", a.num_tiles, LIST_TILES,
             a.max_items, a.split_blocks);
   if (a.max_items == 0) return 0;
-  attention_work_list_kernel<<<1, 256, 0, stream>>>(a, fused);
+  attention_work_list_kernel<<<1, 8 * LIST_LENGTHS, 0, stream>>>(a, fused);
   QRT_LAUNCH_CHECK("attention_work_list");
   return 0;
 }

@@ -86,7 +86,7 @@ class _AttnTileArgs(Structure):
         ("max_items", c_int), ("items", c_void_p),
         ("chunk", c_int), ("cap_in", c_float), ("cap_out", c_float),
         ("gate", c_void_p), ("gate_stride", c_long), ("keep_first", c_int), ("sink", c_int),
-        ("rope_pairs", c_int), ("turn", c_void_p),
+        ("rope_pairs", c_int), ("turn", c_void_p), ("split_most", c_int),
     ]
 
 
@@ -1923,10 +1923,11 @@ class HipOps:
         of one length (as many per sequence as it has) instead of every sequence into equally
         many parts. Measured on 8 to 128 sequences with lengths drawn evenly around 1,024 to
         8,192: the pieces win from a longest length of 1.3 to 1.4 times the mean on (0.80 to 0.9
-        of the time at 1.6 to 1.9), lose 5 to 12 % below it, and lose at any spread while the
-        longest context is under some 2,000 keys (the merge of the parts then weighs too much)."""
-        n, total = len(kv_lens), sum(kv_lens)
-        return n >= 2 and max(kv_lens) * n > self.decode_piece_ratio * total and max(kv_lens) >= 2048
+        of the time at 1.6 to 1.9), lose 5 to 12 % below it, and lose in few keys (the merge of the parts then
+        weighs too much): equal parts and pieces, us, 3 sequences up to 1,200 keys 12.0 and 12.4, 8 up to 600
+        14.4 and 14.7; 30 up to 900 22.9 and 22.2, 32 and 40 up to 1,200 28.4, 37.7 and 25.1, 27.7."""
+        n, total, longest = len(kv_lens), sum(kv_lens), max(kv_lens)
+        return n >= 2 and longest * n > self.decode_piece_ratio * total and (longest >= 2048 or (longest >= 768 and total >= 8192))
 
     def choose_decode_piece(self, kv_lens, nkv: int):
         """Keys per piece for such a launch (a multiple of 32), or None. Equal parts of every
@@ -1942,6 +1943,15 @@ class HipOps:
             return None
         piece = max(512, -(-sum(kv_lens) * nkv // 1536), -(-max(kv_lens) // 32))
         return -(-piece // 32) * 32
+
+    @staticmethod
+    def shortest_decode_piece(kv_lens, piece: int) -> int:
+        """The shortest piece that the work list's kernel may take in place of ``piece`` (the longest is six times that): it
+        looks for the length whose blocks fill the compute units in whole rounds, by the lengths as they are when it
+        runs. No sequence in more than 32. With heads of 128 on 8 key heads, by ``piece`` alone (a sequence's last one shorter)
+        and now, us with the merge: 48 sequences of 136 to 2,606 keys 51.0 and 45.2, 40 to 1,200 37.4 (in equal parts) and 27.7, 16 to 2,600
+        29.9 and 24.8, 64 of 100 to 4,000 128 and 113, 8 of 1,000 to 16,000 46.4 and 44.6."""
+        return max(piece if piece > 512 else 256, -(-max(kv_lens) // 1024) * 32)
 
     # mixed steps: sequences with few rows leave the prompt kernel when their context is this long
     split_launch_min_kv = 1024
@@ -2053,7 +2063,11 @@ class HipOps:
             if piece is None and "attn_splits" not in ctx.scratch:
                 # the lengths as they are; a capture sees its bucket's instead and is told them beside
                 lens = ctx.scratch.get("attn_lens") or kv_lens
-                piece = self.choose_decode_piece([min(n, reach) for n in lens] if reach else lens, nkv)
+                lens = [min(n, reach) for n in lens] if reach else lens
+                piece = self.choose_decode_piece(lens, nkv)
+                if piece:
+                    piece = self.shortest_decode_piece(lens, piece) // 32 * 32
+                    a.split_most = 6 * (piece // 32)
         if piece:
             a.split_blocks = piece // 32
             # 32-key blocks a sequence of this launch can have: all its keys, or those of its
@@ -2094,7 +2108,7 @@ class HipOps:
             list_key = ("attn_items", key, window, chunk, own is not None, piece, a.max_items)
             items = ctx.per_pass.get(list_key)
             if items is None:
-                items = torch.empty((a.max_items, 2), dtype=torch.int32, device=out.device)
+                items = torch.empty(2 * a.max_items + 1, dtype=torch.int32, device=out.device)
                 a.items = items.data_ptr()
                 self._check(lib, lib.qrt_attention_work_list(byref(a), c_int(own is not None), _stream()))
                 ctx.per_pass[list_key] = items

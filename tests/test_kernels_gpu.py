@@ -895,6 +895,32 @@ def test_decode_attention_in_pieces_of_one_length(ops, seqs, nq, nkv, d, ps, win
     close(ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window), want, 2e-2, 2e-2)
 
 
+@pytest.mark.parametrize("lens,nkv,d", [
+    ([100 + 41 * i for i in range(28)], 8, 64),         # none as long as 2,048
+    ([90, 2600, 700, 64, 1500, 33, 4000, 1, 800], 2, 128),
+    ([300] * 56 + [8000] * 8, 1, 64),
+])
+def test_the_list_takes_a_piece_length_by_the_lengths_on_the_device(ops, lens, nkv, d):
+    """The length is one of the range asked for, every sequence's pieces are listed once and no block of keys is left over,
+    and the outputs hold, also after the lengths on the device have changed under the host's view."""
+    q, cache, ctx = build_attention_case([(1, n) for n in lens], 4 * nkv, nkv, d, 16, torch.bfloat16, seed=5, poison=True)
+    scale = d ** -0.5
+    assert ops.decode_in_pieces(lens)
+    shortest = ops.shortest_decode_piece(lens, ops.choose_decode_piece(lens, nkv)) // 32
+    for now in (lens, [max(1, n // 2) for n in lens], [1] * len(lens)):
+        ctx.kv_lens.copy_(torch.tensor(now, dtype=torch.int32))
+        ctx.per_pass.clear()
+        want = R.paged_attention(q, cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, 16,
+                                 4 * nkv, nkv, d, scale, None)
+        close(ops.paged_attention(q, cache, ctx, 4 * nkv, nkv, d, scale, None), want, 2e-2, 2e-2)
+        items = next(v for k, v in ctx.per_pass.items() if k[0] == "attn_items").cpu()
+        most, listed = int(items[-1]), items[:-1].view(-1, 2).tolist()
+        assert shortest <= most <= 6 * shortest
+        blocks = [-(-n // 32) for n in now]
+        per = [-(-b // -(-b // most)) for b in blocks]
+        assert sorted(x for x in listed if x[0] >= 0) == [[i, p] for i in range(len(now)) for p in range(-(-blocks[i] // per[i]))]
+
+
 def test_which_decode_launches_go_in_pieces(ops):
     """Equal lengths keep equal parts; very unequal ones get pieces of at least 512 keys, at most 32
     for the longest sequence, about 1,536 blocks in all."""
