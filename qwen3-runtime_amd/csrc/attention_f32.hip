@@ -15,6 +15,7 @@
 // layout: keys [page, head, offset, D], values [page, head, Dv, offset].
 #include "common.h"
 #include <math.h>
+#include <type_traits>
 
 struct AttnArgs {
   const void* q;         // [T, nq * D]
@@ -167,8 +168,11 @@ __global__ __launch_bounds__(64) void attention_f32_kernel(AttnArgs a) {
 // A row takes nothing from keys it does not see, whatever they hold; but 0 times an infinity is no number, and the tile's rows
 // share the products. A tile with a result that is not finite is therefore made again row by row, as in the kernel above.
 // Head sizes in multiples of 16 up to 256, pages of a multiple of 4 keys; other sizes keep the kernel above.
+// The keys and values of a wave's next block are on their way while one is multiplied (asked for together, under no branch: heads of
+// 32, 64 and 128, FULL, have instances of their own): prompts of 93 and 261 tokens and 6 more tokens of each at the 4B size 56.6 -> 54.5 ms,
+// 252 launches, most of them two tokens behind some 300 keys.
 #define F32_FEW_ROWS 64
-template <int ND, int W>
+template <int ND, int W, bool FULL>
 __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) {
   __shared__ __align__(16) f32x4_t hand[W > 1 ? W / 2 : 1][ND * 64];  // accumulators on their way from wave to wave
   __shared__ float hand_m[W][16], hand_l[W][16];
@@ -194,31 +198,52 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   const float* qr = (const float*)a.q + ((size_t)t * a.nq + h) * D + 4 * q;
 #pragma unroll
   for (int j = 0; j < ND; ++j) {
-    if (j < nd) qv[j] = *(const f32x4_t*)(qr + 16 * j);
+    if (FULL || j < nd) qv[j] = *(const f32x4_t*)(qr + 16 * j);
     acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   float m = -INFINITY, l = 0.f;
   const float* kc = (const float*)a.k_cache;
   const float* vc = (const float*)a.v_cache;
-  // a wave's blocks are those of its number modulo W
-  for (int b = wave < kept ? wave : main0 + ((wave - main0) & (W - 1)); b <= last_block;
-       b = b + W < kept || b >= main0 ? b + W : main0 + ((wave - main0) & (W - 1))) {
-    const int j0 = 16 * b;
-    // K: the lane's key j0 + r; V: its keys j0 + 4 q .. + 3 (one page). Places after the last key, and pages
-    // that were given back, are read as the sequence's last key (its page is there) and count for nothing
-    const int kj = min(j0 + r, hi), vj = j0 + 4 * q;
-    int kp = table[kj / ps], vp = table[min(vj, hi) / ps];
-    const int last_page = table[hi / ps];
-    const bool v_there = vj <= hi && vp >= 0;
+  // K: the lane's key j0 + r; V: its keys j0 + 4 q .. + 3 (one page). Places after the last key, and pages
+  // that were given back, are read as the sequence's last key (its page is there) and count for nothing
+  const int last_page = table[hi / ps];
+  auto key_row = [&](int b) {
+    const int kj = min(16 * b + r, hi);
+    int kp = table[kj / ps];
     kp = kp < 0 ? last_page : kp;
-    vp = v_there ? vp : last_page;
-    const float* kr = kc + (((size_t)kp * a.nkv + kvh) * ps + kj % ps) * D + 4 * q;
-    const float* vr = vc + ((size_t)vp * a.nkv + kvh) * Dv * ps + (v_there ? vj % ps : 0);
+    return kc + (((size_t)kp * a.nkv + kvh) * ps + kj % ps) * D + 4 * q;
+  };
+  auto value_row = [&](int b, bool& there) {
+    const int vj = 16 * b + 4 * q;
+    int vp = table[min(vj, hi) / ps];
+    there = vj <= hi && vp >= 0;
+    vp = there ? vp : last_page;
+    return vc + ((size_t)vp * a.nkv + kvh) * Dv * ps + (there ? vj % ps : 0) + (size_t)r * ps;
+  };
+  struct Block { f32x4_t k[ND], v[ND]; bool v_there; };
+  auto load = [&](int b, Block& blk) {
+    const float* kr = key_row(b);
+    const float* vr = value_row(b, blk.v_there);
+#pragma unroll
+    for (int j = 0; j < ND; ++j) blk.k[j] = *(const f32x4_t*)(kr + 16 * j);
+#pragma unroll
+    for (int j = 0; j < ND; ++j) blk.v[j] = *(const f32x4_t*)(vr + (size_t)(16 * j) * ps);
+  };
+  // a wave's blocks are those of its number modulo W
+  auto after = [&](int b) { return b + W < kept || b >= main0 ? b + W : main0 + ((wave - main0) & (W - 1)); };
+  int b = wave < kept ? wave : main0 + ((wave - main0) & (W - 1));
+  Block now, next;
+  if (FULL && b <= last_block) load(b, now);
+  while (b <= last_block) {
+    const int j0 = 16 * b, vj = j0 + 4 * q, b_next = after(b);
+    const float* kr = nullptr;
+    if (FULL) load(min(b_next, last_block), next);  // behind the wave's last block: one that nobody needs
+    else kr = key_row(b);
     f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < ND; ++j)
-      if (j < nd) {
-        const f32x4_t kv = *(const f32x4_t*)(kr + 16 * j);
+      if (FULL || j < nd) {
+        const f32x4_t kv = FULL ? now.k[j] : *(const f32x4_t*)(kr + 16 * j);
 #pragma unroll
         for (int c = 0; c < 4; ++c) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[c], qv[j][c], sc, 0, 0, 0);
       }
@@ -246,16 +271,19 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
       sc[e] = seen[e] ? expf(sc[e] - m) : 0.f;
       l += sc[e];
     }
+    const float* vr = FULL ? nullptr : value_row(b, now.v_there);
 #pragma unroll
     for (int j = 0; j < ND; ++j)
-      if (j < nv) {
-        f32x4_t vv = *(const f32x4_t*)(vr + (size_t)(16 * j + r) * ps);
+      if (FULL || j < nv) {
+        const f32x4_t vv = FULL ? now.v[j] : *(const f32x4_t*)(vr + (size_t)(16 * j) * ps);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          vv[e] = (v_there && vj + e <= hi) ? vv[e] : 0.f;  // never written: not a number, perhaps
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], sc[e], acc[j], 0, 0, 0);
+          const float value = (now.v_there && vj + e <= hi) ? vv[e] : 0.f;  // never written: not a number, perhaps
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(value, sc[e], acc[j], 0, 0, 0);
         }
       }
+    if (FULL) now = next;
+    b = b_next;
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
@@ -333,12 +361,17 @@ template <int ND>
 static void attention_f32_tiles(const AttnArgs& a, hipStream_t stream) {
   const long g = a.nq / a.nkv;
   const auto grid = [&](long rows) { return dim3((unsigned)((rows + 15) / 16), a.nkv, a.num_seqs); };
-  if constexpr (ND >= 16) {
-    attention_f32_tile_kernel<ND, 8><<<grid(a.max_q_len * g), 512, 0, stream>>>(a);
-  } else {  // sequences of both kinds: both kernels, each leaves the other's alone
-    if (a.min_q_len * g <= F32_FEW_ROWS) attention_f32_tile_kernel<ND, 8><<<grid(min(a.max_q_len * g, (long)F32_FEW_ROWS)), 512, 0, stream>>>(a);
-    if (a.max_q_len * g > F32_FEW_ROWS) attention_f32_tile_kernel<ND, 4><<<grid(a.max_q_len * g), 256, 0, stream>>>(a);
-  }
+  const auto launch = [&](auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    if constexpr (ND >= 16) {
+      attention_f32_tile_kernel<ND, 8, FULL><<<grid(a.max_q_len * g), 512, 0, stream>>>(a);
+    } else {  // sequences of both kinds: both kernels, each leaves the other's alone
+      if (a.min_q_len * g <= F32_FEW_ROWS) attention_f32_tile_kernel<ND, 8, FULL><<<grid(min(a.max_q_len * g, (long)F32_FEW_ROWS)), 512, 0, stream>>>(a);
+      if (a.max_q_len * g > F32_FEW_ROWS) attention_f32_tile_kernel<ND, 4, FULL><<<grid(a.max_q_len * g), 256, 0, stream>>>(a);
+    }
+  };
+  if (ND <= 8 && a.head_dim == 16 * ND && a.value_dim == 16 * ND) launch(std::bool_constant<(ND <= 8)>{});
+  else launch(std::false_type{});
 }
 
 extern "C" int qrt_attention_f32(const AttnArgs* args, int dtype, hipStream_t stream) {
