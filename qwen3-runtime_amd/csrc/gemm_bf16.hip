@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_skinny_kernel(const bf16_t*
         if (nn + r < N) {
           // the gate and the up value are rounded to bfloat16 first, as the unfused kernels see them
           const float g = (float)(bf16_t)sum[r];
-          const float out = GATED ? ep.template apply<GATED>(g, (float)(bf16_t)sum2[r], m) : sum[r];
+          const float out = GATED ? ep.template apply<GATED>(g, (float)(bf16_t)sum2[r], m) : ep.whole(sum[r]);
           C[(size_t)m * N + nn + r] = from_f32<TO>(out);
         }
       }
@@ -240,37 +240,38 @@ static int skinny(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int 
 // 4 h + lane / 16 for k-step h of the pair) then touch every bank once. The activations' 16
 // rows come the same way (rows past M repeat row M - 1; their results are not stored), so the
 // loop holds no load to registers and the waits on the loads' counter can be counted by hand
-// (the compiler does not count them out for direct loads): every pair is 2 (tiles + 1) loads,
+// (the compiler does not count them out for direct loads): every pair is 2 (tiles + 1) loads (FEW, up to
+// 8 rows: one less, operand rows 8 to 15 repeat the others),
 // U pairs are in flight in a ring of the wave's own, and a wave waits until all but the
 // youngest U - 1 pairs have landed. The weights are loaded as data used once, so that the
 // activations stay in the caches (10 % of the time at the large shapes). A block owns NT tiles
-// (and, GATED, the matching up tiles: it writes silu(gate) * up) and part blockIdx.y of K, whose
+// (GATED: one of eight gate rows and their up rows, or one of either: it writes silu(gate) * up) and part blockIdx.y of K, whose
 // result is plane blockIdx.y of the output (the caller adds the planes: used where the result
 // feeds a residual add); its NW waves take the pairs round-robin and meet in LDS, added in
 // wave order.
-template <int NW, int NT, int U, int GATED, typename TO>
+template <int NW, int NT, int U, int GATED, bool FEW, typename TO>
 __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
                                                                   TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep) {
-  constexpr int WT = GATED ? 2 * NT : NT, UNITS = WT + 1, LOADS = 2 * UNITS, SLOT = UNITS * 2048;
+  constexpr bool MIXED = GATED && NT == 1;
+  constexpr int UNITS = NT + 1, LOADS = 2 * UNITS - FEW, SLOT = UNITS * 2048 - (FEW ? 1024 : 0);
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
   static_assert((U - 1) * LOADS < 64, "the loads' counter holds 63");
   extern __shared__ __align__(16) unsigned char rows_lds[];  // [NW][U][UNITS] x 2 KB, then the partial sums
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r16 = lane & 15, quad = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT;
+  const int n0 = blockIdx.x * (MIXED ? 8 : GATED ? 16 : 16 * NT);
   unsigned char* ring = rows_lds + (size_t)wave * U * SLOT;
   const int sub = lane >> 3, piece = (lane & 7) ^ sub;
   const bf16_t* src[UNITS][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int n = min(n0 + 16 * t + 8 * j + sub, N - 1);  // rows past the end repeat the last; not stored
-      src[t][j] = W + (size_t)n * K + 8 * piece;
-      if (GATED) src[NT + t][j] = W + (size_t)(N + n) * K + 8 * piece;
+    for (int t = 0; t < NT; ++t) {  // rows past the end repeat the last; not stored
+      const int n = min(n0 + (MIXED ? 0 : 8 * j) + (GATED ? 0 : 16 * t) + sub, N - 1);
+      src[t][j] = W + ((size_t)(GATED && (MIXED ? j : t) ? N : 0) + n) * K + 8 * piece;
     }
-    src[WT][j] = A + (size_t)min(8 * j + sub, M - 1) * K + 8 * piece;
+    src[NT][j] = A + (size_t)min(8 * j + sub, M - 1) * K + 8 * piece;
   }
   const int all_pairs = K >> 6;
   const int part = (all_pairs + gridDim.y - 1) / gridDim.y;
@@ -284,18 +285,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
     for (int un = 0; un < UNITS; ++un)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if (un < WT)
+        if (un < NT)
           __builtin_amdgcn_global_load_lds((global_ptr_t)(src[un][j] + at), (lds_ptr_t)(dst + un * 2048 + j * 1024), 16, 0, ONCE);
-        else
+        else if (!FEW || j == 0)
           __builtin_amdgcn_global_load_lds((global_ptr_t)(src[un][j] + at), (lds_ptr_t)(dst + un * 2048 + j * 1024), 16, 0, 0);
       }
   };
-  f32x4_t acc[WT];
+  f32x4_t acc[NT];
 #pragma unroll
-  for (int t = 0; t < WT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   int fetched = 0;
   for (; fetched < U && fetched < mine; ++fetched) fetch(fetched, fetched);
   const int read_at[2] = {r16 * 128 + 16 * (quad ^ (r16 & 7)), r16 * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
+  const int ra = FEW ? r16 & 7 : r16, a_at[2] = {ra * 128 + 16 * (quad ^ (r16 & 7)), ra * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
   int slot = 0;
   for (int i = 0; i < mine; ++i) {
     // pair i has landed when at most the U - 1 pairs fetched after it are still on their way;
@@ -303,12 +305,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
     if (fetched - i == U) QRT_WAIT_LOADS((U - 1) * LOADS);
     else QRT_WAIT_LOADS(0);
     const unsigned char* at = ring + slot * SLOT;
-    bf16x8_t w[WT][2], a[2];
+    bf16x8_t w[NT][2], a[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int t = 0; t < WT; ++t) w[t][h] = *(const bf16x8_t*)(at + t * 2048 + read_at[h]);
-      a[h] = *(const bf16x8_t*)(at + WT * 2048 + read_at[h]);
+      for (int t = 0; t < NT; ++t) w[t][h] = *(const bf16x8_t*)(at + t * 2048 + read_at[h]);
+      a[h] = *(const bf16x8_t*)(at + NT * 2048 + a_at[h]);
     }
     QRT_WAIT_LDS();  // the slot is in registers: the next pair may overwrite it
     if (fetched < mine) {
@@ -318,55 +320,51 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int t = 0; t < WT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][h], a[h], acc[t], 0, 0, 0);
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][h], a[h], acc[t], 0, 0, 0);
     slot = slot + 1 == U ? 0 : slot + 1;
   }
   __syncthreads();  // every wave has read its last slot: the rings' room now takes the partial sums
-  float* red = (float*)rows_lds;  // [NW][WT][4][64]
+  float* red = (float*)rows_lds;  // [NW][NT][4][64]
 #pragma unroll
-  for (int t = 0; t < WT; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[((wave * WT + t) * 4 + r) * 64 + lane] = acc[t][r];
+    for (int r = 0; r < 4; ++r) red[((wave * NT + t) * 4 + r) * 64 + lane] = acc[t][r];
   __syncthreads();
-  // one thread per (tile, lane) adds the waves' parts in order
-  for (int i = threadIdx.x; i < NT * 64; i += 64 * NW) {
+  auto total = [&](int t, int l, float (&sum)[4]) {  // the waves' parts in order
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      sum[r] = 0.f;
+      for (int w = 0; w < NW; ++w) sum[r] += red[((w * NT + t) * 4 + r) * 64 + l];
+    }
+  };
+  // one thread per (tile, lane); gated rows of eight: the gate rows' sums in lanes 0 to 31, their up rows' in the others
+  for (int i = threadIdx.x; i < (GATED ? 1 : NT) * 64; i += 64 * NW) {
     const int l = i & 63, t = i >> 6;
     const int m = l & 15;
     const int nn = n0 + 16 * t + 4 * (l >> 4);
-    float sum[4], sum2[4];
+    if (m >= M || (MIXED && l >= 32)) continue;
+    float sum[4], up[4];
+    total(t, l, sum);
+    if (GATED) total(NT - 1, MIXED ? l + 32 : l, up);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v = 0.f, v2 = 0.f;
-      for (int w = 0; w < NW; ++w) {
-        v += red[((w * WT + t) * 4 + r) * 64 + l];
-        if (GATED) v2 += red[((w * WT + NT + t) * 4 + r) * 64 + l];
+    for (int r = 0; r < 4; ++r)
+      if (nn + r < N) {
+        const float g = (float)(bf16_t)sum[r];  // rounded to bfloat16 first, as the unfused kernels see them
+        C[(size_t)m * N + nn + r] = from_f32<TO>(GATED ? ep.template apply<GATED>(g, (float)(bf16_t)up[r], m) : ep.whole(sum[r]));
       }
-      sum[r] = v;
-      sum2[r] = v2;
-    }
-    if (m < M) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (nn + r < N) {
-          const float g = (float)(bf16_t)sum[r];  // rounded to bfloat16 first, as the unfused kernels see them
-          const float out = GATED ? ep.template apply<GATED>(g, (float)(bf16_t)sum2[r], m) : sum[r];
-          C[(size_t)m * N + nn + r] = from_f32<TO>(out);
-        }
-      }
-    }
   }
 }
 
-template <int NW, int NT, int U, int GATED>
+template <int NW, int NT, int U, int GATED, bool FEW>
 static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep,
                        hipStream_t stream, int k_parts) {
-  constexpr int WT = GATED ? 2 * NT : NT;
-  dim3 grid((N + 16 * NT - 1) / (16 * NT), k_parts), block(64 * NW);
-  constexpr size_t smem = (size_t)NW * U * (WT + 1) * 2048;  // the partial sums, NW * WT KB, fit in it
+  constexpr int outputs = GATED ? 8 * NT : 16 * NT;
+  dim3 grid((N + outputs - 1) / outputs, k_parts), block(64 * NW);
+  constexpr size_t ring = (size_t)NW * U * ((NT + 1) * 2048 - (FEW ? 1024 : 0)), meet = (size_t)NW * NT * 1024, smem = ring > meet ? ring : meet;
   static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
 #define GO(TO)                                                                                          \
   do {                                                                                                  \
-    auto kernel = gemm_bf16_rows_kernel<NW, NT, U, GATED, TO>;                                          \
+    auto kernel = gemm_bf16_rows_kernel<NW, NT, U, GATED, FEW, TO>;                                        \
     static bool allowed = false; /* once per kernel: not inside a stream capture again and again */    \
     if (smem > 64 * 1024 && !allowed) {                                                                 \
       if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) \
@@ -383,30 +381,44 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
   return 0;
 }
 
-// Configurations from timing 16 of them (2 to 8 waves, 1 or 2 row tiles a block, 2 to 6 pairs in
-// flight) on the shapes of the 4B, 8B and 32B models at 1, 8 and 16 rows, each on the weight
+// Configurations from timing 14 of them (2 to 8 waves, 1 or 2 row tiles a block, 1 to 4 pairs in
+// flight) on the shapes of the 4B, 8B and 32B models at 1 and 8 rows, each on the weight
 // matrices of 36 layers in turn: four waves everywhere (several small blocks on a compute unit
-// hide each other's ends better than one large one). Gated: one row tile, three pairs in flight
-// (19.1 us at the 4B size, 5.2 TB/s; 81.4 at the 32B size, 6.4 TB/s). The whole result: two tiles a block, except where K is a multiple of 2,048 (the rows of
-// two tiles then start in the same memory channels: 14.0 us against 11.2 for the 8B q/k/v product)
-// and for a few hundred tiles of long rows. K cut into planes: two tiles a block from K = 9,728 on.
-template <int GATED>
+// hide each other's ends better than one large one). us at 1 and 8 rows, by one tile a block and by two:
+//   Gated, three pairs in flight: 4B 17.3, 18.5 by tiles of eight gate and eight up rows, 18.7, 19.2 by a tile of either (5.8 and
+//   5.3 TB/s); 8B 31.3, 31.6 and 32.6, 32.3; 2,048 x 6,144 10.3, 10.5 and 11.2, 11.7; 32B 76.8, 84.2 and 79.4, 81.5, so long rows
+//   of more than two keep a tile of either; at 10 rows level.
+//   The whole result: two tiles a block from 384 tiles on where K is up to 4,096 columns, except between 512 and 768 tiles, whose blocks of two fill
+//   the compute units a little more than once (9,728 x 2,560 10.5, 11.5 and 12.0, 12.8; 12,288 11.5, 12.2 and 12.8, 13.5; at 16 rows
+//   13.6 and 14.1), and up to 4 rows below (6,144 x 2,560 at 1, 4 and 8 rows 7.2, 7.45, 8.1 and 7.35, 7.45, 7.7; 13,312 13.6, 14.7
+//   and 12.9, 13.6). One where K is a multiple of 2,048 (the rows of
+//   two tiles then start in the same memory channels: 14.0 us against 11.2 for the 8B q/k/v product)
+//   and for a few hundred tiles of long rows.
+//   K cut into planes: two tiles a block from K = 9,728 on, one up to 160 tiles of less than 12,288 columns (2,560 x 9,728 9.8, 10.2 and
+//   10.2, 10.8; 3,072 x 9,984 11.5, 12.0 and 11.4, 11.9; 4,096 x 12,288 17.4, 18.3 and 17.4, 17.7).
+// Up to 8 rows (FEW) the activations' unit is half as long: 0.1 to 0.3 us of a product, most where a block has one tile.
+template <int GATED, bool FEW>
 static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep, hipStream_t st,
                     int k_parts) {
   const int tiles = (N + 15) / 16;
-  if (GATED) return launch_rows<4, 1, 3, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-  if (k_parts > 1) {
-    if (K >= 9728) return launch_rows<4, 2, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
-    return launch_rows<4, 1, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
+  if constexpr (GATED) {
+    if constexpr (FEW)
+      if (K <= 4096 || M <= 2) return launch_rows<4, 1, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    return launch_rows<4, 2, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+  } else {
+    if (k_parts > 1) {
+      if (K >= 12288 || (K >= 9728 && tiles > 160)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
+      return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
+    }
+    if (K % 2048 == 0) {
+      if (tiles >= 2048) return launch_rows<4, 1, 3, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+      return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    }
+    if (tiles >= 2048) return launch_rows<4, 2, 3, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    if (tiles >= 384 && K <= 4096 && !(tiles <= 512 ? M <= 4 : tiles <= 768)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    if (tiles >= 384 && K > 4096) return launch_rows<4, 1, 4, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   }
-  if (K % 2048 == 0) {
-    if (tiles >= 2048) return launch_rows<4, 1, 3, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-    return launch_rows<4, 1, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-  }
-  if (tiles >= 2048) return launch_rows<4, 2, 3, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-  if (tiles >= 384 && K <= 4096) return launch_rows<4, 2, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-  if (tiles >= 384) return launch_rows<4, 1, 4, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-  return launch_rows<4, 1, 2, GATED>(a, w, c, out_dtype, M, N, K, ep, st, 1);
 }
 
 // A page of zeros for a wave that has no tile of its own: read at no cost in memory traffic.
@@ -625,7 +637,7 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
           const float g = (float)(bf16_t)acc[t][b][r];
           o[r] = ep.template apply<GATED>(g, (float)(bf16_t)acc[NT + t][b][r], m);
         } else {
-          o[r] = acc[t][b][r];
+          o[r] = ep.whole(acc[t][b][r]);
         }
       }
       store4(C + (size_t)m * N + n, o);
@@ -745,9 +757,12 @@ static int gemm(const void* a, const void* w, void* c, int out_dtype, int M, int
     return mid_rows<8>(A, W, c, out_dtype, M, N, K, ep, gated, stream, k_parts);
   }
   if (M <= 16 && aligned && K % 64 == 0)  // through LDS by direct loads: whole cache lines
-    return gated == 1 ? few_rows<1>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
-           : gated    ? few_rows<2>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
-                      : few_rows<0>(A, W, c, out_dtype, M, N, K, ep, stream, k_parts);
+    return M <= 8 ? (gated == 1 ? few_rows<1, true>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
+                     : gated    ? few_rows<2, true>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
+                                : few_rows<0, true>(A, W, c, out_dtype, M, N, K, ep, stream, k_parts))
+                  : (gated == 1 ? few_rows<1, false>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
+                     : gated    ? few_rows<2, false>(A, W, c, out_dtype, M, N, K, ep, stream, 1)
+                                : few_rows<0, false>(A, W, c, out_dtype, M, N, K, ep, stream, k_parts));
   QRT_CHECK(k_parts == 1, "gemm_bf16: K parts need M <= 16 or the LDS-sharing kernel, and K %% 64 == 0 (M=%d K=%d)", M, K);
   if (M <= 16 && aligned) return gated == 1 ? skinny<1>(A, W, c, out_dtype, M, N, K, ep, stream)
                                 : gated    ? skinny<2>(A, W, c, out_dtype, M, N, K, ep, stream)
@@ -763,6 +778,15 @@ extern "C" int qrt_gemm_bf16(const void* a, const void* w, void* c, int out_dtyp
                              int shared, int k_parts, hipStream_t stream) {
   QRT_CHECK(gated == 0 || gated == 1, "gemm_bf16: unknown mode %d", gated);
   return gemm(a, w, c, out_dtype, M, N, K, gated, shared, k_parts, GatedEpilogue{QRT_ACT_SWIGLU, 0.f, nullptr}, stream);
+}
+
+// The product without a gate and its activation (QRT_ACT_RELU2), bfloat16 out: few rows, or with `shared` the kernel that shares
+// the activations. One kernel less in a decode step (4.7 us of a 4B layer with such a feed-forward).
+extern "C" int qrt_act_gemm_bf16(const void* a, const void* w, void* c, int M, int N, int K, int shared, int act_kind, hipStream_t stream) {
+  QRT_CHECK(act_kind == QRT_ACT_RELU2, "act_gemm_bf16: unknown activation %d", act_kind);
+  QRT_CHECK(shared || (M <= 16 && K % 64 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0),
+            "act_gemm_bf16: needs M <= 16 and K %% 64 == 0, or the LDS-sharing kernel (M=%d K=%d)", M, K);
+  return gemm(a, w, c, QRT_BF16, M, N, K, 0, shared, 1, GatedEpilogue{act_kind, 0.f, nullptr}, stream);
 }
 
 // The gated product with any activation of common.h, row m of the result times row_scale[m] (null: 1).

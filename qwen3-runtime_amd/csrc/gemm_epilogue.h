@@ -5,6 +5,7 @@
 // What the gated products do with a gate and an up value (their template's GATED: 0 no gate, 1 SwiGLU and
 // nothing else, 2 what is given here): an activation of common.h, times a factor per row of the
 // activations (null: 1).
+#define QRT_ACT_RELU2 2  // of a product without a gate: the square of relu
 struct GatedEpilogue {
   int kind;
   float limit;
@@ -14,6 +15,12 @@ struct GatedEpilogue {
     if (GATED == 1) return gated_act(g, u, QRT_ACT_SWIGLU, 0.f);
     const float v = gated_act(g, u, kind, limit);
     return row_scale ? v * row_scale[m] : v;
+  }
+  // a sum without a gate; the activation is of the sum rounded to bfloat16, as a kernel behind the product sees it
+  __device__ __forceinline__ float whole(float x) const {
+    if (kind != QRT_ACT_RELU2) return x;
+    const float v = fmaxf((float)(bf16_t)x, 0.f);
+    return v * v;
   }
 };
 

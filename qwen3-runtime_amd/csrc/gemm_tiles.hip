@@ -151,7 +151,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf16_tiles_kernel(TileAr
         } else {
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            const float o[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            float o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = p.ep.whole(acc[i][j][r]);
             store4((bf16_t*)(row + 32 * j + 8 * quad), o);
           }
         }
@@ -204,17 +206,18 @@ static int by_result(const TileArgs& p, int out_dtype, int gated, hipStream_t st
 }
 
 // C [M, N], or with parts > 1 (not gated, float32) planes [parts, M, N]; tile: a number of TILES in ops/hip.py.
-// act_kind < 0: no gate. Needs N a multiple of 16, K of 64, and operands at multiples of 16 bytes and of less
+// act_kind < 0: no gate; QRT_ACT_RELU2: none, but an activation of the whole result in bfloat16. Needs N a multiple of 16, K of 64, and operands at multiples of 16 bytes and of less
 // than 4 GiB each (their offsets are 32 bits).
 extern "C" int qrt_gemm_tiles(const void* a, const void* w, void* c, int out_dtype, int M, int N, int K, int tile, int parts,
                               int act_kind, float limit, const float* row_scale, hipStream_t stream) {
-  const bool gated = act_kind >= 0;
+  const bool gated = act_kind >= 0 && act_kind != QRT_ACT_RELU2;
   QRT_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiles: bad sizes M=%d N=%d K=%d", M, N, K);
   QRT_CHECK(N % 16 == 0 && K % 64 == 0, "gemm_tiles: needs N %% 16 == 0 and K %% 64 == 0 (N=%d K=%d)", N, K);
   QRT_CHECK(out_dtype == QRT_BF16 || (out_dtype == QRT_F32 && !gated), "gemm_tiles: unknown output dtype %d", out_dtype);
   QRT_CHECK(parts >= 1 && parts <= 64, "gemm_tiles: bad number of K parts %d", parts);
   QRT_CHECK(parts == 1 || (!gated && out_dtype == QRT_F32), "gemm_tiles: K parts need no gate and float32 output");
-  QRT_CHECK(act_kind <= QRT_ACT_CLAMPED, "gemm_tiles: unknown activation %d", act_kind);
+  QRT_CHECK(act_kind <= QRT_ACT_RELU2, "gemm_tiles: unknown activation %d", act_kind);
+  QRT_CHECK(act_kind != QRT_ACT_RELU2 || (out_dtype == QRT_BF16 && !row_scale), "gemm_tiles: an activation without a gate is of whole bfloat16 rows");
   QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0, "gemm_tiles: operands must begin at multiples of 16 bytes");
   const uint64_t limit_bytes = (1ull << 32) - 128;
   QRT_CHECK((uint64_t)M * K * 2 <= limit_bytes && (uint64_t)(gated ? 2 : 1) * N * K * 2 <= limit_bytes,

@@ -68,5 +68,6 @@ class ActMLP(FeedForward):
         self.down = fetch.matrix(self._name("down"))
 
     def forward(self, ctx, x):
-        act = ctx.ops.unary_act(ctx.ops.linear(x, self.up), self.activation)
+        together = getattr(ctx.ops, "act_linear", None)  # product and activation in one kernel
+        act = together(x, self.up, self.activation) if together else ctx.ops.unary_act(ctx.ops.linear(x, self.up), self.activation)
         return ctx.ops.linear_for_residual(act, self.down)

@@ -101,6 +101,37 @@ def test_squared_relu(ops, dtype, shape):
     assert torch.equal(ops.unary_act(x, "relu2"), x.float().clamp(min=0).square().to(dtype))
 
 
+# few rows in every kernel that takes them, tiles, and K that keeps to the two kernels; weight rows: a remainder of 16 goes there too
+@pytest.mark.parametrize("n,k", [(16, 64), (400, 2560), (48, 128), (40, 192), (64, 96)])
+def test_product_and_squared_relu_have_the_bits_of_the_two(ops, n, k):
+    x, w = rnd(300, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=k ** -0.5)
+    for m in (1, 8, 9, 16, 17, 64, 65, 300):
+        assert torch.equal(ops.act_linear(x[:m], w, "relu2"), ops.unary_act(ops.linear(x[:m], w), "relu2")), m
+
+
+# weight rows: 512, 513, 768 and 769 tiles of 16 and a remainder; rows on both sides of 4, 8 and 16
+@pytest.mark.parametrize("n", [8192, 8200, 12288, 12296])
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
+def test_few_rows_at_the_edges_of_their_tiles(ops, m, n):
+    x, w = rnd(m, 192, dtype=torch.bfloat16, seed=3), rnd(n, 192, dtype=torch.bfloat16, seed=4)
+    want = x.double() @ w.double().T
+    # float32 sums of 192 products; the result is not rounded further
+    bound = 192 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((ops.linear(x, w, out_f32=True).double() - want).abs() <= bound).all()
+
+
+# tiles of eight gate and eight up rows or one of either: rows of K up to 4,096 and beyond, on both sides of 2 and 8 rows
+@pytest.mark.parametrize("activation,limit", [("swiglu", 0.0), ("clamped", 0.9)])
+@pytest.mark.parametrize("inter,k", [(8, 64), (20, 4096), (36, 4160)])
+def test_gated_few_rows_at_the_edges_of_their_tiles(ops, inter, k, activation, limit):
+    x, w = rnd(11, k, dtype=torch.bfloat16, seed=5), rnd(2 * inter, k, dtype=torch.bfloat16, seed=6, scale=2 * k ** -0.5)
+    for m in (1, 2, 3, 8, 9, 11):
+        both = (x[:m].double() @ w.double().T).float()
+        want = ops.gated_act(both.to(torch.bfloat16), activation, limit)
+        # both halves rounded to bfloat16 may fall on the other side of a tie: two units of 2^-8, as the result's own
+        close(ops.gated_linear(x[:m], w, activation, limit), want, 2e-2, 2e-2)
+
+
 @pytest.mark.parametrize("tokens", [1, 16, 17, 128, 129, 300])
 @pytest.mark.parametrize("heads,n,k,in_stride,in_offset,out_stride,out_offset",
                          [(3, 4, 64, 64, 0, 4, 0), (2, 60, 128, 160, 24, 72, 8), (4, 384, 128, 192, 0, 448, 0),
