@@ -1566,6 +1566,58 @@ __device__ __forceinline__ void head_as_operand(const bf16_t* __restrict__ x, co
     for (int e = 0; e < 8; ++e) out[i][e] = (bf16_t)v[i][e];
 }
 
+// Heads of 64 and 128 elements: a wave's next block of keys and values comes by direct loads into LDS of its own, whole
+// cache lines, while one is multiplied from registers.
+// Keys: operand row 16 kb + r (key 8 (r / 4) + 4 kb + r % 4 of the block) is a row of D elements, piece c (16 bytes) of it at
+// c ^ (r, or r / 2 where a row is half of the banks), so that the operand reads touch every bank once. Values: element d is
+// a row of 64 bytes, its four groups of eight keys at g ^ (d / 4) % 4. Every load is of 16 bytes a lane, from anywhere: four
+// keys, or sixteen elements of two pages of 16 keys, an instruction. As loads straight to registers the keys came as sixteen half
+// lines an instruction, and two blocks on their way took 128 registers: attention and merge, us, before and now, 8 sequences of 2,054 keys with 32 heads of 128
+// on 8 22.0 and 20.9 in 4 parts, 23.4 and 20.1 in 8; 24 of 800 25.5 and 22.2; 64 of 1,024 53.1 and 51.3; 48 of 136 to 2,606 46.5 and 41.3; 64 of 200 to
+// 8,000 117 and 105. Waiting for keys and values apart, so that either is on its way a little longer, is level (20.9, 21.1).
+constexpr bool DECODE_RING = D % 64 == 0 && DMAX <= 128;
+constexpr int RING_KEYS = 64 * D, RING_WAVE = RING_KEYS + 64 * DV;  // bytes
+
+// Pages of the groups of eight keys of 16 blocks, `step` apart from block `first` on (none after `last`): lane 4 i + g has
+// that of group g of the i-th.
+template <bool P2>
+__device__ __forceinline__ int ring_pages(const int* __restrict__ table, int first, int step, int last, int lo, int pos_max, int ps, int lane) {
+  const int base = min(first + (lane >> 2) * step, last) << 5;
+  return table[page_div<P2>(min(max(base + 8 * (lane & 3), lo & ~7), pos_max & ~7), ps, __builtin_ctz(ps))];
+}
+// Groups that lie outside [lo, pos_max] are read as its first or last one, as block_load does, and masked or zeroed likewise.
+template <bool P2>
+__device__ __forceinline__ void ring_fetch(const AttnTileArgs& a, int kvh, int base, int lo, int pos_max, int pages, int i, int lane,
+                                           unsigned char* ring) {
+  constexpr int ONCE = 2;  // the cache policy of a non-temporal load
+  constexpr int A_ROW = D / 8;  // lanes a key
+  const int ps = a.page_size;
+  auto first_key = [&](int g) { return page_mod<P2>(min(max(base + 8 * g, lo & ~7), pos_max & ~7), ps); };
+#pragma unroll
+  for (int j = 0; j < D / 16; ++j) {
+    const int row = j * (64 / A_ROW) + lane / A_ROW, r = row & 15, g = r >> 2;
+    const int page = __shfl(pages, 4 * i + g, 64), off = first_key(g) + 4 * (row >> 4) + (r & 3);
+    const int piece = (lane % A_ROW) ^ (D % 128 == 0 ? r : r >> 1);
+    const bf16_t* src = a.k_cache + (((size_t)page * a.nkv + kvh) * ps + off) * D + 8 * piece;
+    __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(ring + j * 1024), 16, 0, ONCE);
+  }
+  const int g = (lane & 3) ^ (lane >> 4);
+  const bf16_t* src = a.v_cache + (((size_t)__shfl(pages, 4 * i + g, 64) * a.nkv + kvh) * DV + (lane >> 2)) * ps + first_key(g);
+#pragma unroll
+  for (int j = 0; j < DB; ++j)
+    __builtin_amdgcn_global_load_lds((global_ptr_t)(src + (size_t)16 * j * ps), (lds_ptr_t)(ring + RING_KEYS + j * 1024), 16, 0, ONCE);
+}
+__device__ __forceinline__ void ring_read(const unsigned char* ring, int r16, int quad, KvBlock& blk) {
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int i = 0; i < KFULL; ++i)
+      blk.k[kb][i] = *(const bf16x8_t*)(ring + (16 * kb + r16) * 2 * D + 16 * ((4 * i + quad) ^ (D % 128 == 0 ? r16 : r16 >> 1)));
+#pragma unroll
+  for (int i = 0; i < DB; ++i)
+    blk.v[i] = *(const bf16x8_t*)(ring + RING_KEYS + (16 * i + r16) * 64 + 16 * (quad ^ ((r16 >> 2) & 3)));
+}
+
 constexpr bool DECODE_ONCE = true;  // measured: 2 % off a decode step at batch 1 and at batch 64, level at batch 8
 
 template <bool P2, bool FUSED = false>
@@ -1574,7 +1626,8 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   extern __shared__ float lds[];
   float* lds_m = lds;                 // [DW][16]
   float* lds_l = lds + DW * 16;       // [DW][16]
-  float* lds_o = lds + 2 * DW * 16;   // [DW][16][OROW]
+  float* lds_o = lds + 2 * DW * 16;   // [DW] x O_WAVE: [16][OROW], in the room of the wave's ring
+  constexpr int O_WAVE = DECODE_RING ? RING_WAVE / 4 : 16 * OROW;
 
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r16 = lane & 15, quad = lane >> 4;
@@ -1694,10 +1747,30 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
       if (KTAIL) qtail = load_tail(qp + 32 * KFULL, quad);
     }
 
+    const int last = b + (b1 - 1 - b) / DW * DW;
+    if constexpr (DECODE_RING) {
+      unsigned char* ring = (unsigned char*)(lds_o + wave * O_WAVE);
+      int pages = ring_pages<P2>(table, b, DW, last, lo, pos_max, a.page_size, lane), i = 0;
+      ring_fetch<P2>(a, kvh, b << 5, lo, pos_max, pages, 0, lane, ring);
+      if (FUSED) own_token();  // while the first keys and values are on their way
+      KvBlock blk;
+      for (; b < b1; b += DW) {
+        QRT_WAIT_LOADS(0);
+        ring_read(ring, r16, quad, blk);
+        QRT_WAIT_LDS();  // the block is in registers: the next one may overwrite it
+        if (b + DW < b1) {
+          if (++i == 16) {
+            pages = ring_pages<P2>(table, b + DW, DW, last, lo, pos_max, a.page_size, lane);
+            i = 0;
+          }
+          ring_fetch<P2>(a, kvh, (b + DW) << 5, lo, pos_max, pages, i, lane, ring);
+        }
+        block_compute(blk, qreg, qtail, b << 5, lo, pos_min, pos_max, quad, row_valid, qpos_c, window, a.chunk, a.keep_first, a.cap_in, a.cap_out, a.scale_log2, m, l, o);
+      }
+    } else {
     // two blocks of keys and values are on their way while a third is multiplied, and the page
     // numbers of the two after them; past the wave's last block the loads go on (one shape of
     // loop, no load under a branch) but fetch next to nothing
-    const int last = b + (b1 - 1 - b) / DW * DW;
     KvBlock A, B;
     int pgA[3], pgB[3];
     block_pages<P2>(table, b << 5, lo, pos_max, a.page_size, r16, quad, pgA);
@@ -1718,6 +1791,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
       block_pages<P2>(table, min(b + 4 * DW, last) << 5, lo, pos_max, a.page_size, r16, quad, pgB);
       b += DW;
       if (b >= b1) break;
+    }
     }
   } else if (FUSED) {
     own_token();
@@ -1746,7 +1820,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   }
   if (row_valid)
 #pragma unroll
-    for (int i = 0; i < DB; ++i) *(f32x4_t*)(lds_o + (wave * 16 + r16) * OROW + 16 * i + 4 * quad) = o[i];
+    for (int i = 0; i < DB; ++i) *(f32x4_t*)(lds_o + wave * O_WAVE + r16 * OROW + 16 * i + 4 * quad) = o[i];
   __syncthreads();
 
   const size_t tile_row0 = (size_t)q_begin * a.nq;  // rows of this sequence start here, in units of heads
@@ -1763,7 +1837,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
 #pragma unroll
       for (int w = 0; w < DW; ++w) {
         const float f = exp2f(lds_m[w * 16 + row] - mm);
-        num += f * lds_o[(w * 16 + row) * OROW + d];
+        num += f * lds_o[w * O_WAVE + row * OROW + d];
         den += f * lds_l[w * 16 + row];
       }
     }
@@ -1848,7 +1922,8 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
   const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
   dim3 grid(a.num_tiles, a.nkv, a.num_splits), block(64 * DW);
   if (a.items) grid = dim3(a.nkv, a.max_items, 1);
-  constexpr size_t smem = (size_t)(2 * DW * 16 + DW * 16 * OROW) * sizeof(float);
+  constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (DECODE_RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
+  static_assert(!DECODE_RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
   if (smem > 64 * 1024) {  // head size 256: a little more LDS than a block gets without asking
     static bool allowed = false;  // once: not again inside every stream capture
     if (!allowed) {

@@ -895,6 +895,20 @@ def test_decode_attention_in_pieces_of_one_length(ops, seqs, nq, nkv, d, ps, win
     close(ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window), want, 2e-2, 2e-2)
 
 
+# one part of the keys: a wave walks more blocks than it holds page numbers of (16); pages of one group of keys, of three and of
+# more than a block; a window that begins inside a block and a page
+@pytest.mark.parametrize("d,ps", [(64, 8), (64, 64), (128, 24), (128, 16)])
+@pytest.mark.parametrize("window", [None, 2077])
+def test_decode_attention_over_many_blocks_a_wave(ops, d, ps, window):
+    lens = [4200, 2049, 1, 2048 * 2 + 31]
+    q, cache, ctx = build_attention_case([(1, n) for n in lens], 6, 2, d, ps, torch.bfloat16, seed=9, window=window, poison=True)
+    want = R.paged_attention(q, cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, ps, 6, 2, d,
+                             d ** -0.5, window)
+    for splits in (1, 2):
+        ctx.scratch["attn_splits"] = splits
+        close(ops.paged_attention(q, cache, ctx, 6, 2, d, d ** -0.5, window), want, 2e-2, 2e-2)
+
+
 @pytest.mark.parametrize("lens,nkv,d", [
     ([100 + 41 * i for i in range(28)], 8, 64),         # none as long as 2,048
     ([90, 2600, 700, 64, 1500, 33, 4000, 1, 800], 2, 128),
