@@ -2181,6 +2181,16 @@ class HipOps:
         self._check(self.lib, self.lib.qrt_sample(byref(a), _stream()))
         return tok, lp, work, both
 
+    def force_tokens(self, work, forced, tok, lp):
+        """Where ``forced`` (int32 [R]) is not negative, ``tok`` becomes it and ``lp`` its log-probability under the
+        processed logits ``work`` [R, V]."""
+        r, v = work.shape
+        _need(work, "processed logits", torch.float32)
+        _need(forced, "forced ids", torch.int32, (r,))
+        _need(tok, "ids", torch.int32, (r,))
+        _need(lp, "log-probabilities", torch.float32, (r,))
+        self._check(self.lib, self.lib.qrt_force_tokens(_ptr(work), _ptr(forced), _ptr(tok), _ptr(lp), c_int(r), c_int(v), _stream()))
+
     def count_tokens(self, counts, slots, tokens):
         _need(counts, "counts", torch.int32)
         _need(slots, "slots", torch.int32)

@@ -70,11 +70,15 @@ class Sampler:
         if any_forced:
             # teacher forcing: the given id, scored under the processed logits
             # (reference: qwen3_runtime/sampling.py:319-325)
-            logp = torch.log_softmax(work, dim=-1)
-            for i, f in enumerate(forced):
-                if f is not None:
-                    tok[i] = int(f)
-                    lp[i] = logp[i, int(f)]
+            if tok.device.type == "cuda":
+                ids = torch.tensor([-1 if f is None else int(f) for f in forced], dtype=torch.int32, pin_memory=True)
+                self.ops.force_tokens(work, ids.to(self.device, non_blocking=True), tok, lp)
+            else:
+                logp = torch.log_softmax(work, dim=-1)
+                for i, f in enumerate(forced):
+                    if f is not None:
+                        tok[i] = int(f)
+                        lp[i] = logp[i, int(f)]
         if self.counts is not None:
             self.ops.count_tokens(self.counts, slot_rows, tok)
         if both.device.type != "cuda":

@@ -355,6 +355,27 @@ def test_sampler_greedy_ties_and_logprob():
     assert lp[2] == pytest.approx(float(torch.log_softmax(x[2].cpu(), -1)[1]), abs=1e-5)
 
 
+@pytest.mark.parametrize("vocab", [1, 5, 1023, 1025, 16385, 151936])
+def test_forced_ids_and_their_log_probabilities(vocab):
+    """Rows with a given id and rows without; excluded ids (-inf) among the logits and as the id asked for; against float64: sums of
+    exponentials in any order, each rounded, and the logarithm's own rounding (values up to some 20)."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops, rows = HipOps(), 5
+    work = 4 * torch.randn(rows, vocab, generator=torch.Generator().manual_seed(vocab))
+    work[1, ::2] = float("-inf")
+    forced = [vocab - 1, 0, -1, vocab // 2, min(1, vocab - 1)]
+    want = work.double().log_softmax(-1)
+    tok = torch.full((rows,), 7, dtype=torch.int32, device=DEV)
+    lp = torch.full((rows,), 0.5, device=DEV)
+    ops.force_tokens(work.to(DEV), torch.tensor(forced, dtype=torch.int32, device=DEV), tok, lp)
+    assert tok.tolist() == [7 if f < 0 else f for f in forced]
+    for i, f in enumerate(forced):
+        expect = 0.5 if f < 0 else float(want[i, f])
+        got = float(lp[i])
+        assert (math.isnan(got) and math.isnan(expect)) or got == pytest.approx(expect, abs=1e-5) or got == expect
+
+
 def test_sampler_filters_match_plain_and_draws_follow_the_distribution():
     from qwen3_runtime_amd.sampling.params import SamplingParams
 
