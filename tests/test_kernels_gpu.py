@@ -978,6 +978,21 @@ def test_attention_far_key_stands_out(ops):
         close(got, want, 1e-2, 1e-2)
 
 
+@pytest.mark.parametrize("column", [0, 4, 1])
+@pytest.mark.parametrize("seqs,nq,nkv,d", [([(70, 97), (9, 9), (1, 130)], 8, 2, 128), ([(3, 40), (17, 17)], 4, 1, 80), ([(33, 64)], 2, 2, 16),
+                                           ([(40, 300)], 8, 4, 256), ([(2, 20), (1, 4)], 3, 3, 64)])
+def test_prompt_attention_with_an_output_gate(ops, seqs, nq, nkv, d, column):
+    """The gate's columns of a wider product: at its start, eight bytes in (pieces of four elements) and where only single
+    elements line up; also with an odd row length. The gate is in bf16 and the factor in float32, so the result is the one
+    without a gate times the sigmoid but for the one rounding to bf16 (8 bits: 2^-8 of the value) that each of the two makes."""
+    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, 16, torch.bfloat16)
+    wide = rnd(ctx.num_tokens, nq * d + (4 if column != 1 else 3), dtype=torch.bfloat16, seed=9, scale=3.0)
+    gate = wide[:, column:column + nq * d]
+    plain = ops.paged_attention(q, cache, ctx, nq, nkv, d, 1.0 / math.sqrt(d), None, softcap=20.0)
+    got = ops.paged_attention(q, cache, ctx, nq, nkv, d, 1.0 / math.sqrt(d), None, softcap=20.0, gate=gate)
+    close(got, plain.float() * torch.sigmoid(gate.float()), 1e-6, 1.01 * 2 ** -7)
+
+
 @pytest.mark.parametrize("rise,jump_at", [(0.0, None), (5.0, None), (7.5, None), (3.0, 9), (0.5, 0)])
 def test_prompt_attention_with_scores_that_climb(ops, rise, jump_at):
     """The prompt kernel takes its exponentials against a reference that follows a row's maximum
