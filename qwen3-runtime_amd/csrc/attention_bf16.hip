@@ -441,12 +441,13 @@ __device__ __forceinline__ void block_load(const AttnTileArgs& a, int kvh, int b
 // sees all of them (kend <= the first key of the wave's window): blocks of 32 keys straight from
 // the pages, a handful at most, before (or after) the window's blocks. Loads are clamped into
 // [0, kend - 1], which lies in pages the table keeps.
-template <int RT, bool P2>
+template <int RT, bool P2, class Q>
 __device__ __forceinline__ void kept_keys_pass(const AttnTileArgs& a, const int* __restrict__ table, int kvh, int kend,
                                                int r16, int quad, const bool* row_valid,
-                                               const bf16x8_t (*qreg)[KFULL > 0 ? KFULL : 1], const bf16x8_t* qtail,
+                                               const Q& q_of, const bf16x8_t* qtail,
                                                float* m, float* l, f32x4_t (*o)[DB]) {
   for (int base = 0; base < kend; base += 32) {
+    if (KFULL > 8) asm volatile("" ::: "memory");  // queries that lie in LDS are read for every block
     int pg[3];
     KvBlock blk;
     block_pages<P2>(table, base, 0, kend - 1, a.page_size, r16, quad, pg);
@@ -464,7 +465,7 @@ __device__ __forceinline__ void kept_keys_pass(const AttnTileArgs& a, const int*
       for (int kb = 0; kb < 2; ++kb) {
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < KFULL; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[kb][i], qreg[t][i], acc, 0, 0, 0);
+        for (int i = 0; i < KFULL; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[kb][i], q_of(t, i), acc, 0, 0, 0);
         if (KTAIL) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.kt[kb], qtail[t], acc, 0, 0, 0);
         sc[kb] = acc;
       }
@@ -491,6 +492,14 @@ __device__ __forceinline__ void add_sink(float& m, float& l_total, f32x4_t* o) {
 // four waves, 64 * RT rows. The keys and values of a block of 32 keys are read
 // once into registers and multiplied with all RT tiles, which divides the
 // operand traffic per MFMA by RT.
+// Heads wider than 256 leave no registers for the queries beside the accumulator, a block of keys and values and their
+// addresses. Spilled, they were loaded one 16 bytes at a time, 14 round trips of memory in a row for a head of 448, and came back out
+// of scratch memory for every block; now they lie in LDS, a place of its own for every lane, and the loop spills nothing. One token each of
+// 8 sequences of 1,029 keys, 32 heads of 448 on one, us with the merge 24.1 -> 20.6; of 300 keys 19.5 -> 16.3; of 4,000
+// 39.0 -> 30.0; 32 sequences of 1,029 41.7 -> 32.3. (The first block's page numbers asked for ahead of the queries: 0.5 to 1.5 slower.)
+template <int RT>
+constexpr bool Q_IN_LDS = RT == 1 && KFULL > 8;
+
 template <int RT, bool P2>
 // (Heads wider than 256: a wave's accumulator, queries and one block of keys and values fill most of
 // the 512 registers a lane can have, so one block of waves a compute unit and one tile a wave.)
@@ -518,6 +527,9 @@ __global__ __launch_bounds__(256, (RT <= 2 && DMAX <= 256) ? 2 : 1) void attenti
                                                      // first key that its highest position sees
   size_t row_index[RT];
   bf16x8_t qreg[RT][KFULL > 0 ? KFULL : 1];
+  __shared__ bf16x8_t q_kept[Q_IN_LDS<RT> ? 4 * KFULL * 64 : 1];  // a place for every lane: no wave reads another's
+  bf16x8_t* my_q = q_kept + wave * KFULL * 64 + lane;
+  auto q_of = [&](int t, int i) { return Q_IN_LDS<RT> ? my_q[64 * i] : qreg[t][i]; };
   bf16x8_t qtail[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
@@ -534,6 +546,11 @@ __global__ __launch_bounds__(256, (RT <= 2 && DMAX <= 256) ? 2 : 1) void attenti
     const bf16_t* qp = a.q + row_index[t] * D;
 #pragma unroll
     for (int i = 0; i < KFULL; ++i) qreg[t][i] = *(const bf16x8_t*)(qp + 32 * i + 8 * quad);
+    if (Q_IN_LDS<RT>) {
+#pragma unroll
+      for (int i = 0; i < KFULL; ++i) my_q[64 * i] = qreg[t][i];
+      asm volatile("" ::: "memory");  // from here on they are read out of LDS
+    }
     qtail[t] = load_tail(qp, 2);  // zeros
     if (KTAIL) qtail[t] = load_tail(qp + 32 * KFULL, quad);
   }
@@ -558,7 +575,7 @@ __global__ __launch_bounds__(256, (RT <= 2 && DMAX <= 256) ? 2 : 1) void attenti
   }
 
   if (a.keep_first > 0 && split == 0)
-    kept_keys_pass<RT, P2>(a, table, kvh, min(a.keep_first, lo), r16, quad, row_valid, qreg, qtail, m, l, o);
+    kept_keys_pass<RT, P2>(a, table, kvh, min(a.keep_first, lo), r16, quad, row_valid, q_of, qtail, m, l, o);
 
   // page numbers are looked up one block ahead of the loads that need them; all loads are
   // unconditional (clamped), see block_pages / block_load
@@ -567,6 +584,7 @@ __global__ __launch_bounds__(256, (RT <= 2 && DMAX <= 256) ? 2 : 1) void attenti
     block_pages<P2>(table, b0 << 5, lo, pos_max, ps, r16, quad, pg);
     for (int b = b0; b < b1; ++b) {
       const int base = b << 5;
+      if (Q_IN_LDS<RT>) asm volatile("" ::: "memory");  // the queries are read out of LDS for every block, not kept
       KvBlock blk;
       block_load<P2>(a, kvh, base, lo, pos_max, r16, quad, pg, blk);
       block_pages<P2>(table, min(b + 1, b1 - 1) << 5, lo, pos_max, ps, r16, quad, pg_next);
@@ -586,7 +604,7 @@ __global__ __launch_bounds__(256, (RT <= 2 && DMAX <= 256) ? 2 : 1) void attenti
           f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int i = 0; i < KFULL; ++i)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[kb][i], qreg[t][i], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[kb][i], q_of(t, i), acc, 0, 0, 0);
           if (KTAIL) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.kt[kb], qtail[t], acc, 0, 0, 0);
           s[kb] = acc;
         }
@@ -780,7 +798,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 2 : 1) void attention_bf16_prefil
   }
 
   if (a.keep_first > 0 && split == 0 && grp == 0 && wave_has_rows)
-    kept_keys_pass<RT, P2>(a, table, kvh, min(a.keep_first, lo_w), r16, quad, row_valid, qreg, qtail, m, l, o);
+    kept_keys_pass<RT, P2>(a, table, kvh, min(a.keep_first, lo_w), r16, quad, row_valid, [&](int t, int i) { return qreg[t][i]; }, qtail, m, l, o);
 
   // Who fetches what. A block of 32 keys is four groups of 8 consecutive keys, one per wave.
   // Pages hold a multiple of 8 keys, so a group lies in one page: the wave needs ONE block-table
@@ -1826,7 +1844,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
         for (int i = 0; i < KFULL; ++i) qreg[i] = *(const bf16x8_t*)(qp + 32 * i + 8 * quad);
         if (KTAIL) qtail = load_tail(qp + 32 * KFULL, quad);
       }
-      kept_keys_pass<1, P2>(a, table, kvh, kend, r16, quad, &row_valid, (const bf16x8_t(*)[KFULL > 0 ? KFULL : 1])&qreg, &qtail,
+      kept_keys_pass<1, P2>(a, table, kvh, kend, r16, quad, &row_valid, [&](int, int i) { return qreg[i]; }, &qtail,
                             &m, &l, (f32x4_t(*)[DB])&o);
     }
   }

@@ -1878,9 +1878,15 @@ class HipOps:
     def choose_splits(num_tiles: int, nkv: int, max_kv: int, head_dim: int = 0) -> int:
         """Portions: how many ways to split the keys so that few long sequences still fill the chip.
         Heads wider than 256 (one block of waves a compute unit, and no decode kernel of their own, so
-        that decoded tokens come here too): parts of 64 keys and more, 256 blocks in all."""
+        that decoded tokens come here too): parts of 64 keys and more, 256 blocks in all; parts of 32, one block of keys
+        each, where that makes at most 32 of a sequence and 128 in all (32 heads of 448 on one, us with the merge, 64 and 32 keys a
+        part: 8 sequences of 300 keys 16.3 and 14.4, of 500 17.6 and 16.7, of 640 18.7 and 18.9, of 1,029 20.6 and 26.1; 20 of 300
+        19.8 and 19.8; 8 of 100 in one part 17.8, in four 13.0, of 64 in one 12.0, in two 12.4)."""
         work = num_tiles * nkv
         if head_dim > 256:
+            blocks = (max_kv + 31) // 32
+            if 3 <= blocks <= 32 and work * blocks <= 128:
+                return blocks
             return 1 if max_kv <= 128 or work >= 256 else max(1, min((max_kv + 63) // 64, (256 + work - 1) // work, 64))
         if max_kv <= 512 or work >= 512:
             return 1

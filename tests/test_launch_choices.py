@@ -28,3 +28,11 @@ def test_parts_of_the_keys_of_portions_with_wide_heads(d):
     assert parts((300, 300), (300, 300), (300, 300)) == parts((1000, 1000)) == parts(*[(150, 150)] * 5) == 1
     assert parts((1000, 3000), *[(1, 200)] * 8) == 1
     assert 3 <= parts((200, 4000)) <= 6 and parts((33, 8000)) >= 10
+
+
+@pytest.mark.parametrize("sequences,keys,parts", [
+    (8, 64, 1), (8, 65, 3), (8, 300, 10), (8, 512, 16), (8, 513, 9), (30, 128, 4), (1, 1024, 32), (1, 1025, 17), (16, 256, 8), (17, 256, 4),
+    (8, 1029, 17), (300, 2000, 1),
+])
+def test_parts_of_the_keys_of_decoded_tokens_with_wide_heads(sequences, keys, parts):
+    assert HipOps.choose_splits(sequences, 1, keys, 448) == parts

@@ -117,3 +117,28 @@ def test_a_token_takes_nothing_from_keys_it_does_not_see(value, d, nq, splits, m
                     odd.k[page, :, off, 0] = value
             # one rounding to bfloat16 of results whose probabilities were rounded to it, or were not
             close(attend(odd)[~sees], want[~sees], 2e-2, 2e-2)
+
+
+@pytest.mark.parametrize("d,nq,nkv,seqs,splits,more", [
+    (448, 32, 1, [(1, 1), (1, 33), (1, 96)], None, {}),              # one block of keys a part; a sequence with fewer of them
+    (448, 24, 1, [(1, 64)], None, {}),                               # 24 rows: the second wave's tile half full
+    (320, 8, 2, [(1, 300), (1, 77)], None, {"window": 50}),
+    (320, 72, 2, [(1, 300), (1, 77)], 1, {"window": 50, "keep_first": 37}),  # three waves, one without rows; kept keys: two blocks more
+    (512, 16, 1, [(1, 1030), (2, 40)], None, {"sink": True}),        # the most LDS
+    (512, 16, 1, [(1, 200)], 1, {"chunk": 40}),
+])
+def test_decoded_tokens_with_wide_heads(d, nq, nkv, seqs, splits, more):
+    """The kernel that keeps the queries of heads wider than 256 in LDS, against the oracle."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops, more = HipOps(), dict(more)
+    window = more.pop("window", None)
+    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, 16, torch.bfloat16, poison=True)
+    if splits:
+        ctx.scratch["attn_splits"] = splits
+    scale = 1.0 / math.sqrt(d)
+    want = R.paged_attention(q, cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, 16, nq, nkv, d,
+                             scale, window, **more)
+    got = ops.paged_attention(q, cache, ctx, nq, nkv, d, scale, window, **more)
+    assert next(p for k, p in ctx.scratch.items() if k[0] == "attn_plan")[3] != 3   # not by the kernel of the portions
+    close(got, want, 2e-2, 2e-2)    # as above
