@@ -439,7 +439,6 @@ extern "C" int qrt_count_tokens(int* counts, const int* slot, const int* token, 
   return 0;
 }
 
-// logits[row[i], token[i]] += value[i]   (logit bias; reference: qwen3_runtime/sampling.py:35-41)
 // Teacher forcing: row r's id becomes forced[r] (negative: it keeps the sampled one), its log-probability that id's under the
 // row's processed logits, x - max - log(sum exp(x - max)) as log_softmax has it. A block per row, one pass: a thread follows the
 // maximum of what it has seen, 16 values at a time. Bound by one compute unit's share of the caches: 6 rows of 151,936 take 26 us; the softmax of
@@ -480,6 +479,7 @@ extern "C" int qrt_force_tokens(const float* work, const int* forced, int* token
   return 0;
 }
 
+// logits[row[i], token[i]] += value[i]   (logit bias; reference: qwen3_runtime/sampling.py:35-41)
 __global__ void add_bias_kernel(float* logits, const int* row, const int* token, const float* value, int n, int vocab) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n && token[i] >= 0 && token[i] < vocab) atomicAdd(&logits[(size_t)row[i] * vocab + token[i]], value[i]);
