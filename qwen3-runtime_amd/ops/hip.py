@@ -1932,11 +1932,6 @@ class HipOps:
         for parts in range(2, long_parts + 1):
             if time(parts) < time(best) * 0.999:
                 best = parts
-        # one block to nearly every unit: twice as many of half the length hide each other's starts and ends, as long as they
-        # have 256 keys (8 and 16 sequences of 2,054 keys, us with the merge, in 4 and 2 parts 20.9 and 32.6, in 8 and 4
-        # 20.1 and 30.2; 16 of 1,024 level; 8 of 1,030 in 8 parts 16.2, in 4 15.5)
-        if 1 < best <= 32 and 224 <= work * best <= 256 and blocks // (2 * best) >= 8:
-            return 2 * best
         merge = 180.0 / max(max_kv, 1) if best == 1 else 0.0
         best_time = time(best)
         for parts in range(long_parts + 1, min(blocks // 2, 16) + 1):
