@@ -457,14 +457,15 @@ __global__ __launch_bounds__(1024) void force_tokens_kernel(const float* __restr
     for (int u = 0; u < U; ++u) v[u] = c0 + 1024 * u < vocab ? x[c0 + 1024 * u] : -INFINITY;
 #pragma unroll
     for (int u = 0; u < U; ++u) top = fmaxf(top, v[u]);
-    if (top == -INFINITY) continue;  // nothing but excluded ids so far
-    sum *= expf(m - top);
+    // nothing but excluded ids so far: terms of zero. fmaxf passes a NaN by; the sum has it, and with it the row's result
+    const float base = top == -INFINITY ? 0.f : top;
+    sum *= expf(m - base);
 #pragma unroll
-    for (int u = 0; u < U; ++u) sum += expf(v[u] - top);
+    for (int u = 0; u < U; ++u) sum += expf(v[u] - base);
     m = top;
   }
   const float top = block_max(m, red);
-  const float total = block_sum(m == -INFINITY ? 0.f : sum * expf(m - top), red);
+  const float total = block_sum(m == -INFINITY ? sum : sum * expf(m - top), red);
   if (threadIdx.x == 0) {
     token[row] = id;
     logprob[row] = x[id] - top - logf(total);

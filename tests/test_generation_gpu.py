@@ -376,6 +376,28 @@ def test_forced_ids_and_their_log_probabilities(vocab):
         assert (math.isnan(got) and math.isnan(expect)) or got == pytest.approx(expect, abs=1e-5) or got == expect
 
 
+@pytest.mark.parametrize("vocab", [5, 1025, 16385])
+def test_forced_ids_of_rows_with_a_nan(vocab):
+    """A NaN anywhere in a row makes its log-probability one, also where its thread has seen nothing else but excluded ids; so do
+    an infinite logit and a row of nothing but excluded ids, as log_softmax has it."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    inf, nan = float("inf"), float("nan")
+    work = torch.zeros(6, vocab)
+    work[0, 2] = nan                    # its thread's only id below 1,024, in front of others beyond
+    work[1] = -inf
+    work[1, 0], work[1, vocab - 1] = 1.0, nan
+    work[2] = nan
+    work[3, 1] = inf
+    work[4] = -inf
+    work[5, 1:] = -inf                  # and one that has a value
+    want = work.double().log_softmax(-1)[:, 0]
+    assert want.isnan().tolist() == [True] * 5 + [False]
+    tok, lp = torch.zeros(6, dtype=torch.int32, device=DEV), torch.full((6,), 0.5, device=DEV)
+    HipOps().force_tokens(work.to(DEV), torch.zeros(6, dtype=torch.int32, device=DEV), tok, lp)
+    torch.testing.assert_close(lp.cpu().double(), want, atol=0, rtol=0, equal_nan=True)
+
+
 def test_sampler_filters_match_plain_and_draws_follow_the_distribution():
     from qwen3_runtime_amd.sampling.params import SamplingParams
 
