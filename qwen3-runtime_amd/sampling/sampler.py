@@ -71,8 +71,17 @@ class Sampler:
             # teacher forcing: the given id, scored under the processed logits
             # (reference: qwen3_runtime/sampling.py:319-325)
             if tok.device.type == "cuda":
-                ids = torch.tensor([-1 if f is None else int(f) for f in forced], dtype=torch.int32, pin_memory=True)
+                # an id outside the row is an error here, as an index is; one counted from the row's end is one
+                # there too, and stays the id as given
+                v = work.shape[1]
+                for f in forced:
+                    if f is not None and not -v <= int(f) < v:
+                        raise IndexError(f"given id {int(f)} is out of range for {v} logits")
+                ids = torch.tensor([-1 if f is None else int(f) % v for f in forced], dtype=torch.int32, pin_memory=True)
                 self.ops.force_tokens(work, ids.to(self.device, non_blocking=True), tok, lp)
+                for i, f in enumerate(forced):
+                    if f is not None and int(f) < 0:
+                        tok[i] = int(f)
             else:
                 logp = torch.log_softmax(work, dim=-1)
                 for i, f in enumerate(forced):

@@ -398,6 +398,29 @@ def test_forced_ids_of_rows_with_a_nan(vocab):
     torch.testing.assert_close(lp.cpu().double(), want, atol=0, rtol=0, equal_nan=True)
 
 
+def test_sampler_refuses_a_given_id_outside_the_vocabulary():
+    """Given ids are indices into a row of logits: beyond it an error, counted from its end accepted, in every row of a step."""
+    from qwen3_runtime_amd.sampling.params import SamplingParams
+
+    class Given(_Req):
+        def __init__(self, given):
+            super().__init__(SamplingParams())
+            self.given = given
+
+        def forced_next(self):
+            return self.given
+
+    x = torch.randn(3, 9, generator=torch.Generator().manual_seed(0)).to(DEV)
+    want = x.cpu().double().log_softmax(-1)
+    s, rows = sample_rows(x, [(SamplingParams(), 0)] * 3)
+    for outside in (9, 1 << 20, 1 << 40, -10):
+        with pytest.raises(IndexError):
+            s.sample(x, rows, [Given(None), Given(outside), Given(3)])
+    tok, lp = s.sample(x, rows, [Given(None), Given(8), Given(-2)])
+    assert tok == [int(x[0].argmax()), 8, -2]
+    assert lp == pytest.approx([float(want[0].max()), float(want[1, 8]), float(want[2, -2])], abs=1e-5)
+
+
 def test_sampler_filters_match_plain_and_draws_follow_the_distribution():
     from qwen3_runtime_amd.sampling.params import SamplingParams
 
