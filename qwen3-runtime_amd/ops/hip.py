@@ -1516,6 +1516,8 @@ class HipOps:
         two_i, kw = w_gate_up.shape
         if k != kw or two_i % 2:
             raise OpsError(f"gated_linear: x is {tuple(x.shape)}, weight is {tuple(w_gate_up.shape)}")
+        if ACTIVATIONS[activation] > ACTIVATIONS["clamped"]:  # the kernels take its code, but for a product of another form
+            raise OpsError(f"gated_linear: {activation} has no gate")
         if x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and k % 32 == 0:
             _need(x, "x")
             _need(w_gate_up, "weight")

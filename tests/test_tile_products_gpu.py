@@ -5,7 +5,7 @@ from ctypes import c_float, c_int
 import pytest
 import torch
 
-from qwen3_runtime_amd.ops.hip import BF16, F32, TILES, HipOps, _ptr, _stream
+from qwen3_runtime_amd.ops.hip import BF16, F32, TILES, HipOps, OpsError, _ptr, _stream
 
 DEV = "cuda"
 STAGES = {0: 2, 1: 3, 2: 3, 3: 3, 4: 3, 5: 3, 6: 4, 7: 4, 8: 4, 9: 4, 10: 6, 11: 6, 12: 4, 13: 3}  # in flight
@@ -155,6 +155,17 @@ def test_what_tiles_refuse():
     for a, b in ((x[:, :96].contiguous(), w[:, :96].contiguous()), (x, w[:40])):
         with pytest.raises(Exception, match="gemm_tiles"):
             launch(ops, a, b, out, tile=3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_gated_product_refuses_an_activation_without_a_gate(dtype):
+    """Its code tells the tiles of a product of another form, which would read the gate rows alone."""
+    ops = HipOps()
+    w = rnd(64, 128, seed=2).to(dtype)
+    for m in (1, 16, 64, 300):
+        with pytest.raises(OpsError, match="relu2"):
+            ops.gated_linear(rnd(m, 128, seed=1).to(dtype), w, "relu2")
 
 
 def test_what_the_library_keeps():
