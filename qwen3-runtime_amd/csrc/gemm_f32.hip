@@ -211,6 +211,9 @@ template <int TM_, int TN_, bool PLANES>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int M, int N, int K, int part_len, int group) {
   constexpr int BI = TM_ / 32, BJ = TN_ / 32;  // 16 x 16 blocks a wave, rows of A by rows of W
+  // square whole tiles move a piece of either operand in turn, the others all of A's and then W's: 64 x 64, 2,560 x 9,728 at
+  // 4,096 rows 1,780 us in turn, 1,803 apart; 64 x 32 at 1,024 rows 496 and 487
+  constexpr int IN_TURN = !PLANES && BI == BJ ? BI : BI + BJ;
   __shared__ __align__(16) float as[2][TM_ * F32_LD];
   __shared__ __align__(16) float ws[2][TN_ * F32_LD];
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
@@ -235,9 +238,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
   const int s_first = PLANES ? blockIdx.z * group * per_part : 0, stages = PLANES ? min(all, s_first + group * per_part) : all;
   auto fetch = [&](int buf, int s) {
 #pragma unroll
-    for (int i = 0; i < BI; ++i) ga[buf][i] = load_f32x4_below(ar[i], 32 * s + lk, K);
-#pragma unroll
-    for (int i = 0; i < BJ; ++i) gw[buf][i] = load_f32x4_below(wr[i], 32 * s + lk, K);
+    for (int i = 0; i < IN_TURN; ++i) {
+      const int j = i - (IN_TURN - BJ);
+      if (i < BI) ga[buf][i] = load_f32x4_below(ar[i], 32 * s + lk, K);
+      if (j >= 0) gw[buf][j] = load_f32x4_below(wr[j], 32 * s + lk, K);
+    }
   };
   int left = per_part;
   bool first = true;
@@ -245,9 +250,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     float* da = as[buf];
     float* dw = ws[buf];
 #pragma unroll
-    for (int i = 0; i < BI; ++i) *(f32x4_t*)(da + (lrow + 32 * i) * F32_LD + lk) = ga[buf][i];
-#pragma unroll
-    for (int i = 0; i < BJ; ++i) *(f32x4_t*)(dw + (lrow + 32 * i) * F32_LD + lk) = gw[buf][i];
+    for (int i = 0; i < IN_TURN; ++i) {
+      const int j = i - (IN_TURN - BJ);
+      if (i < BI) *(f32x4_t*)(da + (lrow + 32 * i) * F32_LD + lk) = ga[buf][i];
+      if (j >= 0) *(f32x4_t*)(dw + (lrow + 32 * j) * F32_LD + lk) = gw[buf][j];
+    }
     __syncthreads();  // the stage before last was read before the barrier of the last one: two stages suffice
     // unconditional (under a branch the compiler loses count of the loads in flight and waits for all of
     // them), and held up here (it would move them down to their use): 448 -> 234 us for 354 x 2,560 x 9,728
@@ -257,9 +264,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     for (int h = 0; h < 2; ++h) {
       f32x4_t av[BI], wv[BJ];
 #pragma unroll
-      for (int i = 0; i < BI; ++i) av[i] = *(const f32x4_t*)(da + (wm + 16 * i + r) * F32_LD + 16 * h + 4 * q);
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) wv[j] = *(const f32x4_t*)(dw + (wn + 16 * j + r) * F32_LD + 16 * h + 4 * q);
+      for (int i = 0; i < IN_TURN; ++i) {
+        const int j = i - (IN_TURN - BJ);
+        if (i < BI) av[i] = *(const f32x4_t*)(da + (wm + 16 * i + r) * F32_LD + 16 * h + 4 * q);
+        if (j >= 0) wv[j] = *(const f32x4_t*)(dw + (wn + 16 * j + r) * F32_LD + 16 * h + 4 * q);
+      }
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -267,14 +276,14 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
 #pragma unroll
           for (int j = 0; j < BJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][c], av[i][c], acc[i][j], 0, 0, 0);
     }
-    // a part of K ends. An odd number of stages is followed by one that counts for nothing (zeros, or the next group's
-    // first, whose products are dropped)
-    if (--left == 0 || s + 1 >= stages) {
+    // a part of K ends. An odd number of stages is followed by one that counts for nothing (zeros; in planes the next
+    // group's first, whose products are dropped)
+    if (--left == 0 || (PLANES ? s + 1 >= stages : s + 1 == stages)) {
 #pragma unroll
       for (int i = 0; i < BI; ++i)
 #pragma unroll
         for (int j = 0; j < BJ; ++j) {
-          if (s < stages) total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
+          if (!PLANES || s < stages) total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
           acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
       first = false;
@@ -350,7 +359,10 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // 12 and 6 of them), but alone on its unit a block waits for its own loads: no fewer than 1.3, 1.8 and 2.5 rounds' time.
 // 4B sizes, us, by 64 x 64, 64 x 32, 32 x 32: q/k/v at 64, 180, 354, 1,024 rows 62 47 42, 101 81 76, 146 131 144, 291 309 340;
 // down in planes at 64, 180, 354, 1,024 rows 62 59 49, 97 101 108, 189 195 203, 455 478 521 (whole: 230, 224, 223, 543 by
-// 64 x 64). Larger tiles are slower: 2,048 x 19,456 x 2,560 1,792 us, 1,940 by 128 x 128, 1,854 by 96 x 64.
+// 64 x 64). 128 x 128 where that makes four rounds and more, one block to a unit (its two stages are 80 KB of LDS): 6 % less work a
+// round, but a round is four times as long. By 64 x 64 and 128 x 128, us: 2,560 x 4,096 at 8,192 rows 1,506 and 1,434, 2,560 x 9,728 3,557 and
+// 3,385, 6,144 x 2,560 at 4,096 1,141 and 1,103, 5,120 x 8,192 3,002 and 2,863; 19,456 x 2,560 at 2,048 (9.5 rounds) 1,799 and 1,831, at
+// 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854.
 static int f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
   const long cost = rounds * 100 * round;
@@ -362,6 +374,11 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
   const int c64 = f32_tile_cost(M, N, groups, 64, 64, 606, 130), c32 = f32_tile_cost(M, N, groups, 64, 32, 329, 180),
             c16 = f32_tile_cost(M, N, groups, 32, 32, 190, 250);
   QRT_CHECK((M + 63) / 64 <= 65535, "gemm_f32: M=%d is too large for one launch", M);
+  if constexpr (!PLANES)
+    if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 1024 && f32_tile_cost(M, N, 1, 128, 128, 2324, 0) < c64) {
+      gemm_f32_tile_kernel<128, 128, false><<<dim3((N + 127) / 128, (M + 127) / 128), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts);
+      return 0;
+    }
   if (c64 <= c32 && c64 <= c16)
     gemm_f32_tile_kernel<64, 64, PLANES><<<dim3((N + 63) / 64, (M + 63) / 64, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
   else if (c32 <= c16 || (M + 31) / 32 > 65535)

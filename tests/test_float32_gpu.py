@@ -64,12 +64,36 @@ def test_product_in_planes_is_the_same_for_any_number_of_rows(ops, n, k):
     assert torch.equal(a, b)
 
 
+def tile_of(m, n, groups=1):
+    """The tile that the launch takes by its model of the time (in multiples of a hundredth of a round's)."""
+    tiles, cost = -(-m // 128) * -(-n // 128), {}
+    if groups == 1 and tiles >= 1024:
+        cost[128, 128] = 100 * -(-tiles // 256) * 2324
+    for (tm, tn), (round_time, least) in {(64, 64): (606, 130), (64, 32): (329, 180), (32, 32): (190, 250)}.items():
+        rounds = -(-(-(-m // tm) * -(-n // tn) * groups) // 256)
+        cost[tm, tn] = max(100 * rounds, least) * round_time
+    return min(cost, key=lambda t: (cost[t], t != (64, 64)))
+
+
 def test_product_of_many_rows_in_large_tiles(ops):
-    x, w = rnd(4100, 36, seed=3), rnd(4097, 36, seed=4)   # 33 x 33 tiles of 128, the last of one row and one column
+    x, w = rnd(4100, 36, seed=3), rnd(4097, 36, seed=4)   # 65 x 65 tiles of 64, the last of four rows and one column
     whole = ops.linear(x, w)
     bound = 36 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert ((whole.double() - x.double() @ w.double().T).abs() <= bound).all()
     assert torch.equal(ops.linear(x[4099:].contiguous(), w), whole[4099:])
+
+
+# the last tile of one row and 102 columns, or of two columns; K: one stage a part, two with an odd number in all, 17
+@pytest.mark.parametrize("m,n,k", [(3969, 4070, 36), (4096, 3970, 260), (4000, 4066, 8196)])
+def test_product_of_many_rows_in_tiles_of_128(ops, m, n, k):
+    assert tile_of(m, n) == (128, 128)
+    x, w = rnd(m, k, seed=3), rnd(n, k, seed=4, scale=0.05)
+    whole = ops.linear(x, w)
+    for first in (0, 113, m - 32):
+        part = x[first: first + 32].contiguous()
+        assert torch.equal(ops.linear(part, w), whole[first: first + 32]), first
+        bound = k * 2.0 ** -24 * (part.double().abs() @ w.double().abs().T)   # as above
+        assert ((whole[first: first + 32].double() - part.double() @ w.double().T).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("seqs,nq,nkv,d,dv,ps,more", [
