@@ -14,10 +14,13 @@
 //   of fused multiply-adds per output, as every product had before: 64 x 64 outputs a block, one block per
 //   64 weight rows however few the rows of A.
 //
-// Either MFMA kernel may leave a product for the residual in four planes, the sums of groups of neighbouring parts.
+// Either MFMA kernel may leave a product for the residual in four planes, the sums of groups of neighbouring parts, or (tiles) add
+// those up itself.
 // Error against float64, relative: 3.3e-7 (K 2,560), 4.5e-7 (9,728); the sequential sums': 9.0e-7 and 1.8e-6.
 #include "common.h"
 #include "direct.h"
+#include <limits.h>
+#include <algorithm>
 
 #define TM 64
 #define TN 64
@@ -204,12 +207,15 @@ __global__ __launch_bounds__(64 * PARTS) void gemm_f32_rows_kernel(const float* 
 
 // Tiles of TM x TN outputs, four waves of (TM / 2) x (TN / 2). 32 k of both operands at a time through LDS,
 // two stages; the 32 k after the next come into registers during the products. Rows of 40 floats: 32 bytes
-// modulo 64, with which operand reads meet no bank twice. PLANES: the block makes plane blockIdx.z of the result, the sum
-// of that group of parts; else all parts, from the first to the last.
+// modulo 64, with which operand reads meet no bank twice. The result is all parts, from the first to the last (F32_WHOLE);
+// plane blockIdx.z of it, the sum of that group of parts (F32_PLANES); or the sum of all groups, as a reader of the planes
+// adds them (F32_GROUPS_SUM).
 #define F32_LD 40
-template <int TM_, int TN_, bool PLANES>
+enum { F32_WHOLE, F32_PLANES, F32_GROUPS_SUM };
+template <int TM_, int TN_, int FORM>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int M, int N, int K, int part_len, int group) {
+  constexpr bool PLANES = FORM == F32_PLANES, GROUPS_SUM = FORM == F32_GROUPS_SUM;
   constexpr int BI = TM_ / 32, BJ = TN_ / 32;  // 16 x 16 blocks a wave, rows of A by rows of W
   // square whole tiles move a piece of either operand in turn, the others all of A's and then W's: 64 x 64, 2,560 x 9,728 at
   // 4,096 rows 1,780 us in turn, 1,803 apart; 64 x 32 at 1,024 rows 496 and 487
@@ -233,6 +239,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
   for (int i = 0; i < BI; ++i)
 #pragma unroll
     for (int j = 0; j < BJ; ++j) acc[i][j] = total[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t of_groups[GROUPS_SUM ? BI : 1][GROUPS_SUM ? BJ : 1];
   f32x4_t ga[2][BI], gw[2][BJ];
   const int per_part = part_len / 32, all = (K + 31) / 32;
   const int s_first = PLANES ? blockIdx.z * group * per_part : 0, stages = PLANES ? min(all, s_first + group * per_part) : all;
@@ -244,8 +251,8 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
       if (j >= 0) gw[buf][j] = load_f32x4_below(wr[j], 32 * s + lk, K);
     }
   };
-  int left = per_part;
-  bool first = true;
+  int left = per_part, parts_left = group;
+  bool first = true, first_group = true;
   auto stage = [&](int buf, int s) {
     float* da = as[buf];
     float* dw = ws[buf];
@@ -288,6 +295,18 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
         }
       first = false;
       left = per_part;
+      if (GROUPS_SUM && (--parts_left == 0 || s + 1 == stages)) {
+#pragma unroll
+        for (int i = 0; i < BI; ++i)
+#pragma unroll
+          for (int j = 0; j < BJ; ++j) {
+            f32x4_t& sum = of_groups[GROUPS_SUM ? i : 0][GROUPS_SUM ? j : 0];
+            sum = first_group ? total[i][j] : sum + total[i][j];
+          }
+        first = true;
+        first_group = false;
+        parts_left = group;
+      }
     }
   };
   fetch(0, s_first);
@@ -305,11 +324,12 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     for (int j = 0; j < BJ; ++j) {
       const int n = n0 + wn + 16 * j + 4 * q;
       float* c = C + (size_t)m * N + n;
-      if (N % 4 == 0 && n < N) *(f32x4_t*)c = total[i][j];
+      const f32x4_t v = GROUPS_SUM ? of_groups[GROUPS_SUM ? i : 0][GROUPS_SUM ? j : 0] : total[i][j];
+      if (N % 4 == 0 && n < N) *(f32x4_t*)c = v;
       else
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) c[e] = total[i][j][e];
+          if (n + e < N) c[e] = v[e];
     }
   }
 }
@@ -363,28 +383,36 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // round, but a round is four times as long. By 64 x 64 and 128 x 128, us: 2,560 x 4,096 at 8,192 rows 1,506 and 1,434, 2,560 x 9,728 3,557 and
 // 3,385, 6,144 x 2,560 at 4,096 1,141 and 1,103, 5,120 x 8,192 3,002 and 2,863; 19,456 x 2,560 at 2,048 (9.5 rounds) 1,799 and 1,831, at
 // 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854.
-static int f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
+static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
-  const long cost = rounds * 100 * round;
-  return (int)min(max(cost, (long)least * round), 0x7fffffffL);
+  return std::max(rounds * 100, (long)least) * round;
 }
-template <bool PLANES>
+static long f32_cost_64x64(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 64, 64, 606, 130); }
+static long f32_cost_64x32(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 64, 32, 329, 180); }
+static long f32_cost_32x32(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 32, 32, 190, 250); }
+static long f32_cost_128x128(int M, int N) {
+  return (long)((M + 127) / 128) * ((N + 127) / 128) < 1024 ? LONG_MAX : f32_tile_cost(M, N, 1, 128, 128, 2324, 0);
+}
+template <int TM_, int TN_, int FORM>
+static void f32_tile_launch(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+  const int parts = f32_parts(K);
+  gemm_f32_tile_kernel<TM_, TN_, FORM><<<dim3((N + TN_ - 1) / TN_, (M + TM_ - 1) / TM_, FORM == F32_PLANES ? F32_GROUPS : 1), 256, 0, stream>>>(
+      a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS);
+}
+template <int FORM>
 static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
-  const int parts = f32_parts(K), part_len = f32_part_len(K, parts), groups = PLANES ? F32_GROUPS : 1;
-  const int c64 = f32_tile_cost(M, N, groups, 64, 64, 606, 130), c32 = f32_tile_cost(M, N, groups, 64, 32, 329, 180),
-            c16 = f32_tile_cost(M, N, groups, 32, 32, 190, 250);
+  const int groups = FORM == F32_PLANES ? F32_GROUPS : 1;
+  const long c64 = f32_cost_64x64(M, N, groups), c32 = f32_cost_64x32(M, N, groups), c16 = f32_cost_32x32(M, N, groups);
   QRT_CHECK((M + 63) / 64 <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-  if constexpr (!PLANES)
-    if ((long)((M + 127) / 128) * ((N + 127) / 128) >= 1024 && f32_tile_cost(M, N, 1, 128, 128, 2324, 0) < c64) {
-      gemm_f32_tile_kernel<128, 128, false><<<dim3((N + 127) / 128, (M + 127) / 128), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts);
+  if constexpr (FORM != F32_PLANES)
+    if (f32_cost_128x128(M, N) < c64) {
+      f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
       return 0;
     }
-  if (c64 <= c32 && c64 <= c16)
-    gemm_f32_tile_kernel<64, 64, PLANES><<<dim3((N + 63) / 64, (M + 63) / 64, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
-  else if (c32 <= c16 || (M + 31) / 32 > 65535)
-    gemm_f32_tile_kernel<64, 32, PLANES><<<dim3((N + 31) / 32, (M + 63) / 64, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
-  else
-    gemm_f32_tile_kernel<32, 32, PLANES><<<dim3((N + 31) / 32, (M + 31) / 32, groups), 256, 0, stream>>>(a, w, c, M, N, K, part_len, parts / groups);
+  if constexpr (FORM == F32_GROUPS_SUM) f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
+  else if (c64 <= c32 && c64 <= c16) f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
+  else if (c32 <= c16 || (M + 31) / 32 > 65535) f32_tile_launch<64, 32, FORM>(a, w, c, M, N, K, stream);
+  else f32_tile_launch<32, 32, FORM>(a, w, c, M, N, K, stream);
   return 0;
 }
 
@@ -400,24 +428,34 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
     // 33 to 64 rows: tiles of 32 x 32 where they give every compute unit one and a half (4B gate/up 85 us, as a stream 100;
     // q/k/v 42 either way)
     const bool few = M <= 32 || (M <= 64 && (long)((M + 31) / 32) * ((N + 31) / 32) < 384);
-    if (const int rc = few ? f32_few_rows<0>(a, w, c, M, N, K, 0.f, stream) : f32_tiles<false>(a, w, c, M, N, K, stream)) return rc;
+    if (const int rc = few ? f32_few_rows<0>(a, w, c, M, N, K, 0.f, stream) : f32_tiles<F32_WHOLE>(a, w, c, M, N, K, stream)) return rc;
   }
   QRT_LAUNCH_CHECK("gemm_f32");
   return 0;
 }
 
-// The product in planes [4, M, N] whose sum, from the first to the last, it is (K in multiples of 4 from 256 on): the groups
-// of K's parts, the same whatever the number of rows. Blocks of their own make each, which fills the chip where the weight
-// has few rows. Up to 32 rows as a stream (4B output and down projections at 1, 16, 32 rows 9.5, 10.4, 14.7 and 18.1, 22.9, 31.5 us;
-// all parts in a block 9.7, 12.3, 17.2 and 19.9, 28.1, 40.6), beyond by tiles.
-extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+// The product for the residual (K in multiples of 4 from 256 on), the groups of K's parts added from the first to the last whatever
+// the number of rows: in planes [4, M, N], whose reader adds them, or as their sum [M, N]. Blocks of their own make each plane, which
+// fills the chip where the weight has few rows. Up to 32 rows as a stream (4B output and down projections at 1, 16, 32 rows 9.5, 10.4,
+// 14.7 and 18.1, 22.9, 31.5 us; all parts in a block 9.7, 12.3, 17.2 and 19.9, 28.1, 40.6), beyond by tiles.
+//
+// How many planes: three more of them are written and read, 150 / K of the product's time, so from a round of 64 x 64 tiles on they have to
+// save more than that in part-filled rounds.
+extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
+  if (M <= 32 || N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
+  const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS), f32_cost_64x32(M, N, F32_GROUPS), f32_cost_32x32(M, N, F32_GROUPS)}) / F32_GROUPS;
+  return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1), f32_cost_128x128(M, N)) ? F32_GROUPS : 1;
+}
+extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, int planes, hipStream_t stream) {
   QRT_CHECK(M >= 0 && N > 0 && K >= 256 && K % 4 == 0, "gemm_f32_planes: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(planes == F32_GROUPS || (planes == 1 && M > 32), "gemm_f32_planes: %d planes of %d rows", planes, M);
   QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0, "gemm_f32_planes: operands are read 16 bytes at a time");
   if (M == 0) return 0;
-  if (const int rc = M <= 8    ? f32_rows_planes<1, true>(a, w, c, M, N, K, stream)
-                     : M <= 16 ? f32_rows_planes<1, false>(a, w, c, M, N, K, stream)
-                     : M <= 32 ? f32_rows_planes<2, false>(a, w, c, M, N, K, stream)
-                               : f32_tiles<true>(a, w, c, M, N, K, stream))
+  if (const int rc = planes == 1 ? f32_tiles<F32_GROUPS_SUM>(a, w, c, M, N, K, stream)
+                     : M <= 8    ? f32_rows_planes<1, true>(a, w, c, M, N, K, stream)
+                     : M <= 16   ? f32_rows_planes<1, false>(a, w, c, M, N, K, stream)
+                     : M <= 32   ? f32_rows_planes<2, false>(a, w, c, M, N, K, stream)
+                                 : f32_tiles<F32_PLANES>(a, w, c, M, N, K, stream))
     return rc;
   QRT_LAUNCH_CHECK("gemm_f32_planes");
   return 0;

@@ -96,6 +96,32 @@ def test_product_of_many_rows_in_tiles_of_128(ops, m, n, k):
         assert ((whole[first: first + 32].double() - part.double() @ w.double().T).abs() <= bound).all()
 
 
+# 64 x 64 and 128 x 128, remainders of rows and columns; K: groups of two parts of two stages, the third of one part and the fourth of none;
+# of two parts of five; of four of seventeen
+@pytest.mark.parametrize("m,n,k", [(2049, 2563, 260), (1281, 5123, 1028), (3969, 4070, 1028), (4090, 4096, 8196)])
+def test_product_for_the_residual_of_many_rows_comes_added_up(ops, m, n, k):
+    """One matrix in place of four planes, with the bits of the planes' sum, so that a row's stream and norm do not go by the number of rows."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    planes = HipOps(residual_planes=True)
+    x, w = rnd(m, k, seed=11), rnd(n, k, seed=12, scale=0.05)
+    whole = planes.linear_for_residual(x, w)
+    assert whole.shape == (m, n)
+    res, weight = rnd(m, n, seed=13), torch.ones(n, device=DEV)
+    stream = res.clone()
+    normed = ops.add_rmsnorm(stream, whole, weight, 1e-6, torch.float32)
+    for first, rows in ((0, 1), (63, 9), (130, 33), (m - 200, 200)):
+        at = slice(first, first + rows)
+        few = planes.linear_for_residual(x[at].contiguous(), w)
+        assert few.shape == (4, rows, n)
+        assert torch.equal(((few[0] + few[1]) + few[2]) + few[3], whole[at]), (first, rows)
+        part = res[at].clone()
+        assert torch.equal(ops.add_rmsnorm(part, few, weight, 1e-6, torch.float32), normed[at])
+        assert torch.equal(part, stream[at])
+        bound = k * 2.0 ** -24 * (x[at].double().abs() @ w.double().abs().T)   # as above
+        assert ((whole[at].double() - x[at].double() @ w.double().T).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("seqs,nq,nkv,d,dv,ps,more", [
     ([(1, 16), (1, 17), (1, 130)], 4, 2, 128, 128, 16, {}),                       # decoding: eight waves share the keys
     ([(20, 33), (7, 7), (1, 1)], 5, 1, 48, 48, 4, {}),                            # a tile's 16 rows cut a token's heads
