@@ -402,8 +402,14 @@ static void f32_tile_launch(const float* a, const float* w, float* c, int M, int
 template <int FORM>
 static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
   const int groups = FORM == F32_PLANES ? F32_GROUPS : 1;
+  // a grid holds 65,535 rows of tiles: a result of more rows than that many of 64 is made in two calls (planes are of fewer)
+  constexpr int MOST = 65535 * 64;
+  QRT_CHECK(M <= (FORM == F32_PLANES ? MOST : 2 * MOST), "gemm_f32: M=%d is too large", M);
+  if (M > MOST) {
+    if (const int rc = f32_tiles<FORM>(a, w, c, MOST, N, K, stream)) return rc;
+    a += (size_t)MOST * K, c += (size_t)MOST * N, M -= MOST;
+  }
   const long c64 = f32_cost_64x64(M, N, groups), c32 = f32_cost_64x32(M, N, groups), c16 = f32_cost_32x32(M, N, groups);
-  QRT_CHECK((M + 63) / 64 <= 65535, "gemm_f32: M=%d is too large for one launch", M);
   if constexpr (FORM != F32_PLANES)
     if (f32_cost_128x128(M, N) < c64) {
       f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
@@ -444,6 +450,7 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
 extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
   if (M <= 32 || N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
   const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS), f32_cost_64x32(M, N, F32_GROUPS), f32_cost_32x32(M, N, F32_GROUPS)}) / F32_GROUPS;
+  if (M > 65535 * 64) return 1;  // two calls
   return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1), f32_cost_128x128(M, N)) ? F32_GROUPS : 1;
 }
 extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, int planes, hipStream_t stream) {

@@ -136,6 +136,24 @@ def test_attention_by_tiles(ops, seqs, nq, nkv, d, dv, ps, more):
     if dv != d:
         cache.v = rnd(cache.v.shape[0], nkv, dv, ps, seed=7)
     if more.pop("gate", False):
+@pytest.mark.parametrize("k,planes", [(4, False), (256, True)])
+def test_product_of_more_rows_than_a_grid_has_tiles(k, planes):
+    """65,535 rows of tiles of 64 are 4,194,240; the tiles beyond are in a launch of their own."""
+    from qwen3_runtime_amd.ops.hip import HipOps
+
+    ops, m, n = HipOps(residual_planes=planes), 65535 * 64 + 70, 3
+    gen = torch.Generator(DEV).manual_seed(1)
+    x, w = torch.randn(m, k, device=DEV, generator=gen), rnd(n, k, seed=2)
+    product = ops.linear_for_residual if planes else ops.linear
+    got = product(x, w)
+    assert got.shape == (m, n)
+    for first in (0, 65535 * 64 - 40, 65535 * 64 - 1, m - 64):
+        few = product(x[first: first + 64].contiguous(), w)
+        few = ((few[0] + few[1]) + few[2]) + few[3] if planes else few
+        assert torch.equal(few, got[first: first + 64]), first
+    close(got, x @ w.T, 1e-5 * math.sqrt(k), 1e-5)
+
+
         more["gate"] = rnd(ctx.num_tokens, nq * dv, seed=9)
     window, scale = more.pop("window", None), 1.0 / math.sqrt(d)
     want = R.paged_attention(q.double(), cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, ps,
