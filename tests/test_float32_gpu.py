@@ -75,6 +75,20 @@ def tile_of(m, n, groups=1):
     return min(cost, key=lambda t: (cost[t], t != (64, 64)))
 
 
+# every tile that a whole product takes, a remainder of its rows and columns; K: parts of two, five and seventeen stages of 32, an odd
+# number of stages in all, an end inside a stage and inside a group of four
+@pytest.mark.parametrize("n,tile", [(131, (32, 32)), (2561, (64, 32)), (6148, (64, 64))])
+@pytest.mark.parametrize("k", [260, 1028, 8196])
+def test_whole_product_by_every_tile_has_the_bits_of_few_rows(ops, n, tile, k):
+    assert tile_of(301, n) == tile
+    x, w = rnd(301, k, seed=21), rnd(n, k, seed=22, scale=0.05)
+    whole = ops.linear(x, w)
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)   # as above
+    assert ((whole.double() - x.double() @ w.double().T).abs() <= bound).all()
+    for first, m in ((0, 1), (60, 9), (127, 32), (269, 32)):
+        assert torch.equal(ops.linear(x[first: first + m].contiguous(), w), whole[first: first + m]), (first, m)
+
+
 def test_product_of_many_rows_in_large_tiles(ops):
     x, w = rnd(4100, 36, seed=3), rnd(4097, 36, seed=4)   # 65 x 65 tiles of 64, the last of four rows and one column
     whole = ops.linear(x, w)
@@ -122,20 +136,6 @@ def test_product_for_the_residual_of_many_rows_comes_added_up(ops, m, n, k):
         assert ((whole[at].double() - x[at].double() @ w.double().T).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("seqs,nq,nkv,d,dv,ps,more", [
-    ([(1, 16), (1, 17), (1, 130)], 4, 2, 128, 128, 16, {}),                       # decoding: eight waves share the keys
-    ([(20, 33), (7, 7), (1, 1)], 5, 1, 48, 48, 4, {}),                            # a tile's 16 rows cut a token's heads
-    ([(300, 300), (160, 190)], 8, 8, 32, 16, 24, {}),                             # many tiles: four waves; values of another size
-    ([(40, 90)], 4, 2, 256, 256, 8, {"window": 9, "keep_first": 5, "sink": True}),
-    ([(1, 99), (33, 99)], 6, 2, 64, 80, 16, {"window": 40, "softcap": 5.0}),
-    ([(50, 75)], 4, 4, 16, 32, 12, {"chunk": 24, "gate": True}),
-])
-def test_attention_by_tiles(ops, seqs, nq, nkv, d, dv, ps, more):
-    more = dict(more)
-    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, ps, torch.float32, window=more.get("window"), poison=True)
-    if dv != d:
-        cache.v = rnd(cache.v.shape[0], nkv, dv, ps, seed=7)
-    if more.pop("gate", False):
 @pytest.mark.parametrize("k,planes", [(4, False), (256, True)])
 def test_product_of_more_rows_than_a_grid_has_tiles(k, planes):
     """65,535 rows of tiles of 64 are 4,194,240; the tiles beyond are in a launch of their own."""
@@ -154,6 +154,20 @@ def test_product_of_more_rows_than_a_grid_has_tiles(k, planes):
     close(got, x @ w.T, 1e-5 * math.sqrt(k), 1e-5)
 
 
+@pytest.mark.parametrize("seqs,nq,nkv,d,dv,ps,more", [
+    ([(1, 16), (1, 17), (1, 130)], 4, 2, 128, 128, 16, {}),                       # decoding: eight waves share the keys
+    ([(20, 33), (7, 7), (1, 1)], 5, 1, 48, 48, 4, {}),                            # a tile's 16 rows cut a token's heads
+    ([(300, 300), (160, 190)], 8, 8, 32, 16, 24, {}),                             # many tiles: four waves; values of another size
+    ([(40, 90)], 4, 2, 256, 256, 8, {"window": 9, "keep_first": 5, "sink": True}),
+    ([(1, 99), (33, 99)], 6, 2, 64, 80, 16, {"window": 40, "softcap": 5.0}),
+    ([(50, 75)], 4, 4, 16, 32, 12, {"chunk": 24, "gate": True}),
+])
+def test_attention_by_tiles(ops, seqs, nq, nkv, d, dv, ps, more):
+    more = dict(more)
+    q, cache, ctx = build_attention_case(seqs, nq, nkv, d, ps, torch.float32, window=more.get("window"), poison=True)
+    if dv != d:
+        cache.v = rnd(cache.v.shape[0], nkv, dv, ps, seed=7)
+    if more.pop("gate", False):
         more["gate"] = rnd(ctx.num_tokens, nq * dv, seed=9)
     window, scale = more.pop("window", None), 1.0 / math.sqrt(d)
     want = R.paged_attention(q.double(), cache.k, cache.v, ctx.cu_q.cpu(), ctx.kv_lens.cpu(), cache.group.block_table, ps,
