@@ -394,8 +394,11 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
 //   and 12.9, 13.6). One where K is a multiple of 2,048 (the rows of
 //   two tiles then start in the same memory channels: 14.0 us against 11.2 for the 8B q/k/v product)
 //   and for a few hundred tiles of long rows.
-//   K cut into planes: two tiles a block from K = 9,728 on, one up to 160 tiles of less than 12,288 columns (2,560 x 9,728 9.8, 10.2 and
-//   10.2, 10.8; 3,072 x 9,984 11.5, 12.0 and 11.4, 11.9; 4,096 x 12,288 17.4, 18.3 and 17.4, 17.7).
+//   K cut into planes: two tiles a block from K = 9,728 on, but one where that leaves the busiest compute unit fewer tiles, at most five
+//   of them. Tiles by 8 planes on the busiest of 256 units, one a block and two, and us at 10,240 columns (the same at 9,728 to 14,336):
+//   96 tiles 3 and 4, 7.4, 7.4 and 8.1, 8.0; 128 4 and 4, 8.8, 9.3 and 8.7, 8.9; 144 5 and 6, 10.2, 10.7 and 10.5, 11.1; 160 5 and 6, 10.7, 11.0
+//   and 10.8, 11.6; 164 6 and 6, 11.4, 12.5 and 11.5, 11.5; 192 6 and 6, 12.4, 13.3 and 12.4, 12.2; 224 7 and 8, 14.4, 16.1 and 14.9, 15.0;
+//   320 10 and 10, 19.4, 21.2 and 20.0, 20.7. At 16 rows level.
 // Up to 8 rows (FEW) the activations' unit is half as long: 0.1 to 0.3 us of a product, most where a block has one tile.
 template <int GATED, bool FEW>
 static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep, hipStream_t st,
@@ -407,7 +410,8 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
     return launch_rows<4, 2, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   } else {
     if (k_parts > 1) {
-      if (K >= 12288 || (K >= 9728 && tiles > 160)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
+      const int one = (tiles * k_parts + 255) / 256, two = 2 * (((tiles + 1) / 2 * k_parts + 255) / 256);
+      if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
       return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
     }
     if (K % 2048 == 0) {

@@ -120,6 +120,20 @@ def test_few_rows_at_the_edges_of_their_tiles(ops, m, n):
     assert ((ops.linear(x, w, out_f32=True).double() - want).abs() <= bound).all()
 
 
+# K in eight planes: 128 and 129, 160 and 161 tiles of 16 and a remainder (a block has two, one, one, two), at the shortest K of the rule and
+# in front of it; a part of the pairs of k-steps that is no multiple of the waves
+@pytest.mark.parametrize("n", [2048, 2049, 2560, 2561])
+@pytest.mark.parametrize("k", [9664, 9728, 12352])
+def test_few_rows_in_planes_at_the_edges_of_their_tiles(ops, n, k):
+    x, w = rnd(9, k, dtype=torch.bfloat16, seed=7), rnd(n, k, dtype=torch.bfloat16, seed=8, scale=k ** -0.5)
+    for m in (1, 8, 9):
+        planes = ops.linear_for_residual(x[:m], w)
+        assert planes.shape == (8, m, n)
+        # float32 sums of k products, as above
+        bound = k * 2.0 ** -24 * (x[:m].double().abs() @ w.double().abs().T)
+        assert ((planes.double().sum(0) - x[:m].double() @ w.double().T).abs() <= bound).all()
+
+
 # tiles of eight gate and eight up rows or one of either: rows of K up to 4,096 and beyond, on both sides of 2 and 8 rows
 @pytest.mark.parametrize("activation,limit", [("swiglu", 0.0), ("clamped", 0.9)])
 @pytest.mark.parametrize("inter,k", [(8, 64), (20, 4096), (36, 4160)])
