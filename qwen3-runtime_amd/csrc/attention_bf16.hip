@@ -146,6 +146,7 @@ constexpr int D = QRT_HEAD_DIM;      // of queries and keys
 constexpr int DV = QRT_VALUE_DIM;    // of values and outputs
 constexpr int DMAX = D > DV ? D : DV;
 constexpr int KFULL = D / 32;        // 32-wide steps of the first product
+constexpr bool WIDE_QUERIES = KFULL > 10;  // queries that leave the registers, see Q_IN_LDS
 constexpr bool KTAIL = (D % 32) != 0;  // one 16-wide step more
 constexpr int DB = DV / 16;          // 16-wide blocks of a value
 
@@ -447,7 +448,7 @@ __device__ __forceinline__ void kept_keys_pass(const AttnTileArgs& a, const int*
                                                const Q& q_of, const bf16x8_t* qtail,
                                                float* m, float* l, f32x4_t (*o)[DB]) {
   for (int base = 0; base < kend; base += 32) {
-    if (KFULL > 8) asm volatile("" ::: "memory");  // queries that lie in LDS are read for every block
+    if (WIDE_QUERIES) asm volatile("" ::: "memory");  // queries that lie in LDS are read for every block
     int pg[3];
     KvBlock blk;
     block_pages<P2>(table, base, 0, kend - 1, a.page_size, r16, quad, pg);
@@ -492,13 +493,14 @@ __device__ __forceinline__ void add_sink(float& m, float& l_total, f32x4_t* o) {
 // four waves, 64 * RT rows. The keys and values of a block of 32 keys are read
 // once into registers and multiplied with all RT tiles, which divides the
 // operand traffic per MFMA by RT.
-// Heads wider than 256 leave no registers for the queries beside the accumulator, a block of keys and values and their
-// addresses. Spilled, they were loaded one 16 bytes at a time, 14 round trips of memory in a row for a head of 448, and came back out
-// of scratch memory for every block; now they lie in LDS, a place of its own for every lane, and the loop spills nothing. One token each of
+// Heads of 352 and wider (WIDE_QUERIES) leave no registers for the queries beside the accumulator, a block of keys and values and their
+// addresses (320 spills 2 of them, and reads its queries out of LDS no faster: 32 sequences of 2,000 keys 32.4 us, 33.6 so; 448 spills
+// 128, 72 so). Spilled, they were loaded one 16 bytes at a time, 14 round trips of memory in a row for a head of 448, and came back out
+// of scratch memory for every block; now they lie in LDS, a place of its own for every lane. One token each of
 // 8 sequences of 1,029 keys, 32 heads of 448 on one, us with the merge 24.1 -> 20.6; of 300 keys 19.5 -> 16.3; of 4,000
 // 39.0 -> 30.0; 32 sequences of 1,029 41.7 -> 32.3. (The first block's page numbers asked for ahead of the queries: 0.5 to 1.5 slower.)
 template <int RT>
-constexpr bool Q_IN_LDS = RT == 1 && KFULL > 8;
+constexpr bool Q_IN_LDS = RT == 1 && WIDE_QUERIES;
 
 template <int RT, bool P2>
 // (Heads wider than 256: a wave's accumulator, queries and one block of keys and values fill most of
@@ -1935,8 +1937,6 @@ extern "C" int qrt_attention_work_list(const AttnTileArgs* args, int fused, hipS
   return 0;
 }
 
-// every listed sequence at most 16 rows (q_len * g <= 16) and D <= 256; num_tiles = number of
-// sequences; tile_seq lists them, or is null for all sequences of the step in order
 // Heads of 64 and 128: by the ring, but where blocks that have a compute unit to themselves for long are what the launch waits for:
 // their waves have one block of keys on the way by the ring and two by the loads to registers. Heads of 64 (half the bytes a
 // block): at most one block to a unit, and more than 256 keys to walk for each unit. Heads of 128: two blocks fit a unit, so up to 512 are
@@ -1977,6 +1977,8 @@ static int decode_by_kernel(const AttnTileArgs& a, hipStream_t stream) {
   return p2 ? decode_launch<true, FUSED, false>(a, stream) : decode_launch<false, FUSED, false>(a, stream);
 }
 
+// every listed sequence at most 16 rows (q_len * g <= 16) and D <= 256; num_tiles = number of
+// sequences; tile_seq lists them, or is null for all sequences of the step in order
 extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_total, hipStream_t stream) {
   AttnTileArgs a = *args;
   QRT_CHECK(a.nq > 0 && a.nkv > 0 && a.nq % a.nkv == 0, "attention: %d query heads do not divide into %d key heads",
