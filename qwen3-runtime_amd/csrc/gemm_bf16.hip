@@ -385,9 +385,12 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
 // flight) on the shapes of the 4B, 8B and 32B models at 1 and 8 rows, each on the weight
 // matrices of 36 layers in turn: four waves everywhere (several small blocks on a compute unit
 // hide each other's ends better than one large one). us at 1 and 8 rows, by one tile a block and by two:
-//   Gated, three pairs in flight: 4B 17.3, 18.5 by tiles of eight gate and eight up rows, 18.7, 19.2 by a tile of either (5.8 and
-//   5.3 TB/s); 8B 31.3, 31.6 and 32.6, 32.3; 2,048 x 6,144 10.3, 10.5 and 11.2, 11.7; 32B 76.8, 84.2 and 79.4, 81.5, so long rows
-//   of more than two keep a tile of either; at 10 rows level.
+//   Gated, three pairs in flight, up to 8 rows: tiles of eight gate and eight up rows where they leave the busiest of 256 units less than
+//   blocks of a tile of either do, counted in such tiles; at 10 rows level. us at 1 and 8 rows for K = 2,560 (the same picture at 1,024 to
+//   9,728): 2,048 gate rows, 1 against 2, 6.1, 6.3 and 7.1, 7.8; 2,560, 2 against 2, 8.0, 8.7 and 7.8, 7.9; 4,096, 2 against 2, 9.6, 9.7 and 9.5, 9.4;
+//   4,864, 3 against 4, 11.7, 12.1 and 12.9, 13.3; 6,656, 4 against 4, 14.7, 15.2 and 14.4, 14.3; 9,728, 5 against 6, 18.6, 18.9 and 20.2, 19.7
+//   (5.4 and 4.9 TB/s); 12,288, 6 against 6, 22.5, 22.9 and 22.7, 21.8. Beyond five long rows of more than two keep a tile of either: 25,600 x
+//   5,120, 13 against 14, 81.2, 84.2 and 83.4, 81.5.
 //   The whole result: two tiles a block from 384 tiles on where K is up to 4,096 columns, except between 512 and 768 tiles, whose blocks of two fill
 //   the compute units a little more than once (9,728 x 2,560 10.5, 11.5 and 12.0, 12.8; 12,288 11.5, 12.2 and 12.8, 13.5; at 16 rows
 //   13.6 and 14.1), and up to 4 rows below (6,144 x 2,560 at 1, 4 and 8 rows 7.2, 7.45, 8.1 and 7.35, 7.45, 7.7; 13,312 13.6, 14.7
@@ -405,8 +408,10 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
                     int k_parts) {
   const int tiles = (N + 15) / 16;
   if constexpr (GATED) {
+    // half tiles that the busiest of 256 compute units gets by blocks of eight and eight rows, and by blocks of a tile of either
+    const int mixed = ((N + 7) / 8 + 255) / 256, either = 2 * ((tiles + 255) / 256);
     if constexpr (FEW)
-      if (K <= 4096 || M <= 2) return launch_rows<4, 1, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+      if (mixed < either && (mixed <= 5 || K <= 4096 || M <= 2)) return launch_rows<4, 1, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
     return launch_rows<4, 2, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   } else {
     if (k_parts > 1) {
