@@ -218,7 +218,7 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
     int vp = table[min(vj, hi) / ps];
     there = vj <= hi && vp >= 0;
     vp = there ? vp : last_page;
-    return vc + ((size_t)vp * a.nkv + kvh) * Dv * ps + (there ? vj % ps : 0) + (size_t)r * ps;
+    return vc + ((size_t)vp * a.nkv + kvh) * Dv * ps + (there ? vj % ps : 0) + (FULL ? (size_t)r * ps : 0);
   };
   struct Block { f32x4_t k[ND], v[ND]; bool v_there; };
   auto load = [&](int b, Block& blk) {
@@ -236,9 +236,13 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
   if (FULL && b <= last_block) load(b, now);
   while (b <= last_block) {
     const int j0 = 16 * b, vj = j0 + 4 * q, b_next = after(b);
-    const float* kr = nullptr;
-    if (FULL) load(min(b_next, last_block), next);  // behind the wave's last block: one that nobody needs
-    else kr = key_row(b);
+    const float *kr = nullptr, *vr = nullptr;
+    if (FULL) {
+      load(min(b_next, last_block), next);  // behind the wave's last block: one that nobody needs
+    } else {  // the block's page numbers together: one round trip
+      kr = key_row(b);
+      vr = value_row(b, now.v_there);
+    }
     f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < ND; ++j)
@@ -271,11 +275,10 @@ __global__ __launch_bounds__(64 * W) void attention_f32_tile_kernel(AttnArgs a) 
       sc[e] = seen[e] ? expf(sc[e] - m) : 0.f;
       l += sc[e];
     }
-    const float* vr = FULL ? nullptr : value_row(b, now.v_there);
 #pragma unroll
     for (int j = 0; j < ND; ++j)
       if (FULL || j < nv) {
-        const f32x4_t vv = FULL ? now.v[j] : *(const f32x4_t*)(vr + (size_t)(16 * j) * ps);
+        const f32x4_t vv = FULL ? now.v[j] : *(const f32x4_t*)(vr + (size_t)(16 * j + r) * ps);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float value = (now.v_there && vj + e <= hi) ? vv[e] : 0.f;  // never written: not a number, perhaps
