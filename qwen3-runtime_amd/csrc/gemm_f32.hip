@@ -382,7 +382,7 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // 64 x 64). 128 x 128 where that makes four rounds and more, one block to a unit (its two stages are 80 KB of LDS): 6 % less work a
 // round, but a round is four times as long. By 64 x 64 and 128 x 128, us: 2,560 x 4,096 at 8,192 rows 1,506 and 1,434, 2,560 x 9,728 3,557 and
 // 3,385, 6,144 x 2,560 at 4,096 1,141 and 1,103, 5,120 x 8,192 3,002 and 2,863; 19,456 x 2,560 at 2,048 (9.5 rounds) 1,799 and 1,831, at
-// 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854.
+// 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854. Up to 128 rows they read the weights once: 151,936 x 1,024 at 96 rows 428 and 394.
 static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
   return std::max(rounds * 100, (long)least) * round;
@@ -411,7 +411,7 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
   }
   const long c64 = f32_cost_64x64(M, N, groups), c32 = f32_cost_64x32(M, N, groups), c16 = f32_cost_32x32(M, N, groups);
   if constexpr (FORM != F32_PLANES)
-    if (f32_cost_128x128(M, N) < c64) {
+    if (f32_cost_128x128(M, N) < (M <= 128 ? LONG_MAX : c64)) {
       f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
       return 0;
     }
