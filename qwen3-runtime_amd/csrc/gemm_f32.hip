@@ -14,7 +14,7 @@
 //   of fused multiply-adds per output, as every product had before: 64 x 64 outputs a block, one block per
 //   64 weight rows however few the rows of A.
 //
-// Either MFMA kernel may leave a product for the residual in four planes, the sums of groups of neighbouring parts, or (tiles) add
+// Either MFMA kernel may leave a product for the residual in four planes, the sums of groups of neighbouring parts, or add
 // those up itself.
 // Error against float64, relative: 3.3e-7 (K 2,560), 4.5e-7 (9,728); the sequential sums': 9.0e-7 and 1.8e-6.
 #include "common.h"
@@ -103,7 +103,7 @@ __device__ __forceinline__ f32x4_t load_f32x4_below(const float* __restrict__ ro
 // 6.4 TB/s), and at 16 rows 17, 12, 40, 28 instead of 29, 18, 71, 51.
 template <int MB, int PARTS, int U, bool FEW, int GATED>
 __global__ __launch_bounds__(64 * PARTS) void gemm_f32_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                                   float* __restrict__ C, int M, int N, int K, int part_len, float limit) {
+                                                                   float* __restrict__ C, int M, int N, int K, int part_len, float limit, bool by_groups) {
   constexpr int SLOT = (1 + MB) * 2048 - (FEW ? 1024 : 0), LOADS = 2 + (FEW ? 1 : 2 * MB);
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
   static_assert(!FEW || MB == 1, "up to 8 rows are one block of rows");
@@ -184,6 +184,18 @@ __global__ __launch_bounds__(64 * PARTS) void gemm_f32_rows_kernel(const float* 
   for (int b = 0; b < MB; ++b) sums[(wave * MB + b) * 64 + lane] = acc[b];
   __syncthreads();
   auto total = [&](int i) {
+    if (PARTS >= 2 * F32_GROUPS && by_groups) {  // the whole sum as a reader of the planes adds it
+      constexpr int EACH = PARTS >= 2 * F32_GROUPS ? PARTS / F32_GROUPS : 1;
+      f32x4_t s;
+#pragma unroll
+      for (int g = 0; g < F32_GROUPS; ++g) {
+        f32x4_t of_group = sums[i + g * EACH * MB * 64];
+#pragma unroll
+        for (int p = 1; p < EACH; ++p) of_group += sums[i + (g * EACH + p) * MB * 64];
+        s = g ? s + of_group : of_group;
+      }
+      return s;
+    }
     f32x4_t s = sums[i];
 #pragma unroll
     for (int p = 1; p < PARTS; ++p) s += sums[p * MB * 64 + i];
@@ -336,7 +348,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
 
 // A block's waves: all parts of K, or those of one group (gridDim.y of them, each a plane of the result).
 template <int MB, int PARTS, int U, bool FEW, int GATED>
-static int f32_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, int groups = 1) {
+static int f32_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, bool by_groups, int groups = 1) {
   constexpr size_t smem = (size_t)PARTS * U * ((1 + MB) * 2048 - (FEW ? 1024 : 0));  // the parts' sums fit in it
   static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
   auto kernel = gemm_f32_rows_kernel<MB, PARTS, U, FEW, GATED>;
@@ -346,32 +358,32 @@ static int f32_rows(const float* a, const float* w, float* c, int M, int N, int 
       return qrt_fail("gemm_f32: cannot get %zu bytes of LDS", smem);
     allowed = true;
   }
-  kernel<<<dim3(GATED ? (N + 7) / 8 : (N + 15) / 16, groups), 64 * PARTS, smem, stream>>>(a, w, c, M, N, K, f32_part_len(K, PARTS * groups), limit);
+  kernel<<<dim3(GATED ? (N + 7) / 8 : (N + 15) / 16, groups), 64 * PARTS, smem, stream>>>(a, w, c, M, N, K, f32_part_len(K, PARTS * groups), limit, by_groups);
   return 0;
 }
 template <int MB, bool FEW, int GATED>
-static int f32_rows_parts(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream) {
+static int f32_rows_parts(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, bool by_groups) {
   constexpr int MANY = MB > 1 ? 1 : 2;  // sixteen rings and their slots have to fit LDS
   switch (f32_parts(K)) {
-    case 16: return f32_rows<MB, 16, MANY, FEW, GATED>(a, w, c, M, N, K, limit, stream);
-    case 8: return f32_rows<MB, 8, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
-    case 4: return f32_rows<MB, 4, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
-    case 2: return f32_rows<MB, 2, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
-    default: return f32_rows<MB, 1, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream);
+    case 16: return f32_rows<MB, 16, MANY, FEW, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+    case 8: return f32_rows<MB, 8, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+    case 4: return f32_rows<MB, 4, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+    case 2: return f32_rows<MB, 2, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+    default: return f32_rows<MB, 1, 2, FEW, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
   }
 }
 template <int MB, bool FEW>
 static int f32_rows_planes(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
-  return f32_parts(K) == 16 ? f32_rows<MB, 4, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, F32_GROUPS)
-                            : f32_rows<MB, 2, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, F32_GROUPS);
+  return f32_parts(K) == 16 ? f32_rows<MB, 4, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, false, F32_GROUPS)
+                            : f32_rows<MB, 2, 2, FEW, 0>(a, w, c, M, N, K, 0.f, stream, false, F32_GROUPS);
 }
 template <int GATED>
-static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream) {
+static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, bool by_groups = false) {
   if constexpr (!GATED)
-    if (M > 32) return f32_rows_parts<4, false, 0>(a, w, c, M, N, K, limit, stream);
-  if (M <= 8) return f32_rows_parts<1, true, GATED>(a, w, c, M, N, K, limit, stream);
-  if (M <= 16) return f32_rows_parts<1, false, GATED>(a, w, c, M, N, K, limit, stream);
-  return f32_rows_parts<2, false, GATED>(a, w, c, M, N, K, limit, stream);
+    if (M > 32) return f32_rows_parts<4, false, 0>(a, w, c, M, N, K, limit, stream, by_groups);
+  if (M <= 8) return f32_rows_parts<1, true, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+  if (M <= 16) return f32_rows_parts<1, false, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
+  return f32_rows_parts<2, false, GATED>(a, w, c, M, N, K, limit, stream, by_groups);
 }
 
 // Which tile: the fewest rounds of blocks over the 256 compute units times what a round takes, us for 32 k: a unit's blocks
@@ -382,7 +394,7 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // 64 x 64). 128 x 128 where that makes four rounds and more, one block to a unit (its two stages are 80 KB of LDS): 6 % less work a
 // round, but a round is four times as long. By 64 x 64 and 128 x 128, us: 2,560 x 4,096 at 8,192 rows 1,506 and 1,434, 2,560 x 9,728 3,557 and
 // 3,385, 6,144 x 2,560 at 4,096 1,141 and 1,103, 5,120 x 8,192 3,002 and 2,863; 19,456 x 2,560 at 2,048 (9.5 rounds) 1,799 and 1,831, at
-// 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854. Up to 128 rows they read the weights once: 151,936 x 1,024 at 96 rows 428 and 394.
+// 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854. From 65 to 128 rows they read the weights once: 151,936 x 1,024 at 96 rows 428 and 394.
 static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
   return std::max(rounds * 100, (long)least) * round;
@@ -411,7 +423,7 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
   }
   const long c64 = f32_cost_64x64(M, N, groups), c32 = f32_cost_64x32(M, N, groups), c16 = f32_cost_32x32(M, N, groups);
   if constexpr (FORM != F32_PLANES)
-    if (f32_cost_128x128(M, N) < (M <= 128 ? LONG_MAX : c64)) {
+    if (f32_cost_128x128(M, N) < (M > 64 && M <= 128 ? LONG_MAX : c64)) {
       f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
       return 0;
     }
@@ -445,20 +457,23 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
 // fills the chip where the weight has few rows. Up to 32 rows as a stream (4B output and down projections at 1, 16, 32 rows 9.5, 10.4,
 // 14.7 and 18.1, 22.9, 31.5 us; all parts in a block 9.7, 12.3, 17.2 and 19.9, 28.1, 40.6), beyond by tiles.
 //
-// How many planes: three more of them are written and read, 150 / K of the product's time, so from a round of 64 x 64 tiles on they have to
-// save more than that in part-filled rounds.
+// How many planes. By tiles three more of them are written and read, 150 / K of the product's time, so from a round of 64 x 64 tiles on
+// they have to save more than that in part-filled rounds. As a stream: where 16 weight rows a block leave compute units idle, under
+// 4,096 rows (product and norm, us at 1, 8 and 32 rows, whole and by planes: 2,560 x 4,096 14.4, 14.1, 20.7 and 14.0, 13.9, 19.6; 4,096 x 4,096
+// 17.1, 17.5, 22.4 and 17.5, 18.3, 23.9; 8,192 x 4,096 32.0, 32.3, 47.0 and 35.4, 36.2, 55.8; 8,192 x 256 9.0, 9.5, 12.3 and 11.2, 12.3, 16.9).
 extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
-  if (M <= 32 || N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
+  if (M <= 32) return N < 4096 ? F32_GROUPS : 1;
+  if (N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
   const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS), f32_cost_64x32(M, N, F32_GROUPS), f32_cost_32x32(M, N, F32_GROUPS)}) / F32_GROUPS;
   if (M > 65535 * 64) return 1;  // two calls
   return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1), f32_cost_128x128(M, N)) ? F32_GROUPS : 1;
 }
 extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, int planes, hipStream_t stream) {
   QRT_CHECK(M >= 0 && N > 0 && K >= 256 && K % 4 == 0, "gemm_f32_planes: bad sizes M=%d N=%d K=%d", M, N, K);
-  QRT_CHECK(planes == F32_GROUPS || (planes == 1 && M > 32), "gemm_f32_planes: %d planes of %d rows", planes, M);
+  QRT_CHECK(planes == F32_GROUPS || planes == 1, "gemm_f32_planes: %d planes", planes);
   QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) % 16 == 0, "gemm_f32_planes: operands are read 16 bytes at a time");
   if (M == 0) return 0;
-  if (const int rc = planes == 1 ? f32_tiles<F32_GROUPS_SUM>(a, w, c, M, N, K, stream)
+  if (const int rc = planes == 1 ? (M <= 32 ? f32_few_rows<0>(a, w, c, M, N, K, 0.f, stream, true) : f32_tiles<F32_GROUPS_SUM>(a, w, c, M, N, K, stream))
                      : M <= 8    ? f32_rows_planes<1, true>(a, w, c, M, N, K, stream)
                      : M <= 16   ? f32_rows_planes<1, false>(a, w, c, M, N, K, stream)
                      : M <= 32   ? f32_rows_planes<2, false>(a, w, c, M, N, K, stream)

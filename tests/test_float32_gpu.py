@@ -68,7 +68,7 @@ def tile_of(m, n, groups=1):
     """The tile that the launch takes by its model of the time (in multiples of a hundredth of a round's)."""
     tiles, cost = -(-m // 128) * -(-n // 128), {}
     if groups == 1 and tiles >= 1024:
-        cost[128, 128] = 0 if m <= 128 else 100 * -(-tiles // 256) * 2324   # up to 128 rows: one row of tiles
+        cost[128, 128] = 0 if 64 < m <= 128 else 100 * -(-tiles // 256) * 2324   # one row of tiles
     for (tm, tn), (round_time, least) in {(64, 64): (606, 130), (64, 32): (329, 180), (32, 32): (190, 250)}.items():
         rounds = -(-(-(-m // tm) * -(-n // tn) * groups) // 256)
         cost[tm, tn] = max(100 * rounds, least) * round_time
@@ -113,7 +113,7 @@ def test_product_of_many_rows_in_tiles_of_128(ops, m, n, k):
 # 64 x 64 and 128 x 128, remainders of rows and columns; K: groups of two parts of two stages, the third of one part and the fourth of none;
 # of two parts of five; of four of seventeen
 @pytest.mark.parametrize("m,n,k", [(2049, 2563, 260), (1281, 5123, 1028), (3969, 4070, 1028), (4090, 4096, 8196)])
-def test_product_for_the_residual_of_many_rows_comes_added_up(ops, m, n, k):
+def test_product_for_the_residual_of_many_rows_or_few_of_a_tall_weight_comes_added_up(ops, m, n, k):
     """One matrix in place of four planes, with the bits of the planes' sum, so that a row's stream and norm do not go by the number of rows."""
     from qwen3_runtime_amd.ops.hip import HipOps
 
@@ -124,11 +124,11 @@ def test_product_for_the_residual_of_many_rows_comes_added_up(ops, m, n, k):
     res, weight = rnd(m, n, seed=13), torch.ones(n, device=DEV)
     stream = res.clone()
     normed = ops.add_rmsnorm(stream, whole, weight, 1e-6, torch.float32)
-    for first, rows in ((0, 1), (63, 9), (130, 33), (m - 200, 200)):
+    for first, rows in ((0, 1), (63, 9), (300, 17), (400, 32), (130, 33), (m - 200, 200)):
         at = slice(first, first + rows)
         few = planes.linear_for_residual(x[at].contiguous(), w)
-        assert few.shape == (4, rows, n)
-        assert torch.equal(((few[0] + few[1]) + few[2]) + few[3], whole[at]), (first, rows)
+        assert few.shape == ((rows, n) if n >= 4096 and rows <= 32 else (4, rows, n))   # few rows: by the weight's
+        assert torch.equal(few if few.dim() == 2 else ((few[0] + few[1]) + few[2]) + few[3], whole[at]), (first, rows)
         part = res[at].clone()
         assert torch.equal(ops.add_rmsnorm(part, few, weight, 1e-6, torch.float32), normed[at])
         assert torch.equal(part, stream[at])
