@@ -162,7 +162,8 @@ __device__ __forceinline__ float gate_factor(const bf16_t* __restrict__ gate, lo
 // sum (`inv`) and times the sigmoid of its gate. The gate's elements of eight blocks are asked for before the first is used, four in a
 // load where they line up. Asked for one by one, under a branch each, the 64 loads of a wave's two rows followed one another:
 // three prompts of 301, 589 and 1,151 tokens, 32 heads of 128 on 8, capped scores, took 49 us without a gate and 88 with one,
-// 53 now; one prompt of 2,041 65 and 95, 70 now.
+// 53 now; one prompt of 2,041 65 and 95, 70 now. Heads of 256, whose kernel spills either way, pay for it where there is no gate: a prompt of
+// 300 tokens, 16 heads on 4, 101 -> 79 with a gate and 72 -> 76 without.
 __device__ __forceinline__ void store_row(const AttnTileArgs& a, size_t row, int quad, float inv, const f32x4_t* o) {
   bf16_t* out = a.out + row * DV + 4 * quad;
   if (!a.gate) {
@@ -1421,9 +1422,10 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_o, const f
 // Tiles of at most 16 rows (a decoded token's g query heads, or a very short
 // portion): one block of DW waves per (tile, key head, split). The waves take the
 // block's 32-key blocks round-robin, each with its own running maximum, sum and
-// accumulator; the keys and values of the next two blocks are on their way while
-// one is multiplied, and page numbers are fetched two blocks further ahead, so that
-// no load waits for another. The waves' results meet in LDS. With several splits each
+// accumulator. Keys and values come by loads to registers, those of the next two blocks on their way while
+// one is multiplied and page numbers fetched two blocks further ahead, or (RING: heads of 64 and 128 in
+// most launches, decode_by_ring) by direct loads to LDS, the next block's on its way and page numbers 16 blocks
+// at a time. No load waits for another. The waves' results meet in LDS. With several splits each
 // block writes its normalised part and the base-2 log of its sum, and a second
 // small kernel merges them. (Merging in the block that arrives last at a counter
 // needs a device-scope fence in every block; with one L2 per XCD that fence costs
@@ -1449,8 +1451,8 @@ __device__ __forceinline__ void decode_key_blocks(int kv_len, int q_len, int win
 }
 
 // Blocks of keys in the pieces of a sequence of `blocks`: as few pieces as have at most `most` each, of one length (a last
-// piece of a few keys costs a block's start like any other: 16 sequences of 290 to 2,600 keys, at most 512 a piece, 29.8 us
-// with whole pieces and rests, 27.5 so; 48 of 136 to 2,606, at most 1,024, 47.4 and 45.4).
+// piece of a few keys costs a block's start like any other: with keys by loads to registers 16 sequences of 290 to 2,600, at most 512
+// a piece, 29.8 us with whole pieces and rests, 27.5 so; 48 of 136 to 2,606, at most 1,024, 47.4 and 45.4).
 __device__ __forceinline__ int piece_blocks(int blocks, int most) {
   const int pieces = max(1, (blocks + most - 1) / most);
   return max(1, (blocks + pieces - 1) / pieces);
@@ -1459,10 +1461,12 @@ __device__ __forceinline__ int piece_blocks(int blocks, int most) {
 // The work list of a decode launch in pieces (AttnTileArgs::items). One block; up to LIST_TILES
 // sequences. Every sequence has at least one piece (its last piece also takes the token's own key
 // in the fused form), at most ceil(blocks / split_blocks). Sequences with long pieces come first.
-// Which length: the least of 5 us for every round of blocks (two to each of 256 compute units), of what the longest piece
-// takes times the blocks of the busiest unit (0.6 us for 100 keys of 512 bytes), and of the merge of more than four parts. On 15 sets
-// of 3 to 64 sequences of 60 to 16,000 keys, timed at every multiple of 32 from 128 to 512 and ten lengths beyond, it takes 1.2 %
-// more than the best on average, 5 % at worst; one length for some 1,536 blocks took 13 and 36 %.
+// Which length: the least sum of a weight for every round of blocks (two to each of 256 compute units), of the longest piece times
+// the blocks of the busiest unit, and of the merge of more than four parts. The weights tell lengths apart and are no account of the
+// time, which they give too low: they were fitted with keys by loads to registers. With the ring, on 16 sets of 6 to 64 sequences of 20 to
+// 16,000 keys, seven of them not used for the fit, each timed at 16 lengths from the shortest to six times it, the length taken costs 0.6 %
+// more than the best on average, 4.5 % at worst (48 sequences of 136 to 2,606 keys: 36 blocks, 38.7 us; the best 31, 38.6). The launch is
+// sized for the shortest length, and its blocks without a piece cost another 3 %, 10 at worst.
 constexpr int LIST_TILES = 1024, LIST_LENGTHS = 32;
 __global__ __launch_bounds__(8 * LIST_LENGTHS) void attention_work_list_kernel(AttnTileArgs a, int fused) {
   __shared__ int whole[LIST_TILES + 1], rest[LIST_TILES + 1];  // pieces of each tile, then where they begin
@@ -1612,9 +1616,9 @@ __device__ __forceinline__ void head_as_operand(const bf16_t* __restrict__ x, co
 // c ^ (r, or r / 2 where a row is half of the banks), so that the operand reads touch every bank once. Values: element d is
 // a row of 64 bytes, its four groups of eight keys at g ^ (d / 4) % 4. Every load is of 16 bytes a lane, from anywhere: four
 // keys, or sixteen elements of two pages of 16 keys, an instruction. As loads straight to registers the keys came as sixteen half
-// lines an instruction, and two blocks on their way took 128 registers: attention and merge, us, before and now, 8 sequences of 2,054 keys with 32 heads of 128
-// on 8 22.0 and 20.9 in 4 parts, 23.4 and 20.1 in 8; 24 of 800 25.5 and 22.2; 64 of 1,024 53.1 and 51.3; 48 of 136 to 2,606 46.5 and 41.3; 64 of 200 to
-// 8,000 117 and 105. Waiting for keys and values apart, so that either is on its way a little longer, is level (20.9, 21.1).
+// lines an instruction, and two blocks on their way took 128 registers: attention and merge, us, by registers and by the ring, 32 heads of 128 on
+// 8: 40 sequences of 300 keys 17.8 and 16.4; 20 of 1,030 in 3 parts 23.2 and 22.5; 56 of 1,030 44.5 and 42.5; in pieces 48 of 136 to 2,606 46.5
+// and 41.3, 64 of 200 to 8,000 117 and 105; where it loses, decode_by_ring. Waiting for keys and values apart, so that either is on its way a little longer, is level (20.9, 21.1).
 constexpr bool DECODE_RING = D % 64 == 0 && DMAX <= 128;
 constexpr int RING_KEYS = 64 * D, RING_WAVE = RING_KEYS + 64 * DV;  // bytes
 
@@ -1625,7 +1629,8 @@ __device__ __forceinline__ int ring_pages(const int* __restrict__ table, int fir
   const int base = min(first + (lane >> 2) * step, last) << 5;
   return table[page_div<P2>(min(max(base + 8 * (lane & 3), lo & ~7), pos_max & ~7), ps, __builtin_ctz(ps))];
 }
-// Groups that lie outside [lo, pos_max] are read as its first or last one, as block_load does, and masked or zeroed likewise.
+// Groups of eight keys that lie outside [lo, pos_max] are read as its first or last group, whole (block_load clamps key by key): what that
+// brings of other positions is masked or zeroed as there, and lies in the same pages.
 template <bool P2>
 __device__ __forceinline__ void ring_fetch(const AttnTileArgs& a, int kvh, int base, int lo, int pos_max, int pages, int i, int lane,
                                            unsigned char* ring) {

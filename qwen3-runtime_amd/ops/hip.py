@@ -1962,15 +1962,15 @@ class HipOps:
         return n >= 2 and longest * n > self.decode_piece_ratio * total and (longest >= 2048 or (longest >= 768 and total >= 8192))
 
     def choose_decode_piece(self, kv_lens, nkv: int):
-        """Keys per piece for such a launch (a multiple of 32), or None. Equal parts of every
+        """For such a launch the length that bounds its pieces (keys, a multiple of 32), else None: the list's kernel takes
+        one from ``shortest_decode_piece`` on. Equal parts of every
         sequence make blocks whose work is the sequence's length: with 56 sequences of 300 keys
         and 8 of 8,000 the launch takes 231 us where the two kinds alone take 18 and 48, and more
         parts do not help, because the blocks reach the compute units in launch order, round
-        robin, and heavy blocks a fixed stride apart land on the same few. Pieces of one length,
-        whole ones first in the list: about 1,536 blocks in all, no piece under 512 keys (a block
-        costs some 8 us before its first key arrives) and no sequence in more than 32 (the merge
-        reads every piece's part, up to 64 with all its loads in flight at once: 8 sequences of
-        1,000 to 30,000 keys 91 us in pieces of 1,024, 96 in pieces of 512, 126 in pieces of 4,096)."""
+        robin, and heavy blocks a fixed stride apart land on the same few. Pieces of one length within a sequence, long
+        ones first in the list: this length makes about 1,536 blocks, is 512 keys or more and cuts no sequence into more than
+        32 (the merge reads every piece's part, up to 64 with all its loads in flight at once; with keys by loads to registers 8
+        sequences of 1,000 to 30,000 keys 91 us in pieces of 1,024, 96 in pieces of 512, 126 in pieces of 4,096)."""
         if not self.decode_in_pieces(kv_lens):
             return None
         piece = max(512, -(-sum(kv_lens) * nkv // 1536), -(-max(kv_lens) // 32))
@@ -1980,9 +1980,10 @@ class HipOps:
     def shortest_decode_piece(kv_lens, piece: int) -> int:
         """The shortest piece that the work list's kernel may take in place of ``piece`` (the longest is six times that): it
         looks for the length whose blocks fill the compute units in whole rounds, by the lengths as they are when it
-        runs. No sequence in more than 32. With heads of 128 on 8 key heads, by ``piece`` alone (a sequence's last one shorter)
-        and now, us with the merge: 48 sequences of 136 to 2,606 keys 51.0 and 45.2, 40 to 1,200 37.4 (in equal parts) and 27.7, 16 to 2,600
-        29.9 and 24.8, 64 of 100 to 4,000 128 and 113, 8 of 1,000 to 16,000 46.4 and 44.6."""
+        runs. No sequence in more than 32 at its length now. With heads of 128 on 8 key heads and the ring, lengths in equal ratios, by ``piece``
+        alone (a sequence's last one shorter) and now, us with the merge: 48 sequences of 136 to 2,606 keys 43.2 and 39.1, of 40 to 1,200
+        30.8 (in equal parts) and 23.3, 64 of 100 to 4,000 63.4 and 61.9, 8 of 1,000 to 16,000 42.4 and 41.0, 64 of 200 to 8,000 109.5 and
+        106.1. Where ``piece`` is 512 the parts' scratch is for pieces of 256: 48 sequences of up to 4,096 keys 12.6 MB."""
         return max(piece if piece > 512 else 256, -(-max(kv_lens) // 1024) * 32)
 
     # mixed steps: sequences with few rows leave the prompt kernel when their context is this long

@@ -964,7 +964,7 @@ def test_the_list_takes_a_piece_length_by_the_lengths_on_the_device(ops, lens, n
 
 
 def test_which_decode_launches_go_in_pieces(ops):
-    """Equal lengths keep equal parts; very unequal ones get pieces of at least 512 keys, at most 32
+    """Equal lengths keep equal parts; for very unequal ones the length that bounds the pieces is at least 512 keys, at most 32
     for the longest sequence, about 1,536 blocks in all."""
     assert not ops.decode_in_pieces([2100] * 64) and not ops.decode_in_pieces([2048]) and not ops.decode_in_pieces([1900, 100])
     assert not ops.decode_in_pieces([2000, 3000, 2500, 2600])
