@@ -1423,8 +1423,8 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_o, const f
 // portion): one block of DW waves per (tile, key head, split). The waves take the
 // block's 32-key blocks round-robin, each with its own running maximum, sum and
 // accumulator. Keys and values come by loads to registers, those of the next two blocks on their way while
-// one is multiplied and page numbers fetched two blocks further ahead, or (RING: heads of 64 and 128 in
-// most launches, decode_by_ring) by direct loads to LDS, the next block's on its way and page numbers 16 blocks
+// one is multiplied and page numbers fetched two blocks further ahead, or (heads of 64 and 128,
+// DECODE_RING) by direct loads to LDS, the next block's on its way and page numbers 16 blocks
 // at a time. No load waits for another. The waves' results meet in LDS. With several splits each
 // block writes its normalised part and the base-2 log of its sum, and a second
 // small kernel merges them. (Merging in the block that arrives last at a counter
@@ -1611,14 +1611,17 @@ __device__ __forceinline__ void head_as_operand(const bf16_t* __restrict__ x, co
 }
 
 // Heads of 64 and 128 elements: a wave's next block of keys and values comes by direct loads into LDS of its own, whole
-// cache lines, while one is multiplied from registers (most launches: decode_by_ring).
+// cache lines, while one is multiplied from registers.
 // Keys: operand row 16 kb + r (key 8 (r / 4) + 4 kb + r % 4 of the block) is a row of D elements, piece c (16 bytes) of it at
 // c ^ (r, or r / 2 where a row is half of the banks), so that the operand reads touch every bank once. Values: element d is
 // a row of 64 bytes, its four groups of eight keys at g ^ (d / 4) % 4. Every load is of 16 bytes a lane, from anywhere: four
 // keys, or sixteen elements of two pages of 16 keys, an instruction. As loads straight to registers the keys came as sixteen half
 // lines an instruction, and two blocks on their way took 128 registers: attention and merge, us, by registers and by the ring, 32 heads of 128 on
 // 8: 40 sequences of 300 keys 17.8 and 16.4; 20 of 1,030 in 3 parts 23.2 and 22.5; 56 of 1,030 44.5 and 42.5; in pieces 48 of 136 to 2,606 46.5
-// and 41.3, 64 of 200 to 8,000 117 and 105; where it loses, decode_by_ring. Waiting for keys and values apart, so that either is on its way a little longer, is level (20.9, 21.1).
+// and 41.3, 64 of 200 to 8,000 117 and 105. Launched in a row with their operands partly in the caches some block counts lose (768 with heads of
+// 128: 24 of 1,030 27.6 and 29.6, 48 41.0 and 44.1; up to 256 of long parts with heads of 64: 16 of 2,054 26.6 and 29.1), where keys come
+// from memory none does: whole steps of the 4B size, us, 24 sequences of 1,100 and 2,060 keys 3,524 and 3,433, 4,086 and 3,980, 48 4,213
+// and 4,223, 5,476 and 5,460, 96 of 1,100 6,365 and 6,191; with heads of 64 8 and 16 of 2,060 2,425 and 2,406, 2,790 and 2,779. Waiting for keys and values apart, so that either is on its way a little longer, is level (20.9, 21.1).
 constexpr bool DECODE_RING = D % 64 == 0 && DMAX <= 128;
 constexpr int RING_KEYS = 64 * D, RING_WAVE = RING_KEYS + 64 * DV;  // bytes
 
@@ -1665,14 +1668,14 @@ __device__ __forceinline__ void ring_read(const unsigned char* ring, int r16, in
 
 constexpr bool DECODE_ONCE = true;  // measured: 2 % off a decode step at batch 1 and at batch 64, level at batch 8
 
-template <bool P2, bool FUSED, bool RING>
+template <bool P2, bool FUSED = false>
 __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_decode_kernel(AttnTileArgs a) {
   // per wave: maximum and sum per row, unnormalised accumulator [16][DV]
   extern __shared__ float lds[];
   float* lds_m = lds;                 // [DW][16]
   float* lds_l = lds + DW * 16;       // [DW][16]
   float* lds_o = lds + 2 * DW * 16;   // [DW] x O_WAVE: [16][OROW], in the room of the wave's ring
-  constexpr int O_WAVE = RING ? RING_WAVE / 4 : 16 * OROW;
+  constexpr int O_WAVE = DECODE_RING ? RING_WAVE / 4 : 16 * OROW;
 
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r16 = lane & 15, quad = lane >> 4;
@@ -1793,7 +1796,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     }
 
     const int last = b + (b1 - 1 - b) / DW * DW;
-    if constexpr (RING) {
+    if constexpr (DECODE_RING) {
       unsigned char* ring = (unsigned char*)(lds_o + wave * O_WAVE);
       int pages = ring_pages<P2>(table, b, DW, last, lo, pos_max, a.page_size, lane), i = 0;
       ring_fetch<P2>(a, kvh, b << 5, lo, pos_max, pages, 0, lane, ring);
@@ -1942,46 +1945,6 @@ extern "C" int qrt_attention_work_list(const AttnTileArgs* args, int fused, hipS
   return 0;
 }
 
-// Heads of 64 and 128: by the ring, but where blocks that have a compute unit to themselves for long are what the launch waits for:
-// their waves have one block of keys on the way by the ring and two by the loads to registers. Heads of 64 (half the bytes a
-// block): at most one block to a unit, and more than 256 keys to walk for each unit. Heads of 128: two blocks fit a unit, so up to 512 are
-// one round, and up to 768 a second one of one block a unit. us with the merge, by registers and by the ring. 64: 160 blocks 8.6
-// and 8.6 of 300 keys, 192 8.8 and 8.8 of 300, 12.7 and 13.5 of 515, 240 10.3 and 10.0 of 206, 224 18.3 and 19.4 of 1,027, 256 8.8 and 8.5 of 64, 10.6 and
-// 11.0 of 258, 26.6 and 29.1 of 2,054; 320 blocks 11.3 and 10.3, 448 43.7 and 41.7, 512 46.8 and 44.9, 768 36.8 and 36.0. 128: 256 29.8 and 29.8 of
-// 1,027, 86.7 and 86.0 of 4,000, 384 18.6 and 17.2, 448 44.5 and 42.5, 512 47.6 and 47.9; 640 25.1 and 26.4, 768 27.6 and 29.6, 41.0 and
-// 44.1, 71.0 and 74.5; 960 38.1 and 37.4, 1,024 87.5 and 88.2, 2,048 58.7 and 57.4. The same bits.
-static bool decode_by_ring(const AttnTileArgs& a) {
-  if (a.items || D != DV) return true;
-  const long blocks = (long)a.num_tiles * a.nkv * a.num_splits;
-  if (D > 64) return blocks <= 512 || blocks > 768;
-  const long keys = (long)a.table_width * a.page_size, reach = a.window + a.chunk;  // a window or a chunk, not both
-  return blocks > 256 || (long)a.num_tiles * a.nkv * (reach && reach < keys ? reach : keys) <= 256 * 256;
-}
-template <bool P2, bool FUSED, bool RING>
-static int decode_launch(const AttnTileArgs& a, hipStream_t stream) {
-  constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
-  static_assert(!RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
-  auto kernel = attention_bf16_decode_kernel<P2, FUSED, RING>;
-  if (smem > 64 * 1024) {  // rings of heads of 128, accumulators of 256: a little more LDS than a block gets without asking
-    static bool allowed = false;  // once: not again inside every stream capture
-    if (!allowed) {
-      if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-        return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
-      allowed = true;
-    }
-  }
-  const dim3 grid = a.items ? dim3(a.nkv, a.max_items, 1) : dim3(a.num_tiles, a.nkv, a.num_splits);
-  kernel<<<grid, 64 * DW, smem, stream>>>(a);
-  return 0;
-}
-template <bool FUSED>
-static int decode_by_kernel(const AttnTileArgs& a, hipStream_t stream) {
-  const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
-  if constexpr (DECODE_RING)
-    if (decode_by_ring(a)) return p2 ? decode_launch<true, FUSED, true>(a, stream) : decode_launch<false, FUSED, true>(a, stream);
-  return p2 ? decode_launch<true, FUSED, false>(a, stream) : decode_launch<false, FUSED, false>(a, stream);
-}
-
 // every listed sequence at most 16 rows (q_len * g <= 16) and D <= 256; num_tiles = number of
 // sequences; tile_seq lists them, or is null for all sequences of the step in order
 extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_total, hipStream_t stream) {
@@ -2004,7 +1967,22 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
             "attention (decode): pieces of %d blocks with a list of %d items for %d sequences", a.split_blocks,
             a.max_items, a.num_tiles);
   if (a.num_tiles == 0) return 0;
-  int rc = 0;
+  const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
+  dim3 grid(a.num_tiles, a.nkv, a.num_splits), block(64 * DW);
+  if (a.items) grid = dim3(a.nkv, a.max_items, 1);
+  constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (DECODE_RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
+  static_assert(!DECODE_RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
+  if (smem > 64 * 1024) {  // rings of heads of 128, accumulators of 256: a little more LDS than a block gets without asking
+    static bool allowed = false;  // once: not again inside every stream capture
+    if (!allowed) {
+      if (hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<true>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess ||
+          hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<false>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+        return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
+      allowed = true;
+    }
+  }
   if (a.qkv) {
     // one token per sequence, its query, key and value taken from the product that made them
     if constexpr (D % 64 == 0) {
@@ -2014,12 +1992,24 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
                 a.nq / a.nkv, a.qkv_stride);
       QRT_CHECK(!a.rope || (a.rope_pairs >= 32 && a.rope_pairs % 32 == 0 && a.rope_pairs <= D / 2),
                 "attention (decode, own token from the product): %d pairs turn (multiples of 32 up to %d)", a.rope_pairs, D / 2);
-      rc = decode_by_kernel<true>(a, stream);
+      if (smem > 64 * 1024) {
+        static bool allowed_fused = false;
+        if (!allowed_fused) {
+          if (hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<true, true>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess ||
+              hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<false, true>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+            return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
+          allowed_fused = true;
+        }
+      }
+      if (p2) attention_bf16_decode_kernel<true, true><<<grid, block, smem, stream>>>(a);
+      else attention_bf16_decode_kernel<false, true><<<grid, block, smem, stream>>>(a);
     } else {
       return qrt_fail("attention (decode, own token from the product): head size %d is no multiple of 64", D);
     }
-  } else rc = decode_by_kernel<false>(a, stream);
-  if (rc) return rc;
+  } else if (p2) attention_bf16_decode_kernel<true><<<grid, block, smem, stream>>>(a);
+  else attention_bf16_decode_kernel<false><<<grid, block, smem, stream>>>(a);
   QRT_LAUNCH_CHECK("attention_bf16_decode");
   if (a.num_splits > 1) {
     const int merge_rows = a.merge_tokens ? a.num_merge_tokens * a.nq : num_rows_total;

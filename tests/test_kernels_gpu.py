@@ -909,34 +909,6 @@ def test_decode_attention_over_many_blocks_a_wave(ops, d, ps, window):
         close(ops.paged_attention(q, cache, ctx, 6, 2, d, d ** -0.5, window), want, 2e-2, 2e-2)
 
 
-# blocks of the launch: at the ends of the ranges that load keys to registers (513 and 768 with heads of 128; up to 256 with heads of 64, with
-# more than 65,536 keys in all), and beside them
-@pytest.mark.parametrize("d,n,nkv,splits,kv", [
-    (128, 27, 19, 1, 300), (128, 24, 16, 2, 1030), (128, 32, 16, 1, 90), (128, 11, 70, 1, 90),
-    (64, 23, 7, 1, 410), (64, 16, 8, 2, 1030), (64, 8, 8, 4, 1030), (64, 16, 16, 1, 256), (64, 257, 1, 1, 290),
-])
-def test_decode_attention_by_registers_has_the_rings_bits(ops, d, n, nkv, splits, kv):
-    """Equal parts, by either way of loading keys, against pieces of the same length, which come by the ring; the tokens' keys from the
-    cache and from the product."""
-    ps = 16
-    q, cache, ctx = build_attention_case([(1, kv)] * n, nkv, nkv, d, ps, torch.bfloat16, seed=4, poison=True)
-    table = cache.group.block_table.cpu()
-    cache.group.slots = (table[:, (kv - 1) // ps] * ps + (kv - 1) % ps).to(torch.int32).to(DEV)
-    qkv = rnd(n, 3 * nkv * d, dtype=torch.bfloat16, seed=11)
-    k, v = cache.k.clone(), cache.v.clone()
-    calls = (lambda: ops.paged_attention(q, cache, ctx, nkv, nkv, d, d ** -0.5, None),
-             lambda: ops.decode_attention(qkv, cache, ctx, nkv, nkv, d, d ** -0.5, None, None, None, 0.0, None))
-    for call in calls:
-        got = []
-        for cut in ({"attn_splits": splits}, {"attn_piece": 32 * -(-(-(-kv // 32)) // splits)}):
-            ctx.scratch = dict(cut)
-            ctx.per_pass.clear()
-            cache.k.copy_(k)
-            cache.v.copy_(v)
-            got.append(call())
-        assert torch.isfinite(got[0]).all() and torch.equal(*got)
-
-
 @pytest.mark.parametrize("lens,nkv,d", [
     ([100 + 41 * i for i in range(28)], 8, 64),         # none as long as 2,048
     ([90, 2600, 700, 64, 1500, 33, 4000, 1, 800], 2, 128),
