@@ -213,9 +213,7 @@ class DecodeGraph:
                 self.views_dev = self._views()
                 packed.kv_lens = [self.bucket] * self.batch  # launch shapes are those of the bucket
                 self.ctx = runner._context(packed, self.views_dev)
-                # the bucket's length, not the batch's, now fixes every launch shape (key splits too), which the
-                # attention is told, since the contexts may be far shorter;
-                self.ctx.scratch["attn_bucket"] = True
+                # the bucket's length, not the batch's, now fixes every launch shape (key splits too);
                 # where the lengths are very unequal the attention kernel is told them as they are
                 # now, to choose the length of its pieces by
                 if self.unequal:

@@ -1880,20 +1880,20 @@ class HipOps:
     key_groups_ratio = 0.9
 
     @staticmethod
-    def choose_splits(num_tiles: int, nkv: int, max_kv: int, head_dim: int = 0, bucket: bool = False) -> int:
+    def choose_splits(num_tiles: int, nkv: int, max_kv: int, head_dim: int = 0) -> int:
         """Portions: how many ways to split the keys so that few long sequences still fill the chip.
         Heads wider than 256 (one block of waves a compute unit, and no decode kernel of their own, so
         that decoded tokens come here too): parts of 64 keys and more, 256 blocks in all; parts of 32, one block of keys
         each, where that makes at most 32 of a sequence and 128 in all (32 heads of 448 on one, us with the merge, 64 and 32 keys a
         part: 8 sequences of 300 keys 16.3 and 14.4, of 500 17.6 and 16.7, of 640 18.7 and 18.9, of 1,029 20.6 and 26.1; 20 of 300
-        19.8 and 19.8; 8 of 100 in one part 17.8, in four 13.0, of 64 in one 12.0, in two 12.4). ``bucket``: ``max_kv`` is what a captured
-        step's contexts may grow to, and they may be short: then 32 parts in all, which cost a short context nothing (1 of 100,
-        512 and 1,000 keys in 16 parts 12.0, 12.3, 15.4, in 8 11.9, 14.9, 21.1, in 32 13.7, 13.9, 14.2; 8 of 100, 200 and 400 in 16 15.1, 15.8, 16.4, in 8
-        13.4, 13.8, 17.3; 4 of 100 13.1 and 12.5)."""
+        19.8 and 19.8; 8 of 100 in one part 17.8, in four 13.0, of 64 in one 12.0, in two 12.4). A captured step is cut by its
+        bucket, 512 keys or more; parts of one block are no worse there: a step of a 4B model with nine such layers of 36, us, in
+        8 and 16 parts, 8 sequences of 60, 130, 250 and 400 keys 3,126 and 3,153, 3,145 and 3,143, 3,208 and 3,170, 3,219 and 3,233; 4 of 60, 250 and
+        400 2,843 and 2,847, 2,881 and 2,843, 2,831 and 2,807; one of 700 in 16 and 32 2,478 and 2,462."""
         work = num_tiles * nkv
         if head_dim > 256:
             blocks = (max_kv + 31) // 32
-            if 3 <= blocks <= 32 and work * blocks <= (32 if bucket else 128):
+            if 3 <= blocks <= 32 and work * blocks <= 128:
                 return blocks
             return 1 if max_kv <= 128 or work >= 256 else max(1, min((max_kv + 63) // 64, (256 + work - 1) // work, 64))
         if max_kv <= 512 or work >= 512:
@@ -2078,7 +2078,7 @@ class HipOps:
             ctx.scratch[key] = plan
         tiles, n_tiles, tokens, groups, wide_splits = plan
         splits = ctx.scratch.get("attn_splits") or wide_splits or (
-            self.choose_decode_splits(n_tiles, nkv, seen_kv) if decode else self.choose_splits(n_tiles, nkv, seen_kv, widest, bool(ctx.scratch.get("attn_bucket"))))
+            self.choose_decode_splits(n_tiles, nkv, seen_kv) if decode else self.choose_splits(n_tiles, nkv, seen_kv, widest))
         a = _AttnTileArgs()
         a.chunk = chunk
         # beside a window the sequence's first keys stay in sight; a sink: one more term in the softmax's sum

@@ -49,13 +49,6 @@ def test_first_tokens_of_a_sequence(model_folders):
         assert m.generate(prompt, max_tokens=5) == P.greedy_generate(cfg, w, prompt, 5)
 
 
-def test_a_captured_step_tells_attention_that_its_lengths_are_a_buckets(model_folders):
-    m = llm(model_folders["tiny_b"], dtype="bfloat16", graph=True)
-    m.generate([[5, 6, 7], [8]], max_tokens=6)
-    graphs = list(m.engine.runner._graphs.values())
-    assert graphs and all(g.ctx.scratch["attn_bucket"] and max(g.ctx.kv_lens_host) == g.bucket for g in graphs)
-
-
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_graph_replay_equals_eager(model_folders, dtype):
     cfg, _ = P.read_model(model_folders["tiny_b"])

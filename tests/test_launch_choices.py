@@ -46,9 +46,3 @@ def test_parts_of_the_keys_of_portions_with_wide_heads(d):
 ])
 def test_parts_of_the_keys_of_decoded_tokens_with_wide_heads(sequences, keys, parts):
     assert HipOps.choose_splits(sequences, 1, keys, 448) == parts
-
-
-# by a captured step's bucket, whose contexts may be as short as one key: parts of two blocks, but for one or two sequences
-@pytest.mark.parametrize("sequences,bucket,parts", [(1, 512, 16), (2, 512, 16), (3, 512, 8), (8, 512, 8), (16, 512, 8), (1, 1024, 32), (2, 1024, 16), (8, 2048, 32)])
-def test_parts_of_a_captured_step_with_wide_heads(sequences, bucket, parts):
-    assert HipOps.choose_splits(sequences, 1, bucket, 448, bucket=True) == parts
