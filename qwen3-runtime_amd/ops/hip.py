@@ -1940,6 +1940,15 @@ class HipOps:
         for parts in range(2, long_parts + 1):
             if time(parts) < time(best) * 0.999:
                 best = parts
+        # one block to nearly every unit: twice as many of half the length hide each other's starts and ends, from 256 keys a part on.
+        # A captured step is cut by its bucket, a power of two, so its contexts may have half as many; they gain as well. Whole steps of
+        # the 4B size from graphs, where keys come from memory, us, by as many parts and by twice as many: 8 sequences of 300, 700,
+        # 1,025, 1,300, 1,600, 1,900, 2,054 and 3,300 keys 2,407 and 2,432, 2,518 and 2,526, 2,590 and 2,543, 2,630 and 2,565, 2,689 and 2,638, 2,719 and
+        # 2,702, 2,781 and 2,700, 2,977 and 2,898; 7 of 1,100, 2,060 and 3,000 2,540 and 2,514, 2,762 and 2,696, 2,967 and 2,863; 14 of 1,500 3,073 and 2,986;
+        # 16 of 1,100 to 3,000 0.98 to 1.03 of the time; 12 (480 blocks) 1.03 to 1.07. (The attention alone, launched in a row with part of its
+        # operands in the caches, is level: 8 of 2,054 20.2 and 20.5, of 1,030 15.0 and 14.9.)
+        if 1 < best <= 32 and 224 <= work * best <= 256 and blocks // (2 * best) >= 8:
+            return 2 * best
         merge = 180.0 / max(max_kv, 1) if best == 1 else 0.0
         best_time = time(best)
         for parts in range(long_parts + 1, min(blocks // 2, 16) + 1):
