@@ -1440,7 +1440,7 @@ class HipOps:
                 and k >= 256 and k % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             _need(x, "x")
             _need(w, "weight")
-            # with many rows already added up, in the planes' order
+            # where blocks fill the chip without planes already added up, in the planes' order
             planes = self.lib.qrt_gemm_f32_planes_of(c_int(m), c_int(n), c_int(k))
             out = torch.empty((planes, m, n) if planes > 1 else (m, n), dtype=torch.float32, device=x.device)
             self._check(self.lib, self.lib.qrt_gemm_f32_planes(_ptr(x), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), c_int(planes),
