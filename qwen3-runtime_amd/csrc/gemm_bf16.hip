@@ -11,6 +11,7 @@
 #include "common.h"
 #include "direct.h"
 #include "gemm_epilogue.h"
+#include "row_norm.h"
 #include <type_traits>
 
 template <bool ALIGNED>
@@ -249,10 +250,12 @@ static int skinny(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int 
 // result is plane blockIdx.y of the output (the caller adds the planes: used where the result
 // feeds a residual add); its NW waves take the pairs round-robin and meet in LDS, added in
 // wave order.
-template <int NW, int NT, int U, int GATED, bool FEW, typename TO>
+// SCALED: row m of the activations still lacks the factor 1 / rms of its norm, which multiplies the sums: gemm_residual.hip
+// says why. Its SQUARE_PARTS parts are asked for in front of the weights and added up while those are on their way.
+template <int NW, int NT, int U, int GATED, bool FEW, bool SCALED, typename TO>
 __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
-                                                                  TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep) {
+                                                                  TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep, RowNorm norm) {
   constexpr bool MIXED = GATED && NT == 1;
   constexpr int UNITS = NT + 1, LOADS = 2 * UNITS - FEW, SLOT = UNITS * 2048 - (FEW ? 1024 : 0);
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
@@ -294,8 +297,22 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
   f32x4_t acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  constexpr int MOST = FEW ? 8 : 16, OWN = (MOST + NW - 1) / NW;  // rows whose factor a wave forms
+  __shared__ float factor[SCALED ? MOST : 1];
+  f32x4_t squares[SCALED ? OWN : 1];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int j = 0; j < OWN; ++j) squares[j] = *(const f32x4_t*)(norm.squares + (size_t)min(wave + j * NW, M - 1) * SQUARE_PARTS + 4 * lane);
+  }
   int fetched = 0;
   for (; fetched < U && fetched < mine; ++fetched) fetch(fetched, fetched);
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int j = 0; j < OWN; ++j) {
+      const float f = norm.factor(squares[j]);
+      if (lane == 0 && wave + j * NW < MOST) factor[wave + j * NW] = f;
+    }
+  }
   const int read_at[2] = {r16 * 128 + 16 * (quad ^ (r16 & 7)), r16 * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
   const int ra = FEW ? r16 & 7 : r16, a_at[2] = {ra * 128 + 16 * (quad ^ (r16 & 7)), ra * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
   int slot = 0;
@@ -346,6 +363,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
     float sum[4], up[4];
     total(t, l, sum);
     if (GATED) total(NT - 1, MIXED ? l + 32 : l, up);
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sum[r] *= factor[m];
+        if (GATED) up[r] *= factor[m];
+      }
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (nn + r < N) {
@@ -355,25 +379,26 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
   }
 }
 
-template <int NW, int NT, int U, int GATED, bool FEW>
+template <int NW, int NT, int U, int GATED, bool FEW, bool SCALED>
 static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep,
-                       hipStream_t stream, int k_parts) {
+                       hipStream_t stream, int k_parts, const RowNorm& norm) {
   constexpr int outputs = GATED ? 8 * NT : 16 * NT;
   dim3 grid((N + outputs - 1) / outputs, k_parts), block(64 * NW);
   constexpr size_t ring = (size_t)NW * U * ((NT + 1) * 2048 - (FEW ? 1024 : 0)), meet = (size_t)NW * NT * 1024, smem = ring > meet ? ring : meet;
   static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
 #define GO(TO)                                                                                          \
   do {                                                                                                  \
-    auto kernel = gemm_bf16_rows_kernel<NW, NT, U, GATED, FEW, TO>;                                        \
+    auto kernel = gemm_bf16_rows_kernel<NW, NT, U, GATED, FEW, SCALED, TO>;                                \
     static bool allowed = false; /* once per kernel: not inside a stream capture again and again */    \
     if (smem > 64 * 1024 && !allowed) {                                                                 \
       if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) \
         return qrt_fail("gemm_bf16: cannot get %zu bytes of LDS", smem);                                \
       allowed = true;                                                                                   \
     }                                                                                                   \
-    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ep);                                   \
+    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ep, norm);                             \
   } while (0)
   if (out_dtype == QRT_BF16) GO(bf16_t);
+  else if constexpr (SCALED) return qrt_fail("gemm_bf16: rows that lack their norm's factor give bfloat16 (%d asked for)", out_dtype);
   else if (out_dtype == QRT_F32) GO(float);
   else return qrt_fail("gemm_bf16: unknown output dtype %d", out_dtype);
 #undef GO
@@ -403,30 +428,30 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
 //   and 10.8, 11.6; 164 6 and 6, 11.4, 12.5 and 11.5, 11.5; 192 6 and 6, 12.4, 13.3 and 12.4, 12.2; 224 7 and 8, 14.4, 16.1 and 14.9, 15.0;
 //   320 10 and 10, 19.4, 21.2 and 20.0, 20.7. At 16 rows level.
 // Up to 8 rows (FEW) the activations' unit is half as long: 0.1 to 0.3 us of a product, most where a block has one tile.
-template <int GATED, bool FEW>
+template <int GATED, bool FEW, bool SCALED = false>
 static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep, hipStream_t st,
-                    int k_parts) {
+                    int k_parts, const RowNorm& norm = RowNorm{}) {
   const int tiles = (N + 15) / 16;
   if constexpr (GATED) {
     // half tiles that the busiest of 256 compute units gets by blocks of eight and eight rows, and by blocks of a tile of either
     const int mixed = ((N + 7) / 8 + 255) / 256, either = 2 * ((tiles + 255) / 256);
     if constexpr (FEW)
-      if (mixed < either && (mixed <= 5 || K <= 4096 || M <= 2)) return launch_rows<4, 1, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-    return launch_rows<4, 2, 3, GATED, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+      if (mixed < either && (mixed <= 5 || K <= 4096 || M <= 2)) return launch_rows<4, 1, 3, GATED, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+    return launch_rows<4, 2, 3, GATED, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
   } else {
     if (k_parts > 1) {
       const int one = (tiles * k_parts + 255) / 256, two = 2 * (((tiles + 1) / 2 * k_parts + 255) / 256);
-      if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
-      return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, k_parts);
+      if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
+      return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
     }
     if (K % 2048 == 0) {
-      if (tiles >= 2048) return launch_rows<4, 1, 3, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-      return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+      if (tiles >= 2048) return launch_rows<4, 1, 3, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+      return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
     }
-    if (tiles >= 2048) return launch_rows<4, 2, 3, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-    if (tiles >= 384 && K <= 4096 && !(tiles <= 512 ? M <= 4 : tiles <= 768)) return launch_rows<4, 2, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-    if (tiles >= 384 && K > 4096) return launch_rows<4, 1, 4, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
-    return launch_rows<4, 1, 2, 0, FEW>(a, w, c, out_dtype, M, N, K, ep, st, 1);
+    if (tiles >= 2048) return launch_rows<4, 2, 3, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+    if (tiles >= 384 && K <= 4096 && !(tiles <= 512 ? M <= 4 : tiles <= 768)) return launch_rows<4, 2, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+    if (tiles >= 384 && K > 4096) return launch_rows<4, 1, 4, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+    return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
   }
 }
 
@@ -804,4 +829,23 @@ extern "C" int qrt_gated_gemm_bf16(const void* a, const void* w, void* c, int ou
   QRT_CHECK(act_kind == QRT_ACT_SWIGLU || act_kind == QRT_ACT_CLAMPED, "gated_gemm_bf16: unknown activation %d", act_kind);
   const int mode = act_kind == QRT_ACT_SWIGLU && !row_scale ? 1 : 2;
   return gemm(a, w, c, out_dtype, M, N, K, mode, shared, 1, GatedEpilogue{act_kind, limit, row_scale}, stream);
+}
+
+// The product, or the gated one, of rows that still lack the factor of their RMS norm: C = act(factor * (A W^T)), bfloat16. `a`
+// [M, K] and `squares` [M, SQUARE_PARTS] as qrt_gemm_residual_bf16 left them, `eps` the norm's; M <= 16, K % 64 == 0.
+// The sums' launch shapes are those of the products of whole rows. gated: -1 none, else an activation of common.h.
+extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M, int N, int K, int gated, float limit, const float* squares,
+                                    float eps, hipStream_t stream) {
+  QRT_CHECK(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0, "scaled_gemm_bf16: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)squares) % 16 == 0, "scaled_gemm_bf16: operands off 16 bytes");
+  QRT_CHECK(gated == -1 || gated == QRT_ACT_SWIGLU || gated == QRT_ACT_CLAMPED, "scaled_gemm_bf16: unknown activation %d", gated);
+  if (M == 0) return 0;
+  const bf16_t *A = (const bf16_t*)a, *W = (const bf16_t*)w;
+  const RowNorm norm{squares, 1.0f / (float)K, eps};
+  const GatedEpilogue ep{gated < 0 ? QRT_ACT_SWIGLU : gated, limit, nullptr};
+#define GO(GATED) (M <= 8 ? few_rows<GATED, true, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm) \
+                          : few_rows<GATED, false, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm))
+  if (gated == -1) return GO(0);
+  return gated == QRT_ACT_SWIGLU ? GO(1) : GO(2);
+#undef GO
 }

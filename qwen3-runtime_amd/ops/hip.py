@@ -272,6 +272,37 @@ TILES = (
 SHORT_TILE = 12
 
 
+class PendingProduct:
+    """``x @ w.T`` for the residual stream, not yet made: the norm that adds it makes it in one kernel with the
+    addition (``HipOps.add_rmsnorm`` with ``scaled=True``), or ``made()`` makes it as ``linear_for_residual`` does."""
+
+    __slots__ = ("ops", "x", "w")
+
+    def __init__(self, ops, x, w):
+        self.ops, self.x, self.w = ops, x, w
+
+    def made(self) -> torch.Tensor:
+        return self.ops.linear_for_residual(self.x, self.w)
+
+
+class ScaledRows:
+    """Rows of an RMS norm that lack their factors 1 / rms: ``rows`` = residual * weight in bfloat16, and the parts of the
+    rows' sums of squares. ``linear`` and ``gated_linear`` multiply their sums by the factors; ``made()`` gives the
+    norm's rows, as long as nothing has been added to the residual since."""
+
+    __slots__ = ("ops", "rows", "squares", "residual", "weight", "eps")
+
+    def __init__(self, ops, rows, squares, residual, weight, eps):
+        self.ops, self.rows, self.squares, self.residual, self.weight, self.eps = ops, rows, squares, residual, weight, eps
+
+    @property
+    def shape(self):
+        return self.rows.shape
+
+    def made(self) -> torch.Tensor:
+        return self.ops.add_rmsnorm(self.residual, None, self.weight, self.eps, self.rows.dtype)
+
+
 class HipOps:
     # bfloat16 products with more rows than this are made by tiles or the vendor library
     own_max_rows = 64
@@ -378,10 +409,15 @@ class HipOps:
     def new_rows(self, t, width, dtype, device):
         return torch.empty((t, width), dtype=dtype, device=device)
 
-    def add_rmsnorm(self, residual, delta, weight, eps, out_dtype, rows=None, delta_scale=1.0, delta_norm=None):
-        """``residual += delta_scale * delta`` in place (``delta`` a matrix or float32 planes), then the
+    def add_rmsnorm(self, residual, delta, weight, eps, out_dtype, rows=None, delta_scale=1.0, delta_norm=None, scaled=False):
+        """``residual += delta_scale * delta`` in place (``delta`` a matrix, float32 planes or a ``PendingProduct``), then the
         rows' RMS norm; with ``rows`` only those, and ``residual`` is left alone. ``delta_norm`` =
-        (weight, eps): ``delta`` joins the stream as ``delta / rms(delta) * weight``."""
+        (weight, eps): ``delta`` joins the stream as ``delta / rms(delta) * weight``. ``scaled``: what reads the rows
+        takes ``ScaledRows`` as well, which come where ``delta`` is a ``PendingProduct``."""
+        if isinstance(delta, PendingProduct):
+            if scaled and rows is None and delta_scale == 1.0 and delta_norm is None and out_dtype == torch.bfloat16:
+                return self._product_add_rmsnorm(residual, delta, weight, eps)
+            delta = delta.made()
         if delta_norm is not None:
             return self._norm_add_rmsnorm(residual, delta, delta_norm[0], delta_norm[1], weight, eps, out_dtype, rows)
         t, h = residual.shape
@@ -403,6 +439,29 @@ class HipOps:
             _ptr(residual), _ptr(delta), _CODE[delta.dtype] if delta is not None else F32, _ptr(weight),
             _ptr(rows), _ptr(out), _CODE[out_dtype], c_int(n_out), c_int(h), c_float(eps), c_int(planes),
             c_long(plane_stride), c_float(delta_scale), _stream()))
+        return out
+
+    def _product_add_rmsnorm(self, residual, product, weight, eps):
+        x, w = product.x, product.w
+        (m, k), n = x.shape, w.shape[0]
+        _need(residual, "residual", torch.float32, (m, n))
+        _need(weight, "norm weight", torch.float32, (n,))
+        rows = torch.empty((m, n), dtype=torch.bfloat16, device=residual.device)
+        squares = torch.empty((m, 256), dtype=torch.float32, device=residual.device)
+        self._check(self.lib, self.lib.qrt_gemm_residual_bf16(
+            _ptr(x), _ptr(w), _ptr(residual), _ptr(weight), _ptr(rows), _ptr(squares), c_int(m), c_int(n), c_int(k), _stream()))
+        return ScaledRows(self, rows, squares, residual, weight, eps)
+
+    def _scaled_product(self, x, w, gated=-1, limit=0.0):
+        """The product of ``ScaledRows``, or the gated one by an activation's code; None where the kernels do not take it."""
+        m, k = x.shape
+        if w.dtype != torch.bfloat16 or w.shape[1] != k or w.data_ptr() % 16 or not w.is_contiguous() or not w.is_cuda:
+            return None
+        n = w.shape[0] if gated < 0 else w.shape[0] // 2
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=w.device)
+        self._check(self.lib, self.lib.qrt_scaled_gemm_bf16(
+            _ptr(x.rows), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), c_int(gated), c_float(limit), _ptr(x.squares),
+            c_float(x.eps), _stream()))
         return out
 
     def _norm_add_rmsnorm(self, residual, y, w_after, eps_after, weight, eps, out_dtype, rows):
@@ -1253,6 +1312,9 @@ class HipOps:
 
     # ---- matrix products -------------------------------------------------------
     def linear(self, x, w, out_f32=False):
+        if isinstance(x, ScaledRows):
+            out = None if out_f32 else self._scaled_product(x, w)
+            return self.linear(x.made(), w, out_f32) if out is None else out
         _need(x, "x")
         _need(w, "weight")
         m, k = x.shape
@@ -1467,6 +1529,18 @@ class HipOps:
             c_int(kernel), c_int(parts), _stream()))
         return out
 
+    def product_for_norm(self, x, w):
+        """``linear_for_residual(x, w)`` for a result that goes to ``add_rmsnorm`` and nowhere else: up to 16 rows of
+        bfloat16 come as a ``PendingProduct``. What it takes to make those: whole pairs of k-steps, a residual whose columns
+        256 blocks share at up to 16 each, and that the next product can read in pairs of k-steps."""
+        (m, k), n = x.shape, w.shape[0]
+        if (m <= 16 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape[1] == k and k % 64 == 0 and k > 0 and n % 64 == 0
+                and 256 <= n <= 4096 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
+            _need(x, "x")
+            _need(w, "weight")
+            return PendingProduct(self, x, w)
+        return self.linear_for_residual(x, w)
+
     def linear_planes_with_spare(self, x, w, spare=1):
         """``linear_for_residual(x, w)`` as float32 planes ``[P + spare, T, N]`` of which the last ``spare`` are left
         for the caller to fill with more addends of the same sum (so that the sum costs no
@@ -1521,6 +1595,11 @@ class HipOps:
             raise OpsError(f"gated_linear: x is {tuple(x.shape)}, weight is {tuple(w_gate_up.shape)}")
         if ACTIVATIONS[activation] > ACTIVATIONS["clamped"]:  # the kernels take its code, but for a product of another form
             raise OpsError(f"gated_linear: {activation} has no gate")
+        if isinstance(x, ScaledRows):
+            out = self._scaled_product(x, w_gate_up, ACTIVATIONS[activation], limit) if row_scale is None else None
+            if out is not None:
+                return out
+            x = x.made()
         if x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16 and k % 32 == 0:
             _need(x, "x")
             _need(w_gate_up, "weight")

@@ -50,7 +50,7 @@ import math
 import torch
 
 from ..registry import part_class, register_part
-from .base import Mixer
+from .base import Mixer, for_norm
 from .plan import CacheSpec, PartSpec, TensorDecl
 from .rope import half_frequencies
 
@@ -149,6 +149,10 @@ class GroupedQueryAttention(Mixer):
                 raise ValueError("pairs of neighbours are brought into the order of a half rotation of plain queries and keys")
             n = self.position.dims
             self.row_order = torch.tensor([*range(0, n, 2), *range(1, n, 2), *range(n, self.head_dim)], dtype=torch.long)
+
+    @property
+    def takes_scaled_rows(self):
+        return type(self).forward is GroupedQueryAttention.forward
 
     def children(self):
         return (self.position,) if self.position is not None else ()
@@ -269,7 +273,7 @@ class GroupedQueryAttention(Mixer):
             more = {name: value for name, value in (("chunk", self.chunk), ("softcap", self.softcap),
                                                     ("keep_first", self.keep_first), ("sink", self.sink)) if value}
             attn = ops.paged_attention(q, cache, ctx, nq, nkv, d, self.scale, self.window, **more)
-            return ops.linear_for_residual(attn, self.o)
+            return for_norm(self, ctx, attn, self.o)
         in_place = getattr(self.position, "in_place", False)
         if in_place:
             # biases and an encoding that works on the product where it lies: after it the mixer
@@ -307,7 +311,7 @@ class GroupedQueryAttention(Mixer):
             attn = ops.decode_attention(qkv, cache, ctx, nq, nkv, d, self.scale, self.window,
                                         self.q_norm, self.k_norm, eps, inv_freq,
                                         None if inv_freq is None else self.position.angles_key, **more)
-            return ops.linear_for_residual(attn, self.o)
+            return for_norm(self, ctx, attn, self.o)
         if fused:
             # norm, rotation and the cache write in one pass over qkv
             shape = {k: more[k] for k in ("value_dim", "value_turn") if k in more}
@@ -329,4 +333,4 @@ class GroupedQueryAttention(Mixer):
                 ops.kv_store(k, v, cache)
             q = q.reshape(ctx.num_tokens, nq * d)
         attn = ops.paged_attention(q, cache, ctx, nq, nkv, d, self.scale, self.window, **more)
-        return ops.linear_for_residual(attn, self.o)
+        return for_norm(self, ctx, attn, self.o)

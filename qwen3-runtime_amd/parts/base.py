@@ -79,8 +79,13 @@ class Part:
     # or does anything else a captured HIP graph cannot replay; steps of a model with such a
     # part run eagerly. ``portion_multiple``: a part that works on blocks of this many tokens
     # wants every portion of a prompt but the last to be a multiple of it.
+    # ``takes_scaled_rows``: a mixer or feed-forward that hands its input to ``ops.linear`` and
+    # ``ops.gated_linear`` only may be given rows that lack the factor of their norm. ``before_norm``:
+    # set by a block on the sub-layers whose output it hands to its norms as it is.
     graph_capturable = True
     portion_multiple = 1
+    takes_scaled_rows = False
+    before_norm = False
 
     def __init__(self, tensors: Mapping[str, str] | None = None):
         self.tensor_names: dict[str, str] = dict(tensors or {})
@@ -163,10 +168,21 @@ class PositionEncoding(Part):
 
 class Block(Part):
     role = "block"
+    # The block hands what its sub-layers return to plain RMS norms and nothing else, so that they may
+    # leave the product in front of the addition to the norm (``for_norm``).
+    norms_take_products = False
 
 
 class Entry(Part):
     role = "entry"
+
+
+def for_norm(part, ctx, x, w):
+    """``part``'s last product, whose result joins the residual stream: left to the norm that adds it where
+    the model says that all its norms take products (``DecoderModel.forward``)."""
+    if part.before_norm and ctx.per_pass.get("norms_take_products"):
+        return ctx.ops.product_for_norm(x, w)
+    return ctx.ops.linear_for_residual(x, w)
 
 
 @dataclass

@@ -28,17 +28,30 @@ class PreNormBlock(Block):
         self.feed_forward = feed_forward
         self.norm_in = norms["input"]
         self.norm_post = norms.get("post_mixer")
+        for part in (mixer, feed_forward):
+            if part is not None:
+                part.before_norm = type(self) is PreNormBlock
 
     def children(self):
         return tuple(p for p in (self.norm_in, self.mixer, self.norm_post, self.feed_forward) if p is not None)
 
+    @property
+    def norms_take_products(self):
+        return type(self) is PreNormBlock and all(n is None or getattr(n, "takes_products", False) for n in (self.norm_in, self.norm_post))
+
     def forward(self, ctx, residual, delta, cache):
-        x = self.norm_in.forward(ctx, residual, delta)
+        x = self._normed(ctx, self.norm_in, residual, delta, self.mixer)
         mixed = self.mixer.forward(ctx, x, cache)
         if self.feed_forward is None:  # a layer of a mixer alone
             return residual, mixed
-        x = self.norm_post.forward(ctx, residual, mixed)
+        x = self._normed(ctx, self.norm_post, residual, mixed, self.feed_forward)
         return residual, self.feed_forward.forward(ctx, x)
+
+    @staticmethod
+    def _normed(ctx, norm, residual, delta, reader):
+        if ctx.per_pass.get("norms_take_products") and reader.takes_scaled_rows:
+            return norm.forward(ctx, residual, delta, scaled=True)
+        return norm.forward(ctx, residual, delta)
 
 
 @register_part("block", "sandwich_norm")

@@ -12,7 +12,7 @@ qwen3_runtime/utils/loader.py:51-53); ``silu(g) = g * sigmoid(g)``
 from __future__ import annotations
 
 from ..registry import register_part
-from .base import FeedForward
+from .base import FeedForward, for_norm
 from .plan import TensorDecl
 
 
@@ -29,6 +29,10 @@ class SwiGLU(FeedForward):
         self.gate_up = None
         self.down = None
 
+    @property
+    def takes_scaled_rows(self):
+        return type(self).forward is SwiGLU.forward
+
     def tensor_decls(self):
         h, i = self.hidden_size, self.intermediate_size
         return [
@@ -43,7 +47,7 @@ class SwiGLU(FeedForward):
 
     def forward(self, ctx, x):
         act = ctx.ops.gated_linear(x, self.gate_up, **self.how)
-        return ctx.ops.linear_for_residual(act, self.down)
+        return for_norm(self, ctx, act, self.down)
 
 
 @register_part("feed_forward", "act_mlp")
@@ -70,4 +74,4 @@ class ActMLP(FeedForward):
     def forward(self, ctx, x):
         together = getattr(ctx.ops, "act_linear", None)  # product and activation in one kernel
         act = together(x, self.up, self.activation) if together else ctx.ops.unary_act(ctx.ops.linear(x, self.up), self.activation)
-        return ctx.ops.linear_for_residual(act, self.down)
+        return for_norm(self, ctx, act, self.down)

@@ -42,6 +42,9 @@ class DecoderModel:
         self.final_norm = build_part("norm", plan.final_norm)
         self.head = build_part("head", plan.head)
         self.entries = [build_part("entry", spec) for spec in plan.entries]
+        # what sub-layers return goes to plain RMS norms only: those may make the product in front of the addition too
+        self.norms_take_products = (not self.entries and all(b.norms_take_products for b in self.blocks)
+                                    and getattr(self.final_norm, "takes_products", False))
         self._check_caches()
 
     def _check_caches(self) -> None:
@@ -125,6 +128,8 @@ class DecoderModel:
         the caches.
         """
         ctx.per_pass.clear()
+        if self.norms_take_products and hasattr(ctx.ops, "product_for_norm"):
+            ctx.per_pass["norms_take_products"] = True
         residual = self.embedding.forward(ctx, ids, tuple(embedding_cache)) if embedding_cache else self.embedding.forward(ctx, ids)
         delta = None
         # entries read the embedding's output; the stream itself is updated in place, so they get a copy

@@ -56,6 +56,11 @@ class RMSNorm(Norm):
         if self.delta_scale != 1.0 and (self.streams > 1 or self.has_bias):
             raise ValueError("a scaled residual sum goes with the RMS norm over one stream")
 
+    @property
+    def takes_products(self) -> bool:
+        """Whether ``forward`` with one stream is the plain ``ops.add_rmsnorm``, which takes products that are yet to be made."""
+        return type(self) is RMSNorm and self.streams == 1 and self.groups == 1 and self.delta_scale == 1.0
+
     def tensor_decls(self):
         decls = [TensorDecl(self._name("weight"), (self.size,), init="norm_zero" if self.weight_offset else "norm")]
         if self.has_bias:
@@ -71,12 +76,15 @@ class RMSNorm(Norm):
         if self.streams > 1:
             self.read_all = fetch.constant(torch.ones(self.streams, dtype=torch.float32))
 
-    def forward(self, ctx, residual, delta=None, rows=None, read=None):
-        """Apply ``delta`` to ``residual`` (in place), return its normalised rows.
+    def forward(self, ctx, residual, delta=None, rows=None, read=None, scaled=False):
+        """Apply ``delta`` to ``residual`` (in place), return its normalised rows (``scaled``: or rows that lack
+        the norm's factor, as ``ops.add_rmsnorm`` gives them; for a norm that ``takes_products``).
 
         With ``rows`` (int32 indices) only those rows are normalised and
         returned, packed; ``residual`` is then left as it is.
         """
+        if scaled:
+            return ctx.ops.add_rmsnorm(residual, delta, self.weight, self.eps, ctx.dtype, rows, scaled=True)
         if self.groups > 1 or (isinstance(delta, NormedUpdate) and delta.groups > 1):
             after = None
             if isinstance(delta, NormedUpdate):
