@@ -251,9 +251,10 @@ static int skinny(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int 
 // feeds a residual add); its NW waves take the pairs round-robin and meet in LDS, added in
 // wave order.
 // SCALED: row m of the activations still lacks the factor 1 / rms of its norm, which multiplies the sums: gemm_residual.hip
-// says why. Its SQUARE_PARTS parts are asked for in front of the weights and added up while those are on their way.
+// says why. One more wave adds its SQUARE_PARTS parts up meanwhile (a load to registers in the waves of the ring would have to
+// be waited for with all that is on its way: 9.0 us for 6,144 x 2,560 at 8 rows, 7.7 without the factors).
 template <int NW, int NT, int U, int GATED, bool FEW, bool SCALED, typename TO>
-__global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
+__global__ __launch_bounds__(64 * (NW + SCALED)) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
                                                                   TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep, RowNorm norm) {
   constexpr bool MIXED = GATED && NT == 1;
@@ -279,7 +280,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
   const int all_pairs = K >> 6;
   const int part = (all_pairs + gridDim.y - 1) / gridDim.y;
   const int p_first = blockIdx.y * part, p_end = min(all_pairs, p_first + part);
-  const int mine = max(0, (p_end - p_first - wave + NW - 1) / NW);  // pairs of this wave
+  const int mine = wave < NW ? max(0, (p_end - p_first - wave + NW - 1) / NW) : 0;  // pairs of this wave
   C += (size_t)blockIdx.y * M * N;
   auto fetch = [&](int i, int slot) {  // the wave's i-th pair into a slot of its ring
     const size_t at = (size_t)(p_first + wave + i * NW) * 64;
@@ -297,21 +298,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
   f32x4_t acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  constexpr int MOST = FEW ? 8 : 16, OWN = (MOST + NW - 1) / NW;  // rows whose factor a wave forms
+  constexpr int MOST = FEW ? 8 : 16;
   __shared__ float factor[SCALED ? MOST : 1];
-  f32x4_t squares[SCALED ? OWN : 1];
-  if constexpr (SCALED) {
-#pragma unroll
-    for (int j = 0; j < OWN; ++j) squares[j] = *(const f32x4_t*)(norm.squares + (size_t)min(wave + j * NW, M - 1) * SQUARE_PARTS + 4 * lane);
-  }
   int fetched = 0;
   for (; fetched < U && fetched < mine; ++fetched) fetch(fetched, fetched);
-  if constexpr (SCALED) {
+  if (SCALED && wave == NW) {
+    f32x4_t parts[MOST];
 #pragma unroll
-    for (int j = 0; j < OWN; ++j) {
-      const float f = norm.factor(squares[j]);
-      if (lane == 0 && wave + j * NW < MOST) factor[wave + j * NW] = f;
-    }
+    for (int m = 0; m < MOST; ++m) parts[m] = *(const f32x4_t*)(norm.squares + (size_t)min(m, M - 1) * SQUARE_PARTS + 4 * lane);
+    float f[MOST];
+#pragma unroll
+    for (int m = 0; m < MOST; ++m) f[m] = norm.factor(parts[m]);
+    if (lane == 0)
+#pragma unroll
+      for (int m = 0; m < MOST; ++m) factor[m] = f[m];
   }
   const int read_at[2] = {r16 * 128 + 16 * (quad ^ (r16 & 7)), r16 * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
   const int ra = FEW ? r16 & 7 : r16, a_at[2] = {ra * 128 + 16 * (quad ^ (r16 & 7)), ra * 128 + 16 * ((4 + quad) ^ (r16 & 7))};
@@ -342,10 +342,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
   }
   __syncthreads();  // every wave has read its last slot: the rings' room now takes the partial sums
   float* red = (float*)rows_lds;  // [NW][NT][4][64]
+  if (!SCALED || wave < NW)
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[((wave * NT + t) * 4 + r) * 64 + lane] = acc[t][r];
+      for (int r = 0; r < 4; ++r) red[((wave * NT + t) * 4 + r) * 64 + lane] = acc[t][r];
   __syncthreads();
   auto total = [&](int t, int l, float (&sum)[4]) {  // the waves' parts in order
 #pragma unroll
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_bf16_rows_kernel(const bf16_t* _
     }
   };
   // one thread per (tile, lane); gated rows of eight: the gate rows' sums in lanes 0 to 31, their up rows' in the others
-  for (int i = threadIdx.x; i < (GATED ? 1 : NT) * 64; i += 64 * NW) {
+  for (int i = threadIdx.x; i < (GATED ? 1 : NT) * 64; i += 64 * (NW + SCALED)) {
     const int l = i & 63, t = i >> 6;
     const int m = l & 15;
     const int nn = n0 + 16 * t + 4 * (l >> 4);
@@ -383,7 +384,7 @@ template <int NW, int NT, int U, int GATED, bool FEW, bool SCALED>
 static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep,
                        hipStream_t stream, int k_parts, const RowNorm& norm) {
   constexpr int outputs = GATED ? 8 * NT : 16 * NT;
-  dim3 grid((N + outputs - 1) / outputs, k_parts), block(64 * NW);
+  dim3 grid((N + outputs - 1) / outputs, k_parts), block(64 * (NW + SCALED));
   constexpr size_t ring = (size_t)NW * U * ((NT + 1) * 2048 - (FEW ? 1024 : 0)), meet = (size_t)NW * NT * 1024, smem = ring > meet ? ring : meet;
   static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
 #define GO(TO)                                                                                          \
@@ -486,10 +487,14 @@ __device__ bf16x8_t qrt_zero_tile[64];
 //     batch (the others, read one pair ahead of their products).
 // Within a chunk, loads past the end of K are issued all the same, at clamped addresses, and count
 // as zero; behind the last chunk nothing is fetched, and its waits count accordingly.
-template <int MB, int KW, int NWV, int NT, int KC, int GATED, typename TO>
+// SCALED (up to 16 rows): as in the few-row product. The parts of the factors come to LDS in front of everything else, SQUARE_ROW bytes
+// a row (rows begin in different banks), and are added up when the products are done.
+constexpr int SQUARE_ROW = 4 * SQUARE_PARTS + 16;
+template <int MB, int KW, int NWV, int NT, int KC, int GATED, bool SCALED, typename TO>
 __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const bf16_t* __restrict__ A,
                                                                             const bf16_t* __restrict__ W,
-                                                                            TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep) {
+                                                                            TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep,
+                                                                            RowNorm norm) {
   constexpr int WT = GATED ? 2 * NT : NT;  // weight tiles per wave
   constexpr int PAIRS = KC / 2;            // pairs of k-steps per chunk
   constexpr int ACT = KC * MB / NWV;       // loads of activations a wave issues per chunk
@@ -623,12 +628,33 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
       }
     }
   };
+  static_assert(!SCALED || (MB == 1 && KW == 1), "one block of rows");
+  unsigned char* parts = ring + (size_t)(NWV - nw) * PAIRS * WT * 2048;  // behind the last wave's ring
+  if (SCALED)
+    for (int m = nw; m < 16; m += NWV)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(norm.squares + (size_t)min(m, M - 1) * SQUARE_PARTS + 4 * lane),
+                                       (lds_ptr_t)(parts + m * SQUARE_ROW), 16, 0, 0);
   if (chunks > 0) {  // the same in every wave of the block
     fetch_activations(0);
 #pragma unroll
     for (int p = 0; p < PAIRS; ++p) fetch_weights(0, p);
     for (int c = 0; c + 1 < chunks; ++c) run_chunk(c, std::false_type{});
     run_chunk(chunks - 1, std::true_type{});
+  }
+
+  float factor = 1.f;  // of row r16
+  if constexpr (SCALED) {
+    QRT_WAIT_LOADS(0);
+    __syncthreads();
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const f32x4_t v = *(const f32x4_t*)(parts + r16 * SQUARE_ROW + 256 * quad + 16 * i);
+      sum += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    factor = rsqrtf(sum * norm.inv_width + norm.eps);
   }
 
   if (KW > 1) {  // the K groups' sums meet in group 0, added in group order
@@ -667,6 +693,10 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
       float o[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
+        if (SCALED) {
+          acc[t][b][r] *= factor;
+          if (GATED) acc[NT + t][b][r] *= factor;
+        }
         if (GATED) {  // gate and up value rounded to bfloat16 first, as the unfused kernels see them
           const float g = (float)(bf16_t)acc[t][b][r];
           o[r] = ep.template apply<GATED>(g, (float)(bf16_t)acc[NT + t][b][r], m);
@@ -679,9 +709,9 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
   }
 }
 
-template <int MB, int KW, int NWV, int NT, int KC, int GATED>
+template <int MB, int KW, int NWV, int NT, int KC, int GATED, bool SCALED = false>
 static int launch_mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep,
-                           hipStream_t stream, int k_parts) {
+                           hipStream_t stream, int k_parts, const RowNorm& norm = RowNorm{}) {
   constexpr int WT = GATED ? 2 * NT : NT;
   const int per_block = NWV * NT, tiles = N / 16;
   constexpr int COMPUTE_UNITS = 256;  // of an MI355X
@@ -689,22 +719,23 @@ static int launch_mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dt
                                                 : max(COMPUTE_UNITS / k_parts, (tiles + per_block - 1) / per_block);
   blocks = max(blocks, (tiles + per_block - 1) / per_block);
   dim3 grid(blocks, k_parts), block(64 * KW * NWV);
-  constexpr size_t stage = (size_t)KW * 2 * (KC / 2) * MB * 2048 + (size_t)KW * NWV * (KC / 2) * WT * 2048;
+  constexpr size_t stage = (size_t)KW * 2 * (KC / 2) * MB * 2048 + (size_t)KW * NWV * (KC / 2) * WT * 2048 + (SCALED ? 16 * SQUARE_ROW : 0);
   constexpr size_t meet = (size_t)(KW - 1) * NWV * WT * MB * 1024;
   constexpr size_t smem = stage > meet ? stage : meet;
   static_assert(smem <= 160 * 1024, "the staging of this configuration does not fit LDS");
 #define GO(TO)                                                                                          \
   do {                                                                                                  \
-    auto kernel = gemm_bf16_mid_rows_kernel<MB, KW, NWV, NT, KC, GATED, TO>;                            \
+    auto kernel = gemm_bf16_mid_rows_kernel<MB, KW, NWV, NT, KC, GATED, SCALED, TO>;                          \
     static bool allowed = false; /* once per kernel: not inside a stream capture again and again */    \
     if (smem > 64 * 1024 && !allowed) {                                                                 \
       if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) \
         return qrt_fail("gemm_bf16: cannot get %zu bytes of LDS", smem);                                \
       allowed = true;                                                                                   \
     }                                                                                                   \
-    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ep);                                   \
+    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ep, norm);                             \
   } while (0)
   if (out_dtype == QRT_BF16) GO(bf16_t);
+  else if constexpr (SCALED) return qrt_fail("gemm_bf16: rows that lack their norm's factor give bfloat16 (%d asked for)", out_dtype);
   else if (out_dtype == QRT_F32) GO(float);
   else return qrt_fail("gemm_bf16: unknown output dtype %d", out_dtype);
 #undef GO
@@ -833,9 +864,9 @@ extern "C" int qrt_gated_gemm_bf16(const void* a, const void* w, void* c, int ou
 
 // The product, or the gated one, of rows that still lack the factor of their RMS norm: C = act(factor * (A W^T)), bfloat16. `a`
 // [M, K] and `squares` [M, SQUARE_PARTS] as qrt_gemm_residual_bf16 left them, `eps` the norm's; M <= 16, K % 64 == 0.
-// The sums' launch shapes are those of the products of whole rows. gated: -1 none, else an activation of common.h.
-extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M, int N, int K, int gated, float limit, const float* squares,
-                                    float eps, hipStream_t stream) {
+// `shared` chooses the gated product's kernel as in qrt_gemm_bf16. gated: -1 none, else an activation of common.h.
+extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M, int N, int K, int gated, float limit, int shared,
+                                    const float* squares, float eps, hipStream_t stream) {
   QRT_CHECK(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0, "scaled_gemm_bf16: bad sizes M=%d N=%d K=%d", M, N, K);
   QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)squares) % 16 == 0, "scaled_gemm_bf16: operands off 16 bytes");
   QRT_CHECK(gated == -1 || gated == QRT_ACT_SWIGLU || gated == QRT_ACT_CLAMPED, "scaled_gemm_bf16: unknown activation %d", gated);
@@ -843,6 +874,12 @@ extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M
   const bf16_t *A = (const bf16_t*)a, *W = (const bf16_t*)w;
   const RowNorm norm{squares, 1.0f / (float)K, eps};
   const GatedEpilogue ep{gated < 0 ? QRT_ACT_SWIGLU : gated, limit, nullptr};
+  if (shared) {
+    QRT_CHECK(gated >= 0 && N % 16 == 0 && N <= (1 << 20) && K >= 128, "scaled_gemm_bf16: the LDS-sharing kernel is for gated products, "
+              "N %% 16 == 0, N <= 2^20, K >= 128 (N=%d K=%d)", N, K);
+    return gated == QRT_ACT_SWIGLU ? launch_mid_rows<1, 1, 3, 1, 6, 1, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm)
+                                   : launch_mid_rows<1, 1, 3, 1, 6, 2, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm);
+  }
 #define GO(GATED) (M <= 8 ? few_rows<GATED, true, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm) \
                           : few_rows<GATED, false, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm))
   if (gated == -1) return GO(0);

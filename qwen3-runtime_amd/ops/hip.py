@@ -460,8 +460,8 @@ class HipOps:
         n = w.shape[0] if gated < 0 else w.shape[0] // 2
         out = torch.empty((m, n), dtype=torch.bfloat16, device=w.device)
         self._check(self.lib, self.lib.qrt_scaled_gemm_bf16(
-            _ptr(x.rows), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), c_int(gated), c_float(limit), _ptr(x.squares),
-            c_float(x.eps), _stream()))
+            _ptr(x.rows), _ptr(w), _ptr(out), c_int(m), c_int(n), c_int(k), c_int(gated), c_float(limit),
+            c_int(int(gated >= 0 and self._own_kernel(m, n, k, "gated") == 1)), _ptr(x.squares), c_float(x.eps), _stream()))
         return out
 
     def _norm_add_rmsnorm(self, residual, y, w_after, eps_after, weight, eps, out_dtype, rows):
