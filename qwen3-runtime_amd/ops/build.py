@@ -31,6 +31,8 @@ FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
     # packed float32 instructions stay off: some of their forms have returned wrong results
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # a kernel's first arguments come in registers with its waves instead of by a load that every wave starts with
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 # further hipcc flags (for instance -D switches of a kernel under tuning); part of the libraries' hash
 FLAGS += os.environ.get("QWEN3_RUNTIME_AMD_HIPCC_FLAGS", "").split()
