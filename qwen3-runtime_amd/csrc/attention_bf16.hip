@@ -1563,44 +1563,71 @@ __device__ __forceinline__ void block_compute(KvBlock& blk, const bf16x8_t* qreg
 // queries and keys to memory does. A lane holds elements 32 i + 8 quad .. + 7 of k-step i, so a
 // pair lies in one lane (k-steps i and i + pairs / 32) and the head's sum of squares in the four
 // lanes of a row.
-__device__ __forceinline__ void head_as_operand(const bf16_t* __restrict__ x, const float* __restrict__ w,
-                                                const float* __restrict__ rope, int pairs, float eps, int quad,
-                                                bf16x8_t* out) {
-  constexpr int KF = KFULL > 0 ? KFULL : 1;
+// What it takes is asked for in one go by load_head, in front of the keys: behind them every wait for it would be one for the keys
+// as well (loads come back in order), and weights and angles a trip to memory each.
+// SURE: there are weights, and all pairs turn.
+constexpr int KF = KFULL > 0 ? KFULL : 1, KH = KF > 1 ? KF / 2 : 1;
+struct HeadLoads {
+  bf16x8_t x[KF];
+  f32x4_t w[KF][2], cs[KH][2], sn[KH][2];
+};
+template <bool SURE>
+__device__ __forceinline__ void load_head(const bf16_t* __restrict__ x, const float* __restrict__ w, const float* __restrict__ rope, int pairs,
+                                          int quad, HeadLoads& h) {
+#pragma unroll
+  for (int i = 0; i < KF; ++i) h.x[i] = *(const bf16x8_t*)(x + 32 * i + 8 * quad);
+  if (SURE || w) {
+#pragma unroll
+    for (int i = 0; i < KF; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) h.w[i][e] = *(const f32x4_t*)(w + 32 * i + 8 * quad + 4 * e);
+  }
+  if (SURE || rope) {
+    const int steps = SURE ? KH : pairs >> 5;  // the same for the whole launch
+#pragma unroll
+    for (int i = 0; i < KH; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int j = 32 * min(i, steps - 1) + 8 * quad + 4 * e;
+        h.cs[i][e] = *(const f32x4_t*)(rope + j);
+        h.sn[i][e] = *(const f32x4_t*)(rope + 32 * steps + j);
+      }
+  }
+}
+template <bool SURE>
+__device__ __forceinline__ void head_as_operand(const HeadLoads& h, const f32x4_t (*cs)[2], const f32x4_t (*sn)[2], bool normed, bool turns, int pairs,
+                                                float eps, bf16x8_t* out) {
   float v[KF][8];
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < KF; ++i) {
-    const bf16x8_t r = *(const bf16x8_t*)(x + 32 * i + 8 * quad);
+  for (int i = 0; i < KF; ++i)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[i][e] = (float)r[e];
+      v[i][e] = (float)h.x[i][e];
       ss += v[i][e] * v[i][e];
     }
-  }
-  if (w) {
+  if (SURE || normed) {
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
     const float inv = rsqrtf(ss / (float)D + eps);
 #pragma unroll
     for (int i = 0; i < KF; ++i)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * inv * w[32 * i + 8 * quad + e];
+      for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * inv * h.w[i][e >> 2][e & 3];
   }
-  if (rope) {
-    const int steps = pairs >> 5;  // the same for the whole launch
+  if (SURE || turns) {
+    const int steps = SURE ? KH : pairs >> 5;
 #pragma unroll
-    for (int n = 1; n <= KF / 2; ++n) {
+    for (int n = SURE ? KH : 1; n <= KF / 2; ++n) {
       if (n != steps) continue;
 #pragma unroll
       for (int i = 0; i < n; ++i)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int j = 32 * i + 8 * quad + e;
-          const float cs = rope[j], sn = rope[32 * n + j];
+          const float c = cs[i][e >> 2][e & 3], s = sn[i][e >> 2][e & 3];
           const float x1 = v[i][e], x2 = v[i + n][e];
-          v[i][e] = x1 * cs - x2 * sn;
-          v[i + n][e] = x2 * cs + x1 * sn;
+          v[i][e] = x1 * c - x2 * s;
+          v[i + n][e] = x2 * c + x1 * s;
         }
     }
   }
@@ -1640,17 +1667,18 @@ __device__ __forceinline__ void ring_fetch(const AttnTileArgs& a, int kvh, int b
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
   constexpr int A_ROW = D / 8;  // lanes a key
   const int ps = a.page_size;
+  const int g_last = (pos_max - base) >> 3;  // what a table holds for groups behind it is not looked at
   auto first_key = [&](int g) { return page_mod<P2>(min(max(base + 8 * g, lo & ~7), pos_max & ~7), ps); };
 #pragma unroll
   for (int j = 0; j < D / 16; ++j) {
     const int row = j * (64 / A_ROW) + lane / A_ROW, r = row & 15, g = r >> 2;
-    const int page = __shfl(pages, 4 * i + g, 64), off = first_key(g) + 4 * (row >> 4) + (r & 3);
+    const int page = __shfl(pages, 4 * i + min(g, g_last), 64), off = first_key(g) + 4 * (row >> 4) + (r & 3);
     const int piece = (lane % A_ROW) ^ (D % 128 == 0 ? r : r >> 1);
     const bf16_t* src = a.k_cache + (((size_t)page * a.nkv + kvh) * ps + off) * D + 8 * piece;
     __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(ring + j * 1024), 16, 0, ONCE);
   }
   const int g = (lane & 3) ^ (lane >> 4);
-  const bf16_t* src = a.v_cache + (((size_t)__shfl(pages, 4 * i + g, 64) * a.nkv + kvh) * DV + (lane >> 2)) * ps + first_key(g);
+  const bf16_t* src = a.v_cache + (((size_t)__shfl(pages, 4 * i + min(g, g_last), 64) * a.nkv + kvh) * DV + (lane >> 2)) * ps + first_key(g);
 #pragma unroll
   for (int j = 0; j < DB; ++j)
     __builtin_amdgcn_global_load_lds((global_ptr_t)(src + (size_t)16 * j * ps), (lds_ptr_t)(ring + RING_KEYS + j * 1024), 16, 0, ONCE);
@@ -1668,8 +1696,26 @@ __device__ __forceinline__ void ring_read(const unsigned char* ring, int r16, in
 
 constexpr bool DECODE_ONCE = true;  // measured: 2 % off a decode step at batch 1 and at batch 64, level at batch 8
 
-template <bool P2, bool FUSED = false>
-__global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_decode_kernel(AttnTileArgs a) {
+// What bounds a launch of few or short sequences is its chain of trips to memory, 0.7 to 1 us each: length and pages, keys, and the
+// token's own head. A decode pass of the 4B size, us a step, by what was on the chain: the token's loads behind the keys', weights and angles behind
+// its elements, its value's eight elements one by one under a condition, the first pages behind the length 2,021 (1 request of 2,049 keys)
+// and 2,492 (8); all asked for at one time 1,941 and 2,390.
+// What a wave needs for its first keys comes as arguments of its own, which fill the registers that come with a wave: a structure
+// is loaded by every wave, 0.2 to 0.5 us before anything else. `heads`: 256 key heads + query heads a key head. PLAIN: one token per
+// sequence, equal parts of whole contexts, normed and wholly turned heads, no cap, gate, sink or turned values.
+template <bool P2, bool FUSED = false, bool PLAIN = false>
+__global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_decode_kernel(
+    const int* kv_lens, const int* block_table, const bf16_t* k_cache, const bf16_t* v_cache, const bf16_t* qkv, int table_width, int num_splits,
+    int page_size, int heads, AttnTileArgs args) {
+  static_assert(!PLAIN || (FUSED && DECODE_RING), "the plain form takes keys by the ring");
+  AttnTileArgs a = args;  // the fields known here stand for the structure's
+  a.kv_lens = kv_lens, a.block_table = block_table, a.k_cache = k_cache, a.v_cache = v_cache, a.qkv = qkv;
+  a.table_width = table_width, a.num_splits = num_splits, a.page_size = page_size, a.nkv = heads >> 8, a.nq = a.nkv * (heads & 255);
+  if (PLAIN) {
+    a.items = nullptr, a.tile_seq = nullptr, a.gate = nullptr, a.turn = nullptr;
+    a.window = a.chunk = a.keep_first = a.sink = 0;
+    a.cap_in = a.cap_out = 0.f;
+  }
   // per wave: maximum and sum per row, unnormalised accumulator [16][DV]
   extern __shared__ float lds[];
   float* lds_m = lds;                 // [DW][16]
@@ -1694,18 +1740,30 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     kvh = blockIdx.y;
     split = blockIdx.z;
   }
-  const int g = a.nq / a.nkv;
-  const int q_begin = a.cu_q[seq];
-  const int q_len = a.cu_q[seq + 1] - q_begin;
+  // Equal parts of whole contexts, one token each: the waves of all parts take a sequence's blocks of keys in turn, whatever
+  // their number, so that a wave's first pages are asked for beside the context's length and not behind it. The two that add and
+  // store the token's own key take none where there are parts enough.
+  constexpr bool in_turn = PLAIN;
+  const int turns = a.num_splits * DW - (a.num_splits >= 4 ? 2 : 0);
+  const int* table = a.block_table + (size_t)seq * a.table_width;
+  int pages = 0;
+  if (in_turn) {
+    const int key = ((split * DW + wave + (lane >> 2) * turns) << 5) + 8 * (lane & 3);
+    // (an atomic load because a plain one would be moved down behind the question whether the wave has keys)
+    pages = __hip_atomic_load(table + min(page_div<P2>(key, a.page_size, __builtin_ctz(a.page_size)), a.table_width - 1), __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  const int g = heads & 255;
+  const int q_begin = FUSED ? seq : a.cu_q[seq];
+  const int q_len = FUSED ? 1 : a.cu_q[seq + 1] - q_begin;
   const int kv_len = a.kv_lens[seq];
   const int n_rows = q_len * g;  // <= 16 by the launch condition
   const int first_pos = kv_len - q_len;
   const bool row_valid = r16 < n_rows;
   const int row_c = row_valid ? r16 : max(n_rows - 1, 0);
-  const int tok = row_c / g, hg = row_c - tok * g;
+  const int tok = FUSED ? 0 : row_c / g, hg = row_c - tok * g;
   const int qpos = first_pos + tok;
   const int head = kvh * g + hg;
-  const int* table = a.block_table + (size_t)seq * a.table_width;
 
   f32x4_t o[DB];
 #pragma unroll
@@ -1718,16 +1776,18 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   const int own = FUSED ? 1 : 0;
   const int window = FUSED && a.window > 0 ? a.window - 1 : a.window;
   const int qpos_c = qpos - own;
-  const int pos_min = first_pos - own, pos_max = first_pos + (max(n_rows, 1) - 1) / g - own;
+  const int pos_min = first_pos - own, pos_max = first_pos + (FUSED ? 0 : (max(n_rows, 1) - 1) / g) - own;
   const int lo = max(0, first_seen(first_pos, a.window, a.chunk));
   int blk_begin, blk_end;
   decode_key_blocks(kv_len, q_len, a.window, a.chunk, FUSED, blk_begin, blk_end);
   // equal parts of the sequence's blocks: as many as all sequences have, or as pieces of at most a given length make
-  const int per = a.items ? piece_blocks(blk_end - blk_begin, longest_piece) : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
-  const int last_split = a.items ? max(1, (blk_end - blk_begin + per - 1) / per) - 1 : (int)gridDim.z - 1;
-  const int b0 = blk_begin + split * per;
-  const int b1 = min(blk_end, b0 + per);
+  const int per = in_turn ? 0 : a.items ? piece_blocks(blk_end - blk_begin, longest_piece) : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
+  const int last_split = a.items ? max(1, (blk_end - blk_begin + per - 1) / per) - 1 : a.num_splits - 1;
+  const int b0 = in_turn ? split * DW : blk_begin + split * per;
+  const int b1 = in_turn ? blk_end : min(blk_end, b0 + per);
+  const int step = in_turn ? turns : DW;
   int b = b0 + wave;
+  if (in_turn && b >= turns) b = b1;
 
   bf16x8_t qreg[KFULL > 0 ? KFULL : 1];
   bf16x8_t qtail = load_tail((const bf16_t*)nullptr, 2);  // zeros
@@ -1735,24 +1795,35 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   // token's own key and value, the wave before it stores them into the cache (these have the
   // fewest blocks of cached keys: the blocks go round the waves, and the last split takes what
   // the others left)
-  auto own_token = [&]() {
-    const bf16_t* raw = a.qkv + (size_t)q_begin * a.qkv_stride;
+  const bool at_end = FUSED && split == last_split;
+  const bool adds_own = at_end && wave == DW - 1, stores_own = at_end && wave == (2 * DW - 2) % DW;
+  const bf16_t* raw = a.qkv + (size_t)q_begin * a.qkv_stride;
+  const bf16_t *kraw = raw + ((size_t)a.nq + kvh) * D, *vraw = raw + ((size_t)a.nq + a.nkv) * D + (size_t)kvh * DV;
+  HeadLoads of_query, of_key;
+  bf16_t own_v[DB], kept_v[(DV + 63) / 64];
+  auto load_token = [&]() {
     const float* rope = a.rope ? a.rope + (size_t)q_begin * 2 * a.rope_pairs : nullptr;
-    const float* turn = a.turn ? a.turn + (size_t)q_begin * DV : nullptr;
-    head_as_operand(raw + (size_t)head * D, a.q_weight, rope, a.rope_pairs, a.eps, quad, qreg);
-    const bool at_end = split == last_split;
-    const bool adds_own = at_end && wave == DW - 1, stores_own = at_end && wave == (2 * DW - 2) % DW;
+    load_head<PLAIN>(raw + (size_t)head * D, a.q_weight, rope, a.rope_pairs, quad, of_query);
     if (adds_own || stores_own) {  // uniform over the wave
-      const bf16_t* kraw = raw + ((size_t)a.nq + kvh) * D;
-      const bf16_t* vraw = raw + ((size_t)a.nq + a.nkv) * D + (size_t)kvh * DV;
+      load_head<PLAIN>(kraw, a.k_weight, rope, a.rope_pairs, quad, of_key);
+#pragma unroll
+      for (int i = 0; i < DB; ++i) own_v[i] = vraw[16 * i + r16];
+#pragma unroll
+      for (int k = 0; k < (DV + 63) / 64; ++k) kept_v[k] = vraw[min(lane + 64 * k, DV - 1)];
+    }
+  };
+  auto own_token = [&]() {
+    const float* turn = a.turn ? a.turn + (size_t)q_begin * DV : nullptr;
+    head_as_operand<PLAIN>(of_query, of_query.cs, of_query.sn, a.q_weight, a.rope, a.rope_pairs, a.eps, qreg);
+    if (adds_own || stores_own) {  // uniform over the wave
       bf16x8_t kreg[KFULL > 0 ? KFULL : 1];
-      head_as_operand(kraw, a.k_weight, rope, a.rope_pairs, a.eps, quad, kreg);
+      head_as_operand<PLAIN>(of_key, of_query.cs, of_query.sn, a.k_weight, a.rope, a.rope_pairs, a.eps, kreg);
       // the token's own value, turned by its position where values are
-      auto own_value = [&](int d) -> bf16_t {
-        if (!turn) return vraw[d];
+      auto own_value = [&](int d, bf16_t as_is) -> bf16_t {
+        if (!turn) return as_is;
         const bool low = d < DV / 2;
         const int j = low ? d : d - DV / 2;
-        const float x = (float)vraw[d], y = (float)vraw[low ? d + DV / 2 : j], c = turn[j], sn = turn[DV / 2 + j];
+        const float x = (float)as_is, y = (float)vraw[low ? d + DV / 2 : j], c = turn[j], sn = turn[DV / 2 + j];
         return (bf16_t)(low ? x * c - y * sn : x * c + y * sn);
       };
       if (stores_own) {
@@ -1764,7 +1835,12 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
 #pragma unroll
           for (int i = 0; i < KFULL; ++i) *(bf16x8_t*)(kdst + 32 * i + 8 * quad) = kreg[i];
         }
-        for (int d = lane; d < DV; d += 64) vdst[(size_t)d * a.page_size] = own_value(d);
+#pragma unroll
+        for (int k = 0; k < (DV + 63) / 64; ++k) {
+          const int d = lane + 64 * k;
+          const bf16_t v = own_value(min(d, DV - 1), kept_v[k]);
+          if (d < DV) vdst[(size_t)d * a.page_size] = v;
+        }
       }
       if (adds_own) {
         // a block of keys that holds this one key, in the place of key first_pos: operand row 0
@@ -1780,7 +1856,8 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
         for (int i = 0; i < DB; ++i) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) vv[i][e] = (bf16_t)0.0f;
-          if (quad == 0) vv[i][0] = own_value(16 * i + r16);
+          const bf16_t v = own_value(16 * i + r16, own_v[i]);  // not under the condition: its loads would come one by one
+          vv[i][0] = quad == 0 ? v : (bf16_t)0.0f;
         }
         tile_update(sc, vv, true, first_pos, quad, row_valid, qpos, a.window, a.chunk, 0, 0, a.scale_log2, m, l, o);
       }
@@ -1795,23 +1872,28 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
       if (KTAIL) qtail = load_tail(qp + 32 * KFULL, quad);
     }
 
-    const int last = b + (b1 - 1 - b) / DW * DW;
+    auto last_from = [&](int first) { return first + (b1 - 1 - first) / step * step; };
     if constexpr (DECODE_RING) {
       unsigned char* ring = (unsigned char*)(lds_o + wave * O_WAVE);
-      int pages = ring_pages<P2>(table, b, DW, last, lo, pos_max, a.page_size, lane), i = 0;
+      int i = 0;
+      if (FUSED) load_token();
+      if (!in_turn) pages = ring_pages<P2>(table, b, step, last_from(b), lo, pos_max, a.page_size, lane);
+      // everything so far, which was asked for at one time: the compiler waits for loads in front of direct ones by waiting for all
+      if (FUSED) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       ring_fetch<P2>(a, kvh, b << 5, lo, pos_max, pages, 0, lane, ring);
+      __builtin_amdgcn_sched_barrier(0);  // nothing that waits for the token's loads moves in between the keys'
       if (FUSED) own_token();  // while the first keys and values are on their way
       KvBlock blk;
-      for (; b < b1; b += DW) {
+      for (; b < b1; b += step) {
         QRT_WAIT_LOADS(0);
         ring_read(ring, r16, quad, blk);
         QRT_WAIT_LDS();  // the block is in registers: the next one may overwrite it
-        if (b + DW < b1) {
+        if (b + step < b1) {
           if (++i == 16) {
-            pages = ring_pages<P2>(table, b + DW, DW, last, lo, pos_max, a.page_size, lane);
+            pages = ring_pages<P2>(table, b + step, step, last_from(b + step), lo, pos_max, a.page_size, lane);
             i = 0;
           }
-          ring_fetch<P2>(a, kvh, (b + DW) << 5, lo, pos_max, pages, i, lane, ring);
+          ring_fetch<P2>(a, kvh, (b + step) << 5, lo, pos_max, pages, i, lane, ring);
         }
         block_compute(blk, qreg, qtail, b << 5, lo, pos_min, pos_max, quad, row_valid, qpos_c, window, a.chunk, a.keep_first, a.cap_in, a.cap_out, a.scale_log2, m, l, o);
       }
@@ -1819,8 +1901,10 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     // two blocks of keys and values are on their way while a third is multiplied, and the page
     // numbers of the two after them; past the wave's last block the loads go on (one shape of
     // loop, no load under a branch) but fetch next to nothing
+    const int last = last_from(b);
     KvBlock A, B;
     int pgA[3], pgB[3];
+    if (FUSED) load_token();
     block_pages<P2>(table, b << 5, lo, pos_max, a.page_size, r16, quad, pgA);
     block_pages<P2>(table, min(b + DW, last) << 5, lo, pos_max, a.page_size, r16, quad, pgB);
     block_load<P2, DECODE_ONCE>(a, kvh, b << 5, lo, pos_max, r16, quad, pgA, A);
@@ -1842,6 +1926,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     }
     }
   } else if (FUSED) {
+    load_token();
     own_token();
   }
   if (a.keep_first > 0 && split == 0 && wave == 0 && n_rows > 0) {  // uniform over the wave
@@ -1910,7 +1995,7 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     if (row >= n_rows) continue;
     float mm, den;
     const float val = joined(row, d, mm, den);
-    const int rt = row / g, rh = row - rt * g;
+    const int rt = FUSED ? 0 : row / g, rh = row - rt * g;
     const size_t row_index = tile_row0 + (size_t)rt * a.nq + kvh * g + rh;
     if (a.num_splits == 1) {
       a.out[row_index * DV + d] = (bf16_t)(val * gate_factor(a.gate, a.gate_stride, a.nq, row_index, d));
@@ -1945,6 +2030,35 @@ extern "C" int qrt_attention_work_list(const AttnTileArgs* args, int fused, hipS
   return 0;
 }
 
+template <bool P2, bool FUSED, bool PLAIN>
+static int launch_decode(const AttnTileArgs& a, dim3 grid, hipStream_t stream) {
+  constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (DECODE_RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
+  static_assert(!DECODE_RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
+  auto kernel = attention_bf16_decode_kernel<P2, FUSED, PLAIN>;
+  static bool allowed = false;  // once per kernel: not again inside every stream capture
+  if (smem > 64 * 1024 && !allowed) {  // rings of heads of 128, accumulators of 256: a little more LDS than a block gets without asking
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+      return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
+    allowed = true;
+  }
+  kernel<<<grid, 64 * DW, smem, stream>>>(a.kv_lens, a.block_table, a.k_cache, a.v_cache, a.qkv, a.table_width, a.num_splits, a.page_size,
+                                          a.nkv << 8 | a.nq / a.nkv, a);
+  QRT_LAUNCH_CHECK("attention_bf16_decode");
+  return 0;
+}
+
+// the parts of the keys joined, where there are several
+static int finish_decode(const AttnTileArgs& a, int num_rows_total, hipStream_t stream) {
+  if (a.num_splits > 1) {
+    const int merge_rows = a.merge_tokens ? a.num_merge_tokens * a.nq : num_rows_total;
+    if (merge_rows > 0)
+      attention_merge_kernel<<<dim3(merge_rows), dim3(DV > 128 ? 256 : (DV >= 64 ? 64 : 32)), 0, stream>>>(
+          a.part_o, a.part_lse, a.out, a.num_splits, a.merge_tokens, a.nq, a.gate, a.gate_stride, a.sink, a.turn);
+    QRT_LAUNCH_CHECK("attention_merge");
+  }
+  return 0;
+}
+
 // every listed sequence at most 16 rows (q_len * g <= 16) and D <= 256; num_tiles = number of
 // sequences; tile_seq lists them, or is null for all sequences of the step in order
 extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_total, hipStream_t stream) {
@@ -1968,21 +2082,8 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
             a.max_items, a.num_tiles);
   if (a.num_tiles == 0) return 0;
   const bool p2 = (a.page_size & (a.page_size - 1)) == 0;  // shifts instead of divisions
-  dim3 grid(a.num_tiles, a.nkv, a.num_splits), block(64 * DW);
+  dim3 grid(a.num_tiles, a.nkv, a.num_splits);
   if (a.items) grid = dim3(a.nkv, a.max_items, 1);
-  constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (DECODE_RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
-  static_assert(!DECODE_RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
-  if (smem > 64 * 1024) {  // rings of heads of 128, accumulators of 256: a little more LDS than a block gets without asking
-    static bool allowed = false;  // once: not again inside every stream capture
-    if (!allowed) {
-      if (hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess ||
-          hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<false>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-        return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
-      allowed = true;
-    }
-  }
   if (a.qkv) {
     // one token per sequence, its query, key and value taken from the product that made them
     if constexpr (D % 64 == 0) {
@@ -1992,33 +2093,20 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
                 a.nq / a.nkv, a.qkv_stride);
       QRT_CHECK(!a.rope || (a.rope_pairs >= 32 && a.rope_pairs % 32 == 0 && a.rope_pairs <= D / 2),
                 "attention (decode, own token from the product): %d pairs turn (multiples of 32 up to %d)", a.rope_pairs, D / 2);
-      if (smem > 64 * 1024) {
-        static bool allowed_fused = false;
-        if (!allowed_fused) {
-          if (hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<true, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess ||
-              hipFuncSetAttribute((const void*)attention_bf16_decode_kernel<false, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-            return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
-          allowed_fused = true;
+      if constexpr (DECODE_RING) {
+        const bool plain = !a.items && !a.tile_seq && a.window == 0 && a.chunk == 0 && a.cap_in == 0.f && !a.gate && !a.turn && !a.sink && a.q_weight &&
+                           a.k_weight && a.rope && 2 * a.rope_pairs == D;
+        if (plain) {
+          if (const int rc = p2 ? launch_decode<true, true, true>(a, grid, stream) : launch_decode<false, true, true>(a, grid, stream)) return rc;
+          return finish_decode(a, num_rows_total, stream);
         }
       }
-      if (p2) attention_bf16_decode_kernel<true, true><<<grid, block, smem, stream>>>(a);
-      else attention_bf16_decode_kernel<false, true><<<grid, block, smem, stream>>>(a);
+      if (const int rc = p2 ? launch_decode<true, true, false>(a, grid, stream) : launch_decode<false, true, false>(a, grid, stream)) return rc;
     } else {
       return qrt_fail("attention (decode, own token from the product): head size %d is no multiple of 64", D);
     }
-  } else if (p2) attention_bf16_decode_kernel<true><<<grid, block, smem, stream>>>(a);
-  else attention_bf16_decode_kernel<false><<<grid, block, smem, stream>>>(a);
-  QRT_LAUNCH_CHECK("attention_bf16_decode");
-  if (a.num_splits > 1) {
-    const int merge_rows = a.merge_tokens ? a.num_merge_tokens * a.nq : num_rows_total;
-    if (merge_rows > 0)
-      attention_merge_kernel<<<dim3(merge_rows), dim3(DV > 128 ? 256 : (DV >= 64 ? 64 : 32)), 0, stream>>>(
-          a.part_o, a.part_lse, a.out, a.num_splits, a.merge_tokens, a.nq, a.gate, a.gate_stride, a.sink, a.turn);
-    QRT_LAUNCH_CHECK("attention_merge");
-  }
-  return 0;
+  } else if (const int rc = p2 ? launch_decode<true, false, false>(a, grid, stream) : launch_decode<false, false, false>(a, grid, stream)) return rc;
+  return finish_decode(a, num_rows_total, stream);
 }
 
 extern "C" int qrt_attention_bf16(const AttnTileArgs* args, int num_rows_total, hipStream_t stream) {

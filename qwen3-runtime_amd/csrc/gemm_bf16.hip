@@ -256,7 +256,7 @@ static int skinny(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int 
 template <int NW, int NT, int U, int GATED, bool FEW, bool SCALED, typename TO>
 __global__ __launch_bounds__(64 * (NW + SCALED)) void gemm_bf16_rows_kernel(const bf16_t* __restrict__ A,
                                                                   const bf16_t* __restrict__ W,
-                                                                  TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep, RowNorm norm) {
+                                                                  TO* __restrict__ C, int M, int N, int K, int part, GatedEpilogue ep, RowNorm norm) {
   constexpr bool MIXED = GATED && NT == 1;
   constexpr int UNITS = NT + 1, LOADS = 2 * UNITS - FEW, SLOT = UNITS * 2048 - (FEW ? 1024 : 0);
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
@@ -278,7 +278,6 @@ __global__ __launch_bounds__(64 * (NW + SCALED)) void gemm_bf16_rows_kernel(cons
     src[NT][j] = A + (size_t)min(8 * j + sub, M - 1) * K + 8 * piece;
   }
   const int all_pairs = K >> 6;
-  const int part = (all_pairs + gridDim.y - 1) / gridDim.y;
   const int p_first = blockIdx.y * part, p_end = min(all_pairs, p_first + part);
   const int mine = wave < NW ? max(0, (p_end - p_first - wave + NW - 1) / NW) : 0;  // pairs of this wave
   C += (size_t)blockIdx.y * M * N;
@@ -396,7 +395,7 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
         return qrt_fail("gemm_bf16: cannot get %zu bytes of LDS", smem);                                \
       allowed = true;                                                                                   \
     }                                                                                                   \
-    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ep, norm);                             \
+    kernel<<<grid, block, smem, stream>>>(a, w, (TO*)c, M, N, K, ((K >> 6) + k_parts - 1) / k_parts, ep, norm); \
   } while (0)
   if (out_dtype == QRT_BF16) GO(bf16_t);
   else if constexpr (SCALED) return qrt_fail("gemm_bf16: rows that lack their norm's factor give bfloat16 (%d asked for)", out_dtype);

@@ -21,9 +21,9 @@
 
 // AR rows of activations and WR weight rows, in units of eight, are fetched.
 template <int NW, int U, int AR, int WR>
-__global__ __launch_bounds__(64 * NW) void gemm_residual_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                                                 float* __restrict__ residual, const float* __restrict__ weight,
-                                                                 bf16_t* __restrict__ out, float* __restrict__ squares, int M, int N, int K) {
+__global__ __launch_bounds__(64 * NW) void gemm_residual_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int M, int N,
+                                                                 int K, float* __restrict__ residual, const float* __restrict__ weight,
+                                                                 bf16_t* __restrict__ out, float* __restrict__ squares) {
   constexpr int WL = WR / 8, AL = AR / 8, LOADS = WL + AL, SLOT = LOADS * 1024;
   constexpr int ONCE = 2;  // the cache policy of a non-temporal load
   static_assert(WR <= 16 && AR <= 16 && NW >= 4 && (U - 1) * LOADS < 64, "one MFMA tile, a thread an element, the loads' counter");
@@ -126,7 +126,7 @@ static int launch(const bf16_t* a, const bf16_t* w, float* residual, const float
       return qrt_fail("gemm_residual: cannot get %zu bytes of LDS", smem);
     allowed = true;
   }
-  kernel<<<SQUARE_PARTS, 64 * NW, smem, stream>>>(a, w, residual, weight, out, squares, M, N, K);
+  kernel<<<SQUARE_PARTS, 64 * NW, smem, stream>>>(a, w, M, N, K, residual, weight, out, squares);
   QRT_LAUNCH_CHECK("gemm_residual");
   return 0;
 }
