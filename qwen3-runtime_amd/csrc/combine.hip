@@ -247,30 +247,13 @@ __device__ __forceinline__ void planes_piece(const Planes& y, size_t i, float* v
   }
 }
 
-// wave_sum with the same additions, lanes 32, 16, 8, 4, 2 and 1 apart, but by swaps and rotations of registers: after each of
-// them lanes that far apart hold the same, so a rotation within 16 lanes brings the partner's.
-__device__ __forceinline__ float wave_sum_in_registers(float x) {
-  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-  const unsigned int u = __float_as_uint(x);
-  const u32x2_t a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const unsigned int v = __float_as_uint(x);
-  const u32x2_t b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  x = __uint_as_float(b[0]) + __uint_as_float(b[1]);
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, true));  // row_ror:8
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, true));  // row_ror:4
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xF, 0xF, true));  // row_ror:2
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xF, 0xF, true));  // row_ror:1
-  return x;
-}
-
 // The sum of N values a thread over a block of THREADS threads, with one barrier. The parts are added in the order of the
 // elements, 64 threads' pieces of the row at a time, so that a block of a quarter of the threads with four pieces each sums as the whole one.
 template <int THREADS, int N>
 __device__ __forceinline__ float block_sum_once(const float* x, float* red) {
   float z[N];
 #pragma unroll
-  for (int j = 0; j < N; ++j) z[j] = wave_sum_in_registers(x[j]);
+  for (int j = 0; j < N; ++j) z[j] = wave_sum(x[j]);
   if ((threadIdx.x & 63) == 0)
 #pragma unroll
     for (int j = 0; j < N; ++j) red[j * (THREADS / 64) + (threadIdx.x >> 6)] = z[j];

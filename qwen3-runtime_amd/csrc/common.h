@@ -82,46 +82,53 @@ __device__ __forceinline__ float gated_act(float g, float u, int kind, float lim
   return g / (1.0f + expf(-g)) * u;
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+// What lanes 32, 16, 8, 4, 2 and 1 apart hold, joined step by step: by swaps and rotations of registers, where a shuffle through
+// LDS takes some 60 cycles a step (after each step lanes that far apart hold the same, so a rotation within 16 lanes brings the
+// partner's). Every lane of the wave takes part. A norm's block sums and the serial loop they ended with took 1 of 5.8 us.
+template <class Join>
+__device__ __forceinline__ float wave_join(float x, Join join) {
+  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+  const unsigned int u = __float_as_uint(x);
+  const u32x2_t a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  x = join(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const unsigned int v = __float_as_uint(x);
+  const u32x2_t b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  x = join(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  x = join(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, true)));  // row_ror:8
+  x = join(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, true)));  // row_ror:4
+  x = join(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xF, 0xF, true)));  // row_ror:2
+  x = join(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xF, 0xF, true)));  // row_ror:1
   return x;
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  return wave_join(x, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
-  return x;
+  return wave_join(x, [](float a, float b) { return fmaxf(a, b); });
 }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.
-// `red` is shared memory of at least 17 floats. Order of additions is fixed.
-__device__ __forceinline__ float block_sum(float x, float* red) {
-  x = wave_sum(x);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nw = (blockDim.x + 63) >> 6;
+// Sum over a block of up to 1024 threads, in whole waves; every thread gets the result, from
+// parts that all of them add in the order of the waves. `red` is shared memory of at least 16 floats.
+template <class Join>
+__device__ __forceinline__ float block_join(float x, float* red, float none, Join join) {
+  x = wave_join(x, join);
+  const int wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   __syncthreads();
-  if (lane == 0) red[wave] = x;
+  if ((threadIdx.x & 63) == 0) red[wave] = x;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int i = 0; i < nw; ++i) s += red[i];
-    red[16] = s;
+  float s = none;
+  if (nw <= 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s = i < nw ? join(s, red[i]) : s;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s = i < nw ? join(s, red[i]) : s;
   }
-  __syncthreads();
-  return red[16];
+  return s;
+}
+__device__ __forceinline__ float block_sum(float x, float* red) {
+  return block_join(x, red, 0.f, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float block_max(float x, float* red) {
-  x = wave_max(x);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nw = (blockDim.x + 63) >> 6;
-  __syncthreads();
-  if (lane == 0) red[wave] = x;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = red[0];
-    for (int i = 1; i < nw; ++i) s = fmaxf(s, red[i]);
-    red[16] = s;
-  }
-  __syncthreads();
-  return red[16];
+  return block_join(x, red, -INFINITY, [](float a, float b) { return fmaxf(a, b); });
 }

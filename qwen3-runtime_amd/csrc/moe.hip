@@ -248,14 +248,35 @@ __global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restri
     float acc[TB];
 #pragma unroll
     for (int t = 0; t < TB; ++t) acc[t] = 0.f;
-#pragma unroll (TB > 1 ? 2 : 8)
-    for (int c = lane * 4; c < hidden; c += 256) {
-      const f32x4_t wv = *(const f32x4_t*)(wr + c);
+    if (TB == 1) {  // pieces of ROUTE_AHEAD at a time, all asked for before the first is used (beyond the row: its last, not used)
+      constexpr int ROUTE_AHEAD = 12;
+      for (int c0 = lane * 4; c0 < hidden; c0 += 256 * ROUTE_AHEAD) {
+        f32x4_t wv[ROUTE_AHEAD];
+        xvec_t xv[ROUTE_AHEAD];
 #pragma unroll
-      for (int t = 0; t < TB; ++t) {
-        const xvec_t xv = TB > 1 ? *(const xvec_t*)(xs + (size_t)t * hidden + c) : *(const xvec_t*)(x + (size_t)t0 * hidden + c);
+        for (int i = 0; i < ROUTE_AHEAD; ++i) {
+          const int c = min(c0 + 256 * i, hidden - 4);
+          wv[i] = *(const f32x4_t*)(wr + c);
+          xv[i] = *(const xvec_t*)(x + (size_t)t0 * hidden + c);
+        }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc[t] = fmaf(to_f32<T>(xv[k]), wv[k], acc[t]);
+        for (int i = 0; i < ROUTE_AHEAD; ++i) {
+          float sum = acc[0];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) sum = fmaf(to_f32<T>(xv[i][k]), wv[i][k], sum);
+          acc[0] = c0 + 256 * i < hidden ? sum : acc[0];  // no branch: loads would move into it
+        }
+      }
+    } else {
+#pragma unroll 2
+      for (int c = lane * 4; c < hidden; c += 256) {
+        const f32x4_t wv = *(const f32x4_t*)(wr + c);
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+          const xvec_t xv = *(const xvec_t*)(xs + (size_t)t * hidden + c);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) acc[t] = fmaf(to_f32<T>(xv[k]), wv[k], acc[t]);
+        }
       }
     }
 #pragma unroll
