@@ -320,6 +320,8 @@ class HipOps:
     shared_from_rows = {"whole": 17, "gated": 12, "planes": 9}
     # steps of single tokens: norm, rotation, cache write and attention in one kernel
     fuse_decode = True
+    # ``latent_store`` takes ``norm``, ``heads_linear`` takes ``gate`` and ``rotation``
+    launches_together = True
     # tiles of 16 rows per wave in the attention kernel for long portions (1 or 2)
     prefill_row_tiles = 2
     # long portions: keys and values go through LDS, shared by the four waves of a block
@@ -563,13 +565,14 @@ class HipOps:
                                                            c_float(eps), _ptr(out), _CODE[y.dtype], c_int(t), _stream()))
         return out
 
-    def latent_store(self, y, first, rank, rot_dim, weight, eps, positions, freq, cache, neighbours=False, magnitude=1.0):
+    def latent_store(self, y, first, rank, rot_dim, weight, eps, positions, freq, cache, neighbours=False, magnitude=1.0, norm=None):
         """Columns ``first .. first + rank`` of ``y`` RMS-normed (the latent ``c``) and the ``rot_dim``
         columns behind them rotated (rotate-half over the first ``2 len(freq)``; ``neighbours``: element
         2i against 2i + 1; cosines and sines times ``magnitude``) go into the cache of
-        one key/value head: the key row ``[c | k_rot]``, the value row ``[c | 0]``."""
+        one key/value head: the key row ``[c | k_rot]``, the value row ``[c | 0]``. ``norm`` (first, width, weight): in the
+        same launch ``rmsnorm_columns`` of those, with the same ``eps``; its result is returned."""
         if cache is None:
-            return
+            return None if norm is None else self.rmsnorm_columns(y, *norm, eps)
         t, w = y.shape
         width = rank + rot_dim
         _need(y, "y")
@@ -582,10 +585,18 @@ class HipOps:
         _need(cache.group.slots, "slots", torch.int32, (t,))
         if not 0 <= first <= first + width <= w or 2 * pairs > rot_dim:
             raise OpsError(f"latent_store: columns {first}..{first + width} of {w}, {pairs} pairs in {rot_dim}")
+        normed, (q_first, q_width, q_weight) = None, norm or (0, 0, None)
+        if norm is not None:
+            _need(q_weight, "norm weight", torch.float32, (q_width,))
+            if not 0 <= q_first <= q_first + q_width <= w:
+                raise OpsError(f"columns {q_first}..{q_first + q_width} of {w}")
+            normed = torch.empty((t, q_width), dtype=y.dtype, device=y.device)
         self._check(self.lib, self.lib.qrt_latent_store(
             _ptr(y), c_long(w), c_int(first), c_int(rank), c_int(rot_dim), _ptr(weight), c_float(eps), _ptr(positions),
             _ptr(freq), c_int(pairs), _ptr(cache.group.slots), _ptr(cache.k), _ptr(cache.v), c_int(cache.group.page_size),
-            c_long(pages), _CODE[y.dtype], c_int(t), c_int(bool(neighbours)), c_float(magnitude), _stream()))
+            c_long(pages), _CODE[y.dtype], c_int(t), c_int(bool(neighbours)), c_float(magnitude), c_int(q_first), c_int(q_width),
+            _ptr(q_weight), _ptr(normed), _stream()))
+        return normed
 
     def rotate_half(self, x, in_stride, in_offset, out, out_stride, out_offset, heads, width, positions, freq,
                     scale_from_head=None, scale=1.0, neighbours=False, magnitude=1.0):
@@ -594,6 +605,14 @@ class HipOps:
         against element i + len(freq), by ``position * freq[i]``); heads from ``scale_from_head`` on are
         multiplied by ``scale``. ``neighbours``: element 2i turns against element 2i + 1 instead; cosines and
         sines are multiplied by ``magnitude``. ``out`` may be float32 for a bfloat16 ``x``."""
+        a = self._rotation(x, in_stride, in_offset, out, out_stride, out_offset, heads, width, positions, freq, scale_from_head, scale,
+                           neighbours, magnitude)
+        self._check(self.lib, self.lib.qrt_rotate_half(byref(a), _CODE[x.dtype], _CODE[out.dtype], c_int(x.shape[0]), _stream()))
+        return out
+
+    @staticmethod
+    def _rotation(x, in_stride, in_offset, out, out_stride, out_offset, heads, width, positions, freq, scale_from_head=None, scale=1.0,
+                  neighbours=False, magnitude=1.0):
         t = x.shape[0]
         _need(x, "x")
         _need(out, "out", shape=(t, out.shape[1]))
@@ -607,8 +626,7 @@ class HipOps:
             a.positions = _need(positions, "positions", torch.int32, (t,)).data_ptr()
         a.scale_from_head, a.scale = heads if scale_from_head is None else scale_from_head, scale
         a.neighbours, a.magnitude = int(bool(neighbours)), magnitude
-        self._check(self.lib, self.lib.qrt_rotate_half(byref(a), _CODE[x.dtype], _CODE[out.dtype], c_int(t), _stream()))
-        return out
+        return a
 
     # bfloat16 steps with more tokens than this whose rows are no whole pieces of 16 bytes take the per-head products
     # to the vendor library; rows that are take the tile kernel at any number of tokens, which is faster than both
@@ -618,9 +636,11 @@ class HipOps:
     # batched product makes of their strides
     heads_linear_own_max_rows = 16
 
-    def heads_linear(self, x, in_stride, in_offset, w, out, out_stride, out_offset):
+    def heads_linear(self, x, in_stride, in_offset, w, out, out_stride, out_offset, gate=None, rotation=None):
         """A product per head on strided rows: ``out[t, h * out_stride + out_offset + n] =
-        sum_k w[h, n, k] x[t, h * in_stride + in_offset + k]``; ``w`` [heads, N, K]."""
+        sum_k w[h, n, k] x[t, h * in_stride + in_offset + k]``; ``w`` [heads, N, K]. ``gate``: then
+        ``sigmoid_gate(out, gate)``, in the same kernel where it goes by tiles. ``rotation`` (the arguments of ``rotate_half`` by name, without
+        ``x`` and ``out``): ``rotate_half`` from ``x`` into other elements of ``out``, in the same launch where both go by pieces of 16 bytes."""
         t = x.shape[0]
         heads, n, k = w.shape
         _need(x, "x")
@@ -633,6 +653,19 @@ class HipOps:
                  and (x.shape[1] | in_stride | in_offset) % 8 == 0
                  and (out.shape[1] | out_stride | out_offset) % 4 == 0
                  and (x.data_ptr() | w.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0)
+        if gate is not None and not (tiles and gate.dtype == out.dtype and tuple(gate.shape) == tuple(out.shape) and gate.stride(1) == 1
+                                     and heads * out_stride == out.shape[1] and n == out_stride and gate.stride(0) % 4 == 0
+                                     and gate.stride(0) >= out.shape[1] and gate.data_ptr() % 8 == 0):
+            return self.sigmoid_gate(self.heads_linear(x, in_stride, in_offset, w, out, out_stride, out_offset), gate)
+        turn = None
+        if rotation is not None:
+            a = self._rotation(x, out=out, **rotation)
+            if (tiles and not a.neighbours and a.pairs <= 512
+                    and (a.pairs | a.width | a.in_stride | a.in_offset | a.out_stride | a.out_offset | a.x_row | a.out_row) % 8 == 0
+                    and out.data_ptr() % 16 == 0):
+                turn = a
+            else:
+                self.rotate_half(x, out=out, **rotation)
         if not tiles and x.dtype == torch.bfloat16 and t > self.heads_linear_own_max_rows:
             src = x.view(t, -1)[:, : heads * in_stride].view(t, heads, in_stride)[:, :, in_offset: in_offset + k]
             res = torch.bmm(src.transpose(0, 1).contiguous(), w.transpose(1, 2).contiguous())  # [heads, T, N]
@@ -641,7 +674,9 @@ class HipOps:
             return out
         self._check(self.lib, self.lib.qrt_heads_linear(
             _ptr(x), c_long(x.shape[1]), c_int(in_stride), c_int(in_offset), _ptr(w), c_int(heads), c_int(n), c_int(k),
-            _ptr(out), c_long(out.shape[1]), c_int(out_stride), c_int(out_offset), _CODE[x.dtype], c_int(t), c_int(tiles), _stream()))
+            _ptr(out), c_long(out.shape[1]), c_int(out_stride), c_int(out_offset), _CODE[x.dtype], c_int(t), c_int(tiles),
+            None if gate is None else c_void_p(gate.data_ptr()), c_long(0 if gate is None else gate.stride(0)),
+            None if turn is None else byref(turn), _stream()))
         return out
 
     def retention_prepare(self, y, heads, dim, vdim, positions, freq, k_scale):
@@ -653,15 +688,14 @@ class HipOps:
         if c > w:
             raise OpsError(f"retention_prepare: {c} channels in {w} columns")
         out = torch.empty((t, c), dtype=torch.float32, device=y.device)
-        self.rotate_half(y, dim, 0, out, dim, 0, 2 * heads, dim, positions, freq, scale_from_head=heads, scale=k_scale)
+        a = self._rotation(y, dim, 0, out, dim, 0, 2 * heads, dim, positions, freq, scale_from_head=heads, scale=k_scale)
         # the values: a copy into float32 behind them
-        a = _RotateArgs()
-        _need(y, "y")
-        a.x, a.x_row, a.in_stride, a.in_offset = y.data_ptr() + 2 * heads * dim * y.element_size(), w, vdim, 0
-        a.out, a.out_row, a.out_stride, a.out_offset = out.data_ptr() + 2 * heads * dim * 4, c, vdim, 0
-        a.heads, a.width, a.pairs, a.scale_from_head, a.scale = heads, vdim, 0, heads, 1.0
-        a.magnitude = 1.0
-        self._check(self.lib, self.lib.qrt_rotate_half(byref(a), _CODE[y.dtype], F32, c_int(t), _stream()))
+        b = _RotateArgs()
+        b.x, b.x_row, b.in_stride, b.in_offset = y.data_ptr() + 2 * heads * dim * y.element_size(), w, vdim, 0
+        b.out, b.out_row, b.out_stride, b.out_offset = out.data_ptr() + 2 * heads * dim * 4, c, vdim, 0
+        b.heads, b.width, b.pairs, b.scale_from_head, b.scale = heads, vdim, 0, heads, 1.0
+        b.magnitude = 1.0
+        self._check(self.lib, self.lib.qrt_rotate_half_two(byref(a), byref(b), _CODE[y.dtype], F32, c_int(t), _stream()))
         return out
 
     def retention_rule(self, ctx, qkv, decay, state, heads, dim, vdim):

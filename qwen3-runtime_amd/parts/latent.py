@@ -154,24 +154,39 @@ class LatentAttention(Mixer):
         n, w, dr = self.heads, self.latent_width, self.dim + self.rot_dim
         turn = {"neighbours": True, "magnitude": self.magnitude} if self.neighbours or self.magnitude != 1.0 else {}
         y = ops.linear(x, self.down)
-        if self.q_rank is None:
-            q, at = y, self.query_width  # the queries are the product's first columns
-        else:
-            q, at = ops.linear(ops.rmsnorm_columns(y, 0, self.q_rank, self.dq_norm, self.eps), self.uq), self.q_rank
+        q, at = y, self.query_width  # the queries are the product's first columns, or their latent is
+        if self.q_rank is not None:
+            at = self.q_rank
+        norm = None if self.q_rank is None else (0, self.q_rank, self.dq_norm)
+        one_launch = getattr(ops, "launches_together", False)
         if self.own_latent:
             # norm of the latent, rotation of the shared key part, and the cache write, in one pass
-            ops.latent_store(y, at, self.kv_rank, self.rot_dim, self.dkv_norm, self.eps, ctx.positions, self.freq,
-                             cache if cache.writes else None, **turn)
+            if norm is not None and one_launch:
+                turn["norm"] = norm
+            q_latent = ops.latent_store(y, at, self.kv_rank, self.rot_dim, self.dkv_norm, self.eps, ctx.positions, self.freq,
+                                        cache if cache.writes else None, **turn)
+            turn.pop("norm", None)
             at += w
         elif cache.writes:
             raise ValueError("a layer without a latent of its own reads a cache that another layer writes")
+        if norm is not None:
+            q = ops.linear(q_latent if self.own_latent and one_launch else ops.rmsnorm_columns(y, *norm, self.eps), self.uq)
         # queries as the cached rows see them: [W_uk^T q_plain | rotated part] per head
         ql = ops.new_rows(ctx.num_tokens, n * w, q.dtype, x.device)
-        ops.heads_linear(q, dr, 0, self.uk_t, ql, w, 0)
-        ops.rotate_half(q, dr, self.dim, ql, w, self.kv_rank, n, self.rot_dim, ctx.positions, self.freq, **turn)
+        rotation = dict(in_stride=dr, in_offset=self.dim, out_stride=w, out_offset=self.kv_rank, heads=n, width=self.rot_dim,
+                        positions=ctx.positions, freq=self.freq, **turn)
+        if one_launch:
+            ops.heads_linear(q, dr, 0, self.uk_t, ql, w, 0, rotation=rotation)
+        else:
+            ops.heads_linear(q, dr, 0, self.uk_t, ql, w, 0)
+            ops.rotate_half(q, out=ql, **rotation)
         attn = ops.paged_attention(ql, cache, ctx, n, 1, w, self.scale, self.window)
         out = ops.new_rows(ctx.num_tokens, n * self.vdim, q.dtype, x.device)
-        ops.heads_linear(attn, w, 0, self.uv, out, self.vdim, 0)
-        if self.output_gate:
-            ops.sigmoid_gate(out, y[:, at: at + n * self.vdim])
+        gate = y[:, at: at + n * self.vdim] if self.output_gate else None
+        if gate is not None and one_launch:
+            ops.heads_linear(attn, w, 0, self.uv, out, self.vdim, 0, gate=gate)
+        else:
+            ops.heads_linear(attn, w, 0, self.uv, out, self.vdim, 0)
+            if gate is not None:
+                ops.sigmoid_gate(out, gate)
         return ops.linear_for_residual(out, self.o)
