@@ -489,12 +489,14 @@ __device__ bf16x8_t qrt_zero_tile[64];
 // SCALED (up to 16 rows): as in the few-row product. The parts of the factors come to LDS in front of everything else, SQUARE_ROW bytes
 // a row (rows begin in different banks), and are added up when the products are done.
 constexpr int SQUARE_ROW = 4 * SQUARE_PARTS + 16;
+constexpr int MIXED_WAVES = 5;
 template <int MB, int KW, int NWV, int NT, int KC, int GATED, bool SCALED, typename TO>
 __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const bf16_t* __restrict__ A,
                                                                             const bf16_t* __restrict__ W,
                                                                             TO* __restrict__ C, int M, int N, int K, GatedEpilogue ep,
                                                                             RowNorm norm) {
-  constexpr int WT = GATED ? 2 * NT : NT;  // weight tiles per wave
+  constexpr bool MIXED = GATED && NT == 1 && NWV == MIXED_WAVES;  // a wave's tile: eight gate rows and their up rows
+  constexpr int WT = GATED && !MIXED ? 2 * NT : NT;  // weight tiles per wave
   constexpr int PAIRS = KC / 2;            // pairs of k-steps per chunk
   constexpr int ACT = KC * MB / NWV;       // loads of activations a wave issues per chunk
   constexpr int WLOADS = 2 * WT;           // loads of weights per pair
@@ -507,7 +509,7 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
   const int kg = wave / NWV, nw = wave % NWV;
   const int r16 = lane & 15, quad = lane >> 4;
   const int sub = lane >> 3, piece = (lane & 7) ^ sub;
-  const int ntiles = N >> 4;
+  const int ntiles = MIXED ? N >> 3 : N >> 4;
   const int tile_lo = (int)(blockIdx.x * (unsigned)ntiles / gridDim.x);  // N <= 2^20: no overflow
   const int tile_hi = (int)((blockIdx.x + 1) * (unsigned)ntiles / gridDim.x);
   const int tile0 = tile_lo + nw * NT;
@@ -536,9 +538,9 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
     wpair[t] = mine ? 64 : 0;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const size_t row = (size_t)16 * (tile0 + t) + 8 * j + sub;
+      const size_t row = MIXED ? (size_t)j * N + 8 * (tile0 + t) + sub : (size_t)16 * (tile0 + t) + 8 * j + sub;
       wsrc[t][j] = mine ? W + row * K + 8 * piece : (const bf16_t*)qrt_zero_tile + 8 * lane;
-      if (GATED) wsrc[NT + t][j] = mine ? W + ((size_t)N + row) * K + 8 * piece : (const bf16_t*)qrt_zero_tile + 8 * lane;
+      if (GATED && !MIXED) wsrc[NT + t][j] = mine ? W + ((size_t)N + row) * K + 8 * piece : (const bf16_t*)qrt_zero_tile + 8 * lane;
     }
   }
   // activations: load u = nw + NWV j of a chunk is (pair u / (2 MB), row block (u / 2) % MB, half u % 2)
@@ -684,21 +686,24 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     if (tile0 + t >= tile_hi) continue;
-    const int n = 16 * (tile0 + t) + 4 * quad;
+    const int n = (MIXED ? 8 : 16) * (tile0 + t) + 4 * quad;
 #pragma unroll
     for (int b = 0; b < MB; ++b) {
       const int m = 16 * b + r16;
-      if (m >= M) continue;
+      f32x4_t up;  // of the same outputs: a tile of up rows, or the tile's other half, 32 lanes on
+#pragma unroll
+      for (int r = 0; r < 4; ++r) up[r] = MIXED ? __shfl_xor(acc[t][b][r], 32, 64) : GATED ? acc[WT - NT + t][b][r] : 0.f;
+      if (m >= M || (MIXED && quad >= 2)) continue;
       float o[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (SCALED) {
           acc[t][b][r] *= factor;
-          if (GATED) acc[NT + t][b][r] *= factor;
+          up[r] *= factor;
         }
         if (GATED) {  // gate and up value rounded to bfloat16 first, as the unfused kernels see them
           const float g = (float)(bf16_t)acc[t][b][r];
-          o[r] = ep.template apply<GATED>(g, (float)(bf16_t)acc[NT + t][b][r], m);
+          o[r] = ep.template apply<GATED>(g, (float)(bf16_t)up[r], m);
         } else {
           o[r] = ep.whole(acc[t][b][r]);
         }
@@ -711,8 +716,9 @@ __global__ __launch_bounds__(64 * KW * NWV) void gemm_bf16_mid_rows_kernel(const
 template <int MB, int KW, int NWV, int NT, int KC, int GATED, bool SCALED = false>
 static int launch_mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep,
                            hipStream_t stream, int k_parts, const RowNorm& norm = RowNorm{}) {
-  constexpr int WT = GATED ? 2 * NT : NT;
-  const int per_block = NWV * NT, tiles = N / 16;
+  constexpr bool MIXED = GATED && NT == 1 && NWV == MIXED_WAVES;
+  constexpr int WT = GATED && !MIXED ? 2 * NT : NT;
+  const int per_block = NWV * NT, tiles = MIXED ? N / 8 : N / 16;
   constexpr int COMPUTE_UNITS = 256;  // of an MI355X
   int blocks = tiles <= COMPUTE_UNITS / k_parts ? tiles
                                                 : max(COMPUTE_UNITS / k_parts, (tiles + per_block - 1) / per_block);
@@ -755,9 +761,22 @@ static int launch_mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dt
 // or three with chunks of four where K is a multiple of 2,048; up to 64 rows only: beyond, every
 // block would have to fetch more activations than weights, and the vendor library is faster.
 // Very many tiles (the vocabulary head): eight tiles on the staged activations.
+// Gated, up to 64 rows: five waves with tiles of eight gate and eight up rows where that leaves the busiest compute unit less than tiles of either
+// do, counted in such tiles, and no more than the five. us, three waves with a gate and an up tile each and five of eight and eight at 12, 24, 48 and
+// 64 rows: 9,728 x 2,560 (6 against 5) 19.2, 20.5, 22.5, 23.8 and 18.4, 19.7, 21.5, 23.0; 6,144 x 2,048 (4, 3) 13.0, 14.4, 16.1, 17.1 and 12.1, 13.1,
+// 14.5, 15.9; 4,864 x 2,560 (4, 3) 15.5, 17.2, 19.5, 20.6 and 13.6, 14.8, 16.4, 17.9; 2,048 x 2,560 (2, 1) 14.0, 15.8, 17.9, 19.1 and 13.3, 14.4, 16.2,
+// 17.8; level counts lose, 3,072 x 1,024 (2, 2) 7.8, 8.8, 9.7, 10.4 and 8.0, 8.9, 9.8, 10.9, and six, 12,288 x 4,096 (6, 6) 32.4, 33.0, 34.2, 35.5 and 40.3,
+// 44.9, 48.8, 53.5.
+static bool mixed_mid_rows(int N) {
+  const int mixed = (N / 8 + 255) / 256;
+  return mixed <= MIXED_WAVES && mixed < 2 * ((N / 16 + 255) / 256);
+}
 template <int MB>
 static int mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep, int gated,
                     hipStream_t st, int k_parts) {
+  if constexpr (MB <= 4)
+    if (gated && mixed_mid_rows(N)) return gated == 1 ? launch_mid_rows<MB, 1, MIXED_WAVES, 1, 10, 1>(a, w, c, out_dtype, M, N, K, ep, st, 1)
+                                                      : launch_mid_rows<MB, 1, MIXED_WAVES, 1, 10, 2>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (gated == 1) return launch_mid_rows<MB, 1, 3, 1, 6, 1>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (gated) return launch_mid_rows<MB, 1, 3, 1, 6, 2>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (k_parts > 1) {
@@ -876,6 +895,9 @@ extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M
   if (shared) {
     QRT_CHECK(gated >= 0 && N % 16 == 0 && N <= (1 << 20) && K >= 128, "scaled_gemm_bf16: the LDS-sharing kernel is for gated products, "
               "N %% 16 == 0, N <= 2^20, K >= 128 (N=%d K=%d)", N, K);
+    if (mixed_mid_rows(N))
+      return gated == QRT_ACT_SWIGLU ? launch_mid_rows<1, 1, MIXED_WAVES, 1, 10, 1, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm)
+                                     : launch_mid_rows<1, 1, MIXED_WAVES, 1, 10, 2, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm);
     return gated == QRT_ACT_SWIGLU ? launch_mid_rows<1, 1, 3, 1, 6, 1, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm)
                                    : launch_mid_rows<1, 1, 3, 1, 6, 2, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm);
   }
