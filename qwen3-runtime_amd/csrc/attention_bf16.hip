@@ -1700,22 +1700,11 @@ constexpr bool DECODE_ONCE = true;  // measured: 2 % off a decode step at batch 
 // token's own head. A decode pass of the 4B size, us a step, by what was on the chain: the token's loads behind the keys', weights and angles behind
 // its elements, its value's eight elements one by one under a condition, the first pages behind the length 2,021 (1 request of 2,049 keys)
 // and 2,492 (8); all asked for at one time 1,941 and 2,390.
-// What a wave needs for its first keys comes as arguments of its own, which fill the registers that come with a wave: a structure
-// is loaded by every wave, 0.2 to 0.5 us before anything else. `heads`: 256 key heads + query heads a key head. PLAIN: one token per
-// sequence, equal parts of whole contexts, normed and wholly turned heads, no cap, gate, sink or turned values.
-template <bool P2, bool FUSED = false, bool PLAIN = false>
-__global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_decode_kernel(
-    const int* kv_lens, const int* block_table, const bf16_t* k_cache, const bf16_t* v_cache, const bf16_t* qkv, int table_width, int num_splits,
-    int page_size, int heads, AttnTileArgs args) {
-  static_assert(!PLAIN || (FUSED && DECODE_RING), "the plain form takes keys by the ring");
-  AttnTileArgs a = args;  // the fields known here stand for the structure's
-  a.kv_lens = kv_lens, a.block_table = block_table, a.k_cache = k_cache, a.v_cache = v_cache, a.qkv = qkv;
-  a.table_width = table_width, a.num_splits = num_splits, a.page_size = page_size, a.nkv = heads >> 8, a.nq = a.nkv * (heads & 255);
-  if (PLAIN) {
-    a.items = nullptr, a.tile_seq = nullptr, a.gate = nullptr, a.turn = nullptr;
-    a.window = a.chunk = a.keep_first = a.sink = 0;
-    a.cap_in = a.cap_out = 0.f;
-  }
+enum { DECODE_PARTS = 0, DECODE_PLAIN = 1, DECODE_LIST = 2 };
+// One block's part: keys of one sequence, key head and split (a piece from the list: with the length of the longest).
+template <bool P2, bool FUSED, int FORM>
+__device__ __forceinline__ void decode_part(const AttnTileArgs& a, int heads, int seq, int kvh, int split, int longest_piece) {
+  constexpr bool PLAIN = FORM == DECODE_PLAIN, LIST = FORM == DECODE_LIST;
   // per wave: maximum and sum per row, unnormalised accumulator [16][DV]
   extern __shared__ float lds[];
   float* lds_m = lds;                 // [DW][16]
@@ -1725,21 +1714,6 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
 
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
   const int r16 = lane & 15, quad = lane >> 4;
-  // every sequence is one tile here, so without a list the block's number is the sequence's: one
-  // dependent load less before the first key arrives. A list names the sequences of a launch
-  // that covers only some of the step's.
-  int seq, kvh, split, longest_piece = 0;
-  if (a.items) {  // pieces from the work list: (key head, item)
-    longest_piece = a.items[2 * a.max_items];
-    seq = a.items[2 * blockIdx.y];
-    if (seq < 0) return;  // past the end of the list
-    split = a.items[2 * blockIdx.y + 1];
-    kvh = blockIdx.x;
-  } else {
-    seq = a.tile_seq ? a.tile_seq[blockIdx.x] : blockIdx.x;
-    kvh = blockIdx.y;
-    split = blockIdx.z;
-  }
   // Equal parts of whole contexts, one token each: the waves of all parts take a sequence's blocks of keys in turn, whatever
   // their number, so that a wave's first pages are asked for beside the context's length and not behind it. The two that add and
   // store the token's own key take none where there are parts enough.
@@ -1781,8 +1755,8 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
   int blk_begin, blk_end;
   decode_key_blocks(kv_len, q_len, a.window, a.chunk, FUSED, blk_begin, blk_end);
   // equal parts of the sequence's blocks: as many as all sequences have, or as pieces of at most a given length make
-  const int per = in_turn ? 0 : a.items ? piece_blocks(blk_end - blk_begin, longest_piece) : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
-  const int last_split = a.items ? max(1, (blk_end - blk_begin + per - 1) / per) - 1 : a.num_splits - 1;
+  const int per = in_turn ? 0 : LIST ? piece_blocks(blk_end - blk_begin, longest_piece) : (blk_end - blk_begin + a.num_splits - 1) / a.num_splits;
+  const int last_split = LIST ? max(1, (blk_end - blk_begin + per - 1) / per) - 1 : a.num_splits - 1;
   const int b0 = in_turn ? split * DW : blk_begin + split * per;
   const int b1 = in_turn ? blk_end : min(blk_end, b0 + per);
   const int step = in_turn ? turns : DW;
@@ -2005,13 +1979,46 @@ __global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_d
     }
   }
   // the pieces this sequence does not have count as empty splits (their parts are never read)
-  if (a.items && split == 0) {
+  if (LIST && split == 0) {
     const int missing = a.num_splits - 1 - last_split;
     for (int idx = threadIdx.x; idx < n_rows * missing; idx += 64 * DW) {
       const int row = idx % n_rows, s = last_split + 1 + idx / n_rows;
       const int rt = row / g, rh = row - rt * g;
       a.part_lse[(tile_row0 + (size_t)rt * a.nq + kvh * g + rh) * a.num_splits + s] = -INFINITY;
     }
+  }
+}
+
+// What a wave needs for its first keys comes as arguments of its own, which fill the registers that come with a wave: a structure
+// is loaded by every wave, 0.2 to 0.5 us before anything else. `heads`: 256 key heads + query heads a key head. PLAIN: one token per
+// sequence, equal parts of whole contexts, normed and wholly turned heads, no cap, gate, sink or turned values; `second` is then the
+// values' cache, else the list of pieces (null: none).
+template <bool P2, bool FUSED, int FORM>
+__global__ __launch_bounds__(64 * DW, DMAX <= 128 ? 2 : 1) void attention_bf16_decode_kernel(
+    const int* __restrict__ kv_lens, const int* __restrict__ block_table, const bf16_t* k_cache, const void* second, const bf16_t* __restrict__ qkv,
+    int table_width, int num_splits, int page_size, int heads, AttnTileArgs args) {
+  constexpr bool PLAIN = FORM == DECODE_PLAIN;
+  static_assert(!PLAIN || (FUSED && DECODE_RING), "the plain form takes keys by the ring");
+  AttnTileArgs a = args;  // the fields known here stand for the structure's
+  a.kv_lens = kv_lens, a.block_table = block_table, a.k_cache = k_cache, a.qkv = qkv;
+  a.table_width = table_width, a.num_splits = num_splits, a.page_size = page_size, a.nkv = heads >> 8, a.nq = a.nkv * (heads & 255);
+  if constexpr (PLAIN) {
+    a.v_cache = (const bf16_t*)second;
+    a.items = nullptr, a.gate = nullptr, a.turn = nullptr;
+    a.window = a.chunk = a.keep_first = a.sink = 0;
+    a.cap_in = a.cap_out = 0.f;
+    decode_part<P2, FUSED, FORM>(a, heads, blockIdx.x, blockIdx.y, blockIdx.z, 0);
+  } else if constexpr (FORM == DECODE_LIST) {  // (key head, item)
+    const int2 item = ((const int2* __restrict__)second)[blockIdx.y];
+    asm volatile("" ::"s"(item.x), "s"(item.y));  // both in one load
+    if (item.x < 0) return;  // past the end of the list
+    decode_part<P2, FUSED, FORM>(a, heads, item.x, blockIdx.x, item.y, ((const int* __restrict__)second)[2 * a.max_items]);
+  } else {
+    // every sequence is one tile here, so without a list the block's number is the sequence's: one
+    // dependent load less before the first key arrives. A list of tiles names the sequences of a launch
+    // that covers only some of the step's.
+    a.items = nullptr;
+    decode_part<P2, FUSED, FORM>(a, heads, a.tile_seq ? a.tile_seq[blockIdx.x] : blockIdx.x, blockIdx.y, blockIdx.z, 0);
   }
 }
 
@@ -2030,18 +2037,18 @@ extern "C" int qrt_attention_work_list(const AttnTileArgs* args, int fused, hipS
   return 0;
 }
 
-template <bool P2, bool FUSED, bool PLAIN>
+template <bool P2, bool FUSED, int FORM>
 static int launch_decode(const AttnTileArgs& a, dim3 grid, hipStream_t stream) {
   constexpr size_t smem = (size_t)(2 * DW * 16) * sizeof(float) + (DECODE_RING ? (size_t)DW * RING_WAVE : (size_t)DW * 16 * OROW * sizeof(float));
   static_assert(!DECODE_RING || RING_WAVE >= 16 * OROW * (int)sizeof(float), "a wave's accumulator passes through the room of its ring");
-  auto kernel = attention_bf16_decode_kernel<P2, FUSED, PLAIN>;
+  auto kernel = attention_bf16_decode_kernel<P2, FUSED, FORM>;
   static bool allowed = false;  // once per kernel: not again inside every stream capture
   if (smem > 64 * 1024 && !allowed) {  // rings of heads of 128, accumulators of 256: a little more LDS than a block gets without asking
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
       return qrt_fail("attention (decode): cannot get %zu bytes of LDS", smem);
     allowed = true;
   }
-  kernel<<<grid, 64 * DW, smem, stream>>>(a.kv_lens, a.block_table, a.k_cache, a.v_cache, a.qkv, a.table_width, a.num_splits, a.page_size,
+  kernel<<<grid, 64 * DW, smem, stream>>>(a.kv_lens, a.block_table, a.k_cache, FORM == DECODE_PLAIN ? (const void*)a.v_cache : (const void*)a.items, a.qkv, a.table_width, a.num_splits, a.page_size,
                                           a.nkv << 8 | a.nq / a.nkv, a);
   QRT_LAUNCH_CHECK("attention_bf16_decode");
   return 0;
@@ -2093,19 +2100,20 @@ extern "C" int qrt_attention_bf16_decode(const AttnTileArgs* args, int num_rows_
                 a.nq / a.nkv, a.qkv_stride);
       QRT_CHECK(!a.rope || (a.rope_pairs >= 32 && a.rope_pairs % 32 == 0 && a.rope_pairs <= D / 2),
                 "attention (decode, own token from the product): %d pairs turn (multiples of 32 up to %d)", a.rope_pairs, D / 2);
-      if constexpr (DECODE_RING) {
-        const bool plain = !a.items && !a.tile_seq && a.window == 0 && a.chunk == 0 && a.cap_in == 0.f && !a.gate && !a.turn && !a.sink && a.q_weight &&
-                           a.k_weight && a.rope && 2 * a.rope_pairs == D;
-        if (plain) {
-          if (const int rc = p2 ? launch_decode<true, true, true>(a, grid, stream) : launch_decode<false, true, true>(a, grid, stream)) return rc;
-          return finish_decode(a, num_rows_total, stream);
-        }
-      }
-      if (const int rc = p2 ? launch_decode<true, true, false>(a, grid, stream) : launch_decode<false, true, false>(a, grid, stream)) return rc;
+      int rc = 0;
+      if (a.items) rc = p2 ? launch_decode<true, true, DECODE_LIST>(a, grid, stream) : launch_decode<false, true, DECODE_LIST>(a, grid, stream);
+      else if (DECODE_RING && !a.tile_seq && a.window == 0 && a.chunk == 0 && a.cap_in == 0.f && !a.gate && !a.turn && !a.sink && a.q_weight &&
+               a.k_weight && a.rope && 2 * a.rope_pairs == D) {
+        if constexpr (DECODE_RING)
+          rc = p2 ? launch_decode<true, true, DECODE_PLAIN>(a, grid, stream) : launch_decode<false, true, DECODE_PLAIN>(a, grid, stream);
+      } else rc = p2 ? launch_decode<true, true, DECODE_PARTS>(a, grid, stream) : launch_decode<false, true, DECODE_PARTS>(a, grid, stream);
+      if (rc) return rc;
     } else {
       return qrt_fail("attention (decode, own token from the product): head size %d is no multiple of 64", D);
     }
-  } else if (const int rc = p2 ? launch_decode<true, false, false>(a, grid, stream) : launch_decode<false, false, false>(a, grid, stream)) return rc;
+  } else if (a.items) {
+    if (const int rc = p2 ? launch_decode<true, false, DECODE_LIST>(a, grid, stream) : launch_decode<false, false, DECODE_LIST>(a, grid, stream)) return rc;
+  } else if (const int rc = p2 ? launch_decode<true, false, DECODE_PARTS>(a, grid, stream) : launch_decode<false, false, DECODE_PARTS>(a, grid, stream)) return rc;
   return finish_decode(a, num_rows_total, stream);
 }
 
