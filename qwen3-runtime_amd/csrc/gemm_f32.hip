@@ -346,6 +346,135 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
   }
 }
 
+// The same tiles, parts and sums (the same bits) where rows are whole stages of 32 k and offsets fit 32 bits: operands come to LDS by direct loads,
+// S stages of 32 k in a ring, piece c (16 bytes) of row r at 128 r + 16 (c ^ (r & 7)), so that operand reads meet no bank twice. What bounded
+// the kernel above beside its matrix instructions were the others, which do not overlap with them on a SIMD: addresses, a row's end and the way
+// through registers were 1.9 vector instructions an MFMA; here a load costs its wave two scalar ones. Blocks of one stretch of
+// weight rows follow one another on an XCD, whose L2 then has it for all of them.
+#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_buffer(const void* p, unsigned bytes) {
+  constexpr int RAW = 0x00020000;  // a buffer of bytes
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, RAW);
+}
+#endif
+template <int TM_, int TN_, int S, int FORM>
+__global__ __launch_bounds__(256) void gemm_f32_ring_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M,
+                                                            int N, int K, int part_len, int group, int tiles, int row_tiles) {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr bool PLANES = FORM == F32_PLANES, GROUPS_SUM = FORM == F32_GROUPS_SUM;
+  constexpr int BI = TM_ / 32, BJ = TN_ / 32;  // 16 x 16 blocks a wave, and its loads of 8 rows of A and of W a stage
+  constexpr int LOADS = BI + BJ, STAGE = (TM_ + TN_) * 128;
+  static_assert((S - 1) * LOADS < 64, "the loads' counter holds 63");
+  extern __shared__ __align__(16) unsigned char ring[];
+  const int per_xcd = (tiles + 7) >> 3, tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= tiles) return;
+  const int lane = threadIdx.x & 63, wave = uniform_wave_number();
+  const int r = lane & 15, q = lane >> 4;
+  const int m0 = tile % row_tiles * TM_, n0 = tile / row_tiles * TN_;
+  const int wm = (wave >> 1) * (TM_ / 2), wn = (wave & 1) * (TN_ / 2);
+  const unsigned piece = 16 * ((lane & 7) ^ (lane >> 3));
+  const __amdgpu_buffer_rsrc_t a_buf = f32_buffer(A, (unsigned)M * (unsigned)K * 4u), w_buf = f32_buffer(W, (unsigned)N * (unsigned)K * 4u);
+  unsigned aoff[BI], woff[BJ];  // rows past the end repeat the last; not stored
+#pragma unroll
+  for (int i = 0; i < BI; ++i) aoff[i] = (unsigned)min(m0 + 8 * (wave + 4 * i) + (lane >> 3), M - 1) * (unsigned)K * 4u + piece;
+#pragma unroll
+  for (int j = 0; j < BJ; ++j) woff[j] = (unsigned)min(n0 + 8 * (wave + 4 * j) + (lane >> 3), N - 1) * (unsigned)K * 4u + piece;
+  const int per_part = part_len / 32, all = K / 32;
+  const int s_first = PLANES ? blockIdx.z * group * per_part : 0, s_end = PLANES ? min(all, s_first + group * per_part) : all;
+  const int stages = max(0, s_end - s_first);
+  auto fetch = [&](int s, int slot) {
+    unsigned char* dst = ring + slot * STAGE + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buf, (lds_ptr_t)(dst + i * 4096), 16, aoff[i], (s_first + s) * 128, 0, 0);
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf, (lds_ptr_t)(dst + TM_ * 128 + j * 4096), 16, woff[j], (s_first + s) * 128, 0, 0);
+  };
+  f32x4_t acc[BI][BJ], total[BI][BJ], of_groups[GROUPS_SUM ? BI : 1][GROUPS_SUM ? BJ : 1];
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) acc[i][j] = total[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int left = per_part, parts_left = group, slot = 0;
+  bool first = true, first_group = true;
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < stages) fetch(s, s);
+  const unsigned char* a_at = ring + (wm + r) * 128;
+  const unsigned char* w_at = ring + (TM_ + wn + r) * 128;
+  const int read_at[2] = {16 * (q ^ (r & 7)), 16 * ((4 + q) ^ (r & 7))};
+  for (int s = 0; s < stages; ++s) {
+    // stage s has landed when at most the S - 2 behind it are on their way; behind the barrier it has for every wave, and
+    // every wave has the stage before in registers, whose slot takes the S - 1st from here
+    if (s + S - 1 <= stages) QRT_WAIT_LOADS((S - 2) * LOADS);
+    else QRT_WAIT_LOADS(0);
+    QRT_WAIT_LDS();
+    QRT_BARRIER();
+    const int free_slot = slot == 0 ? S - 1 : slot - 1;
+    if (s + S - 1 < stages) fetch(s + S - 1, free_slot);
+    const int base = slot * STAGE;
+    f32x4_t av[2][BI], wv[2][BJ];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < BI; ++i) av[h][i] = *(const f32x4_t*)(a_at + base + i * 2048 + read_at[h]);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) wv[h][j] = *(const f32x4_t*)(w_at + base + j * 2048 + read_at[h]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < BI; ++i)
+#pragma unroll
+          for (int j = 0; j < BJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[h][j][c], av[h][i][c], acc[i][j], 0, 0, 0);
+    if (--left == 0 || s + 1 == stages) {  // a part of K ends
+#pragma unroll
+      for (int i = 0; i < BI; ++i)
+#pragma unroll
+        for (int j = 0; j < BJ; ++j) {
+          total[i][j] = first ? acc[i][j] : total[i][j] + acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      first = false;
+      left = per_part;
+      if (GROUPS_SUM && (--parts_left == 0 || s + 1 == stages)) {
+#pragma unroll
+        for (int i = 0; i < BI; ++i)
+#pragma unroll
+          for (int j = 0; j < BJ; ++j) {
+            f32x4_t& sum = of_groups[GROUPS_SUM ? i : 0][GROUPS_SUM ? j : 0];
+            sum = first_group ? total[i][j] : sum + total[i][j];
+          }
+        first = true;
+        first_group = false;
+        parts_left = group;
+      }
+    }
+    slot = slot + 1 == S ? 0 : slot + 1;
+  }
+  if (PLANES) C += (size_t)blockIdx.z * M * N;
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    const int m = m0 + wm + 16 * i + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) {
+      const int n = n0 + wn + 16 * j + 4 * q;
+      float* c = C + (size_t)m * N + n;
+      const f32x4_t v = GROUPS_SUM ? of_groups[GROUPS_SUM ? i : 0][GROUPS_SUM ? j : 0] : total[i][j];
+      if (N % 4 == 0 && n < N) *(f32x4_t*)c = v;
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) c[e] = v[e];
+    }
+  }
+#endif
+}
+
 // A block's waves: all parts of K, or those of one group (gridDim.y of them, each a plane of the result).
 template <int MB, int PARTS, int U, bool FEW, int GATED>
 static int f32_rows(const float* a, const float* w, float* c, int M, int N, int K, float limit, hipStream_t stream, bool by_groups, int groups = 1) {
@@ -395,21 +524,50 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // round, but a round is four times as long. By 64 x 64 and 128 x 128, us: 2,560 x 4,096 at 8,192 rows 1,506 and 1,434, 2,560 x 9,728 3,557 and
 // 3,385, 6,144 x 2,560 at 4,096 1,141 and 1,103, 5,120 x 8,192 3,002 and 2,863; 19,456 x 2,560 at 2,048 (9.5 rounds) 1,799 and 1,831, at
 // 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854. From 65 to 128 rows they read the weights once: 151,936 x 1,024 at 96 rows 428 and 394.
+//
+// Where the ring takes the product (f32_ring) a round costs less and its start more; 64 x 64 run four to a unit (two slots), and a lone fifth takes
+// as long as a lone first. us, through registers and by the ring, 64 x 64, 64 x 32 and 32 x 32 each, weights of eight layers in turn:
+//   19,456 x 2,560 at 128 rows 146 131 144 and 133 118 117, at 354 378 378 391 and 331 318 316, at 512 476 480 510 and 416 402 412,
+//     at 2,048 1,788 1,884 2,008 and 1,542 1,684 1,691 (132, 121, 121 TFLOP/s);
+//   6,144 x 2,560 at 128 61 60 49 and 66 51 42, at 354 146 130 139 and 131 118 105, at 512 147 160 165 and 131 133 136, at 2,048 571 604 639 and
+//     496 533 541;
+//   2,560 x 9,728 in planes at 128 98 78 70 and 88 66 60, at 354 186 192 193 and 160 162 159, at 512 230 239 256 and 209 202 208, at 2,048
+//     889 937 1,003 and 768 842 857.
+// 128 x 128 tiles do not pay beside them (19,456 x 2,560 at 2,048 rows 1,918 by a ring, 1,809 through registers). Slots of a ring: two for
+// 64 x 64 (four blocks a compute unit in place of three: 1,542 and 1,597), three otherwise (in sums of groups 64 x 64 has more in registers
+// anyway: 2,560 x 9,728 at 2,048 828 by two, 793 by three); four are slower everywhere (1,673).
+static bool f32_ring(int M, int N, int K) { return K % 32 == 0 && (long)M * K < 1 << 29 && (long)N * K < 1 << 29; }
 static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
   return std::max(rounds * 100, (long)least) * round;
 }
-static long f32_cost_64x64(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 64, 64, 606, 130); }
-static long f32_cost_64x32(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 64, 32, 329, 180); }
-static long f32_cost_32x32(int M, int N, int groups) { return f32_tile_cost(M, N, groups, 32, 32, 190, 250); }
-static long f32_cost_128x128(int M, int N) {
-  return (long)((M + 127) / 128) * ((N + 127) / 128) < 1024 ? LONG_MAX : f32_tile_cost(M, N, 1, 128, 128, 2324, 0);
+static long f32_cost_64x64(int M, int N, int groups, bool ring) {
+  if (!ring) return f32_tile_cost(M, N, groups, 64, 64, 606, 130);
+  const long rounds = ((long)((M + 63) / 64) * ((N + 63) / 64) * groups + 255) / 256;
+  return (rounds * 100 + (rounds % 4 == 1 ? 60 : 0)) * 507;
+}
+static long f32_cost_64x32(int M, int N, int groups, bool ring) { return f32_tile_cost(M, N, groups, 64, 32, ring ? 278 : 329, ring ? 225 : 180); }
+static long f32_cost_32x32(int M, int N, int groups, bool ring) { return f32_tile_cost(M, N, groups, 32, 32, ring ? 140 : 190, ring ? 370 : 250); }
+static long f32_cost_128x128(int M, int N, bool ring) {
+  return ring || (long)((M + 127) / 128) * ((N + 127) / 128) < 1024 ? LONG_MAX : f32_tile_cost(M, N, 1, 128, 128, 2324, 0);
 }
 template <int TM_, int TN_, int FORM>
-static void f32_tile_launch(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
+static int f32_tile_launch(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
   const int parts = f32_parts(K);
+  if constexpr (TM_ < 128)
+    if (f32_ring(M, N, K)) {
+      constexpr int S = TM_ == 64 && TN_ == 64 && FORM != F32_GROUPS_SUM ? 2 : 3;
+      constexpr size_t smem = (size_t)S * (TM_ + TN_) * 128;
+      static_assert(smem <= 64 * 1024, "what a block gets without asking");
+      const long tiles = (long)((N + TN_ - 1) / TN_) * ((M + TM_ - 1) / TM_);
+      QRT_CHECK(tiles < 1l << 28, "gemm_f32: %ld tiles", tiles);  // a result of 2^38 elements
+      gemm_f32_ring_kernel<TM_, TN_, S, FORM><<<dim3((unsigned)((tiles + 7) / 8 * 8), 1, FORM == F32_PLANES ? F32_GROUPS : 1), 256, smem, stream>>>(
+          a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS, (int)tiles, (M + TM_ - 1) / TM_);
+      return 0;
+    }
   gemm_f32_tile_kernel<TM_, TN_, FORM><<<dim3((N + TN_ - 1) / TN_, (M + TM_ - 1) / TM_, FORM == F32_PLANES ? F32_GROUPS : 1), 256, 0, stream>>>(
       a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS);
+  return 0;
 }
 template <int FORM>
 static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
@@ -421,17 +579,14 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
     if (const int rc = f32_tiles<FORM>(a, w, c, MOST, N, K, stream)) return rc;
     a += (size_t)MOST * K, c += (size_t)MOST * N, M -= MOST;
   }
-  const long c64 = f32_cost_64x64(M, N, groups), c32 = f32_cost_64x32(M, N, groups), c16 = f32_cost_32x32(M, N, groups);
+  const bool ring = f32_ring(M, N, K);
+  const long c64 = f32_cost_64x64(M, N, groups, ring), c32 = f32_cost_64x32(M, N, groups, ring), c16 = f32_cost_32x32(M, N, groups, ring);
   if constexpr (FORM != F32_PLANES)
-    if (f32_cost_128x128(M, N) < (M > 64 && M <= 128 ? LONG_MAX : c64)) {
-      f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
-      return 0;
-    }
-  if constexpr (FORM == F32_GROUPS_SUM) f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
-  else if (c64 <= c32 && c64 <= c16) f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
-  else if (c32 <= c16 || (M + 31) / 32 > 65535) f32_tile_launch<64, 32, FORM>(a, w, c, M, N, K, stream);
-  else f32_tile_launch<32, 32, FORM>(a, w, c, M, N, K, stream);
-  return 0;
+    if (f32_cost_128x128(M, N, ring) < (M > 64 && M <= 128 ? LONG_MAX : c64)) return f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
+  if constexpr (FORM == F32_GROUPS_SUM) return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
+  else if (c64 <= c32 && c64 <= c16) return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
+  else if (c32 <= c16 || (!ring && (M + 31) / 32 > 65535)) return f32_tile_launch<64, 32, FORM>(a, w, c, M, N, K, stream);
+  else return f32_tile_launch<32, 32, FORM>(a, w, c, M, N, K, stream);
 }
 
 extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
@@ -464,9 +619,10 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
 extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
   if (M <= 32) return N < 4096 ? F32_GROUPS : 1;
   if (N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
-  const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS), f32_cost_64x32(M, N, F32_GROUPS), f32_cost_32x32(M, N, F32_GROUPS)}) / F32_GROUPS;
+  const bool ring = f32_ring(M, N, K);
+  const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS, ring), f32_cost_64x32(M, N, F32_GROUPS, ring), f32_cost_32x32(M, N, F32_GROUPS, ring)}) / F32_GROUPS;
   if (M > 65535 * 64) return 1;  // two calls
-  return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1), f32_cost_128x128(M, N)) ? F32_GROUPS : 1;
+  return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1, ring), f32_cost_128x128(M, N, ring)) ? F32_GROUPS : 1;
 }
 extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, int planes, hipStream_t stream) {
   QRT_CHECK(M >= 0 && N > 0 && K >= 256 && K % 4 == 0, "gemm_f32_planes: bad sizes M=%d N=%d K=%d", M, N, K);
