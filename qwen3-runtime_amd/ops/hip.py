@@ -316,8 +316,7 @@ class HipOps:
     # matrix over and over, the sharing kernel looks 15 to 40 % faster than the few-row kernel
     # down to one row, because a matrix of up to some 100 MB then stays in the memory-side
     # cache; in a step it is 5 % slower at 8 rows, and a decode step with it from one row on
-    # lost 3 % at batch 8 and 9 % at batch 1.) Gated from 12 rows on, and from 9 on where its tiles are of eight
-    # gate and eight up rows (csrc/gemm_bf16.hip, mixed_mid_rows); under 4,096 outputs, which give it few blocks, never up to 16: us at 9 and 16 rows
+    # lost 3 % at batch 8 and 9 % at batch 1.) Gated under 4,096 outputs, which give it few blocks, never up to 16: us at 9 and 16 rows
     # by the few-row kernel and by this one 9,728 x 2,560 19.2, 20.5 and 18.4, 18.5; 6,144 x 2,048 12.6, 13.1 and 12.0, 12.2; 4,864 x 2,560 13.2, 14.2 and
     # 13.3, 13.6; 12,288 x 4,096 32.8, 32.5 and 32.4, 32.4; 3,072 x 1,024 5.0, 5.1 and 8.0, 8.2; 2,048 x 2,560 7.7, 8.3 and 13.0, 13.2.
     shared_from_rows = {"whole": 17, "gated": 12, "planes": 9}
@@ -1524,9 +1523,6 @@ class HipOps:
             least = self.shared_from_rows[form]
             if form == "gated" and n < 4096:
                 least = 17
-            elif form == "gated" and 9 <= m < least:
-                tiles = n // 16
-                least = 9 if -(-2 * tiles // 256) < 2 * -(-tiles // 256) and 2 * tiles <= 5 * 256 else least
             if m >= least:
                 return 1
         if m <= min(16, limit):
