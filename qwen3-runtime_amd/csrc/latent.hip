@@ -398,69 +398,79 @@ __global__ __launch_bounds__(256) void heads_linear_rows_kernel(const T* __restr
 // make it. HL_ROTATE: blocks behind those of the tiles turn and copy another part of the heads, as rotate_half does (`ys` a token).
 // A launch less either way: 8 tokens of 32 heads in a traced step, 384 -> 128 and the gate 11.9 and 8.8 us, 128 -> 384 and the rotation
 // of 64 elements 9.6 and 5.3.
+//
+// Few tokens: tiles of 32 tokens x 64 outputs with eight stages in the ring, while they are no more than one for each of 256 compute units. What
+// bounds the pass then is a stage's latency after the other's, and few blocks: 512 columns of K come at one time here, 32 heads of 128 outputs are 64
+// blocks. Same sums, same bits. us by tiles of 128 tokens and these, from a graph:
+//   32 heads, 384 -> 128 and the gate, at 1, 8, 32, 64 and 128 tokens 8.9, 8.1, 9.8, 13.2, 13.2 and 5.3, 5.0, 5.25, 5.3, 5.4; without it 6.5, 6.6, 6.9, 7.6, 8.3
+//   and 4.2, 4.3, 4.6, 4.7, 4.7; 128 -> 384 beside the rotation at 1, 8 and 32 4.5, 4.6, 5.0 and 3.6, 3.75, 4.0 (at 33, 384 tiles, 5.0 and 5.5);
+//   128 heads, 512 -> 128 at 8 and 33 (512 tiles) 8.8, 9.3 and 6.4, 9.6.
 enum { HL_PLAIN = 0, HL_GATE = 1, HL_ROTATE = 2 };
-template <int BN, int MORE>
-__global__ __launch_bounds__(256, 2) void heads_linear_tile_kernel(const bf16_t* __restrict__ x, long x_row, int in_stride, int in_offset,
+template <int BM, int BN, int S, int MORE>
+__global__ __launch_bounds__(256, BM == 128 ? 2 : 1) void heads_linear_tile_kernel(const bf16_t* __restrict__ x, long x_row, int in_stride, int in_offset,
                                                                    const bf16_t* __restrict__ w, int heads, int n, int k,
                                                                    bf16_t* __restrict__ out, long out_row, int out_stride, int out_offset,
                                                                    int num_tokens, const bf16_t* __restrict__ gate, long gate_row,
                                                                    RotateArgs turn, int tile_blocks, int ys) {
-  extern __shared__ __align__(16) unsigned char lds[];  // [2][128 tokens | BN weight rows] x 128 bytes
+  extern __shared__ __align__(16) unsigned char lds[];  // [S][BM tokens | BN weight rows] x 128 bytes
   if (MORE == HL_ROTATE && (int)blockIdx.x >= tile_blocks) {  // the whole block turns here, before any other barrier
     const int b = blockIdx.x - tile_blocks;
     rotate_token<bf16_t, bf16_t>(turn, b / ys, b % ys, ys, (float*)lds, (float*)lds + ROTATE_MAX_PAIRS);
     return;
   }
-  constexpr int STAGE = (128 + BN) * 128, LOADS = (128 + BN) / 32, WN = BN / 2, JT = BN / 32;
-  const int col_tiles = (n + BN - 1) / BN, row_tiles = (num_tokens + 127) / 128;
+  constexpr int STAGE = (BM + BN) * 128, LOADS = (BM + BN) / 32, WM = BM / 2, WN = BN / 2, IT = BM / 32, JT = BN / 32;
+  static_assert((S & (S - 1)) == 0 && (S - 1) * LOADS < 64, "slots by a mask, the loads' counter");
+  const int col_tiles = (n + BN - 1) / BN, row_tiles = (num_tokens + BM - 1) / BM;
   const int total = heads * col_tiles * row_tiles, per = (total + 7) >> 3;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
   const int h = tile / (col_tiles * row_tiles), rest = tile % (col_tiles * row_tiles);
-  const int t0 = rest / col_tiles * 128, n0 = rest % col_tiles * BN;
+  const int t0 = rest / col_tiles * BM, n0 = rest % col_tiles * BN;
   const int lane = threadIdx.x & 63, wave = uniform_wave_number();
-  const int r16 = lane & 15, quad = lane >> 4, wm = (wave >> 1) * 64, wn = (wave & 1) * WN;
+  const int r16 = lane & 15, quad = lane >> 4, wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
   const int sub = lane >> 3, piece = (lane & 7) ^ sub;
   // a wave's loads of a stage, 8 rows x 128 bytes each; rows past the end repeat the last and are not stored
   const bf16_t* src[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     const int r = (wave * LOADS + i) * 8 + sub;
-    src[i] = r < 128 ? x + (size_t)min(t0 + r, num_tokens - 1) * x_row + (size_t)h * in_stride + in_offset + 8 * piece
-                     : w + ((size_t)h * n + min(n0 + r - 128, n - 1)) * k + 8 * piece;
+    src[i] = r < BM ? x + (size_t)min(t0 + r, num_tokens - 1) * x_row + (size_t)h * in_stride + in_offset + 8 * piece
+                     : w + ((size_t)h * n + min(n0 + r - BM, n - 1)) * k + 8 * piece;
   }
   unsigned char* dst = lds + wave * LOADS * 1024;
   auto fetch = [&](int s) {
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[i] + (size_t)s * 64), (lds_ptr_t)(dst + (s & 1) * STAGE + i * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[i] + (size_t)s * 64), (lds_ptr_t)(dst + (s & (S - 1)) * STAGE + i * 1024), 16, 0, 0);
   };
-  f32x4_t acc[4][JT];
+  f32x4_t acc[IT][JT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int stages = k >> 6;
-  fetch(0);
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+    if (s < stages) fetch(s);
   for (int s = 0; s < stages; ++s) {
-    if (s + 1 < stages) {
-      fetch(s + 1);
-      QRT_WAIT_LOADS(LOADS);
+    if (s + S - 1 < stages) {
+      fetch(s + S - 1);
+      QRT_WAIT_LOADS((S - 1) * LOADS);
     } else {
       QRT_WAIT_LOADS(0);
     }
     QRT_BARRIER();
-    const unsigned char* at = lds + (s & 1) * STAGE;
+    const unsigned char* at = lds + (s & (S - 1)) * STAGE;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int col = 16 * ((4 * e + quad) ^ (r16 & 7));
-      bf16x8_t xv[4], wv[JT];
+      bf16x8_t xv[IT], wv[JT];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) xv[i] = *(const bf16x8_t*)(at + (wm + 16 * i + r16) * 128 + col);
+      for (int i = 0; i < IT; ++i) xv[i] = *(const bf16x8_t*)(at + (wm + 16 * i + r16) * 128 + col);
 #pragma unroll
-      for (int j = 0; j < JT; ++j) wv[j] = *(const bf16x8_t*)(at + (128 + wn + 16 * j + r16) * 128 + col);
+      for (int j = 0; j < JT; ++j) wv[j] = *(const bf16x8_t*)(at + (BM + wn + 16 * j + r16) * 128 + col);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < IT; ++i)
 #pragma unroll
         for (int j = 0; j < JT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j], xv[i], acc[i][j], 0, 0, 0);
     }
@@ -469,7 +479,7 @@ __global__ __launch_bounds__(256, 2) void heads_linear_tile_kernel(const bf16_t*
   }
   // acc[i][j]: token t0 + wm + 16 i + r16, four outputs from n0 + wn + 16 j + 4 quad on
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < IT; ++i) {
     const int t = t0 + wm + 16 * i + r16;
     if (t >= num_tokens) continue;
     bf16_t* o = out + (size_t)t * out_row + (size_t)h * out_stride + out_offset;
@@ -508,19 +518,36 @@ extern "C" int qrt_heads_linear(const void* x, long x_row, int in_stride, int in
     QRT_CHECK(!gate || (gate_row >= (long)heads * out_stride && gate_row % 4 == 0 && (uintptr_t)gate % 8 == 0),
               "heads_linear: gate rows of %ld elements in pieces of 8 bytes", gate_row);
     QRT_CHECK(!turn || rotate_in_pieces(*turn), "heads_linear: the rotation beside it goes by pieces of 16 bytes");
-    const bool narrow = n <= 64;
-    const long blocks = (long)heads * ((n + (narrow ? 63 : 127)) / (narrow ? 64 : 128)) * ((num_tokens + 127) / 128);
+    const bool few = (long)heads * ((n + 63) / 64) * ((num_tokens + 31) / 32) <= 256, narrow = few || n <= 64;
+    const int rows = few ? 32 : 128, columns = narrow ? 64 : 128;
+    const long blocks = (long)heads * ((n + columns - 1) / columns) * ((num_tokens + rows - 1) / rows);
     const int ys = turn ? (num_tokens >= 512 ? 1 : min((turn->heads * turn->width / 8 + 255) / 256, 64)) : 0;
     QRT_CHECK(blocks < (1l << 30) && (long)num_tokens * ys < (1l << 30), "heads_linear: too many tiles");
     const unsigned grid = (unsigned)((blocks + 7) / 8 * 8);
-#define GO(BN, MORE)                                                                                                                 \
-  heads_linear_tile_kernel<BN, MORE><<<grid + (unsigned)(num_tokens * ys), 256, BN == 64 ? 48 * 1024 : 64 * 1024, stream>>>(          \
-      (const bf16_t*)x, x_row, in_stride, in_offset, (const bf16_t*)w, heads, n, k, (bf16_t*)out, out_row, out_stride, out_offset,    \
-      num_tokens, (const bf16_t*)gate, gate_row, turn ? *turn : RotateArgs{}, (int)grid, ys)
-    if (gate) { if (narrow) GO(64, HL_GATE); else GO(128, HL_GATE); }
-    else if (turn) { if (narrow) GO(64, HL_ROTATE); else GO(128, HL_ROTATE); }
-    else if (narrow) GO(64, HL_PLAIN);
-    else GO(128, HL_PLAIN);
+#define GO(BM, BN, S, MORE)                                                                                                          \
+  do {                                                                                                                               \
+    auto kernel = heads_linear_tile_kernel<BM, BN, S, MORE>;                                                                         \
+    constexpr int smem = S * (BM + BN) * 128;                                                                                        \
+    static bool allowed = false; /* once per kernel: not inside a stream capture again and again */                                 \
+    if (smem > 64 * 1024 && !allowed) {                                                                                              \
+      if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess)                  \
+        return qrt_fail("heads_linear: cannot get %d bytes of LDS", smem);                                                           \
+      allowed = true;                                                                                                                \
+    }                                                                                                                                \
+    kernel<<<grid + (unsigned)(num_tokens * ys), 256, smem, stream>>>(                                                               \
+        (const bf16_t*)x, x_row, in_stride, in_offset, (const bf16_t*)w, heads, n, k, (bf16_t*)out, out_row, out_stride, out_offset, \
+        num_tokens, (const bf16_t*)gate, gate_row, turn ? *turn : RotateArgs{}, (int)grid, ys);                                      \
+  } while (0)
+#define BY_SIZE(MORE)                       \
+  do {                                      \
+    if (few) GO(32, 64, 8, MORE);           \
+    else if (narrow) GO(128, 64, 2, MORE);  \
+    else GO(128, 128, 2, MORE);             \
+  } while (0)
+    if (gate) BY_SIZE(HL_GATE);
+    else if (turn) BY_SIZE(HL_ROTATE);
+    else BY_SIZE(HL_PLAIN);
+#undef BY_SIZE
 #undef GO
     QRT_LAUNCH_CHECK("heads_linear_tile");
     return 0;
