@@ -1874,7 +1874,10 @@ __device__ __forceinline__ void decode_part(const AttnTileArgs& a, int heads, in
     } else {
     // two blocks of keys and values are on their way while a third is multiplied, and the page
     // numbers of the two after them; past the wave's last block the loads go on (one shape of
-    // loop, no load under a branch) but fetch next to nothing
+    // loop, no load under a branch) but fetch next to nothing. The token's loads go first and its operands are made
+    // behind the first block's: beside two blocks of heads of 256 they do not fit the registers (404 bytes of scratch a lane,
+    // here 88). us at 1, 8 and 32 requests of up to 2,078 keys, 16 / 4 heads: behind both blocks 15.2, 21.0, 39.9 (heads of 192) and 25.2,
+    // 43.5, 77.8 (256), here 14.1, 19.3, 36.3 and 18.4, 26.9, 53.1; all loads of the token behind the keys 18.5, 24.8, 45.0 and 23.6, 33.3, 62.0
     const int last = last_from(b);
     KvBlock A, B;
     int pgA[3], pgB[3];
@@ -1882,10 +1885,10 @@ __device__ __forceinline__ void decode_part(const AttnTileArgs& a, int heads, in
     block_pages<P2>(table, b << 5, lo, pos_max, a.page_size, r16, quad, pgA);
     block_pages<P2>(table, min(b + DW, last) << 5, lo, pos_max, a.page_size, r16, quad, pgB);
     block_load<P2, DECODE_ONCE>(a, kvh, b << 5, lo, pos_max, r16, quad, pgA, A);
+    if (FUSED) own_token();  // while the first keys and values are on their way
     block_load<P2, DECODE_ONCE>(a, kvh, min(b + DW, last) << 5, lo, pos_max, r16, quad, pgB, B, b + DW <= last);
     block_pages<P2>(table, min(b + 2 * DW, last) << 5, lo, pos_max, a.page_size, r16, quad, pgA);
     block_pages<P2>(table, min(b + 3 * DW, last) << 5, lo, pos_max, a.page_size, r16, quad, pgB);
-    if (FUSED) own_token();  // while the first keys and values are on their way
     while (true) {
       block_compute(A, qreg, qtail, b << 5, lo, pos_min, pos_max, quad, row_valid, qpos_c, window, a.chunk, a.keep_first, a.cap_in, a.cap_out, a.scale_log2, m, l, o);
       block_load<P2, DECODE_ONCE>(a, kvh, min(b + 2 * DW, last) << 5, lo, pos_max, r16, quad, pgA, A, b + 2 * DW <= last);
