@@ -526,30 +526,48 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // 1,024 (4.75) 906 and 917; 96 x 64 at 2,048 1,854. From 65 to 128 rows they read the weights once: 151,936 x 1,024 at 96 rows 428 and 394.
 //
 // Where the ring takes the product (f32_ring) a round costs less and its start more; 64 x 64 run four to a unit (two slots), and a lone fifth takes
-// as long as a lone first. us, through registers and by the ring, 64 x 64, 64 x 32 and 32 x 32 each, weights of eight layers in turn:
-//   19,456 x 2,560 at 128 rows 146 131 144 and 133 118 117, at 354 378 378 391 and 331 318 316, at 512 476 480 510 and 416 402 412,
-//     at 2,048 1,788 1,884 2,008 and 1,542 1,684 1,691 (132, 121, 121 TFLOP/s);
+// longer than a share of four. us, through registers and by the ring, 64 x 64, 64 x 32 and 32 x 32 each, weights of eight layers in turn:
+//   19,456 x 2,560 at 128 rows 146 131 144 and 133 118 117, at 354 378 378 391 and 331 318 316 (on another device 336 329 341), at 512 476 480 510
+//     and 416 402 412 (418 424 461), at 2,048 1,788 1,884 2,008 and 1,542 1,684 1,691 (132, 121, 121 TFLOP/s);
 //   6,144 x 2,560 at 128 61 60 49 and 66 51 42, at 354 146 130 139 and 131 118 105, at 512 147 160 165 and 131 133 136, at 2,048 571 604 639 and
 //     496 533 541;
 //   2,560 x 9,728 in planes at 128 98 78 70 and 88 66 60, at 354 186 192 193 and 160 162 159, at 512 230 239 256 and 209 202 208, at 2,048
 //     889 937 1,003 and 768 842 857.
+// A round of n blocks to a unit takes next to the same whatever the sizes, us for 32 k at 1, 2, 3, 4, 5, 8, 16 and 38 rounds: 64 x 64 0.78, 1.17, 1.67,
+// 2.13, 2.79, 4.2, 8.2, 19.7; 64 x 32 0.47, 0.62, 0.90, 1.15, 1.49, 2.20, 4.45, 10.4; 32 x 32 0.3, 0.38, 0.53, 0.66, 0.79, 1.23, 2.35, 5.7: the costs below. Over 477
+// products, 24 weights of 768 to 19,456 rows at 65 to 2,048 rows, the tile they choose takes 0.4 % longer than the best of the three
+// on average. Most where short K or a last round that is half empty counts: 1,024 x 3,072 in planes at 600 rows 43.0, 32 x 32 38.8;
+// 5,120 x 5,120 at 480 251 and 232; 3,584 x 18,944 in planes at 101 173, 64 x 32 162.
 // 128 x 128 tiles do not pay beside them (19,456 x 2,560 at 2,048 rows 1,918 by a ring, 1,809 through registers). Slots of a ring: two for
 // 64 x 64 (four blocks a compute unit in place of three: 1,542 and 1,597), three otherwise (in sums of groups 64 x 64 has more in registers
 // anyway: 2,560 x 9,728 at 2,048 828 by two, 793 by three); four are slower everywhere (1,673).
 static bool f32_ring(int M, int N, int K) { return K % 32 == 0 && (long)M * K < 1 << 29 && (long)N * K < 1 << 29; }
+static long f32_rounds(int M, int N, int groups, int tm, int tn) { return ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256; }
 static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
-  const long rounds = ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256;
-  return std::max(rounds * 100, (long)least) * round;
+  return std::max(f32_rounds(M, N, groups, tm, tn) * 100, (long)least) * round;
 }
 static long f32_cost_64x64(int M, int N, int groups, bool ring) {
   if (!ring) return f32_tile_cost(M, N, groups, 64, 64, 606, 130);
-  const long rounds = ((long)((M + 63) / 64) * ((N + 63) / 64) * groups + 255) / 256;
-  return (rounds * 100 + (rounds % 4 == 1 ? 60 : 0)) * 507;
+  const long rounds = f32_rounds(M, N, groups, 64, 64);
+  return 100 * (515 * rounds + (rounds % 4 == 1 ? 280 : 150));
 }
-static long f32_cost_64x32(int M, int N, int groups, bool ring) { return f32_tile_cost(M, N, groups, 64, 32, ring ? 278 : 329, ring ? 225 : 180); }
-static long f32_cost_32x32(int M, int N, int groups, bool ring) { return f32_tile_cost(M, N, groups, 32, 32, ring ? 140 : 190, ring ? 370 : 250); }
+static long f32_cost_64x32(int M, int N, int groups, bool ring) {
+  return ring ? 100 * std::max(278 * f32_rounds(M, N, groups, 64, 32) + 55, 480l) : f32_tile_cost(M, N, groups, 64, 32, 329, 180);
+}
+static long f32_cost_32x32(int M, int N, int groups, bool ring) {
+  return ring ? 100 * std::max(147 * f32_rounds(M, N, groups, 32, 32) + 62, 340l) : f32_tile_cost(M, N, groups, 32, 32, 190, 250);
+}
 static long f32_cost_128x128(int M, int N, bool ring) {
   return ring || (long)((M + 127) / 128) * ((N + 127) / 128) < 1024 ? LONG_MAX : f32_tile_cost(M, N, 1, 128, 128, 2324, 0);
+}
+enum { F32_128x128, F32_64x64, F32_64x32, F32_32x32 };
+static int f32_tile_of(int M, int N, int K, int form) {
+  const int groups = form == F32_PLANES ? F32_GROUPS : 1;
+  const bool ring = f32_ring(M, N, K);
+  const long c64 = f32_cost_64x64(M, N, groups, ring), c32 = f32_cost_64x32(M, N, groups, ring), c16 = f32_cost_32x32(M, N, groups, ring);
+  if (form != F32_PLANES && f32_cost_128x128(M, N, ring) < (M > 64 && M <= 128 ? LONG_MAX : c64)) return F32_128x128;
+  if (form == F32_GROUPS_SUM || (c64 <= c32 && c64 <= c16)) return F32_64x64;
+  return c32 <= c16 || (!ring && (M + 31) / 32 > 65535) ? F32_64x32 : F32_32x32;
 }
 template <int TM_, int TN_, int FORM>
 static int f32_tile_launch(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
@@ -571,7 +589,6 @@ static int f32_tile_launch(const float* a, const float* w, float* c, int M, int 
 }
 template <int FORM>
 static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
-  const int groups = FORM == F32_PLANES ? F32_GROUPS : 1;
   // a grid holds 65,535 rows of tiles: a result of more rows than that many of 64 is made in two calls (planes are of fewer)
   constexpr int MOST = 65535 * 64;
   QRT_CHECK(M <= (FORM == F32_PLANES ? MOST : 2 * MOST), "gemm_f32: M=%d is too large", M);
@@ -579,14 +596,19 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
     if (const int rc = f32_tiles<FORM>(a, w, c, MOST, N, K, stream)) return rc;
     a += (size_t)MOST * K, c += (size_t)MOST * N, M -= MOST;
   }
-  const bool ring = f32_ring(M, N, K);
-  const long c64 = f32_cost_64x64(M, N, groups, ring), c32 = f32_cost_64x32(M, N, groups, ring), c16 = f32_cost_32x32(M, N, groups, ring);
+  const int tile = f32_tile_of(M, N, K, FORM);
   if constexpr (FORM != F32_PLANES)
-    if (f32_cost_128x128(M, N, ring) < (M > 64 && M <= 128 ? LONG_MAX : c64)) return f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
-  if constexpr (FORM == F32_GROUPS_SUM) return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
-  else if (c64 <= c32 && c64 <= c16) return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
-  else if (c32 <= c16 || (!ring && (M + 31) / 32 > 65535)) return f32_tile_launch<64, 32, FORM>(a, w, c, M, N, K, stream);
-  else return f32_tile_launch<32, 32, FORM>(a, w, c, M, N, K, stream);
+    if (tile == F32_128x128) return f32_tile_launch<128, 128, FORM>(a, w, c, M, N, K, stream);
+  if constexpr (FORM != F32_GROUPS_SUM) {
+    if (tile == F32_64x32) return f32_tile_launch<64, 32, FORM>(a, w, c, M, N, K, stream);
+    if (tile == F32_32x32) return f32_tile_launch<32, 32, FORM>(a, w, c, M, N, K, stream);
+  }
+  return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
+}
+// For tests: the tile of a product by tiles, its whole result, its planes or their sum (4, 1 planes; else 0), as rows * 1000 + columns.
+extern "C" int qrt_gemm_f32_tile_of(int M, int N, int K, int planes) {
+  const int sizes[] = {128128, 64064, 64032, 32032};
+  return sizes[f32_tile_of(M, N, K, planes == 0 ? F32_WHOLE : planes == 1 ? F32_GROUPS_SUM : F32_PLANES)];
 }
 
 extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
@@ -612,8 +634,9 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
 // fills the chip where the weight has few rows. Up to 32 rows as a stream (4B output and down projections at 1, 16, 32 rows 9.5, 10.4,
 // 14.7 and 18.1, 22.9, 31.5 us; all parts in a block 9.7, 12.3, 17.2 and 19.9, 28.1, 40.6), beyond by tiles.
 //
-// How many planes. By tiles three more of them are written and read, 150 / K of the product's time, so from a round of 64 x 64 tiles on
-// they have to save more than that in part-filled rounds. As a stream: where 16 weight rows a block leave compute units idle, under
+// How many planes. By tiles three more of them are written and read, 150 / K of the product's time (of the ring's, which is shorter, 300), so from a
+// round of 64 x 64 tiles on they have to save more than that in part-filled rounds (product and norm at 181 sizes of 360 to 2,048 rows by 1,024 to 5,120
+// columns: 0.5 % above the best of both forms and all tiles on average, most at 2,048 x 2,048 and 710 rows, 70.9 and 66.3 us). As a stream: where 16 weight rows a block leave compute units idle, under
 // 4,096 rows (product and norm, us at 1, 8 and 32 rows, whole and by planes: 2,560 x 4,096 14.4, 14.1, 20.7 and 14.0, 13.9, 19.6; 4,096 x 4,096
 // 17.1, 17.5, 22.4 and 17.5, 18.3, 23.9; 8,192 x 4,096 32.0, 32.3, 47.0 and 35.4, 36.2, 55.8; 8,192 x 256 9.0, 9.5, 12.3 and 11.2, 12.3, 16.9).
 extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
@@ -622,7 +645,7 @@ extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
   const bool ring = f32_ring(M, N, K);
   const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS, ring), f32_cost_64x32(M, N, F32_GROUPS, ring), f32_cost_32x32(M, N, F32_GROUPS, ring)}) / F32_GROUPS;
   if (M > 65535 * 64) return 1;  // two calls
-  return cut + cut * 150 / K < std::min(f32_cost_64x64(M, N, 1, ring), f32_cost_128x128(M, N, ring)) ? F32_GROUPS : 1;
+  return cut + cut * (ring ? 300 : 150) / K < std::min(f32_cost_64x64(M, N, 1, ring), f32_cost_128x128(M, N, ring)) ? F32_GROUPS : 1;
 }
 extern "C" int qrt_gemm_f32_planes(const float* a, const float* w, float* c, int M, int N, int K, int planes, hipStream_t stream) {
   QRT_CHECK(M >= 0 && N > 0 && K >= 256 && K % 4 == 0, "gemm_f32_planes: bad sizes M=%d N=%d K=%d", M, N, K);
