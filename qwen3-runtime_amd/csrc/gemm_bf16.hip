@@ -385,13 +385,13 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
                        hipStream_t stream, int k_parts, const RowNorm& norm) {
   constexpr int outputs = GATED ? 8 * NT : 16 * NT;
   dim3 grid((N + outputs - 1) / outputs, k_parts), block(64 * (NW + SCALED));
-  constexpr size_t ring = (size_t)NW * U * ((NT + 1) * 2048 - (FEW ? 1024 : 0)), meet = (size_t)NW * NT * 1024, smem = ring > meet ? ring : meet;
-  static_assert(smem <= 160 * 1024, "the rings of this configuration do not fit LDS");
+  constexpr size_t ring = (size_t)NW * U * ((NT + 1) * 2048 - (FEW ? 1024 : 0)), meet = (size_t)NW * NT * 1024, smem = ring > meet ? ring : meet, factors = SCALED ? 64 : 0;
+  static_assert(smem + factors <= 160 * 1024, "the rings of this configuration do not fit LDS");
 #define GO(TO)                                                                                          \
   do {                                                                                                  \
     auto kernel = gemm_bf16_rows_kernel<NW, NT, U, GATED, FEW, SCALED, TO>;                                \
     static bool allowed = false; /* once per kernel: not inside a stream capture again and again */    \
-    if (smem > 64 * 1024 && !allowed) {                                                                 \
+    if (smem + factors > 64 * 1024 && !allowed) {                                                       \
       if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) \
         return qrt_fail("gemm_bf16: cannot get %zu bytes of LDS", smem);                                \
       allowed = true;                                                                                   \
@@ -440,11 +440,12 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
       if (mixed < either && (mixed <= 5 || K <= 4096 || M <= 2)) return launch_rows<4, 1, 3, GATED, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
     return launch_rows<4, 2, 3, GATED, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
   } else {
-    if (k_parts > 1) {
-      const int one = (tiles * k_parts + 255) / 256, two = 2 * (((tiles + 1) / 2 * k_parts + 255) / 256);
-      if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
-      return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
-    }
+    if constexpr (!SCALED)  // K of scaled rows is a residual's width, and whole
+      if (k_parts > 1) {
+        const int one = (tiles * k_parts + 255) / 256, two = 2 * (((tiles + 1) / 2 * k_parts + 255) / 256);
+        if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW, false>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
+        return launch_rows<4, 1, 2, 0, FEW, false>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
+      }
     if (out_dtype == QRT_BF16 && even_takes(M, N)) return even_product(a, w, (bf16_t*)c, M, N, K, ep, SCALED ? &norm : nullptr, st);
     if (K % 2048 == 0) {
       if (tiles >= 2048) return launch_rows<4, 1, 3, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
@@ -452,7 +453,8 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
     }
     if (tiles >= 2048) return launch_rows<4, 2, 3, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
     if (tiles >= 384 && K <= 4096 && !(tiles <= 512 ? M <= 4 : tiles <= 768)) return launch_rows<4, 2, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
-    if (tiles >= 384 && K > 4096) return launch_rows<4, 1, 4, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
+    if constexpr (!SCALED)
+      if (tiles >= 384 && K > 4096) return launch_rows<4, 1, 4, 0, FEW, false>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
     return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
   }
 }
@@ -883,11 +885,12 @@ extern "C" int qrt_gated_gemm_bf16(const void* a, const void* w, void* c, int ou
 }
 
 // The product, or the gated one, of rows that still lack the factor of their RMS norm: C = act(factor * (A W^T)), bfloat16. `a`
-// [M, K] and `squares` [M, SQUARE_PARTS] as qrt_gemm_residual_bf16 left them, `eps` the norm's; M <= 16, K % 64 == 0.
+// [M, K] and `squares` [M, SQUARE_PARTS] as qrt_gemm_residual_bf16 left them, `eps` the norm's; M <= 16, K % 64 == 0 and, as
+// there, up to 4,096.
 // `shared` chooses the gated product's kernel as in qrt_gemm_bf16. gated: -1 none, else an activation of common.h.
 extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M, int N, int K, int gated, float limit, int shared,
                                     const float* squares, float eps, hipStream_t stream) {
-  QRT_CHECK(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0, "scaled_gemm_bf16: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0 && K <= 16 * SQUARE_PARTS, "scaled_gemm_bf16: bad sizes M=%d N=%d K=%d", M, N, K);
   QRT_CHECK(((uintptr_t)a | (uintptr_t)w | (uintptr_t)squares) % 16 == 0, "scaled_gemm_bf16: operands off 16 bytes");
   QRT_CHECK(gated == -1 || gated == QRT_ACT_SWIGLU || gated == QRT_ACT_CLAMPED, "scaled_gemm_bf16: unknown activation %d", gated);
   if (M == 0) return 0;
