@@ -642,7 +642,10 @@ class HipOps:
         """A product per head on strided rows: ``out[t, h * out_stride + out_offset + n] =
         sum_k w[h, n, k] x[t, h * in_stride + in_offset + k]``; ``w`` [heads, N, K]. ``gate``: then
         ``sigmoid_gate(out, gate)``, in the same kernel where it goes by tiles. ``rotation`` (the arguments of ``rotate_half`` by name, without
-        ``x`` and ``out``): ``rotate_half`` from ``x`` into other elements of ``out``, in the same launch where both go by pieces of 16 bytes."""
+        ``x`` and ``out``): ``rotate_half`` from ``x`` into other elements of ``out``, in the same launch where both go by pieces of 16 bytes.
+        Not both: the gate is one of all of ``out``."""
+        if gate is not None and rotation is not None:
+            raise OpsError("heads_linear: a gate or a rotation beside the product, not both")
         t = x.shape[0]
         heads, n, k = w.shape
         _need(x, "x")
