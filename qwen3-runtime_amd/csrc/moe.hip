@@ -16,6 +16,7 @@
 // order: it depends on neither the batch nor the other pairs. This form streams an expert's
 // matrices once per pair and suits steps of few tokens (decoding).
 #include "common.h"
+#include <type_traits>
 #include <math.h>
 
 // sum over lanes of x[c] * w[c], c < n: 16-byte loads of w where the row allows them
@@ -204,12 +205,16 @@ __global__ __launch_bounds__(1024) void route_top_kernel(const T* __restrict__ x
 // taken once. 2,041 tokens 33 -> 12 us, 8 tokens
 // 9.8 -> 8.7; with softmax scores in groups 38 -> 15 and 11.7 -> 10.8, and 10.2 -> 8.8 in a traced step of 8 tokens since a lane
 // asks the lanes of its own group alone (before, all of them, with a division each to find their groups); 9.5 -> 7.2 with all of a row's
-// loads at one time, sums in registers and rounds without branches.
+// loads at one time, sums in registers and rounds without branches. One token a block: as many of its pieces at a time as there are, up to AHEAD:
+// 12, and 4 where two blocks share a compute unit (40 registers; with 66 there was room for one: 64 experts of 256 at 512 tokens 28.1 us). Always asking for 12 cost
+// short rows more than it gave: us at 1, 8 and 512 tokens, one piece after the other, always 12, and this, 64 experts of 256 7.0, 7.2, 8.9 and 15.8, 16.1, 28.4 and
+// 6.4, 6.6, 8.2; of 2,560 15.2, 15.6, 25.5 and 15.8, 16.1, 28.4 and 13.8, 14.4, 24.2 (routers of 600 layers in turn 18.2, 19.7, 25.3 and 16.5, 17.1, 28.5 and
+// 14.3, 15.0, 23.6); 16 of 2,560 5.7, 5.9, 8.8 and 5.7, 5.9, 9.7 and 5.2, 5.5, 8.4.
 __device__ __forceinline__ float lane_value(float x, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
-template <typename T, int TB>
-__global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restrict__ x, const float* __restrict__ router,
+template <typename T, int TB, int AHEAD>
+__global__ __launch_bounds__(1024, AHEAD == 4 ? 8 : 4) void route_top_lanes_kernel(const T* __restrict__ x, const float* __restrict__ router,
                                                                const float* __restrict__ bias, int* __restrict__ index,
                                                                float* __restrict__ weight, int num_tokens, int hidden, int experts,
                                                                int top, int sigmoid_scores, int groups, int keep, int group_max,
@@ -244,28 +249,39 @@ __global__ __launch_bounds__(1024) void route_top_lanes_kernel(const T* __restri
       }
     }
   }
+  const int all_pieces = (hidden + 255) >> 8, rounds = AHEAD ? (all_pieces + AHEAD - 1) / AHEAD : 1, a_time = (all_pieces + rounds - 1) / rounds;
   for (int e = wave; e < experts; e += 16) {
     const float* wr = router + (size_t)e * hidden;
     float acc[TB];
 #pragma unroll
     for (int t = 0; t < TB; ++t) acc[t] = 0.f;
-    if (TB == 1) {  // pieces of ROUTE_AHEAD at a time, all asked for before the first is used (beyond the row: its last, not used)
-      constexpr int ROUTE_AHEAD = 12;
-      for (int c0 = lane * 4; c0 < hidden; c0 += 256 * ROUTE_AHEAD) {
-        f32x4_t wv[ROUTE_AHEAD];
-        xvec_t xv[ROUTE_AHEAD];
+    if (TB == 1) {  // pieces of 256 elements, as many at a time as there are, up to AHEAD, all asked for before the first is used
+      auto pieces = [&](auto count, int c0) {
+        constexpr int N = decltype(count)::value;
+        f32x4_t wv[N];
+        xvec_t xv[N];
 #pragma unroll
-        for (int i = 0; i < ROUTE_AHEAD; ++i) {
-          const int c = min(c0 + 256 * i, hidden - 4);
+        for (int i = 0; i < N; ++i) {  // lanes beyond the row: its last elements, not used
+          const int at = c0 + 256 * i + 4 * lane, c = i < N - 1 ? at : min(at, hidden - 4);
           wv[i] = *(const f32x4_t*)(wr + c);
           xv[i] = *(const xvec_t*)(x + (size_t)t0 * hidden + c);
         }
+        float sum = acc[0];
 #pragma unroll
-        for (int i = 0; i < ROUTE_AHEAD; ++i) {
-          float sum = acc[0];
+        for (int i = 0; i < N; ++i) {
+          if (i == N - 1) acc[0] = sum;
 #pragma unroll
           for (int k = 0; k < 4; ++k) sum = fmaf(to_f32<T>(xv[i][k]), wv[i][k], sum);
-          acc[0] = c0 + 256 * i < hidden ? sum : acc[0];  // no branch: loads would move into it
+        }
+        acc[0] = c0 + 256 * (N - 1) + 4 * lane < hidden ? sum : acc[0];  // no branch: loads would move into it
+      };
+      for (int left = all_pieces; left > 0; left -= a_time) {
+        const int c0 = (all_pieces - left) << 8;
+        const int n = min(left, a_time);
+        switch (n) {
+#define GO(N) case N: if constexpr (N <= AHEAD) pieces(std::integral_constant<int, N>{}, c0); break
+          GO(1); GO(2); GO(3); GO(4); GO(5); GO(6); GO(7); GO(8); GO(9); GO(10); GO(11); GO(12);
+#undef GO
         }
       }
     } else {
@@ -372,14 +388,15 @@ static int route_lanes(const T* x, const float* router, const float* bias, int* 
   // a block per token goes in rounds of 256, and eight tokens a block take as long as two to three of those: 16 experts of 2,560
   // 9.0 us at 512 tokens, 11.7 at 513, by eights 10.5; 48 of 1,000 14.8 at 768, 17.7 at 800, by eights 16.7
   if (num_tokens > (hidden >= 2048 ? 512 : 768) && smem <= 128 * 1024) {
-    auto kernel = route_top_lanes_kernel<T, TB>;
+    auto kernel = route_top_lanes_kernel<T, TB, 0>;
     static bool allowed = false;  // once: not again inside every stream capture
     if (!allowed && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess)
       return qrt_fail("route_top: cannot get 128 KB of LDS");
     allowed = true;
     kernel<<<(num_tokens + TB - 1) / TB, 1024, smem, stream>>>(x, router, bias, index, weight, num_tokens, hidden, experts, top, scores, groups, keep, group_max, correction, renormalise, weight_scale, gate);
   } else {
-    route_top_lanes_kernel<T, 1><<<num_tokens, 1024, 0, stream>>>(x, router, bias, index, weight, num_tokens, hidden, experts, top, scores, groups, keep, group_max, correction, renormalise, weight_scale, gate);
+    auto kernel = num_tokens <= 256 ? route_top_lanes_kernel<T, 1, 12> : route_top_lanes_kernel<T, 1, 4>;
+    kernel<<<num_tokens, 1024, 0, stream>>>(x, router, bias, index, weight, num_tokens, hidden, experts, top, scores, groups, keep, group_max, correction, renormalise, weight_scale, gate);
   }
   QRT_LAUNCH_CHECK("route_top");
   return 0;
