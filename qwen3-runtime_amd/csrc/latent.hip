@@ -13,6 +13,7 @@
 //   takes the same two options;
 // * a product per head, out[t, h, :] = W[h] x[t, h, :], on strided rows: W [heads, N, K].
 #include "common.h"
+#include <type_traits>
 #include "direct.h"
 #include <math.h>
 
@@ -42,29 +43,75 @@ struct LatentArgs {
   int neighbours; float magnitude;
 };
 
-// A row's elements stay in registers up to LATENT_KEEP a thread, asked for with their weights in one go (the rest of a wider row is read again).
-constexpr int LATENT_KEEP = 4;
+// A row in pieces of 256 elements, one a thread each. KEEP, the first of up to four, stay in registers, asked for with their weights in one go;
+// the rest of a row over 1,024 is read again, four pieces at a time (`put` stores, and no load would be moved up in front of a store).
+// us at 8 and 2,048 rows by an element at a time, four always in registers and the rest one at a time, and this: rows of 64 2.5, 3.1 and 2.3, 3.3 and 2.3, 3.0;
+// of 1,536 3.7, 5.7 and 3.1, 5.7 and 2.9, 5.3; of 2,560 4.6, 7.3 and 3.9, 8.2 and 3.3, 6.9; of 8,192 9.7, 23.0 and 9.0, 30.0 and 5.7, 18.7.
+template <int N>
+struct RowPieces {  // of which the last may be part of one: its threads beyond the row read the last element and count for nothing
+  float v[N];
+  template <typename T>
+  __device__ __forceinline__ void load(const T* __restrict__ row, int from, int width) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const int i = from + 256 * k + (int)threadIdx.x;
+      v[k] = to_f32<T>(row[k < N - 1 ? i : min(i, width - 1)]);
+    }
+  }
+};
+template <typename T, int KEEP, class Put>
+__device__ __forceinline__ void rms_normed(const T* __restrict__ row, int width, const float* __restrict__ weight, float eps, float* red, Put put) {
+  float ss = 0.f, inv;
+  auto add = [&](auto& x, int from) {
+    constexpr int N = sizeof(x.v) / sizeof(float);
+#pragma unroll
+    for (int k = 0; k < N; ++k) ss += k < N - 1 || from + 256 * k + (int)threadIdx.x < width ? x.v[k] * x.v[k] : 0.f;
+  };
+  auto store = [&](auto& x, auto& w, int from) {
+    constexpr int N = sizeof(x.v) / sizeof(float);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const int i = from + 256 * k + (int)threadIdx.x;
+      if (k < N - 1 || i < width) put(i, from_f32<T>(x.v[k] * inv * w.v[k]));
+    }
+  };
+  auto rest = [&](auto each) {  // four pieces at a time, then the one to four that are left; the same in the whole block
+    int from = 1024;
+    for (; width - from > 1024; from += 1024) each(std::integral_constant<int, 4>{}, from);
+    switch ((width - from + 255) >> 8) {
+      case 1: each(std::integral_constant<int, 1>{}, from); break;
+      case 2: each(std::integral_constant<int, 2>{}, from); break;
+      case 3: each(std::integral_constant<int, 3>{}, from); break;
+      case 4: each(std::integral_constant<int, 4>{}, from); break;
+    }
+  };
+  RowPieces<KEEP> kept, kept_weight;
+  kept.load(row, 0, width);
+  kept_weight.load(weight, 0, width);
+  add(kept, 0);
+  if (KEEP == 4)
+    rest([&](auto count, int from) {
+      RowPieces<decltype(count)::value> x;
+      x.load(row, from, width);
+      add(x, from);
+    });
+  ss = block_sum(ss, red);
+  inv = 1.0f / sqrtf(ss / (float)width + eps);
+  store(kept, kept_weight, 0);
+  if (KEEP == 4)
+    rest([&](auto count, int from) {
+      RowPieces<decltype(count)::value> x, w;
+      x.load(row, from, width);
+      w.load(weight, from, width);
+      store(x, w, from);
+    });
+}
 template <typename T, class Put>
 __device__ __forceinline__ void rms_normed(const T* __restrict__ row, int width, const float* __restrict__ weight, float eps, float* red, Put put) {
-  float v[LATENT_KEEP], w[LATENT_KEEP], ss = 0.f;
-#pragma unroll
-  for (int k = 0; k < LATENT_KEEP; ++k) {
-    const int i = min((int)threadIdx.x + 256 * k, width - 1);
-    v[k] = to_f32<T>(row[i]);
-    w[k] = weight[i];
-  }
-#pragma unroll
-  for (int k = 0; k < LATENT_KEEP; ++k) ss += (int)threadIdx.x + 256 * k < width ? v[k] * v[k] : 0.f;
-  for (int i = threadIdx.x + 256 * LATENT_KEEP; i < width; i += 256) {
-    const float x = to_f32<T>(row[i]);
-    ss += x * x;
-  }
-  ss = block_sum(ss, red);
-  const float inv = 1.0f / sqrtf(ss / (float)width + eps);
-#pragma unroll
-  for (int k = 0; k < LATENT_KEEP; ++k)
-    if ((int)threadIdx.x + 256 * k < width) put(threadIdx.x + 256 * k, from_f32<T>(v[k] * inv * w[k]));
-  for (int i = threadIdx.x + 256 * LATENT_KEEP; i < width; i += 256) put(i, from_f32<T>(to_f32<T>(row[i]) * inv * weight[i]));
+  if (width <= 256) rms_normed<T, 1>(row, width, weight, eps, red, put);  // the same branch in the whole block
+  else if (width <= 512) rms_normed<T, 2>(row, width, weight, eps, red, put);
+  else if (width <= 768) rms_normed<T, 3>(row, width, weight, eps, red, put);
+  else rms_normed<T, 4>(row, width, weight, eps, red, put);
 }
 
 template <typename T>
