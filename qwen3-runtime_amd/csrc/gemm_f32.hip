@@ -541,8 +541,15 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // 128 x 128 tiles do not pay beside them (19,456 x 2,560 at 2,048 rows 1,918 by a ring, 1,809 through registers). Slots of a ring: two for
 // 64 x 64 (four blocks a compute unit in place of three: 1,542 and 1,597), three otherwise (in sums of groups 64 x 64 has more in registers
 // anyway: 2,560 x 9,728 at 2,048 828 by two, 793 by three); four are slower everywhere (1,673).
-static bool f32_ring(int M, int N, int K) { return K % 32 == 0 && (long)M * K < 1 << 29 && (long)N * K < 1 << 29; }
 static long f32_rounds(int M, int N, int groups, int tm, int tn) { return ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256; }
+// A block alone on its unit waits for its stages one after the other, through the ring longer where they come from L2. So weights of up to 4 MB, which may
+// be there from the pass before, go through registers where 32 x 32 tiles are no more than the units: us through registers and by the ring from L2 and from
+// beyond, 1,024 x 1,024 at 65 rows 10.3, 12.4 and 13.2, 12.7; 256 x 512 at 300 6.5, 7.5 and 7.1, 7.2; 16 x 2,048 at 300 18.3, 24.3 and 23.8, 23.8 (K of 96 and less level or
+// better by the ring); 2,048 x 2,048 at 65 18.4, 22.9 and 30.6, 23.8.
+static bool f32_ring(int M, int N, int K, int groups) {
+  if (K % 32 != 0 || (long)M * K >= 1 << 29 || (long)N * K >= 1 << 29) return false;
+  return K < 128 || (long)N * K > 1 << 20 || f32_rounds(M, N, groups, 32, 32) > 1;
+}
 static long f32_tile_cost(int M, int N, int groups, int tm, int tn, int round, int least) {  // in units of 1 / 100 of 1 / 1000 us
   return std::max(f32_rounds(M, N, groups, tm, tn) * 100, (long)least) * round;
 }
@@ -563,7 +570,7 @@ static long f32_cost_128x128(int M, int N, bool ring) {
 enum { F32_128x128, F32_64x64, F32_64x32, F32_32x32 };
 static int f32_tile_of(int M, int N, int K, int form) {
   const int groups = form == F32_PLANES ? F32_GROUPS : 1;
-  const bool ring = f32_ring(M, N, K);
+  const bool ring = f32_ring(M, N, K, groups);
   const long c64 = f32_cost_64x64(M, N, groups, ring), c32 = f32_cost_64x32(M, N, groups, ring), c16 = f32_cost_32x32(M, N, groups, ring);
   if (form != F32_PLANES && f32_cost_128x128(M, N, ring) < (M > 64 && M <= 128 ? LONG_MAX : c64)) return F32_128x128;
   if (form == F32_GROUPS_SUM || (c64 <= c32 && c64 <= c16)) return F32_64x64;
@@ -573,12 +580,12 @@ template <int TM_, int TN_, int FORM>
 static int f32_tile_launch(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
   const int parts = f32_parts(K);
   if constexpr (TM_ < 128)
-    if (f32_ring(M, N, K)) {
+    if (f32_ring(M, N, K, FORM == F32_PLANES ? F32_GROUPS : 1)) {
+      const long tiles = (long)((N + TN_ - 1) / TN_) * ((M + TM_ - 1) / TM_);
+      QRT_CHECK(tiles < 1l << 28, "gemm_f32: %ld tiles", tiles);  // a result of 2^38 elements
       constexpr int S = TM_ == 64 && TN_ == 64 && FORM != F32_GROUPS_SUM ? 2 : 3;
       constexpr size_t smem = (size_t)S * (TM_ + TN_) * 128;
       static_assert(smem <= 64 * 1024, "what a block gets without asking");
-      const long tiles = (long)((N + TN_ - 1) / TN_) * ((M + TM_ - 1) / TM_);
-      QRT_CHECK(tiles < 1l << 28, "gemm_f32: %ld tiles", tiles);  // a result of 2^38 elements
       gemm_f32_ring_kernel<TM_, TN_, S, FORM><<<dim3((unsigned)((tiles + 7) / 8 * 8), 1, FORM == F32_PLANES ? F32_GROUPS : 1), 256, smem, stream>>>(
           a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS, (int)tiles, (M + TM_ - 1) / TM_);
       return 0;
@@ -605,11 +612,13 @@ static int f32_tiles(const float* a, const float* w, float* c, int M, int N, int
   }
   return f32_tile_launch<64, 64, FORM>(a, w, c, M, N, K, stream);
 }
-// For tests: the tile of a product by tiles, its whole result, its planes or their sum (4, 1 planes; else 0), as rows * 1000 + columns.
+// For tests: the tile of a product by tiles, its whole result, its planes or their sum (4, 1 planes; else 0), as rows * 1000 + columns, and
+// whether it goes through the ring.
 extern "C" int qrt_gemm_f32_tile_of(int M, int N, int K, int planes) {
   const int sizes[] = {128128, 64064, 64032, 32032};
   return sizes[f32_tile_of(M, N, K, planes == 0 ? F32_WHOLE : planes == 1 ? F32_GROUPS_SUM : F32_PLANES)];
 }
+extern "C" int qrt_gemm_f32_ring_of(int M, int N, int K, int planes) { return f32_ring(M, N, K, planes == F32_GROUPS ? F32_GROUPS : 1); }
 
 extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int N, int K, hipStream_t stream) {
   QRT_CHECK(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -642,7 +651,7 @@ extern "C" int qrt_gemm_f32(const float* a, const float* w, float* c, int M, int
 extern "C" int qrt_gemm_f32_planes_of(int M, int N, int K) {
   if (M <= 32) return N < 4096 ? F32_GROUPS : 1;
   if (N <= 0 || K <= 0 || (long)((M + 63) / 64) * ((N + 63) / 64) < 256) return F32_GROUPS;
-  const bool ring = f32_ring(M, N, K);
+  const bool ring = f32_ring(M, N, K, 1);
   const long cut = std::min({f32_cost_64x64(M, N, F32_GROUPS, ring), f32_cost_64x32(M, N, F32_GROUPS, ring), f32_cost_32x32(M, N, F32_GROUPS, ring)}) / F32_GROUPS;
   if (M > 65535 * 64) return 1;  // two calls
   return cut + cut * (ring ? 300 : 150) / K < std::min(f32_cost_64x64(M, N, 1, ring), f32_cost_128x128(M, N, ring)) ? F32_GROUPS : 1;

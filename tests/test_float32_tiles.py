@@ -35,3 +35,12 @@ def test_whole_product_by_square_tiles(m, n, k):
     assert ops.lib.qrt_gemm_f32_tile_of(m, n, k, 0) == 64064
     x, w = rnd(m, k, seed=5), rnd(n, k, seed=6, scale=0.05)
     check(ops.linear(x, w), x, w, lambda rows: ops.linear(rows, w))
+
+
+# blocks that are alone on their units, with weights that lie in L2 from the pass before: through registers (us through them and by the ring 10.3 and 12.4,
+# 6.5 and 7.5, 18.3 and 24.3); short K, larger weights, more blocks than units, four planes of them: by the ring
+@pytest.mark.parametrize("m,n,k,planes,ring", [(65, 1024, 1024, 0, 0), (300, 256, 512, 0, 0), (300, 16, 2048, 0, 0), (65, 256, 768, 4, 0),
+                                               (65, 1024, 96, 0, 1), (65, 2048, 2048, 0, 1), (300, 1024, 1024, 0, 1), (300, 256, 768, 4, 1),
+                                               (300, 2048, 2050, 0, 0)])
+def test_what_goes_through_the_ring(m, n, k, planes, ring):
+    assert HipOps().lib.qrt_gemm_f32_ring_of(m, n, k, planes) == ring
