@@ -18,6 +18,7 @@
 // those up itself.
 // Error against float64, relative: 3.3e-7 (K 2,560), 4.5e-7 (9,728); the sequential sums': 9.0e-7 and 1.8e-6.
 #include "common.h"
+#include <type_traits>
 #include "direct.h"
 #include <limits.h>
 #include <algorithm>
@@ -539,8 +540,9 @@ static int f32_few_rows(const float* a, const float* w, float* c, int M, int N, 
 // on average. Most where short K or a last round that is half empty counts: 1,024 x 3,072 in planes at 600 rows 43.0, 32 x 32 38.8;
 // 5,120 x 5,120 at 480 251 and 232; 3,584 x 18,944 in planes at 101 173, 64 x 32 162.
 // 128 x 128 tiles do not pay beside them (19,456 x 2,560 at 2,048 rows 1,918 by a ring, 1,809 through registers). Slots of a ring: two for
-// 64 x 64 (four blocks a compute unit in place of three: 1,542 and 1,597), three otherwise (in sums of groups 64 x 64 has more in registers
-// anyway: 2,560 x 9,728 at 2,048 828 by two, 793 by three); four are slower everywhere (1,673).
+// 64 x 64 (four blocks a compute unit in place of three: 1,542 and 1,597), three otherwise; four are slower everywhere (1,673). In sums of groups two
+// where a unit's blocks make fewer fours than threes, by two and by three: 2,048 x 768 at 2,048 rows (4 rounds) 56.5 and 70.2, 2,560 x
+// 4,096 at 1,300 (4) 265 and 285, 5,120 x 2,048 at 1,300 (7) 238 and 245, 2,560 x 9,728 at 1,300 (4) 623 and 669; else three: at 2,048 (5) 834 and 800, 512 (2) 336 and 329.
 static long f32_rounds(int M, int N, int groups, int tm, int tn) { return ((long)((M + tm - 1) / tm) * ((N + tn - 1) / tn) * groups + 255) / 256; }
 // A block alone on its unit waits for its stages one after the other, through the ring longer where they come from L2. So weights of up to 4 MB, which may
 // be there from the pass before, go through registers where 32 x 32 tiles are no more than the units: us through registers and by the ring from L2 and from
@@ -583,11 +585,18 @@ static int f32_tile_launch(const float* a, const float* w, float* c, int M, int 
     if (f32_ring(M, N, K, FORM == F32_PLANES ? F32_GROUPS : 1)) {
       const long tiles = (long)((N + TN_ - 1) / TN_) * ((M + TM_ - 1) / TM_);
       QRT_CHECK(tiles < 1l << 28, "gemm_f32: %ld tiles", tiles);  // a result of 2^38 elements
-      constexpr int S = TM_ == 64 && TN_ == 64 && FORM != F32_GROUPS_SUM ? 2 : 3;
-      constexpr size_t smem = (size_t)S * (TM_ + TN_) * 128;
-      static_assert(smem <= 64 * 1024, "what a block gets without asking");
-      gemm_f32_ring_kernel<TM_, TN_, S, FORM><<<dim3((unsigned)((tiles + 7) / 8 * 8), 1, FORM == F32_PLANES ? F32_GROUPS : 1), 256, smem, stream>>>(
-          a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS, (int)tiles, (M + TM_ - 1) / TM_);
+      auto go = [&](auto slots) {
+        constexpr int S = decltype(slots)::value;
+        constexpr size_t smem = (size_t)S * (TM_ + TN_) * 128;
+        static_assert(smem <= 64 * 1024, "what a block gets without asking");
+        gemm_f32_ring_kernel<TM_, TN_, S, FORM><<<dim3((unsigned)((tiles + 7) / 8 * 8), 1, FORM == F32_PLANES ? F32_GROUPS : 1), 256, smem, stream>>>(
+            a, w, c, M, N, K, f32_part_len(K, parts), parts / F32_GROUPS, (int)tiles, (M + TM_ - 1) / TM_);
+      };
+      if constexpr (FORM == F32_GROUPS_SUM) {
+        const long rounds = f32_rounds(M, N, 1, TM_, TN_);
+        if ((rounds + 3) / 4 < (rounds + 2) / 3) go(std::integral_constant<int, 2>{});
+        else go(std::integral_constant<int, 3>{});
+      } else go(std::integral_constant<int, TM_ == 64 && TN_ == 64 ? 2 : 3>{});
       return 0;
     }
   gemm_f32_tile_kernel<TM_, TN_, FORM><<<dim3((N + TN_ - 1) / TN_, (M + TM_ - 1) / TM_, FORM == F32_PLANES ? F32_GROUPS : 1), 256, 0, stream>>>(

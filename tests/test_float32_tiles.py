@@ -1,12 +1,14 @@
 """Which tiles float32 products take: the choice beside what the three of them were measured to take, and a product by each."""
 
+from ctypes import c_int
+
 import pytest
 import torch
 
 from test_float32_ring_gpu import check
 from test_kernels_gpu import rnd
 
-from qwen3_runtime_amd.ops.hip import HipOps
+from qwen3_runtime_amd.ops.hip import HipOps, _ptr, _stream
 
 TILES = (64064, 64032, 32032)
 
@@ -44,3 +46,19 @@ def test_whole_product_by_square_tiles(m, n, k):
                                                (300, 2048, 2050, 0, 0)])
 def test_what_goes_through_the_ring(m, n, k, planes, ring):
     assert HipOps().lib.qrt_gemm_f32_ring_of(m, n, k, planes) == ring
+
+
+# sums of groups: four and seven blocks to a unit (two slots in the ring), five and six (three), remainders of either side
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(2041, 1987), (2041, 3267), (2049, 1987), (2049, 2563)])
+@pytest.mark.parametrize("k", [256, 288, 1056, 8224])
+def test_sums_of_groups_by_square_tiles(m, n, k):
+    ops = HipOps(residual_planes=True)
+    x, w = rnd(m, k, seed=7), rnd(n, k, seed=8, scale=0.05)
+
+    def product(rows, planes):
+        out = torch.full((planes, rows.shape[0], n), float("nan"), device=x.device)
+        ops._check(ops.lib, ops.lib.qrt_gemm_f32_planes(_ptr(rows), _ptr(w), _ptr(out), c_int(rows.shape[0]), c_int(n), c_int(k), c_int(planes), _stream()))
+        return out[0] if planes == 1 else ((out[0] + out[1]) + out[2]) + out[3]
+
+    check(product(x, 1), x, w, lambda rows: product(rows, 4))
