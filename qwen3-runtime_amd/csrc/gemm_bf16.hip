@@ -417,10 +417,11 @@ static int launch_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype,
 //   4,864, 3 against 4, 11.7, 12.1 and 12.9, 13.3; 6,656, 4 against 4, 14.7, 15.2 and 14.4, 14.3; 9,728, 5 against 6, 18.6, 18.9 and 20.2, 19.7
 //   (5.4 and 4.9 TB/s); 12,288, 6 against 6, 22.5, 22.9 and 22.7, 21.8. Beyond five long rows of more than two keep a tile of either: 25,600 x
 //   5,120, 13 against 14, 81.2, 84.2 and 83.4, 81.5.
-//   The whole result: in bfloat16 evenly shared rows where the busiest unit would get a tile more than others (gemm_even.hip); otherwise two tiles a block from 384 tiles on where K is up to 4,096 columns, except between 512 and 768 tiles, whose blocks of two fill
-//   the compute units a little more than once (9,728 x 2,560 10.5, 11.5 and 12.0, 12.8; 12,288 11.5, 12.2 and 12.8, 13.5; at 16 rows
-//   13.6 and 14.1), and up to 4 rows below (6,144 x 2,560 at 1, 4 and 8 rows 7.2, 7.45, 8.1 and 7.35, 7.45, 7.7; 13,312 13.6, 14.7
-//   and 12.9, 13.6). One where K is a multiple of 2,048 (the rows of
+//   The whole result: in bfloat16 evenly shared rows where the busiest unit would get a tile more than others (even_takes in gemm_even.h says where).
+//   Otherwise two tiles a block from 384 tiles on where K is up to 4,096 columns, except between 512 and 768 tiles, whose blocks of two fill
+//   the compute units a little more than once, and up to 4 rows below. The times that drew these lines are of bfloat16 at sizes that are mostly shared evenly
+//   now; float32 results of the same sizes go by them: 9,728 x 2,560 10.5, 11.5 and 12.0, 12.8; 12,288 11.5, 12.2 and 12.8, 13.5 (at 16 rows
+//   13.6 and 14.1); 6,144 x 2,560 at 1, 4 and 8 rows 7.2, 7.45, 8.1 and 7.35, 7.45, 7.7; 13,312 13.6, 14.7 and 12.9, 13.6. One where K is a multiple of 2,048 (the rows of
 //   two tiles then start in the same memory channels: 14.0 us against 11.2 for the 8B q/k/v product)
 //   and for a few hundred tiles of long rows.
 //   K cut into planes: two tiles a block from K = 9,728 on, but one where that leaves the busiest compute unit fewer tiles, at most five
@@ -446,7 +447,7 @@ static int few_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, in
         if (K >= 9728 && !(one < two && one <= 5)) return launch_rows<4, 2, 2, 0, FEW, false>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
         return launch_rows<4, 1, 2, 0, FEW, false>(a, w, c, out_dtype, M, N, K, ep, st, k_parts, norm);
       }
-    if (out_dtype == QRT_BF16 && even_takes(M, N)) return even_product(a, w, (bf16_t*)c, M, N, K, ep, SCALED ? &norm : nullptr, st);
+    if (out_dtype == QRT_BF16 && even_takes(M, N, K)) return even_product(a, w, (bf16_t*)c, M, N, K, ep, SCALED ? &norm : nullptr, st);
     if (K % 2048 == 0) {
       if (tiles >= 2048) return launch_rows<4, 1, 3, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);
       return launch_rows<4, 1, 2, 0, FEW, SCALED>(a, w, c, out_dtype, M, N, K, ep, st, 1, norm);

@@ -141,10 +141,13 @@ static int by_rows(const bf16_t* a, const bf16_t* w, bf16_t* c, int M, int N, in
 }
 
 int even_product(const bf16_t* a, const bf16_t* w, bf16_t* c, int M, int N, int K, const GatedEpilogue& ep, const RowNorm* norm, hipStream_t stream) {
-  QRT_CHECK(even_takes(M, N) && M > 0 && M <= 16 && K > 0 && K % 64 == 0, "gemm_even: bad sizes M=%d N=%d K=%d", M, N, K);
+  QRT_CHECK(even_takes(M, N, K) && M > 0 && M <= 16 && K > 0 && K % 64 == 0, "gemm_even: bad sizes M=%d N=%d K=%d", M, N, K);
   switch (even_units(N)) {
     case 3: return by_rows<3, 3>(a, w, c, M, N, K, ep, norm, stream);
     case 5: return by_rows<2, 5>(a, w, c, M, N, K, ep, norm, stream);
     default: return by_rows<2, 6>(a, w, c, M, N, K, ep, norm, stream);
   }
 }
+
+// For tests: whether few rows of a bfloat16 result are shared evenly.
+extern "C" int qrt_gemm_even_takes(int M, int N, int K) { return even_takes(M, N, K); }
