@@ -772,15 +772,22 @@ static int launch_mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dt
 // 14.5, 15.9; 4,864 x 2,560 (4, 3) 15.5, 17.2, 19.5, 20.6 and 13.6, 14.8, 16.4, 17.9; 2,048 x 2,560 (2, 1) 14.0, 15.8, 17.9, 19.1 and 13.3, 14.4, 16.2,
 // 17.8; level counts lose, 3,072 x 1,024 (2, 2) 7.8, 8.8, 9.7, 10.4 and 8.0, 8.9, 9.8, 10.9, and six, 12,288 x 4,096 (6, 6) 32.4, 33.0, 34.2, 35.5 and 40.3,
 // 44.9, 48.8, 53.5.
-static bool mixed_mid_rows(int N) {
+// And where K is long enough: five waves ask for chunks of ten k-steps, three for six, of which more is beyond a short K's end, and the ring's start counts. us, three and
+// five waves at 17, 48 and 64 rows: 9,728 x 128 4.7, 5.2, 5.8 and 5.4, 6.5, 7.3; 9,728 x 2,048 2 to 5 % slower from 12 rows on; 2,048 x 768 9 to 12 %, x 2,304 up to 4 %;
+// 1,536 x 768 2 to 10 %, x 1,536 4 to 9 % faster; 5,120 x 768 up to 8 % slower, x 1,024 level to 7 % faster. (8,448 x 4,096 is 6 to 9 % slower up to 24 rows, the sizes beside it 4 to 7 % faster.)
+static bool mixed_mid_rows(int N, int K) {
   const int mixed = (N / 8 + 255) / 256;
-  return mixed <= MIXED_WAVES && mixed < 2 * ((N / 16 + 255) / 256);
+  const int least_k = mixed == 1 ? (N <= 1536 ? 1536 : 2560) : mixed == 3 ? 1024 : 2560;
+  return mixed <= MIXED_WAVES && mixed < 2 * ((N / 16 + 255) / 256) && K >= least_k;
 }
+// For tests: whether gated products of 12 or 17 to 64 rows go by five waves.
+extern "C" int qrt_gated_gemm_mixed(int N, int K) { return mixed_mid_rows(N, K); }
+
 template <int MB>
 static int mid_rows(const bf16_t* a, const bf16_t* w, void* c, int out_dtype, int M, int N, int K, const GatedEpilogue& ep, int gated,
                     hipStream_t st, int k_parts) {
   if constexpr (MB <= 4)
-    if (gated && mixed_mid_rows(N)) return gated == 1 ? launch_mid_rows<MB, 1, MIXED_WAVES, 1, 10, 1>(a, w, c, out_dtype, M, N, K, ep, st, 1)
+    if (gated && mixed_mid_rows(N, K)) return gated == 1 ? launch_mid_rows<MB, 1, MIXED_WAVES, 1, 10, 1>(a, w, c, out_dtype, M, N, K, ep, st, 1)
                                                       : launch_mid_rows<MB, 1, MIXED_WAVES, 1, 10, 2>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (gated == 1) return launch_mid_rows<MB, 1, 3, 1, 6, 1>(a, w, c, out_dtype, M, N, K, ep, st, 1);
   if (gated) return launch_mid_rows<MB, 1, 3, 1, 6, 2>(a, w, c, out_dtype, M, N, K, ep, st, 1);
@@ -901,7 +908,7 @@ extern "C" int qrt_scaled_gemm_bf16(const void* a, const void* w, void* c, int M
   if (shared) {
     QRT_CHECK(gated >= 0 && N % 16 == 0 && N <= (1 << 20) && K >= 128, "scaled_gemm_bf16: the LDS-sharing kernel is for gated products, "
               "N %% 16 == 0, N <= 2^20, K >= 128 (N=%d K=%d)", N, K);
-    if (mixed_mid_rows(N))
+    if (mixed_mid_rows(N, K))
       return gated == QRT_ACT_SWIGLU ? launch_mid_rows<1, 1, MIXED_WAVES, 1, 10, 1, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm)
                                      : launch_mid_rows<1, 1, MIXED_WAVES, 1, 10, 2, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm);
     return gated == QRT_ACT_SWIGLU ? launch_mid_rows<1, 1, 3, 1, 6, 1, true>(A, W, c, QRT_BF16, M, N, K, ep, stream, 1, norm)

@@ -2,6 +2,8 @@
 
 import pytest
 
+import test_gated_rows_gpu as gated
+
 from qwen3_runtime_amd.ops.hip import HipOps
 
 
@@ -15,3 +17,22 @@ from qwen3_runtime_amd.ops.hip import HipOps
 ])
 def test_rows_that_are_shared_evenly(m, n, k, evenly):
     assert HipOps().lib.qrt_gemm_even_takes(m, n, k) == evenly
+
+
+# gated rows by five waves (csrc/gemm_bf16.hip), us by three and five at 64 rows: 9,728 x 128 5.8, 7.3; 2,048 x 768 11 % apart; 9,728 x 2,048 5 %; 5,120 x 768 2 %
+@pytest.mark.parametrize("n,k,five", [
+    (256, 1536, 1), (1536, 1536, 1), (2048, 2560, 1), (4352, 1024, 1), (6144, 2048, 1), (9728, 2560, 1), (10240, 5120, 1),
+    (256, 1024, 0), (1536, 1472, 0), (1552, 1536, 0), (2048, 2304, 0), (5120, 768, 0), (9728, 128, 0), (9728, 2048, 0), (3072, 4096, 0), (12288, 4096, 0),
+])
+def test_gated_rows_by_five_waves(n, k, five):
+    assert HipOps().lib.qrt_gated_gemm_mixed(n, k) == five
+
+
+# rows: ends of the blocks of 16; outputs: fewer tiles than compute units, one tile to some of three, five to all; K: two k-steps less than a chunk of ten,
+# whole chunks, a chunk and a part
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [9, 16, 17, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(48, 1536), (48, 1600), (1536, 1664), (4112, 1088), (10240, 2560), (10240, 2624)])
+def test_gated_products_by_five_waves(m, n, k):
+    assert HipOps().lib.qrt_gated_gemm_mixed(n, k) == 1
+    gated.test_gated_rows(m, n, k)
