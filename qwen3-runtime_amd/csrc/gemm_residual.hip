@@ -3,7 +3,8 @@
 // residual[M, N] += A[M, K] W[N, K]^T in float32; out[M, N] = residual * weight in bfloat16, the norm's rows but for their factor
 // 1 / rms, which the products that read them multiply their sums by (gemm_bf16.hip, SCALED): a factor of a whole row passes through
 // a product, and a rounding to bfloat16 is as large in relation to its value before it as behind it. What the factor is made of leaves
-// as squares[M, SQUARE_PARTS]: each block's part of the rows' sums of squares, which every consumer adds up in the same order.
+// as squares[M, SQUARE_PARTS]: each block's part of the rows' sums of squares, which every consumer adds up in an order of its own (few-row products
+// as RowNorm::factor has it, the product that shares activations a quad of lanes at a time), whatever the other rows.
 //
 // Until there was this kernel K was cut over blocks, whose planes a kernel of a block a row added up and normed: 3 to 4 us of a
 // boundary and two trips to memory for 40 KB a row. Here K stays whole in a block and the 256 compute units share the weight rows
@@ -13,6 +14,9 @@
 // what was there: results of columns that are not stored). us, the product in planes and the norm against this
 // kernel, weights of 36 layers in turn, from a graph, 1, 8 and 16 rows:
 //   2,560 x 4,096  9.0, 9.4, 10.5 and 6.2, 6.6, 7.6;  2,560 x 9,728  13.5, 14.2, 15.6 and 10.3, 11.3, 13.6.
+// Narrower and wider residuals, with the product that reads the rows behind it, in planes and by this kernel: 256 x 256 (and 768 x 256) 6.6, 6.9, 6.9 and 5.2, 5.6,
+// 6.2; 1,024 x 3,072 (4,096) 9.8, 10.1, 13.1 and 7.8, 8.2, 9.8; 2,048 x 6,144 (4,096) 14.1, 14.6, 16.7 and 11.9, 12.8, 14.5; 4,096 x 14,336 (6,144) 33.5, 34.4, 34.9 and
+// 30.4, 30.9, 34.6; least at 16 rows of 4,096 x 12,288, in front of a gated product of 12,288 outputs 54.4 and 54.7.
 // Four waves of eight pairs 6.7, 7.2 and 10.7, 11.6; sixteen of two 6.3, 6.8 and 10.6, 11.7; tiles of 16 rows on 160 compute units 6.6, 7.4
 // and 11.0, 13.1; of eight rows on 320 7.4, 8.2 and 12.8, 15.6.
 #include "common.h"

@@ -48,7 +48,7 @@ def test_stream_and_rows(ops, m, n, k):
     # one rounding of the rows and one of the result to bfloat16 (2^-9 each), and the sums' own
     allowed = size * (2.0 ** -9 + (n + 64) * 2.0 ** -23) + sums.abs() * 2.0 ** -8
     assert ((got.double() - sums).abs() <= allowed).all()
-    # whole tiles of 16 from 4,096 outputs on go to the kernel that shares the activations, from 12 rows on or, in tiles of eight and eight, from 9
+    # whole tiles of 16 from 4,096 outputs on go to the kernel that shares the activations from 12 rows on, up to 11 rows to the few-row kernel
     for half in (88, 4096, 6160) if (n, k) == (2112, 576) else (88, 96):
         gate_up = rnd(2 * half, n, seed=half, scale=n ** -0.5, dtype=torch.bfloat16)
         _, gu, gu_size = exact(before, x, w, weight, gate_up)
